@@ -155,6 +155,19 @@ int m2_mixer_core_fwd(const void* xproj, const float* proj_bias, const float* u,
 int m2_fftconv_fwd(const void* x, const float* spec, void* y, int B, int L, int d, int act_dtype, void* stream);
 
 /* ---------------------------------------------------------------------------------------------
+ * The two dense projections around the mixer core (in_linear, out_linear of MonarchMixerSequenceMixing,
+ * bert/src/mm/monarch_mixer_sequence_mixer.py:70-71,103,152), bf16 MFMA with fp32 accumulation, between row-major
+ * activations and the channel-major ones the core reads and writes:
+ *   to_channels    out (N, M) = w (N, K) x (M, K)^T
+ *   from_channels  out (M, N) = x (K, M)^T w (N, K)^T + bias (N, fp32 or NULL)
+ * m2_dense_supported: M and N multiples of 8, K a multiple of 64, either operand below 4 GB.
+ * ------------------------------------------------------------------------------------------- */
+int m2_dense_supported(int M, int N, int K);
+int m2_dense_to_channels_fwd(const void* x, const void* w, void* out, int M, int N, int K, void* stream);
+int m2_dense_from_channels_fwd(const void* x, const void* w, const float* bias, void* out, int M, int N, int K,
+                               void* stream);
+
+/* ---------------------------------------------------------------------------------------------
  * Block-diagonal ("Monarch") linear layers of the GLU MLP, bf16 MFMA with fp32 accumulation.
  * Stand in for: bert/src/mm/blockdiag_multiply.py:49-60 (BlockdiagMultiply.forward, bf16 under
  * autocast), bert/src/mm/structured_linear.py:65-69 (bias add) and bert/src/bert_layers.py:482-506

@@ -1,0 +1,261 @@
+// Dense and block-diagonal bf16 matrix products on the tile engine (gemm_engine.h) and, for few rows, on a kernel that
+// splits K over the waves of a workgroup.
+#include "gemm_engine.h"
+
+namespace m2 {
+
+// ---------------------------------------------------------------------------------------------
+// Few rows: a 32 x 32 tile of OUT[j][i] per workgroup, K split over its NW waves, every wave's operands requested at
+// once straight into registers (no LDS stage, no loop: one memory latency), partial sums added through LDS.  GLU: two
+// products (gate block and value block of a gated block-diagonal layer) and gelu(gate) * value on the sums.
+// ---------------------------------------------------------------------------------------------
+constexpr int kRedRow = 36;      // floats between two j of a partial tile
+
+template <int NW, int KSMAX, bool QKM, bool GLU>
+struct SmallShape {
+  static constexpr int kProd = GLU ? 2 : 1;
+  static constexpr int kRed = NW * kProd * 32 * kRedRow * 4;
+  static constexpr int kStage = QKM ? NW * KSMAX * 2048 : 0;
+  static constexpr int kLds = kRed > kStage ? kRed : kStage;
+};
+
+template <int NW, int KSMAX, bool QKM, bool GLU>
+__global__ __launch_bounds__(64 * NW) void small_gemm_kernel(GemmArgs g) {
+  using S = SmallShape<NW, KSMAX, QKM, GLU>;
+  static_assert(!(QKM && GLU), "the gated product reads row-major activations");
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  const int tid = threadIdx.x, lane = tid & 63, i16 = lane & 15, q4 = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int ntiles = g.ti * g.tj;
+  const int xcd = blockIdx.x & 7;
+  const int tile = (int)((long)xcd * ntiles / 8) + (int)(blockIdx.x >> 3);
+  if (tile >= (int)((long)(xcd + 1) * ntiles / 8)) return;
+  int i0, j0, blk;
+  tile_origin<32, 32>(g, tile, i0, j0, blk);
+  const int nks = (g.nk + 31) / 32;
+  const int s0 = wave * nks / NW, ns = (wave + 1) * nks / NW - s0;
+  const u32x4 zero = {0u, 0u, 0u, 0u};
+
+  u32x4 pf[S::kProd][KSMAX][2], qf[S::kProd][KSMAX][2];
+  static_for<0, S::kProd>([&](auto dd) {
+    constexpr int D = decltype(dd)::value;
+    // GLU: gated columns of weight block blk (gate, read against the same block of Q) and of block blk + nblk (value)
+    const int wb = blk + D * g.nblk, qb = GLU ? wb : blk;
+    const uint16_t* pb = g.p + wb * g.pblk + 32 * s0 + 8 * q4;
+    const uint16_t* qbase = g.q + (long)qb * g.nk + 32 * s0 + 8 * q4;
+    static_for<0, 2>([&](auto tt) {
+      constexpr int t = decltype(tt)::value;
+      int i = i0 + 8 * (i16 >> 2) + 4 * t + (i16 & 3);
+      i = i < g.ni ? i : g.ni - 1;
+      int j = j0 + 16 * t + i16;
+      j = j < g.nj ? j : g.nj - 1;
+      static_for<0, KSMAX>([&](auto ss) {
+        constexpr int s = decltype(ss)::value;
+        pf[D][s][t] = zero;
+        if constexpr (!QKM) qf[D][s][t] = zero;
+        if (s < ns && 32 * (s0 + s) + 8 * q4 < g.nk) {
+          pf[D][s][t] = *reinterpret_cast<const u32x4*>(pb + (long)i * g.ldp + 32 * s);
+          if constexpr (!QKM) qf[D][s][t] = *reinterpret_cast<const u32x4*>(qbase + (long)j * g.ldq + 32 * s);
+        }
+      });
+    });
+  });
+  if constexpr (QKM) {
+    // the wave's k rows (64 bytes = 32 j each) through its own LDS rows, read back transposed
+    const unsigned lds0 = (unsigned)(uintptr_t)smem + wave * (KSMAX * 2048);
+    int j = j0 + 8 * (lane & 3);
+    j = j <= g.nj - 8 ? j : g.nj - 8;
+    const unsigned voff = (unsigned)(((long)(lane >> 2) * g.ldq + j) * 2);
+    for (int s = 0; s < 2 * ns; ++s)
+      load_to_lds(lds0 + s * 1024, voff, (const unsigned char*)g.q + (32l * s0 + 16 * s) * g.ldq * 2);
+    __builtin_amdgcn_s_waitcnt(kWaitVm0);
+    asm volatile("" ::: "memory");
+    typedef __attribute__((address_space(3))) s16x4 lds4;
+    const unsigned a0 = lds0 + (8 * q4 + (i16 >> 2)) * 64 + 8 * (i16 & 3);
+    static_for<0, KSMAX>([&](auto ss) {
+      constexpr int s = decltype(ss)::value;
+      static_for<0, 2>([&](auto tt) {
+        constexpr int t = decltype(tt)::value;
+        qf[0][s][t] = zero;
+        if (s < ns) {
+          const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds4*)(uintptr_t)(a0 + s * 2048 + 32 * t));
+          const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds4*)(uintptr_t)(a0 + s * 2048 + 32 * t + 256));
+          qf[0][s][t] = __builtin_bit_cast(u32x4, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+        }
+      });
+    });
+  }
+  floatx4 acc[S::kProd][2][2];
+  static_for<0, S::kProd>([&](auto dd) {
+    constexpr int D = decltype(dd)::value;
+    static_for<0, 4>([&](auto tt) {
+      constexpr int t = decltype(tt)::value >> 1, u = decltype(tt)::value & 1;
+      floatx4 a = {0.f, 0.f, 0.f, 0.f};
+      static_for<0, KSMAX>([&](auto ss) {
+        constexpr int s = decltype(ss)::value;
+        a = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, pf[D][s][t]), __builtin_bit_cast(bf16x8, qf[D][s][u]), a, 0, 0, 0);
+      });
+      acc[D][t][u] = a;
+    });
+  });
+  float* red = reinterpret_cast<float*>(smem);
+  if constexpr (QKM) __syncthreads();      // every wave has read its stage: the partial sums take its place
+  static_for<0, S::kProd>([&](auto dd) {
+    constexpr int D = decltype(dd)::value;
+    static_for<0, 4>([&](auto tt) {
+      constexpr int t = decltype(tt)::value >> 1, u = decltype(tt)::value & 1;
+      *reinterpret_cast<floatx4*>(red + ((wave * S::kProd + D) * 32 + 16 * u + i16) * kRedRow + 8 * q4 + 4 * t) = acc[D][t][u];
+    });
+  });
+  __syncthreads();
+  if (tid >= 256) return;
+  const int j = tid >> 3, i4 = 4 * (tid & 7);
+  floatx4 sum[S::kProd];
+  static_for<0, S::kProd>([&](auto dd) {
+    constexpr int D = decltype(dd)::value;
+    floatx4 v = {0.f, 0.f, 0.f, 0.f};
+    static_for<0, NW>([&](auto ww) {
+      v += *reinterpret_cast<const floatx4*>(red + ((decltype(ww)::value * S::kProd + D) * 32 + j) * kRedRow + i4);
+    });
+    sum[D] = v;
+  });
+  const int i = i0 + i4;
+  if (i >= g.ni || j0 + j >= g.nj) return;
+  const long o = (long)(j0 + j) * g.ldo + blk * g.ni + i;
+  float r[4];
+  if constexpr (GLU) {
+    static_for<0, 4>([&](auto e) { r[decltype(e)::value] = gelu_erf_poly(sum[0][decltype(e)::value]) * sum[1][decltype(e)::value]; });
+  } else {
+    static_for<0, 4>([&](auto e) { r[decltype(e)::value] = sum[0][decltype(e)::value]; });
+    if (g.bias) static_for<0, 4>([&](auto e) { r[decltype(e)::value] += g.bias[blk * g.ni + i + decltype(e)::value]; });
+    if (g.resid) {
+      const u32x2 rr = *reinterpret_cast<const u32x2*>(g.resid + o);
+      r[0] += __uint_as_float(rr.x << 16); r[1] += __uint_as_float(rr.x & 0xffff0000u);
+      r[2] += __uint_as_float(rr.y << 16); r[3] += __uint_as_float(rr.y & 0xffff0000u);
+    }
+  }
+  u32x2 pk = {pack_bf16x2(r[0], r[1]), pack_bf16x2(r[2], r[3])};
+  *reinterpret_cast<u32x2*>(g.out + o) = pk;
+}
+
+template <int NW, int KSMAX, bool QKM, bool GLU>
+static int launch_small(GemmArgs g, hipStream_t st) {
+  using S = SmallShape<NW, KSMAX, QKM, GLU>;
+  auto kern = small_gemm_kernel<NW, KSMAX, QKM, GLU>;
+  g.ti = g.nblk * ((g.ni + 31) / 32);
+  g.tj = (g.nj + 31) / 32;
+  if (S::kLds > 64 * 1024) {
+    hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, S::kLds);
+    if (e != hipSuccess) return set_error(M2_ERR_LAUNCH, "hipFuncSetAttribute(small_gemm): %s", hipGetErrorString(e));
+  }
+  const int nt = g.ti * g.tj;
+  hipLaunchKernelGGL(kern, dim3(8 * ((nt + 7) / 8)), dim3(64 * NW), S::kLds, st, g);
+  return check_launch("small_gemm");
+}
+
+template <int BI, int BJ, int WI, int WJ, int STAGES, bool QKM, int OCC>
+static int launch_engine(GemmArgs g, hipStream_t st) {
+  using S = GemmShape<BI, BJ, WI, WJ, STAGES, QKM>;
+  auto kern = gemm_kernel<BI, BJ, WI, WJ, STAGES, QKM, OCC>;
+  hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, S::kLds);
+  if (e != hipSuccess) return set_error(M2_ERR_LAUNCH, "hipFuncSetAttribute(gemm): %s", hipGetErrorString(e));
+  g.ti = g.nblk * ((g.ni + BI - 1) / BI);
+  g.tj = (g.nj + BJ - 1) / BJ;
+  const int nt = g.ti * g.tj;
+  const int per_xcd = num_cus() / 8 * (160 * 1024 / S::kLds > 2 ? 2 : 160 * 1024 / S::kLds);
+  const int need = (nt + 7) / 8;
+  hipLaunchKernelGGL(kern, dim3(8 * (need < per_xcd ? need : per_xcd)), dim3(S::kThreads), S::kLds, st, g);
+  return check_launch("gemm");
+}
+
+// ---------------------------------------------------------------------------------------------
+// Which kernel for which size.  A tile step (64 of K) of a workgroup takes a time that depends on its tile and on whether
+// the compute unit holds a second workgroup; a launch takes about 2.5 us.  Measured on MI355X (us per step, one / two
+// workgroups per compute unit; K = 768 and 1536, M = 128 .. 32768): the table below.  What bounds a step: the small
+// tiles their loads (a compute unit gets 50 - 65 GB/s out of L2) and the latency of a step, the two large ones the power
+// budget (the clock falls to 1.6 - 1.8 GHz under them).  The model picks the measured best, or one within 10 % of it, at
+// all of 4 widths x 9 row counts.
+// ---------------------------------------------------------------------------------------------
+enum DenseVariant { kVarSmall, kVar64, kVar128, kVarMid, kVarWide, kVar256, kVariants };
+struct VariantShape {
+  int bi, bj, per_cu;       // tile (QKM: i and j exchanged where they differ), workgroups of a compute unit
+  float t1, t2;             // us per step with one and with per_cu workgroups on it
+};
+static const VariantShape kVariantShapes[kVariants] = {
+    {32, 32, 4, 0.f, 0.f},       {64, 128, 2, 0.47f, 0.80f},  {128, 128, 2, 0.64f, 1.12f},
+    {128, 192, 2, 1.05f, 1.68f}, {256, 192, 1, 1.55f, 1.55f}, {256, 256, 1, 1.90f, 1.90f}};
+
+static float variant_cost(int v, const GemmArgs& g, bool swap) {
+  const VariantShape& s = kVariantShapes[v];
+  const int bi = swap ? s.bj : s.bi, bj = swap ? s.bi : s.bj;
+  const long tiles = (long)g.nblk * ((g.ni + bi - 1) / bi) * ((g.nj + bj - 1) / bj);
+  // few rows: the launch, one memory latency, and 64 operand rows per tile at about 13 TB/s
+  if (v == kVarSmall) return g.nk > 2048 ? 1e30f : 4.0f + 128e-6f * (float)tiles * (float)g.nk / 13.f;
+  const long cus = num_cus(), slots = cus * s.per_cu;
+  const long full = tiles / slots, rest = tiles - full * slots;
+  return 2.5f + (float)(g.nk / kGK) * ((float)full * s.t2 + (rest == 0 ? 0.f : rest <= cus ? s.t1 : s.t2));
+}
+// swap: the long side of the tiles along i instead of j
+static int pick_variant(const GemmArgs& g, bool swap) {
+  int best = kVarSmall;
+  float cost = 1e30f;
+  for (int v = 0; v < kVariants; ++v) {
+    if (v != kVarSmall && g.nk % kGK != 0) continue;
+    const float c = variant_cost(v, g, swap);
+    if (c < cost) { cost = c; best = v; }
+  }
+  return best;
+}
+
+template <bool QKM>
+static int dense_launch(int variant, GemmArgs g, hipStream_t st) {
+  switch (variant) {
+    case kVarSmall: {
+      // the tiles of an XCD keep the larger operand's rows together: weights are read by one L2 only
+      g.jfast = QKM;
+      const int ks = ((g.nk + 31) / 32 + 7) / 8;
+      if (ks <= 3) return launch_small<8, 3, QKM, false>(g, st);
+      if (ks <= 4) return launch_small<8, 4, QKM, false>(g, st);
+      if (ks <= 6) return launch_small<8, 6, QKM, false>(g, st);
+      return launch_small<8, 8, QKM, false>(g, st);
+    }
+    case kVar64: return QKM ? launch_engine<128, 64, 2, 2, 3, QKM, 2>(g, st) : launch_engine<64, 128, 2, 2, 3, QKM, 2>(g, st);
+    case kVar128: return launch_engine<128, 128, 2, 2, 2, QKM, 2>(g, st);
+    case kVarMid: return QKM ? launch_engine<192, 128, 2, 2, 2, QKM, 2>(g, st) : launch_engine<128, 192, 2, 2, 2, QKM, 2>(g, st);
+    case kVarWide: return QKM ? launch_engine<192, 256, 2, 4, 2, QKM, 2>(g, st) : launch_engine<256, 192, 4, 2, 2, QKM, 2>(g, st);
+    default: return launch_engine<256, 256, 2, 4, 2, QKM, 2>(g, st);
+  }
+}
+
+static int check_dense(const char* who, const void* x, const void* w, const void* out, int M, int N, int K) {
+  if (!x || !w || !out) return set_error(M2_ERR_ARG, "%s: null pointer", who);
+  if (M <= 0 || N <= 0 || K <= 0) return set_error(M2_ERR_ARG, "%s: sizes must be positive (M=%d N=%d K=%d)", who, M, N, K);
+  if (!m2_dense_supported(M, N, K))
+    return set_error(M2_ERR_UNSUPPORTED, "%s: needs M and N multiples of 8, K a multiple of 64 and operands below 4 GB (M=%d N=%d K=%d)", who, M, N, K);
+  return M2_OK;
+}
+
+}  // namespace m2
+
+using namespace m2;
+
+extern "C" int m2_dense_supported(int M, int N, int K) {
+  if (M < 8 || N < 8 || K < 64 || M % 8 || N % 8 || K % 64) return 0;
+  // the direct loads of the tile engine take 32-bit byte offsets
+  return ((long)M * K * 2 < (1l << 32) && (long)N * K * 2 < (1l << 32)) ? 1 : 0;
+}
+
+extern "C" int m2_dense_to_channels_fwd(const void* x, const void* w, void* out, int M, int N, int K, void* stream) {
+  const int rc = check_dense("m2_dense_to_channels_fwd", x, w, out, M, N, K);
+  if (rc) return rc;
+  GemmArgs g{(const uint16_t*)x, (const uint16_t*)w, (uint16_t*)out, nullptr, nullptr, K, K, M, M, N, K, 1, 0, 0, 0, 1};
+  return dense_launch<false>(pick_variant(g, false), g, (hipStream_t)stream);
+}
+
+extern "C" int m2_dense_from_channels_fwd(const void* x, const void* w, const float* bias, void* out, int M, int N, int K,
+                                          void* stream) {
+  const int rc = check_dense("m2_dense_from_channels_fwd", x, w, out, M, N, K);
+  if (rc) return rc;
+  GemmArgs g{(const uint16_t*)w, (const uint16_t*)x, (uint16_t*)out, bias, nullptr, K, M, N, N, M, K, 1, 0, 0, 0, 0};
+  return dense_launch<true>(pick_variant(g, true), g, (hipStream_t)stream);
+}

@@ -6,10 +6,10 @@ in the reference (bert/src/bert_layers.py:131-252 BertEmbeddings, :457-508 BertG
 layer so that no activation is transposed or re-read in between:
 
     h32 (M,d) f32, h16 (M,d) bf16, hT (d,M) f32   <- LayerNorm of the previous layer (three forms, one kernel)
-    xproj (3d,M) bf16 = W_in h16^T                library GEMM, channel-major output (bias added by K2)
+    xproj (3d,M) bf16 = W_in h16^T                own kernel or library GEMM, channel-major output (bias added by K2)
     spec              = filter spectra            K1 (hidden MLP, projection+decay) + spectrum FFT
     y (d,M) bf16      = mixer core(xproj, hT)     K2
-    a (M,d) bf16      = y^T W_out^T + b           library GEMM
+    a (M,d) bf16      = y^T W_out^T + b           own kernel or library GEMM
     g (M,I) bf16      = GLU(blockdiag(a, Wg))     K3
     s (M,d) f32       = blockdiag(g, Wo) + b + a  K3
     LayerNorm(s)      -> next layer's three forms
@@ -247,20 +247,13 @@ class BertLayer(nn.Module):
         d = at.d_model
         if at.hyena_training_additions:      # extra input LayerNorm: needs the fp32 form, replaces h16 / hT
             _, h16, hT = at.pre_norm(h32, want_f32=False, want_bf16=True)
-        w_in = at._cast("in_w", at.in_linear.weight, torch.bfloat16)
-        w_out = at._cast("out_w", at.out_linear.weight, torch.bfloat16)
-        b_out = at._cast("out_b", at.out_linear.bias, torch.bfloat16)
-        # (3d, M) channel-major, bias added in the core.  Written as h16 @ W^T into the transposed view of the
-        # output: the same product as W @ h16^T, for which the library picks a faster kernel (126 against 144 us at
-        # M = 32768, d = 768)
-        xproj = torch.empty(3 * d, B * L, dtype=torch.bfloat16, device=h16.device)
-        torch.mm(h16, w_in.t(), out=xproj.t())
+        xproj = at.project_in(h16)                   # (3d, M) channel-major, bias added in the core
         if spec_ready is not None:
             torch.cuda.current_stream().wait_event(spec_ready)
         y = at.core(xproj.view(3 * d, B, L), hT.view(d, B, L) if at.residual_long_conv else None, B, L, spec=spec)
         if after_core is not None:
             after_core()
-        a16 = torch.addmm(b_out, y.view(d, B * L).t(), w_out.t())                    # (M, d)
+        a16 = at.project_out(y.view(d, B * L))                                       # (M, d)
         pre = at.hyena_training_additions        # the next layer then reads the fp32 form only
         return self.mlp.normed(a16, want_f32, not pre, not pre)
 

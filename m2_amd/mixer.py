@@ -3,10 +3,10 @@ HIP mixer core (bert/src/mm/monarch_mixer_sequence_mixer.py:12-154).
 
 Data flow of `forward(u)`, u (B, L, d):
 
-    xproj (3d, B*L) = in_linear.weight @ u^T + bias       one library GEMM, written CHANNEL-major
+    xproj (3d, B*L) = in_linear.weight @ u^T + bias       written CHANNEL-major (own kernel or library GEMM, by size)
     spec            = spectra of the two bidirectional implicit filters (skip weights folded in)
     y (d, B*L)      = m2_mixer_core_fwd(xproj, u^T, short_filter, spec)
-    out (B*L, d)    = y^T @ out_linear.weight^T + bias     one library GEMM
+    out (B*L, d)    = y^T @ out_linear.weight^T + bias     own kernel or library GEMM, by size
 
 so the three `transpose` passes of the reference disappear into GEMM operand orientation.  With fp32
 input outside autocast everything is fp32; with bf16 input or under CUDA autocast the projections
@@ -133,6 +133,26 @@ class MonarchMixerSequenceMixing(nn.Module):
         return ops.layernorm(h32, ln.weight.detach().float(), ln.bias.detach().float(), ln.eps, want_f32=want_f32,
                              want_bf16=want_bf16, want_channel_major=self.residual_long_conv)
 
+    def project_in(self, x: torch.Tensor) -> torch.Tensor:
+        """x (M, d) -> in_linear.weight @ x^T without the bias, (3d, M) channel-major, in x's dtype (bf16 or fp32)."""
+        M, d = x.shape
+        w = self._cast("in_w", self.in_linear.weight, x.dtype)
+        if x.dtype == torch.bfloat16 and x.data_ptr() % 16 == 0 and ops.own_to_channels(M, d):
+            return ops.dense_to_channels(x, w)
+        # Written as x @ W^T into the transposed view of the output: the same product as W @ x^T, for which the library
+        # picks a faster kernel (126 against 144 us at M = 32768, d = 768)
+        out = torch.empty(3 * d, M, dtype=x.dtype, device=x.device)
+        torch.mm(x, w.t(), out=out.t())
+        return out
+
+    def project_out(self, y: torch.Tensor) -> torch.Tensor:
+        """y (d, M) channel-major -> y^T @ out_linear.weight^T + bias, (M, d), in y's dtype (bf16 or fp32)."""
+        d, M = y.shape
+        w = self._cast("out_w", self.out_linear.weight, y.dtype)
+        if y.dtype == torch.bfloat16 and ops.own_from_channels(M, d):
+            return ops.dense_from_channels(y, w, self._cast("out_b", self.out_linear.bias, torch.float32))
+        return torch.addmm(self._cast("out_b", self.out_linear.bias, y.dtype), y.t(), w.t())
+
     # -- reference API -----------------------------------------------------------------------
     def forward(self, u, **kwargs):
         if not u.is_cuda:
@@ -143,9 +163,6 @@ class MonarchMixerSequenceMixing(nn.Module):
         low = u.dtype == torch.bfloat16 or torch.is_autocast_enabled()
         act = torch.bfloat16 if low else torch.float32
         u2 = u.reshape(B * L, d)
-        w_in = self._cast("in_w", self.in_linear.weight, act)
-        w_out = self._cast("out_w", self.out_linear.weight, act)
-        b_out = self._cast("out_b", self.out_linear.bias, act)
         with torch.autocast("cuda", enabled=False):
             u_cm = None
             if self.hyena_training_additions:
@@ -154,12 +171,11 @@ class MonarchMixerSequenceMixing(nn.Module):
                 u2, u16, u_cm = self.pre_norm(u2.float().contiguous(), want_f32=not low, want_bf16=low)
                 if low:
                     u2 = u16
-            xproj = torch.empty(3 * d, B * L, dtype=act, device=u.device)               # (3d, B*L), bias added in the core
-            torch.mm(u2.to(act), w_in.t(), out=xproj.t())
+            xproj = self.project_in(u2.to(act).contiguous())                             # (3d, B*L), bias added in the core
             if u_cm is None and self.residual_long_conv:
                 u_cm = u2.float().t().contiguous()                                       # (d, B*L)
             if not self.residual_long_conv:
                 u_cm = None
             y = self.core(xproj.view(3 * d, B, L), None if u_cm is None else u_cm.view(d, B, L), B, L)
-            out = torch.addmm(b_out, y.view(d, B * L).t(), w_out.t())                   # (B*L, d)
+            out = self.project_out(y.view(d, B * L))                                    # (B*L, d)
         return out.view(B, L, d), None

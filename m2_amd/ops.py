@@ -230,6 +230,48 @@ def fftconv(x: Tensor, spec: Tensor, B: int, L: int, d: int) -> Tensor:
     return out
 
 
+# The library's own projection kernels against torch's (hipBLASLt), MI355X, us per call (own / torch):
+#   to_channels    d = 768: M = 4096 22 / 27, 8192 33 / 47, 16384 66 / 62, 32768 130 / 127; d = 960: 4096 27 / 25,
+#                  8192 49 / 49, 16384 101 / 85; d = 1536: 2048 36 / 30, 4096 66 / 58, 8192 120 / 102; d = 1792: 2048 42 / 46,
+#                  4096 91 / 72.  Below that torch's call costs 19 us whatever the size (its host side), own 8 .. 20.
+#   from_channels  d = 768: 4096 13 / 20, 16384 25 / 27, 32768 45 / 49; d = 960: 8192 23 / 29, 16384 36 / 48, 32768 69 / 74;
+#                  d = 1536: 2048 22 / 20, 4096 30 / 27, 8192 41 / 41, 16384 84 / 77; d = 1792: 4096 35 / 32, 8192 58 / 51.
+# So the own kernels serve products of up to about 29 GFLOP (to_channels), and every one of d <= 1024 (from_channels).
+_OWN_DENSE_FLOPS = 2.95e10
+
+
+def own_to_channels(M: int, d: int) -> bool:
+    return 6.0 * M * d * d <= _OWN_DENSE_FLOPS and bool(lib.m2_dense_supported(M, 3 * d, d))
+
+
+def own_from_channels(M: int, d: int) -> bool:
+    return (d <= 1024 or 6.0 * M * d * d <= _OWN_DENSE_FLOPS) and bool(lib.m2_dense_supported(M, d, d))
+
+
+def dense_to_channels(x: Tensor, w: Tensor) -> Tensor:
+    """w @ x^T: x (M, K) bf16, w (N, K) bf16 -> (N, M) bf16, fp32 accumulation."""
+    M, K = x.shape
+    N = w.shape[0]
+    _require(x, "x", torch.bfloat16)
+    _require(w, "w", torch.bfloat16, (N, K))
+    out = torch.empty(N, M, dtype=torch.bfloat16, device=x.device)
+    check(lib.m2_dense_to_channels_fwd(_ptr(x), _ptr(w), _ptr(out), M, N, K, _stream()))
+    return out
+
+
+def dense_from_channels(x: Tensor, w: Tensor, bias: Optional[Tensor] = None) -> Tensor:
+    """x^T @ w^T + bias: x (K, M) bf16, w (N, K) bf16, bias (N) fp32 -> (M, N) bf16, fp32 accumulation."""
+    K, M = x.shape
+    N = w.shape[0]
+    _require(x, "x", torch.bfloat16)
+    _require(w, "w", torch.bfloat16, (N, K))
+    if bias is not None:
+        _require(bias, "bias", torch.float32, (N,))
+    out = torch.empty(M, N, dtype=torch.bfloat16, device=x.device)
+    check(lib.m2_dense_from_channels_fwd(_ptr(x), _ptr(w), _ptr(bias), _ptr(out), M, N, K, _stream()))
+    return out
+
+
 def blockdiag_glu(x: Tensor, w: Tensor, out: Optional[Tensor] = None) -> Tensor:
     """gelu_erf(h[:, :I]) * h[:, I:] with h = blockdiag_multiply(x, w); x (M, in) bf16, w (nb, 2I/nb, in/nb) bf16."""
     M, in_f = x.shape
