@@ -977,6 +977,7 @@ extern "C" int m2_blockdiag_glu_fwd(const void* x, const void* w, void* out, int
   const int p = in_features / nblocks, q = 2 * intermediate / nblocks;
   int rc = check_blockdiag("m2_blockdiag_glu_fwd", M, nblocks, p, q, true);
   if (rc) return rc;
+  if (glu_few_rows_pays(M, nblocks, p)) return glu_few_rows(x, w, out, M, nblocks, p, q, (hipStream_t)stream);
   if (p % 64 != 0 || q % 64 != 0) {               // block sizes off the tile grid (d = 960: 240-wide blocks): the masked kernel
     hipStream_t st = (hipStream_t)stream;
     return q >= 128 ? launch_blockdiag<2, 2, true, uint16_t, 2, true>(x, w, nullptr, nullptr, out, M, nblocks, p, q, intermediate, st)
@@ -1015,24 +1016,22 @@ extern "C" int m2_blockdiag_linear_fwd(const void* x, const void* w, const float
   int rc = check_blockdiag("m2_blockdiag_linear_fwd", M, nblocks, p, q, false);
   if (rc) return rc;
   hipStream_t st = (hipStream_t)stream;
-  if (p % 64 != 0 || q % 64 != 0) {               // block sizes off the tile grid: the masked kernel
-    if (out_dtype == M2_DTYPE_F32)
-      return q >= 128 ? launch_blockdiag<2, 2, false, float, 1, true>(x, w, bias, residual, out, M, nblocks, p, q, out_features, st)
-                      : launch_blockdiag<4, 1, false, float, 1, true>(x, w, bias, residual, out, M, nblocks, p, q, out_features, st);
+  if (out_dtype == M2_DTYPE_BF16) {
+    // the row offsets of the tile engine's direct loads are 32 bits wide
+    if (p % 64 == 0 && (long)M * in_features * 2 < (1l << 32) && (long)nblocks * q * p * 2 < (1l << 32))
+      return blockdiag_linear_engine(x, w, bias, residual, out, M, nblocks, p, q, st);
     return q >= 128 ? launch_blockdiag<2, 2, false, uint16_t, 1, true>(x, w, bias, residual, out, M, nblocks, p, q, out_features, st)
                     : launch_blockdiag<4, 1, false, uint16_t, 1, true>(x, w, bias, residual, out, M, nblocks, p, q, out_features, st);
   }
+  if (p % 64 != 0 || q % 64 != 0)                 // block sizes off the tile grid: the masked kernel
+    return q >= 128 ? launch_blockdiag<2, 2, false, float, 1, true>(x, w, bias, residual, out, M, nblocks, p, q, out_features, st)
+                    : launch_blockdiag<4, 1, false, float, 1, true>(x, w, bias, residual, out, M, nblocks, p, q, out_features, st);
   // 256 x 192 tiles once there is at least one per compute unit (measured at d = 768 and 1536: below that the
   // smaller tiles of the general kernel fill the chip better)
   if (q % kWideBN == 0 && (long)((M + kWideBM - 1) / kWideBM) * (nblocks * q / kWideBN) >= num_cus())
-    return out_dtype == M2_DTYPE_F32 ? launch_blockdiag_wide<float>(x, w, bias, residual, out, M, nblocks, p, q, st)
-                                     : launch_blockdiag_wide<uint16_t>(x, w, bias, residual, out, M, nblocks, p, q, st);
-  const bool wide = q % 128 == 0;
-  if (out_dtype == M2_DTYPE_F32)
-    return wide ? launch_blockdiag<2, 2, false, float, 1>(x, w, bias, residual, out, M, nblocks, p, q, out_features, st)
-                : launch_blockdiag<4, 1, false, float, 1>(x, w, bias, residual, out, M, nblocks, p, q, out_features, st);
-  return wide ? launch_blockdiag<2, 2, false, uint16_t, 1>(x, w, bias, residual, out, M, nblocks, p, q, out_features, st)
-              : launch_blockdiag<4, 1, false, uint16_t, 1>(x, w, bias, residual, out, M, nblocks, p, q, out_features, st);
+    return launch_blockdiag_wide<float>(x, w, bias, residual, out, M, nblocks, p, q, st);
+  return q % 128 == 0 ? launch_blockdiag<2, 2, false, float, 1>(x, w, bias, residual, out, M, nblocks, p, q, out_features, st)
+                      : launch_blockdiag<4, 1, false, float, 1>(x, w, bias, residual, out, M, nblocks, p, q, out_features, st);
 }
 
 extern "C" int m2_blockdiag_linear_f32_fwd(const float* x, const float* w, const float* bias, float* out, int M,

@@ -173,8 +173,8 @@ static int launch_engine(GemmArgs g, hipStream_t st) {
 // the compute unit holds a second workgroup; a launch takes about 2.5 us.  Measured on MI355X (us per step, one / two
 // workgroups per compute unit; K = 768 and 1536, M = 128 .. 32768): the table below.  What bounds a step: the small
 // tiles their loads (a compute unit gets 50 - 65 GB/s out of L2) and the latency of a step, the two large ones the power
-// budget (the clock falls to 1.6 - 1.8 GHz under them).  The model picks the measured best, or one within 10 % of it, at
-// all of 4 widths x 9 row counts.
+// budget (the clock falls to 1.6 - 1.8 GHz under them).  At 4 widths x 9 row counts the model picks the measured best or
+// one within about 10 % of it.
 // ---------------------------------------------------------------------------------------------
 enum DenseVariant { kVarSmall, kVar64, kVar128, kVarMid, kVarWide, kVar256, kVariants };
 struct VariantShape {
@@ -182,8 +182,8 @@ struct VariantShape {
   float t1, t2;             // us per step with one and with per_cu workgroups on it
 };
 static const VariantShape kVariantShapes[kVariants] = {
-    {32, 32, 4, 0.f, 0.f},       {64, 128, 2, 0.47f, 0.80f},  {128, 128, 2, 0.64f, 1.12f},
-    {128, 192, 2, 1.05f, 1.68f}, {256, 192, 1, 1.55f, 1.55f}, {256, 256, 1, 1.90f, 1.90f}};
+    {32, 32, 4, 0.f, 0.f},       {64, 128, 2, 0.52f, 0.86f},  {128, 128, 2, 0.80f, 1.14f},
+    {128, 192, 2, 1.08f, 1.70f}, {256, 192, 1, 1.65f, 1.65f}, {256, 256, 1, 2.00f, 2.00f}};
 
 static float variant_cost(int v, const GemmArgs& g, bool swap) {
   const VariantShape& s = kVariantShapes[v];
@@ -224,6 +224,55 @@ static int dense_launch(int variant, GemmArgs g, hipStream_t st) {
     case kVarMid: return QKM ? launch_engine<192, 128, 2, 2, 2, QKM, 2>(g, st) : launch_engine<128, 192, 2, 2, 2, QKM, 2>(g, st);
     case kVarWide: return QKM ? launch_engine<192, 256, 2, 4, 2, QKM, 2>(g, st) : launch_engine<256, 192, 4, 2, 2, QKM, 2>(g, st);
     default: return launch_engine<256, 256, 2, 4, 2, QKM, 2>(g, st);
+  }
+}
+
+// ---- block-diagonal products (declared in m2_internal.h) ----
+// weights along i (P), rows of x along j (Q)
+static GemmArgs blockdiag_args(const void* x, const void* w, const float* bias, const void* resid, void* out, int M, int nb,
+                               int p, int q) {
+  return GemmArgs{(const uint16_t*)w, (const uint16_t*)x, (uint16_t*)out, bias, (const uint16_t*)resid, p, (long)nb * p,
+                  (long)nb * q, q, M, p, nb, (long)q * p, 0, 0, 0};
+}
+template <int NW>
+static int launch_small_glu(const GemmArgs& g, hipStream_t st) {
+  const int ks = ((g.nk + 31) / 32 + NW - 1) / NW;
+  if (ks <= 2) return launch_small<NW, 2, false, true>(g, st);
+  if (ks <= 3) return launch_small<NW, 3, false, true>(g, st);
+  return launch_small<NW, 4, false, true>(g, st);
+}
+// The gated product + GLU for few rows.  us per call at M = 128 / 256, this against the next best: d = 768 5.5 / 7.0 (the
+// weight-stationary kernel 10.1 / 10.4), d = 960 5.2 / 7.7 (the streaming kernel 8.2 / 8.4), d = 1536 10.5 / 19.6
+// (12.7 / 13.3): every 32 x 32 tile reads its operands again, so it ends where M times the width passes about 250 thousand.
+bool glu_few_rows_pays(int M, int nb, int p) { return (long)M * nb * p <= 245760 && p <= 512; }
+int glu_few_rows(const void* x, const void* w, void* out, int M, int nb, int p, int q, hipStream_t st) {
+  GemmArgs g = blockdiag_args(x, w, nullptr, nullptr, out, M, nb, p, q);
+  g.nblk = nb / 2;
+  g.ldo = (long)nb / 2 * q;
+  g.jfast = 1;
+  return launch_small_glu<4>(g, st);
+}
+// wo + bias + residual in bf16, p % 64 == 0 and q % 8 == 0.  us per call, this against the LDS-tiled kernels it took over
+// from: d = 768 M = 128 5.3 / 13.2, 1024 8.8 / 15.5; d = 1536 M = 512 14 / 22, 1024 15 / 23, 2048 20 / 24, 4096 29 / 33,
+// 8192 44 / 48; d = 1792 M = 128 9 / 26, 1024 18 / 31, 4096 36 / 42, 8192 60 / 81; d = 960 (240-wide blocks) M = 128
+// 6 / 17, 1024 10 / 17, 8192 23 / 27, 32768 107 / 117.
+int blockdiag_linear_engine(const void* x, const void* w, const float* bias, const void* resid, void* out, int M, int nb, int p,
+                            int q, hipStream_t st) {
+  GemmArgs g = blockdiag_args(x, w, bias, resid, out, M, nb, p, q);
+  switch (pick_variant(g, true)) {
+    case kVarSmall: {
+      g.jfast = 1;
+      const int ks = ((p + 31) / 32 + 7) / 8;
+      if (ks <= 3) return launch_small<8, 3, false, false>(g, st);
+      if (ks <= 4) return launch_small<8, 4, false, false>(g, st);
+      if (ks <= 6) return launch_small<8, 6, false, false>(g, st);
+      return launch_small<8, 8, false, false>(g, st);
+    }
+    case kVar64: return launch_engine<128, 64, 2, 2, 3, false, 2>(g, st);
+    case kVar128: return launch_engine<128, 128, 2, 2, 2, false, 2>(g, st);
+    case kVarMid: return launch_engine<192, 128, 2, 2, 2, false, 2>(g, st);
+    case kVarWide: return launch_engine<192, 256, 2, 4, 2, false, 2>(g, st);
+    default: return launch_engine<256, 256, 2, 4, 2, false, 2>(g, st);
   }
 }
 

@@ -73,7 +73,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     const uint16_t* __restrict__ x,             // (M, 4 p) bf16
     const unsigned char* __restrict__ wpk,      // the gated weight as packed by glu_stream_pack_kernel
     uint16_t* __restrict__ out,                 // (M, I) bf16
-    int M, int I, int ntiles, int p) {
+    int M, int I, int ntiles, int p, int nsplit) {
   constexpr int kSKS = KS, kSStage = GluShape<KS>::kStage, kSBatch = GluShape<KS>::kBatch, kSStages = GluShape<KS>::kStages;
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   const int tid = threadIdx.x, lane = tid & 63, i16 = lane & 15, q4 = lane >> 4;
@@ -81,13 +81,16 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   // Workgroup ids are dealt round-robin to the 8 XCDs (one L2 each): XCD e works on r = 2 (e % 2), 2 (e % 2) + 1, which
   // read the same two blocks of x, and on the row tiles = e / 2 (mod 4); neighbouring workgroups of an XCD take the
   // same row tile with the two r, so the second read of its x rows is an L2 hit and an L2 holds half of the weights.
+  // With nsplit > 1 a workgroup takes one of nsplit runs of the chunks of its r (gated columns are independent).
   const int xcd = blockIdx.x & 7, slot = (int)(blockIdx.x >> 3);
   const int r = 2 * (xcd & 1) + (slot & 1);
-  const int tile_step = 2 * (int)(gridDim.x >> 3);
-  int tile = 4 * (slot >> 1) + (xcd >> 1);
+  const int split = (slot >> 1) % nsplit, tslots = (int)(gridDim.x >> 4) / nsplit;
+  const int tile_step = 4 * tslots;
+  int tile = 4 * ((slot >> 1) / nsplit) + (xcd >> 1);
   if (tile >= ntiles) return;
   const int IS = I >> 2;                  // gated columns of this r
-  const int nchunks = IS / kSChunk;
+  const int chunk0 = split * (IS / kSChunk) / nsplit;
+  const int nchunks = (split + 1) * (IS / kSChunk) / nsplit - chunk0;
   const int gb = r >> 1;                  // gate block; the value block is gb + 2
   const int d = 4 * p;
 
@@ -117,7 +120,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   // chunk it + 2 of a tile, or the first chunks of the next tile (same r, same weights) at a tile's end.
   const unsigned lds0 = (unsigned)(uintptr_t)smem;
   const unsigned voff = 16 * lane;
-  const unsigned char* wr = wpk + (long)r * nchunks * kSStage;
+  const unsigned char* wr = wpk + ((long)r * (IS / kSChunk) + chunk0) * kSStage;
   auto dma_one = [&](int stage, int chunk, auto jj) __attribute__((always_inline)) {
     constexpr int j = decltype(jj)::value;
     load_to_lds(lds0 + stage * kSStage + (wave + 8 * j) * kSBlk, voff, wr + (long)chunk * kSStage + (wave + 8 * j) * kSBlk);
@@ -148,7 +151,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     for (int s = 0; s < kSKS; ++s) asm volatile("" : "+v"(xa[s]), "+v"(xb[s]));
     const int row = tile * kSRows + 16 * wave + i16;
     const int rowc = row < M ? row : M - 1;
-    uint16_t* orow = out + (long)rowc * I + r * IS + 8 * q4;
+    uint16_t* orow = out + (long)rowc * I + r * IS + kSChunk * chunk0 + 8 * q4;
 
     // gelu(gate) * value of the chunk whose accumulators sit in gp / vp: eight chains side by side, one 16-byte store
     auto finish_chunk = [&](int chunk) __attribute__((always_inline)) {
@@ -264,12 +267,12 @@ extern "C" int m2_glu_stream_pack(const void* w_gated, void* packed, int in_feat
 
 template <int KS>
 static int launch_glu_stream(const void* x, const void* w_packed, void* out, int M, int intermediate, int p, int per_xcd,
-                             int ntiles, hipStream_t stream) {
+                             int ntiles, int nsplit, hipStream_t stream) {
   auto kern = glu_stream_kernel<KS>;
   hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, GluShape<KS>::kLds);
   if (e != hipSuccess) return set_error(M2_ERR_LAUNCH, "hipFuncSetAttribute(glu_stream): %s", hipGetErrorString(e));
   hipLaunchKernelGGL(kern, dim3(8 * per_xcd), dim3(512), GluShape<KS>::kLds, stream, (const uint16_t*)x,
-                     (const unsigned char*)w_packed, (uint16_t*)out, M, intermediate, ntiles, p);
+                     (const unsigned char*)w_packed, (uint16_t*)out, M, intermediate, ntiles, p, nsplit);
   return check_launch("glu_stream");
 }
 
@@ -284,11 +287,23 @@ extern "C" int m2_glu_stream_fwd(const void* x, const void* w_packed, void* out,
   // one persistent workgroup per compute unit (its LDS stages take most of it), an even number per XCD
   int per_xcd = (num_cus() / 8) & ~1;
   if (per_xcd < 2) per_xcd = 2;      // a device (or partition) with fewer than 16 compute units: work is dealt to 8 x per_xcd slots whatever the real count
-  if (per_xcd > 2 * ((ntiles + 3) / 4)) per_xcd = 2 * ((ntiles + 3) / 4);
+  // The 128-row tiles of the four r rarely fill the compute units in whole rounds: the chunks of an r are then dealt to
+  // nsplit workgroups.  A workgroup costs its chunks plus about four (launch, x rows, first chunk).  us at d = 1536, without
+  // and with: M = 128 60 / 13, 1024 61 / 18, 2048 62 / 26, 4096 69 / 47; d = 1792, M = 1024 82 / 22, 4096 88 / 60.
+  const int half = per_xcd / 2, tslots = (ntiles + 3) / 4, nchunks = intermediate / 4 / kSChunk;
+  int nsplit = 1;
+  long best = -1;
+  for (int n = 1; n <= half && n <= nchunks; ++n) {
+    const bool one_round = tslots * n <= half;
+    if (!one_round && half % n != 0) continue;      // a workgroup keeps its run of chunks from tile to tile
+    const long cost = (one_round ? 1l : (tslots * n + half - 1) / half) * ((nchunks + n - 1) / n + 4);
+    if (best < 0 || cost < best) { best = cost; nsplit = n; }
+  }
+  if (tslots * nsplit < half) per_xcd = 2 * tslots * nsplit;
   const int p = in_features / 4;
   switch (glu_stream_ksteps(p)) {
-    case 12: return launch_glu_stream<12>(x, w_packed, out, M, intermediate, p, per_xcd, ntiles, (hipStream_t)stream);
-    case 14: return launch_glu_stream<14>(x, w_packed, out, M, intermediate, p, per_xcd, ntiles, (hipStream_t)stream);
-    default: return launch_glu_stream<8>(x, w_packed, out, M, intermediate, p, per_xcd, ntiles, (hipStream_t)stream);
+    case 12: return launch_glu_stream<12>(x, w_packed, out, M, intermediate, p, per_xcd, ntiles, nsplit, (hipStream_t)stream);
+    case 14: return launch_glu_stream<14>(x, w_packed, out, M, intermediate, p, per_xcd, ntiles, nsplit, (hipStream_t)stream);
+    default: return launch_glu_stream<8>(x, w_packed, out, M, intermediate, p, per_xcd, ntiles, nsplit, (hipStream_t)stream);
   }
 }

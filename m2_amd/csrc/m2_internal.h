@@ -14,6 +14,12 @@ int check_launch(const char* what);
 // Compute units of the current device (cached per device).
 int num_cus();
 
+// Block-diagonal products on the dense kernels (dense_kernels.hip): x (M, nb p) bf16, w (nb, q, p) bf16.
+bool glu_few_rows_pays(int M, int nb, int p);
+int glu_few_rows(const void* x, const void* w, void* out, int M, int nb, int p, int q, hipStream_t stream);
+int blockdiag_linear_engine(const void* x, const void* w, const float* bias, const void* resid, void* out, int M, int nb, int p,
+                            int q, hipStream_t stream);
+
 // round-to-nearest-even float -> bfloat16 bits (NaN stays NaN)
 // float -> bf16 bits, round to nearest even (host restatement of what v_cvt_pk_bf16_f32 does)
 __host__ __device__ __forceinline__ uint16_t f32_to_bf16_bits(float f) {

@@ -147,7 +147,9 @@ class BertGatedLinearUnitMLP(nn.Module):
     def presum(self, a16: torch.Tensor) -> torch.Tensor:
         """a16 (M, d) bf16 -> wo(glu(a16)) + bias + a16, (M, d) fp32 (the LayerNorm input; bf16 with `bf16_presum`)."""
         sum_dtype = torch.bfloat16 if self.bf16_presum else torch.float32
-        if self.fuse_mlp and ops.mlp_fused_supported(a16.shape[1], self.config.intermediate_size,
+        # up to 512 rows the one-kernel MLP leaves most compute units idle (21.5 us whatever the row count); the two
+        # products as kernels of their own take 11 us at M = 128, 12.5 at 256, 19 at 512, 20 at 1024
+        if self.fuse_mlp and a16.shape[0] > 512 and ops.mlp_fused_supported(a16.shape[1], self.config.intermediate_size,
                                                      self.config.monarch_mlp_nblocks):
             wg, wo = self.gated_layers.weight_bf16(), self.wo.weight_bf16()
             # the packed copy the kernel streams: rebuilt whenever one of the bf16 copies has been rebuilt
@@ -168,7 +170,8 @@ class BertGatedLinearUnitMLP(nn.Module):
     def glu(self, a16: torch.Tensor) -> torch.Tensor:
         """a16 (M, d) bf16 -> gelu(gate) * value of gated_layers(a16), (M, I) bf16."""
         wg = self.gated_layers.weight_bf16()
-        if self.stream_glu and ops.glu_stream_supported(a16.shape[1], self.config.intermediate_size,
+        few = a16.shape[0] * a16.shape[1] <= 245760          # m2_blockdiag_glu_fwd has a kernel for few rows
+        if self.stream_glu and not few and ops.glu_stream_supported(a16.shape[1], self.config.intermediate_size,
                                                         self.config.monarch_mlp_nblocks):
             if self._packed_glu is None or self._packed_glu[0] is not wg:      # rebuilt with the bf16 copy
                 self._packed_glu = (wg, ops.glu_stream_pack(wg))

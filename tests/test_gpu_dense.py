@@ -44,3 +44,58 @@ def test_dense_unsupported_sizes_are_refused(gpu):
         with pytest.raises(RuntimeError, match="multiples of 8"):
             ops.dense_to_channels(torch.zeros(M, K, dtype=torch.bfloat16, device=gpu),
                                   torch.zeros(N, K, dtype=torch.bfloat16, device=gpu))
+
+
+def _blockdiag(x, w):
+    nb, q, p = w.shape
+    return torch.cat([x[:, k * p:(k + 1) * p] @ w[k].T for k in range(nb)], dim=1)
+
+
+# wo with bias and residual on the tile engine: few rows, 240-wide blocks, each tile variant, ragged rows
+@pytest.mark.parametrize("M,nb,q,p", [(1, 4, 8, 64), (33, 4, 192, 768), (128, 4, 240, 960), (1000, 4, 384, 1536), (2049, 2, 448, 1792),
+                                      (4100, 4, 384, 1536), (8192, 4, 384, 1536), (5000, 4, 448, 1792), (40, 2, 24, 2112)])
+def test_blockdiag_linear_bf16(gpu, M, nb, q, p):
+    from m2_amd import ops
+    g = torch.Generator().manual_seed(M + p)
+    x, w, res, bias = _bf16(g, M, nb * p), _bf16(g, nb, q, p) * 0.05, _bf16(g, M, nb * q), torch.randn(nb * q, generator=g)
+    ref, absref = _blockdiag(x.double(), w.double()), _blockdiag(x.double().abs(), w.double().abs())
+    _within_bf16(ops.blockdiag_linear(x.to(gpu), w.to(gpu)), ref, absref)
+    _within_bf16(ops.blockdiag_linear(x.to(gpu), w.to(gpu), bias.to(gpu), res.to(gpu)), ref + bias.double() + res.double(),
+                 absref + bias.double().abs() + res.double().abs())
+
+
+def _glu(x, w):
+    nb, q, p = w.shape
+    h = _blockdiag(x.double(), w.double())
+    gate, val = h[:, :nb * q // 2], h[:, nb * q // 2:]
+    return torch.nn.functional.gelu(gate) * val, val
+
+
+def _within_glu(got, ref, val):
+    """The GELU polynomial's 2.5e-4 of the value and one bf16 rounding, as for the other GLU kernels."""
+    err = (got.double().cpu() - ref).abs()
+    assert (err <= ref.abs() * 2.0 ** -7 + 2.5e-4 * (val.abs() + 1)).all(), err.max()
+
+
+# the gated product of few rows: block widths off 32, one row, the last row count of its range and one beyond it
+@pytest.mark.parametrize("M,nb,q,p", [(1, 4, 96, 192), (128, 4, 1536, 192), (256, 4, 1920, 240), (257, 4, 1920, 240), (64, 4, 3072, 384),
+                                      (137, 4, 3584, 448), (70, 2, 40, 504)])
+def test_blockdiag_glu_few_rows(gpu, M, nb, q, p):
+    from m2_amd import ops
+    g = torch.Generator().manual_seed(M + p)
+    x, w = _bf16(g, M, nb * p), _bf16(g, nb, q, p) * (3 / p ** 0.5)
+    _within_glu(ops.blockdiag_glu(x.to(gpu), w.to(gpu)), *_glu(x, w))
+
+
+# the streaming kernel with the chunks of a block row dealt to several workgroups: one tile, uneven runs (30 and 56 chunks
+# over 5, 8 and 16), several rounds of a split
+@pytest.mark.parametrize("M,d", [(300, 960), (1100, 960), (700, 1536), (2000, 1536), (10300, 1536), (500, 1792), (10240, 1792)])
+def test_glu_stream_split_chunks(gpu, M, d):
+    from m2_amd import ops
+    g = torch.Generator().manual_seed(M + d)
+    x, w = _bf16(g, M, d), _bf16(g, 4, 2 * d, d // 4) * (3 / (d / 4) ** 0.5)
+    got = ops.glu_stream(x.to(gpu), w.to(gpu))
+    tiled = ops.blockdiag_glu(x.to(gpu), w.to(gpu))
+    rows = torch.cat([torch.arange(min(M, 40)), torch.arange(max(0, M - 140), M)]).unique()
+    _within_glu(got[rows.to(gpu)], *_glu(x[rows], w))
+    assert (got.float() - tiled.float()).abs().max() <= 2.0 ** -6 * tiled.float().abs().max()
