@@ -274,6 +274,36 @@ int m2_embed_layernorm_fwd(const long long* input_ids, const long long* token_ty
                            float* out_f32, void* out_bf16, float* out_channel_major, int* bad_index, int B, int L,
                            int d, void* stream);
 
+/* ---------------------------------------------------------------------------------------------
+ * The fused schedule of a stack of encoder layers (BertEncoder.forward, bert/src/bert_layers.py:691-813, with
+ * BertLayer :575-599), bf16 GEMMs, enqueued by one call.  `layers` is a HOST array of device pointers; `spectra` holds
+ * the layers' filter spectra one after the other (m2_mixer_filters_fwd); `h16` (M, d) bf16 and `h_channel_major` (d, M) fp32
+ * are the two forms of the input; out_f32[i] receives layer i's output (M, d) fp32 or is NULL.  The workspace holds
+ * m2_encoder_layers_workspace_bytes.  Sizes: m2_dense_supported for both projections and what the other entry points
+ * take.  `mlp_packed` (m2_mlp_fused_pack) selects the one-kernel MLP, else `glu_packed` (m2_glu_stream_pack) the streaming
+ * gated product, else m2_blockdiag_glu_fwd.
+ * ------------------------------------------------------------------------------------------- */
+typedef struct m2_layer_params {
+  const void* in_w;        /* (3d, d) bf16                                  */
+  const float* in_b;       /* (3d) or NULL                                  */
+  const float* short_w;    /* (3d, 3)                                       */
+  const float* short_b;    /* (3d)                                          */
+  const void* out_w;       /* (d, d) bf16                                   */
+  const float* out_b;      /* (d) or NULL                                   */
+  const void* w_gated;     /* (nblocks, 2I/nblocks, d/nblocks) bf16         */
+  const void* w_out;       /* (nblocks, d/nblocks, I/nblocks) bf16          */
+  const void* mlp_packed;  /* or NULL                                       */
+  const void* glu_packed;  /* or NULL                                       */
+  const float* wo_b;       /* (d) or NULL                                   */
+  const float* ln_gamma;   /* (d)                                           */
+  const float* ln_beta;    /* (d)                                           */
+  int residual;            /* 1: the mixer has a second (residual) long convolution */
+} m2_layer_params;
+size_t m2_encoder_layers_workspace_bytes(int M, int d, int intermediate);
+int m2_encoder_layers_fwd(const m2_layer_params* layers, int nlayers, const float* spectra, const void* h16,
+                          const float* h_channel_major, float* const* out_f32, void* workspace, int B, int L, int d,
+                          int intermediate, int nblocks, float eps, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

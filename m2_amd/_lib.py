@@ -25,6 +25,12 @@ class HyenaFilterParams(ctypes.Structure):
         "rw0", "rb0", "rw1", "rb1", "rw2", "rb2", "rw3")]
 
 
+class LayerParams(ctypes.Structure):
+    """Mirror of `m2_layer_params`."""
+    _fields_ = [(n, c_void_p) for n in ("in_w", "in_b", "short_w", "short_b", "out_w", "out_b", "w_gated", "w_out",
+                                        "mlp_packed", "glu_packed", "wo_b", "ln_gamma", "ln_beta")] + [("residual", c_int)]
+
+
 def _load() -> ctypes.CDLL:
     if not os.path.exists(LIB_PATH):
         raise ImportError(
@@ -99,6 +105,10 @@ def _load() -> ctypes.CDLL:
     lib.m2_embed_layernorm_fwd.restype = c_int
     lib.m2_embed_layernorm_fwd.argtypes = ([c_void_p] * 6 + [c_int] * 3 + [c_void_p] * 2 + [c_float] + [c_void_p] * 4
                                            + [c_int, c_int, c_int, c_void_p])
+    lib.m2_encoder_layers_workspace_bytes.restype = c_size_t
+    lib.m2_encoder_layers_workspace_bytes.argtypes = [c_int] * 3
+    lib.m2_encoder_layers_fwd.restype = c_int
+    lib.m2_encoder_layers_fwd.argtypes = [c_void_p, c_int] + [c_void_p] * 5 + [c_int] * 5 + [c_float, c_void_p]
     return lib
 
 
@@ -107,7 +117,7 @@ lib = _load()
 EXPORTS = ["m2_version", "m2_last_error", "m2_hyena_filter_workspace_bytes", "m2_hyena_filter_fwd", "m2_hyena_filter_fwd_static", "m2_mixer_filters_workspace_bytes", "m2_mixer_filters_fwd",
            "m2_fftconv_supported_seqlen", "m2_filter_spectrum_bytes", "m2_filter_spectrum_fwd", "m2_mixer_core_fwd",
            "m2_fftconv_fwd", "m2_dense_supported", "m2_dense_to_channels_fwd", "m2_dense_from_channels_fwd", "m2_blockdiag_glu_fwd", "m2_blockdiag_linear_fwd", "m2_blockdiag_linear_f32_fwd", "m2_mlp_fused_supported", "m2_mlp_fused_packed_bytes", "m2_mlp_fused_pack", "m2_mlp_fused_fwd", "m2_glu_stream_supported", "m2_glu_stream_packed_bytes", "m2_glu_stream_pack", "m2_glu_stream_fwd", "m2_layernorm_fwd", "m2_layernorm_bf16_fwd",
-           "m2_embed_layernorm_fwd", "m2_blockdiag_linear_layernorm_supported", "m2_blockdiag_linear_layernorm_fwd"]
+           "m2_embed_layernorm_fwd", "m2_blockdiag_linear_layernorm_supported", "m2_blockdiag_linear_layernorm_fwd", "m2_encoder_layers_workspace_bytes", "m2_encoder_layers_fwd"]
 
 
 def check(rc: int) -> None:

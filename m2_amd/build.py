@@ -14,7 +14,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libm2_amd.so")
 SOURCES = ["common.hip", "fftconv_kernels.hip", "fftconv_real_kernels.hip", "fftconv_split_kernels.hip", "hyena_filter_kernels.hip", "filter_fused_kernels.hip", "blockdiag_kernels.hip", "wo_layernorm_kernels.hip",
-           "mlp_fused_kernels.hip", "glu_stream_kernels.hip", "dense_kernels.hip"]
+           "mlp_fused_kernels.hip", "glu_stream_kernels.hip", "dense_kernels.hip", "encoder_schedule.hip"]
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 # packed fp32 VALU instructions are switched off on purpose (device flag, the host pass warns about it)
 FLAGS = ["-std=c++17", "-O3", "--offload-arch=gfx950", "-fPIC", "-Xclang", "-target-feature", "-Xclang",
@@ -45,10 +45,30 @@ def _compile(src: str, incremental: bool = False) -> str:
     return obj
 
 
+def _build_param_check(incremental: bool = False) -> str:
+    """m2_amd/_param_check.so, a host-only CPython extension against torch's headers."""
+    import sysconfig
+
+    import torch
+    from torch.utils.cpp_extension import include_paths, library_paths
+    src, out = os.path.join(CSRC, "param_check.cpp"), os.path.join(HERE, "_param_check.so")
+    if incremental and os.path.exists(out) and os.path.getmtime(src) < os.path.getmtime(out):
+        return out
+    cmd = ["g++", "-std=c++17", "-O2", "-fPIC", "-shared", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           *[f"-I{p}" for p in include_paths()], f"-I{sysconfig.get_paths()['include']}", src, "-o", out,
+           *[f"-L{p}" for p in library_paths()], "-lc10", "-ltorch_cpu", "-ltorch_python"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"g++ failed for param_check.cpp:\n{r.stderr}")
+    return out
+
+
 def build(verbose: bool = True, incremental: bool = False) -> str:
     """Compiles every source (or, with incremental=True, only those older than their .hip / headers) and links."""
     with ThreadPoolExecutor(max_workers=min(8, len(SOURCES))) as ex:
+        check = ex.submit(_build_param_check, incremental)
         objs = list(ex.map(lambda src: _compile(src, incremental), SOURCES))
+        check.result()
     cmd = [HIPCC, "-shared", "-fPIC", "--offload-arch=gfx950", "-o", LIB, *objs]
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:

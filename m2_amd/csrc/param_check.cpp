@@ -1,0 +1,126 @@
+// CPython extension m2_amd._param_check: "are these still the tensors a plan was made from?"
+//
+// A plan of the native schedule (m2_amd/schedule.py) holds device addresses of some fifty tensors per layer and copies
+// derived from four of them.  Before every use each tensor is looked up again where the modules keep it and its address
+// (and, for those that copies were made from, its version counter) compared; so is every module on the way there.  For
+// 12 layers that is about 1,100 look-ups: 0.1 ms in Python, 15 us here.
+#define PY_SSIZE_T_CLEAN
+#include <Python.h>
+#include <torch/csrc/autograd/python_variable.h>
+
+#include <vector>
+
+namespace {
+
+struct ModuleSlot {
+  PyObject *dict, *key, *expected;
+};
+struct TensorSlot {
+  PyObject *dict, *key;
+  const void* data;
+  int64_t version;      // -1: not compared
+};
+struct Checker {
+  PyObject_HEAD
+  std::vector<ModuleSlot>* modules;
+  std::vector<TensorSlot>* tensors;
+};
+
+bool read_tensor(PyObject* dict, PyObject* key, const void** data, int64_t* version) {
+  PyObject* o = PyDict_GetItemWithError(dict, key);
+  if (!o || !THPVariable_Check(o)) return false;
+  const at::Tensor& t = THPVariable_Unpack(o);
+  if (!t.defined()) return false;
+  *data = t.const_data_ptr();
+  if (*version >= 0) *version = t.is_inference() ? 0 : t._version();
+  return true;
+}
+
+void checker_dealloc(PyObject* self) {
+  Checker* c = reinterpret_cast<Checker*>(self);
+  if (c->modules) {
+    for (auto& m : *c->modules) { Py_DECREF(m.dict); Py_DECREF(m.key); Py_DECREF(m.expected); }
+    delete c->modules;
+  }
+  if (c->tensors) {
+    for (auto& t : *c->tensors) { Py_DECREF(t.dict); Py_DECREF(t.key); }
+    delete c->tensors;
+  }
+  Py_TYPE(self)->tp_free(self);
+}
+
+// Checker(modules, tensors): sequences of (dict, key) and (dict, key, compare_version); the present state is recorded.
+PyObject* checker_new(PyTypeObject* type, PyObject* args, PyObject*) {
+  PyObject *mods, *tens;
+  if (!PyArg_ParseTuple(args, "O!O!", &PyList_Type, &mods, &PyList_Type, &tens)) return nullptr;
+  Checker* c = reinterpret_cast<Checker*>(type->tp_alloc(type, 0));
+  if (!c) return nullptr;
+  c->modules = new std::vector<ModuleSlot>();
+  c->tensors = new std::vector<TensorSlot>();
+  for (Py_ssize_t i = 0; i < PyList_GET_SIZE(mods); ++i) {
+    PyObject *dict, *key;
+    if (!PyArg_ParseTuple(PyList_GET_ITEM(mods, i), "O!O", &PyDict_Type, &dict, &key)) { Py_DECREF(c); return nullptr; }
+    PyObject* o = PyDict_GetItemWithError(dict, key);
+    if (!o) {
+      if (!PyErr_Occurred()) PyErr_SetObject(PyExc_KeyError, key);
+      Py_DECREF(c);
+      return nullptr;
+    }
+    Py_INCREF(dict); Py_INCREF(key); Py_INCREF(o);
+    c->modules->push_back({dict, key, o});
+  }
+  for (Py_ssize_t i = 0; i < PyList_GET_SIZE(tens); ++i) {
+    PyObject *dict, *key;
+    int ver;
+    if (!PyArg_ParseTuple(PyList_GET_ITEM(tens, i), "O!Op", &PyDict_Type, &dict, &key, &ver)) { Py_DECREF(c); return nullptr; }
+    TensorSlot s{dict, key, nullptr, ver ? 0 : -1};
+    if (!read_tensor(dict, key, &s.data, &s.version)) {
+      if (!PyErr_Occurred()) PyErr_SetObject(PyExc_KeyError, key);
+      Py_DECREF(c);
+      return nullptr;
+    }
+    Py_INCREF(dict); Py_INCREF(key);
+    c->tensors->push_back(s);
+  }
+  return reinterpret_cast<PyObject*>(c);
+}
+
+// unchanged() -> bool
+PyObject* checker_unchanged(PyObject* self, PyObject*) {
+  Checker* c = reinterpret_cast<Checker*>(self);
+  for (const auto& m : *c->modules)
+    if (PyDict_GetItemWithError(m.dict, m.key) != m.expected) {
+      if (PyErr_Occurred()) return nullptr;
+      Py_RETURN_FALSE;
+    }
+  for (const auto& t : *c->tensors) {
+    const void* data;
+    int64_t version = t.version < 0 ? -1 : 0;
+    if (!read_tensor(t.dict, t.key, &data, &version) || data != t.data || version != t.version) {
+      if (PyErr_Occurred()) return nullptr;
+      Py_RETURN_FALSE;
+    }
+  }
+  Py_RETURN_TRUE;
+}
+
+PyMethodDef checker_methods[] = {{"unchanged", checker_unchanged, METH_NOARGS, "True if every module and tensor is as recorded."},
+                                 {nullptr, nullptr, 0, nullptr}};
+PyTypeObject CheckerType = {PyVarObject_HEAD_INIT(nullptr, 0) "m2_amd._param_check.Checker"};
+PyModuleDef module_def = {PyModuleDef_HEAD_INIT, "_param_check", nullptr, -1, nullptr};
+
+}  // namespace
+
+PyMODINIT_FUNC PyInit__param_check() {
+  CheckerType.tp_basicsize = sizeof(Checker);
+  CheckerType.tp_flags = Py_TPFLAGS_DEFAULT;
+  CheckerType.tp_new = checker_new;
+  CheckerType.tp_dealloc = checker_dealloc;
+  CheckerType.tp_methods = checker_methods;
+  if (PyType_Ready(&CheckerType) < 0) return nullptr;
+  PyObject* m = PyModule_Create(&module_def);
+  if (!m) return nullptr;
+  Py_INCREF(&CheckerType);
+  PyModule_AddObject(m, "Checker", reinterpret_cast<PyObject*>(&CheckerType));
+  return m;
+}

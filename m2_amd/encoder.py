@@ -25,7 +25,7 @@ from typing import List, Optional
 import torch
 import torch.nn as nn
 
-from . import ops
+from . import ops, schedule
 from .blockdiag import BlockdiagLinear
 from .config import M2BertConfig
 from .mixer import MonarchMixerSequenceMixing
@@ -144,19 +144,32 @@ class BertGatedLinearUnitMLP(nn.Module):
     # B = 4; per-layer deviation from the fp32 oracle 0.89 % instead of 0.78 % (max), end to end unchanged.
     bf16_presum = True
 
+    def mlp_route(self, M: int):
+        """(one-kernel MLP?, few rows?) for M rows.  Up to 512 rows the one-kernel MLP leaves most compute units idle
+        (21.5 us whatever the row count) and the two products as kernels of their own take 11 us at M = 128, 12.5 at 256,
+        19 at 512, 20 at 1024.  For few rows m2_blockdiag_glu_fwd has a kernel that beats the streaming one."""
+        d = self.config.hidden_size
+        fused = M > 512 and ops.mlp_fused_supported(d, self.config.intermediate_size, self.config.monarch_mlp_nblocks)
+        return fused, M * d <= 245760
+
+    def packed_mlp(self, wg: torch.Tensor, wo: torch.Tensor) -> torch.Tensor:
+        """The packed copy the one-kernel MLP streams: rebuilt whenever one of the bf16 copies has been rebuilt."""
+        if self._packed is None or self._packed[0] is not wg or self._packed[1] is not wo:
+            self._packed = (wg, wo, ops.mlp_fused_pack(wg, wo))
+        return self._packed[2]
+
+    def packed_glu(self, wg: torch.Tensor) -> torch.Tensor:
+        if self._packed_glu is None or self._packed_glu[0] is not wg:      # rebuilt with the bf16 copy
+            self._packed_glu = (wg, ops.glu_stream_pack(wg))
+        return self._packed_glu[1]
+
     def presum(self, a16: torch.Tensor) -> torch.Tensor:
         """a16 (M, d) bf16 -> wo(glu(a16)) + bias + a16, (M, d) fp32 (the LayerNorm input; bf16 with `bf16_presum`)."""
         sum_dtype = torch.bfloat16 if self.bf16_presum else torch.float32
-        # up to 512 rows the one-kernel MLP leaves most compute units idle (21.5 us whatever the row count); the two
-        # products as kernels of their own take 11 us at M = 128, 12.5 at 256, 19 at 512, 20 at 1024
-        if self.fuse_mlp and a16.shape[0] > 512 and ops.mlp_fused_supported(a16.shape[1], self.config.intermediate_size,
-                                                     self.config.monarch_mlp_nblocks):
+        if self.fuse_mlp and self.mlp_route(a16.shape[0])[0]:
             wg, wo = self.gated_layers.weight_bf16(), self.wo.weight_bf16()
-            # the packed copy the kernel streams: rebuilt whenever one of the bf16 copies has been rebuilt
-            if self._packed is None or self._packed[0] is not wg or self._packed[1] is not wo:
-                self._packed = (wg, wo, ops.mlp_fused_pack(wg, wo))
             return ops.mlp_fused(a16, wg, wo, self.wo.bias.detach().float().contiguous(), a16, out_dtype=sum_dtype,
-                                 packed=self._packed[2])
+                                 packed=self.packed_mlp(wg, wo))
         g = self.glu(a16)
         return ops.blockdiag_linear(g, self.wo.weight_bf16(), self.wo.bias.detach().float().contiguous(), a16,
                                     out_dtype=sum_dtype)
@@ -170,12 +183,9 @@ class BertGatedLinearUnitMLP(nn.Module):
     def glu(self, a16: torch.Tensor) -> torch.Tensor:
         """a16 (M, d) bf16 -> gelu(gate) * value of gated_layers(a16), (M, I) bf16."""
         wg = self.gated_layers.weight_bf16()
-        few = a16.shape[0] * a16.shape[1] <= 245760          # m2_blockdiag_glu_fwd has a kernel for few rows
-        if self.stream_glu and not few and ops.glu_stream_supported(a16.shape[1], self.config.intermediate_size,
-                                                        self.config.monarch_mlp_nblocks):
-            if self._packed_glu is None or self._packed_glu[0] is not wg:      # rebuilt with the bf16 copy
-                self._packed_glu = (wg, ops.glu_stream_pack(wg))
-            return ops.glu_stream(a16, wg, packed=self._packed_glu[1])
+        if self.stream_glu and not self.mlp_route(a16.shape[0])[1] and ops.glu_stream_supported(
+                a16.shape[1], self.config.intermediate_size, self.config.monarch_mlp_nblocks):
+            return ops.glu_stream(a16, wg, packed=self.packed_glu(wg))
         return ops.blockdiag_glu(a16, wg)
 
     def ln_params(self):
@@ -241,8 +251,9 @@ class BertLayer(nn.Module):
 
     def fused(self, h16: Optional[torch.Tensor], hT: Optional[torch.Tensor], B: int, L: int, want_f32: bool,
               spec: Optional[torch.Tensor] = None, spec_ready=None, after_core=None,
-              h32: Optional[torch.Tensor] = None):
-        """One layer of the fused schedule.  h16 (M,d) bf16, hT (d,M) f32 -> (f32 | None, bf16, (d,M) f32).
+              h32: Optional[torch.Tensor] = None, last: bool = False):
+        """One layer of the fused schedule.  h16 (M,d) bf16, hT (d,M) f32 -> (f32 | None, bf16, (d,M) f32); the two forms
+        for the next layer are None behind the last one.
         `spec`: this layer's filter spectra when the caller has generated them already (`spec_ready`: the event
         the current stream must wait for before reading them); `after_core()` is called once the mixer core
         has been enqueued."""
@@ -258,7 +269,7 @@ class BertLayer(nn.Module):
             after_core()
         a16 = at.project_out(y.view(d, B * L))                                       # (M, d)
         pre = at.hyena_training_additions        # the next layer then reads the fp32 form only
-        return self.mlp.normed(a16, want_f32, not pre, not pre)
+        return self.mlp.normed(a16, want_f32, not (pre or last), not (pre or last))
 
 
 class BertEncoder(nn.Module):
@@ -297,6 +308,11 @@ class BertEncoder(nn.Module):
         self.overlap_filters = None
         self._filter_stream = None
         self._filter_table = None
+        # native_schedule = True (default): forwards whose projections run on the library's own kernels (short ones) are
+        #   enqueued by three library calls instead of layer by layer (m2_amd/schedule.py); filter generation is then on
+        #   the main stream.  Same kernels, same results.
+        self.native_schedule = True
+        self._native_plans = {}
         # nn.Module.load_state_dict of a parent never calls a child's load_state_dict, but it does run the
         # post hooks of every module it recursed into: new weights drop the captured graphs
         self.register_load_state_dict_post_hook(BertEncoder._drop_graphs_after_load)
@@ -307,6 +323,7 @@ class BertEncoder(nn.Module):
 
     def _apply(self, fn, *args, **kwargs):
         self._graphs = {}
+        self._native_plans = {}
         return super()._apply(fn, *args, **kwargs)
 
     @staticmethod
@@ -326,6 +343,9 @@ class BertEncoder(nn.Module):
                     h16 = h32.to(torch.bfloat16)
                 if hT is None:
                     hT = h32.t().contiguous()
+                plan = schedule.stack_plan(self, None, B, L)
+                if plan is not None:
+                    return plan.run(B, all_layers, h16, hT)
             outs = []
             n = len(self.layer)
             o32 = h32
@@ -404,41 +424,50 @@ class BertEncoder(nn.Module):
                             ev.record(cur)
                             generate(i + 1, ev)
                 o32, h16, hT = layer.fused(h16, hT, B, L, want_f32=keep32, spec=spec, spec_ready=ready,
-                                           after_core=hook, h32=o32)
+                                           after_core=hook, h32=o32, last=i == n - 1)
                 if want:
                     outs.append(o32)
             if overlap and overlap != "inline-batched":
                 cur.wait_stream(self._filter_stream)
         return outs
 
-    def _batched_filter_plan(self, L: int):
-        """(pointer table of all layers' filters, [(first layer, count), ...]) when the filters of all layers are
-        generated by batched calls, else None."""
+    def _batched_filter_groups(self, L: int):
+        """[(first layer, count), ...] when the filters of all layers are generated by batched calls, else None."""
         if not self.batch_filters:
             return None
         mixers = [lay.attention for lay in self.layer]
         m0 = mixers[0]
+        f0 = m0.filter_fn
         if any(m.cache_filters for m in mixers):
             return None
-        same = all(m.d_model == m0.d_model and m.residual_long_conv == m0.residual_long_conv
-                   and m.bidirectional == m0.bidirectional and m.filter_fn.order == m0.filter_fn.order
-                   and m.filter_fn.emb_dim == m0.filter_fn.emb_dim and m.filter_fn.w_mod == m0.filter_fn.w_mod
-                   and m.filter_fn.modulation.shift == m0.filter_fn.modulation.shift for m in mixers)
+        alike = (m0.d_model, m0.residual_long_conv, m0.bidirectional, f0.order, f0.emb_dim, f0.w_mod, f0.modulation.shift)
+        for m in mixers:
+            f = m.filter_fn
+            if (m.d_model, m.residual_long_conv, m.bidirectional, f.order, f.emb_dim, f.w_mod, f.modulation.shift) != alike:
+                return None
         d, n = m0.d_model, len(mixers)
-        if not same or n * ops.lib.m2_filter_spectrum_bytes(d, L) > self.UPFRONT_MAX_BYTES:
+        if n * ops.lib.m2_filter_spectrum_bytes(d, L) > self.UPFRONT_MAX_BYTES:
             return None
+        per = max(1, ops.lib.m2_mixer_filters_workspace_bytes(1, 2 if m0.residual_long_conv else 1, L, d, f0.order))
+        group = max(1, min(n, self.FILTER_WORKSPACE_BYTES // per))
+        return [(i, min(group, n - i)) for i in range(0, n, group)]
+
+    def _batched_filter_plan(self, L: int):
+        """(pointer table of all layers' filters, [(first layer, count), ...]) when the filters of all layers are
+        generated by batched calls, else None."""
+        groups = self._batched_filter_groups(L)
+        if groups is None:
+            return None
+        mixers = [lay.attention for lay in self.layer]
+        m0 = mixers[0]
         entries = [m.filter_table_entry() for m in mixers]
         probe = (L,) + tuple(t.data_ptr() for filters, skips in entries for f in filters for v in f.values()
                              for t in (v if isinstance(v, list) else [v])) + tuple(b.data_ptr() for _, skips in entries
                                                                                    for b in skips)
         if self._filter_table is None or self._filter_table[0] != probe:
-            self._filter_table = (probe, ops.FilterTable([e[0] for e in entries], [e[1] for e in entries], L, d,
+            self._filter_table = (probe, ops.FilterTable([e[0] for e in entries], [e[1] for e in entries], L, m0.d_model,
                                                          m0.filter_fn.order, m0.filter_fn.emb_dim))
-        table = self._filter_table[1]
-        fpm = table.fpm
-        per = max(1, ops.lib.m2_mixer_filters_workspace_bytes(1, fpm, L, d, table.order))
-        group = max(1, min(n, self.FILTER_WORKSPACE_BYTES // per))
-        return table, [(i, min(group, n - i)) for i in range(0, n, group)]
+        return self._filter_table[1], groups
 
     def _run_graphed(self, h32: Optional[torch.Tensor], B: int, L: int, all_layers: bool,
                      h16: Optional[torch.Tensor] = None, hT: Optional[torch.Tensor] = None) -> List[torch.Tensor]:
@@ -525,6 +554,25 @@ class BertModel(nn.Module):
         self.validate_ids = True
         self.register_load_state_dict_post_hook(lambda module, keys: module.encoder.reset_graphs())
 
+    def _run_native(self, ids, tt, pos, all_layers: bool):
+        """Embeddings and layers by the native schedule, or None where it does not apply (other dtypes, indices the
+        embedding call would refuse, ...: the Python schedule then runs, or reports the error)."""
+        B, L = ids.shape
+        emb = self.embeddings
+        if (emb.training and emb.dropout.p > 0) or ids.dtype != torch.int64 or not ids.is_cuda:
+            return None
+        if tt is not None or pos is not None:
+            if any(t is not None and (t.dtype != torch.int64 or not t.is_cuda) for t in (tt, pos)):
+                return None
+            tt = None if tt is None else tt.expand(B, L).contiguous()
+            pos = None if pos is None else pos.expand(B, L).contiguous()
+        if pos is not None and not emb.use_positional_encodings:
+            return None
+        if pos is None and emb.use_positional_encodings and emb.position_embeddings.weight.shape[0] < L:
+            return None
+        plan = schedule.stack_plan(self.encoder, emb, B, L)
+        return None if plan is None else plan.run(B, all_layers, None, None, ids.contiguous(), tt, pos)
+
     def get_input_embeddings(self):
         return self.embeddings.word_embeddings
 
@@ -540,6 +588,9 @@ class BertModel(nn.Module):
         pre_norm = self.encoder.layer[0].attention.hyena_training_additions
 
         def run(ids, tt, pos):
+            outs = self._run_native(ids, tt, pos, all_layers)
+            if outs is not None:
+                return outs
             # the embedding LayerNorm writes the bf16 and channel-major forms the first layer reads itself
             # (or the fp32 form when the layers start with their own LayerNorm)
             h32, h16, hT = self.embeddings.forward_forms(ids, tt, pos, want_f32=pre_norm, want_bf16=not pre_norm,
@@ -572,12 +623,13 @@ class BertModel(nn.Module):
                     dst.copy_(src)
             graph.replay()
             outs = [o.clone() for o in static_out]
-        if self.validate_ids and not torch.cuda.is_current_stream_capturing():
-            self.embeddings.check_indices()
         enc = [o.view(B, L, -1) for o in outs]
         pooled = None
         if self.pooler is not None:
             if attention_mask is None:
                 attention_mask = torch.ones_like(input_ids)
             pooled = self.pooler(enc[-1], mask=attention_mask)
+        # last, behind everything that is to be enqueued: it waits for the stream
+        if self.validate_ids and not torch.cuda.is_current_stream_capturing():
+            self.embeddings.check_indices()
         return (enc if output_all_encoded_layers else enc[-1]), pooled

@@ -157,6 +157,27 @@ class FilterTable:
         self.table = torch.tensor(rows, dtype=torch.int64).to(dev)
         self.skip = torch.tensor(skip_row, dtype=torch.int64).to(dev)
 
+    @classmethod
+    def of_rows(cls, rows: Sequence[Sequence[Optional[Tensor]]], skips: Sequence[Tensor], fpm: int, L: int, d: int, order: int,
+                emb_dim: int) -> "FilterTable":
+        """The same table from the tensors themselves: per filter z, t, freq, deltas and the seven of either MLP (None for a
+        missing reverse one), fp32, contiguous and of the shapes of their modules; one skip weight per filter."""
+        shapes = [(order, emb_dim), (order,), (order, order), (order,), (order, order), (order,), (d, order)] * 2
+        for row in rows:
+            if row[0].numel() < L * emb_dim or row[0].shape[-1] != emb_dim or row[1].numel() < L or row[2].numel() != order \
+                    or row[3].numel() != d or any(t is not None and t.shape != s for t, s in zip(row[4:], shapes)):
+                raise ValueError("filter tensors of unexpected shapes")
+        if any(b.shape != (d,) for b in skips):
+            raise ValueError("skip weights of unexpected shapes")
+        self = cls.__new__(cls)
+        self.nmixers, self.fpm = len(rows) // fpm, fpm
+        self.L, self.d, self.order, self.emb_dim = L, d, order, emb_dim
+        self.keep = [t for row in rows for t in row if t is not None] + list(skips)
+        both = torch.tensor([[0 if t is None else t.data_ptr() for t in row] + [b.data_ptr()] for row, b in zip(rows, skips)],
+                            dtype=torch.int64).to(rows[0][0].device)
+        self.table, self.skip = both[:, :-1].contiguous(), both[:, -1].contiguous()
+        return self
+
     def spectrum_floats(self) -> int:
         return lib.m2_filter_spectrum_bytes(self.d, self.L) // 4
 

@@ -1,0 +1,187 @@
+"""The native schedule of an encoder: embeddings, filter generation and all layers enqueued by three library calls.
+
+`BertEncoder._run_layers` walks over its layers in Python, about 170 us of host time per layer and 0.2 ms more for the
+filter table, which is what a short forward then costs whatever the GPU does (L = 128, B = 1: 2.4 ms for 0.75 ms of
+kernels).  A `StackPlan` holds what the calls need: the layers' device pointers, the bf16 and packed copies of the
+weights, the filter pointer table.  It is made once and, before each use, compared tensor by tensor with what the modules
+hold now (address, and version counter for the weights that copies were made from): `_param_check.Checker`.
+
+Same kernels in the same order on the current stream as the Python schedule, hence the same bits.  It serves row counts
+whose projections run on the library's own kernels; larger forwards, whose host time hides behind the GPU's, and encoders
+with per-layer options stay with the Python schedule.
+"""
+from __future__ import annotations
+
+import ctypes
+from typing import List, Optional
+
+import torch
+
+from . import ops
+from ._lib import LayerParams, check, lib
+
+try:
+    from . import _param_check
+except ImportError as e:
+    raise ImportError("m2_amd/_param_check.so is missing or does not fit this torch: build it with `python m2_amd/build.py`") from e
+
+
+_IN_PLACE, _COPIED = False, True       # read at its address / a copy was made from it: compare the version too
+
+
+class StackPlan:
+    """Device pointers of an encoder's layers (and of the embeddings in front of it) for one length and MLP route."""
+
+    def __init__(self, encoder, embeddings, L: int, fused_mlp: bool, few_rows: bool):
+        # (dict, key) of every module and (dict, key, compare the version) of every tensor the plan depends on
+        mods, tens = [(encoder._modules, "layer")], []
+
+        def child(mod, key):
+            mods.append((mod._modules, key))
+            return mod._modules[key]
+
+        def tensor(mod, key, how=_IN_PLACE):
+            where = mod._parameters if key in mod._parameters else mod._buffers
+            tens.append((where, key, how))
+            t = where[key]
+            if not (t.is_cuda and t.dtype == torch.float32 and t.is_contiguous()):
+                raise ValueError("parameters that are not plain fp32")
+            return t
+
+        stack = encoder._modules["layer"]
+        n = len(stack._modules)
+        self.layers = n
+        self.array = (LayerParams * n)()
+        self.keep: List[torch.Tensor] = []
+        rows, skips = [], []
+        for i, key in enumerate(stack._modules):
+            lay = child(stack, key)
+            at, mlp = child(lay, "attention"), child(lay, "mlp")
+            for name in ("filter_fn", "filter_fn2")[:2 if at.residual_long_conv else 1]:
+                f = child(at, name)
+                skips.append(tensor(f, "bias"))
+                emb = child(f, "pos_emb")
+                fwd = child(f, "implicit_filter")
+                row = [tensor(emb, "z"), tensor(emb, "t"), tensor(child(fwd, "1"), "freq"), tensor(child(f, "modulation"), "deltas")]
+                for seq in (fwd, child(f, "implicit_filter_rev") if at.bidirectional else None):
+                    if seq is None:
+                        row += [None] * 7
+                        continue
+                    for k in "024":
+                        lin = child(seq, k)
+                        row += [tensor(lin, "weight"), tensor(lin, "bias")]
+                    row.append(tensor(child(seq, "6"), "weight"))
+                rows.append(row)
+            lin_in, lin_out, short = child(at, "in_linear"), child(at, "out_linear"), child(at, "short_filter")
+            gated, wo, ln = child(mlp, "gated_layers"), child(mlp, "wo"), child(mlp, "layernorm")
+            in_place = [tensor(lin_in, "bias"), tensor(lin_out, "bias"), tensor(short, "weight"), tensor(short, "bias"),
+                        tensor(wo, "bias"), tensor(ln, "weight"), tensor(ln, "bias")]
+            for m in (lin_in, lin_out, gated, wo):
+                tensor(m, "weight", _COPIED)
+            w_in, w_out = at._cast("in_w", lin_in.weight, torch.bfloat16), at._cast("out_w", lin_out.weight, torch.bfloat16)
+            wg16, wo16 = gated.weight_bf16(), wo.weight_bf16()
+            self.keep += [w_in, w_out, wg16, wo16]
+            p = self.array[i]
+            p.in_w, p.out_w, p.w_gated, p.w_out = w_in.data_ptr(), w_out.data_ptr(), wg16.data_ptr(), wo16.data_ptr()
+            (p.in_b, p.out_b, p.short_w, p.short_b, p.wo_b, p.ln_gamma, p.ln_beta) = [t.data_ptr() for t in in_place]
+            p.residual = 1 if at.residual_long_conv else 0
+            if i == 0:
+                f0 = at.filter_fn
+                self.d, self.I, self.nb = at.d_model, mlp.config.intermediate_size, mlp.config.monarch_mlp_nblocks
+                self.eps = float(ln.eps)
+                self.w_mod, self.shift = float(f0.w_mod), float(f0.modulation.shift)
+                stream_glu = not fused_mlp and not few_rows and ops.glu_stream_supported(self.d, self.I, self.nb)
+            elif (mlp.config.intermediate_size, mlp.config.monarch_mlp_nblocks, float(ln.eps)) != (self.I, self.nb, self.eps):
+                raise ValueError("layers that differ")
+            if fused_mlp:
+                self.keep.append(mlp.packed_mlp(wg16, wo16))
+                p.mlp_packed = self.keep[-1].data_ptr()
+            elif stream_glu:
+                self.keep.append(mlp.packed_glu(wg16))
+                p.glu_packed = self.keep[-1].data_ptr()
+        self.table = ops.FilterTable.of_rows(rows, skips, len(rows) // n, L, self.d, f0.order, f0.emb_dim)
+        self.embed = None
+        if embeddings is not None:
+            e = embeddings
+            word, typ = tensor(child(e, "word_embeddings"), "weight"), tensor(child(e, "token_type_embeddings"), "weight")
+            pos = tensor(child(e, "position_embeddings"), "weight") if e.use_positional_encodings else None
+            ln = child(e, "LayerNorm")
+            g, b = tensor(ln, "weight"), tensor(ln, "bias")
+            tens.append((e._buffers, "_bad_index", _IN_PLACE))
+            if any(t is not None and (t.dim() != 2 or t.shape[1] != self.d) for t in (word, typ, pos)) or g.shape != (self.d,):
+                raise ValueError("embedding tables of another width")
+            self.embed = (word.data_ptr(), typ.data_ptr(), None if pos is None else pos.data_ptr(), word.shape[0], typ.shape[0],
+                          0 if pos is None else pos.shape[0], g.data_ptr(), b.data_ptr(), float(ln.eps))
+            self.bad_index = e._bad_index.data_ptr()
+        self.checker = _param_check.Checker(mods, tens)
+        self.L = L
+        self.spec_bytes = lib.m2_filter_spectrum_bytes(self.d, L)
+        self.filter_ws = lib.m2_mixer_filters_workspace_bytes(n, self.table.fpm, L, self.d, self.table.order)
+
+    def __reduce__(self):                    # a plan belongs to its modules: copies and pickles of them make their own
+        return type(None), ()
+
+    def run(self, B: int, all_layers: bool, h16: Optional[torch.Tensor], hT: Optional[torch.Tensor], ids=None, tt=None, pos=None):
+        """Enqueues the stack on the current stream; input either as h16 / hT or as token ids for the embeddings."""
+        n, L, d = self.layers, self.L, self.d
+        M = B * L
+        dev = ids.device if ids is not None else h16.device
+        stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+        up = lambda v: (v + 255) & ~255      # noqa: E731
+        o_spec = up(self.filter_ws)
+        o_act = o_spec + up(n * self.spec_bytes)
+        o_in = o_act + up(lib.m2_encoder_layers_workspace_bytes(M, d, self.I))
+        ws = torch.empty(o_in + (up(2 * M * d) + 4 * M * d if ids is not None else 0), dtype=torch.uint8, device=dev)
+        base = ws.data_ptr()
+        outs = [torch.empty(M, d, dtype=torch.float32, device=dev) for _ in range(n if all_layers else 1)]
+        ptrs = (ctypes.c_void_p * n)()
+        for i, o in enumerate(outs):
+            ptrs[n - len(outs) + i] = o.data_ptr()
+        t = self.table
+        check(lib.m2_mixer_filters_fwd(t.table.data_ptr(), t.skip.data_ptr(), n, t.fpm, L, d, t.order, t.emb_dim, self.w_mod, self.shift,
+                                       base, base + o_spec, stream))
+        if ids is not None:
+            p16, pT = base + o_in, base + o_in + up(2 * M * d)
+            w, ty, pe, nw, nt, npos, g, b, eps = self.embed
+            check(lib.m2_embed_layernorm_fwd(ids.data_ptr(), None if tt is None else tt.data_ptr(), None if pos is None else pos.data_ptr(),
+                                             w, ty, pe, nw, nt, npos, g, b, eps, None, p16, pT, self.bad_index, B, L, d, stream))
+        else:
+            p16, pT = h16.data_ptr(), hT.data_ptr()
+        check(lib.m2_encoder_layers_fwd(self.array, n, base + o_spec, p16, pT, ptrs, base + o_act, B, L, d, self.I, self.nb, self.eps, stream))
+        return outs
+
+
+def stack_plan(encoder, embeddings, B: int, L: int) -> Optional[StackPlan]:
+    """The plan for (B, L), made or re-used, or None where the Python schedule serves."""
+    if not encoder.native_schedule or not encoder.batch_filters or encoder.overlap_filters not in (None, False):
+        return None
+    layers = encoder._modules["layer"]._modules.values()
+    M = B * L
+    for lay in layers:
+        at, mlp = lay._modules["attention"], lay._modules["mlp"]
+        if (at.cache_filters or at.hyena_training_additions or mlp.fuse_wo_layernorm or not mlp.fuse_mlp or not mlp.bf16_presum
+                or not mlp.stream_glu):
+            return None
+    d = at.d_model
+    if at.in_linear.weight.dtype != torch.float32 or not at.in_linear.weight.is_cuda:
+        return None
+    if not ops.own_to_channels(M, d) or not ops.own_from_channels(M, d):
+        return None
+    fused, few = mlp.mlp_route(M)
+    key = (L, fused, few, embeddings is not None)
+    plan = encoder._native_plans.get(key)
+    if plan is not None and plan.layers == len(layers) and plan.checker.unchanged():
+        return plan
+    if torch.cuda.is_current_stream_capturing():
+        return None                                  # the filter table is copied from the host: not inside a capture
+    groups = encoder._batched_filter_groups(L)       # the same rule: layers alike, spectra small enough, ...
+    if groups is None or len(groups) != 1:
+        return None
+    try:
+        plan = StackPlan(encoder, embeddings, L, fused, few)
+    except ValueError:
+        return None
+    if len(encoder._native_plans) >= 8:              # a handful of lengths: drop the oldest
+        encoder._native_plans.pop(next(iter(encoder._native_plans)))
+    encoder._native_plans[key] = plan
+    return plan

@@ -1,0 +1,142 @@
+"""The native schedule of an encoder (m2_amd/schedule.py) against the Python schedule: the same bits in every form, and plans
+that follow their modules."""
+import copy
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _model(cfg, gpu, seed, **kw):
+    import m2_amd
+    model = m2_amd.BertModel(cfg, **kw)
+    model.load_state_dict(m2_amd.seeded_state_dict(cfg, seed))
+    return model.to(gpu).eval()
+
+
+def _both(model, *args, **kw):
+    """(native result, Python-schedule result); the native one must really have run."""
+    model.encoder.native_schedule = True
+    got = model(*args, **kw)
+    assert any(p.checker.unchanged() for p in model.encoder._native_plans.values())
+    model.encoder.native_schedule = False
+    want = model(*args, **kw)
+    model.encoder.native_schedule = True
+    return got, want
+
+
+def _ids(cfg, B, L, seed, gpu):
+    return torch.randint(0, cfg.vocab_size, (B, L), generator=torch.Generator().manual_seed(seed)).to(gpu)
+
+
+# few rows, one-kernel MLP, streaming GLU with and without few rows, l_max beyond L
+@pytest.mark.parametrize("helper,l_max,B,L", [("m2_bert_80m", 128, 1, 128), ("m2_bert_80m", 512, 3, 512), ("m2_bert_80m", 1024, 5, 256),
+                                              ("m2_bert_110m", 128, 1, 128), ("m2_bert_large", 256, 3, 256), ("m2_bert_341m", 128, 2, 128)])
+def test_native_schedule_matches_python_schedule(gpu, helper, l_max, B, L):
+    import m2_amd
+    cfg = getattr(m2_amd, helper)(l_max)
+    cfg.num_hidden_layers = 3
+    model = _model(cfg, gpu, 5)
+    ids = _ids(cfg, B, L, 6, gpu)
+    mask = torch.ones_like(ids)
+    (seq, pooled), (wseq, wpooled) = _both(model, ids, attention_mask=mask)
+    assert torch.equal(seq, wseq) and torch.equal(pooled, wpooled)
+    (all_, _), (wall, _) = _both(model, ids, output_all_encoded_layers=True)
+    assert len(all_) == 3 and all(torch.equal(a, b) for a, b in zip(all_, wall))
+    tt = (ids % 2).contiguous()
+    pos = torch.arange(L, device=gpu).flip(0)[None]
+    (a, _), (b, _) = _both(model, ids, token_type_ids=tt, position_ids=pos)
+    assert torch.equal(a, b) and not torch.equal(a, seq)
+    h = torch.randn(B, L, cfg.hidden_size, generator=torch.Generator().manual_seed(7)).to(gpu)
+    outs = model.encoder(h)
+    model.encoder.native_schedule = False
+    want = model.encoder(h)
+    assert len(outs) == 3 and all(torch.equal(a, b) for a, b in zip(outs, want))
+
+
+def test_plans_follow_their_modules(gpu):
+    import m2_amd
+    cfg = m2_amd.m2_bert_80m(128)
+    cfg.num_hidden_layers = 2
+    model = _model(cfg, gpu, 8)
+    ids = _ids(cfg, 2, 128, 9, gpu)
+    (prev, _), _ = _both(model, ids)
+    lay = model.encoder.layer[1]
+
+    def changed(what):
+        nonlocal prev
+        (got, _), (want, _) = _both(model, ids)
+        assert torch.equal(got, want) and not torch.equal(got, prev), what
+        prev = got
+
+    with torch.no_grad():
+        lay.attention.out_linear.weight.mul_(1.5)                              # in place: a copy has to be made again
+        changed("weight in place")
+        lay.mlp.wo.bias.add_(0.5)                                              # read in place
+        changed("bias in place")
+        lay.attention.filter_fn.implicit_filter[6].weight.mul_(2.0)
+        changed("filter in place")
+        lay.mlp.gated_layers.weight = torch.nn.Parameter(lay.mlp.gated_layers.weight.detach() * 1.2)
+        changed("parameter replaced")
+        lay.attention.in_linear.weight.data = lay.attention.in_linear.weight.data * 1.1
+        changed("data replaced")
+    new = torch.nn.LayerNorm(768, eps=cfg.layer_norm_eps).to(gpu)
+    torch.nn.init.constant_(new.weight, 0.7)
+    lay.mlp.layernorm = new
+    changed("module replaced")
+    model.embeddings.word_embeddings = torch.nn.Embedding.from_pretrained(model.embeddings.word_embeddings.weight.detach() * 0.5)
+    changed("embedding replaced")
+    model.load_state_dict(m2_amd.seeded_state_dict(cfg, 10))
+    changed("state dict loaded")
+    model.encoder.layer.append(copy.deepcopy(lay))                             # one more layer
+    changed("layer added")
+    fresh = _model(cfg, gpu, 10)
+    want, _ = fresh(ids)
+    got, _ = copy.deepcopy(fresh)(ids)                                         # a copy makes plans of its own
+    assert torch.equal(got, want)
+    lay.mlp.bf16_presum = False                                                # an option the native schedule has no path for
+    opt, _ = model(ids)
+    assert not torch.equal(opt, prev)
+
+
+def test_native_schedule_in_a_graph_and_on_streams(gpu):
+    """Captured and replayed with other work in between; eager calls on two streams at once."""
+    import m2_amd
+    cfg = m2_amd.m2_bert_80m(256)
+    cfg.num_hidden_layers = 2
+    model, graphed = _model(cfg, gpu, 11), _model(cfg, gpu, 11, use_hip_graph=True)
+    for it in range(4):
+        ids = _ids(cfg, 3, 256, 20 + it, gpu)
+        want, _ = model(ids)
+        scratch = torch.randn(512, 512, device=gpu) @ torch.randn(512, 512, device=gpu)
+        got, _ = graphed(ids)
+        torch.cuda.synchronize()
+        assert torch.equal(got, want), it
+        del scratch
+    model.validate_ids = False
+    batches = [_ids(cfg, 3, 256, 30 + i, gpu) for i in range(6)]
+    wants = [model(b)[0].clone() for b in batches]
+    torch.cuda.synchronize()
+    streams = [torch.cuda.Stream() for _ in range(2)]
+    outs = []
+    for i, b in enumerate(batches):
+        with torch.cuda.stream(streams[i % 2]):
+            outs.append(model(b)[0])
+    torch.cuda.synchronize()
+    assert all(torch.equal(a, b) for a, b in zip(outs, wants))
+
+
+def test_bad_indices_are_reported_by_the_native_schedule(gpu):
+    import m2_amd
+    cfg = m2_amd.m2_bert_80m(128)
+    cfg.num_hidden_layers = 1
+    model = _model(cfg, gpu, 12)
+    ids = _ids(cfg, 1, 128, 13, gpu)
+    model(ids)
+    assert model.encoder._native_plans
+    ids[0, 5] = cfg.vocab_size
+    with pytest.raises(IndexError):
+        model(ids)
+    ids[0, 5] = 0
+    model(ids)
