@@ -469,6 +469,11 @@ class BertEncoder(nn.Module):
                                                          m0.filter_fn.order, m0.filter_fn.emb_dim))
         return self._filter_table[1], groups
 
+    def _graph_reads(self) -> tuple:
+        """What a graph captured just now reads beside parameters: pointer tables and packed weights, which forwards of
+        other lengths replace here and which therefore have to live as long as the graph."""
+        return self._filter_table, tuple(self._native_plans.values())
+
     def _run_graphed(self, h32: Optional[torch.Tensor], B: int, L: int, all_layers: bool,
                      h16: Optional[torch.Tensor] = None, hT: Optional[torch.Tensor] = None) -> List[torch.Tensor]:
         given = [t for t in (h32, h16, hT) if t is not None]
@@ -485,9 +490,9 @@ class BertEncoder(nn.Module):
             graph = torch.cuda.CUDAGraph()
             with torch.cuda.graph(graph):
                 static_out = self._run_layers(static[0], B, L, all_layers, h16=static[1], hT=static[2])
-            entry = (graph, static, static_out)
+            entry = (graph, static, static_out, self._graph_reads())
             self._graphs[key] = entry
-        graph, static, static_out = entry
+        graph, static, static_out, _ = entry
         for dst, src in zip(static, (h32, h16, hT)):
             if dst is not None:
                 dst.copy_(src)
@@ -615,9 +620,9 @@ class BertModel(nn.Module):
                 graph = torch.cuda.CUDAGraph()
                 with torch.cuda.graph(graph):
                     static_out = run(*static)
-                entry = (graph, static, static_out)
+                entry = (graph, static, static_out, self.encoder._graph_reads())
                 self.encoder._graphs[key] = entry
-            graph, static, static_out = entry
+            graph, static, static_out, _ = entry
             for dst, src in zip(static, given):
                 if dst is not None:
                     dst.copy_(src)

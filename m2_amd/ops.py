@@ -173,9 +173,10 @@ class FilterTable:
         self.nmixers, self.fpm = len(rows) // fpm, fpm
         self.L, self.d, self.order, self.emb_dim = L, d, order, emb_dim
         self.keep = [t for row in rows for t in row if t is not None] + list(skips)
-        both = torch.tensor([[0 if t is None else t.data_ptr() for t in row] + [b.data_ptr()] for row, b in zip(rows, skips)],
-                            dtype=torch.int64).to(rows[0][0].device)
-        self.table, self.skip = both[:, :-1].contiguous(), both[:, -1].contiguous()
+        # two blocking copies from the host: nothing is left on this stream that a call on another one would have to wait for
+        dev = rows[0][0].device
+        self.table = torch.tensor([[0 if t is None else t.data_ptr() for t in row] for row in rows], dtype=torch.int64).to(dev)
+        self.skip = torch.tensor([b.data_ptr() for b in skips], dtype=torch.int64).to(dev)
         return self
 
     def spectrum_floats(self) -> int:

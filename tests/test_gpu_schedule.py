@@ -140,3 +140,30 @@ def test_bad_indices_are_reported_by_the_native_schedule(gpu):
         model(ids)
     ids[0, 5] = 0
     model(ids)
+
+
+def test_a_graph_keeps_what_it_reads(gpu):
+    """Forwards of other lengths replace the pointer tables of plans and schedules: a captured graph holds on to its own."""
+    import m2_amd
+    cfg = m2_amd.m2_bert_80m(512)
+    cfg.num_hidden_layers = 1
+    for native in (True, False):
+        model = _model(cfg, gpu, 14, use_hip_graph=True)
+        model.encoder.native_schedule = native
+        ids = _ids(cfg, 2, 128, 15, gpu)
+        first, _ = model(ids)
+        table = next(iter(model.encoder._native_plans.values())).table if native else model.encoder._filter_table[1]
+        held, address = table.table, table.table.data_ptr()
+        gone = __import__("weakref").ref(table)
+        del table, held
+        model.encoder._native_plans.clear()
+        model.encoder._filter_table = None
+        for L in (256, 512):
+            model(_ids(cfg, 2, L, L, gpu))
+        assert gone() is not None and gone().table.data_ptr() == address
+        again, _ = model(ids)
+        assert torch.equal(again, first)
+        model.encoder.reset_graphs()
+        model.encoder._native_plans.clear()
+        model.encoder._filter_table = None
+        assert gone() is None
