@@ -275,6 +275,27 @@ int m2_embed_layernorm_fwd(const long long* input_ids, const long long* token_ty
                            int d, void* stream);
 
 /* ---------------------------------------------------------------------------------------------
+ * fp32 matrix products on the bf16 matrix cores (the dense projections and the block-diagonal MLP of fp32 callers outside
+ * autocast: bert/src/mm/monarch_mixer_sequence_mixer.py:108,152, bert/src/mm/blockdiag_multiply.py:19-60).  An operand is
+ * split into three bf16 parts per value, x = hi + mid + lo; the products use all terms down to 2^-24 relative and accumulate
+ * in fp32.  A split operand of `rows` rows of `nblocks` blocks of `p` values takes m2_split_bytes (0: unsupported): p a
+ * multiple of 4, below 4 GB.
+ *   m2_split_rows_fwd      x (M, nblocks p) fp32 -> parts; channel_major: NULL or (p, M) fp32, receives x^T (nblocks 1, M % 4 == 0)
+ *   m2_split_channels_fwd  x (K, M) fp32 -> parts of x^T; M % 4 == 0
+ * Weights (nblocks, q, p) are split as nblocks q rows of one block.
+ *   m2_split_to_channels_fwd  out (N, M) fp32 = w x^T; M % 4 == 0
+ *   m2_split_linear_fwd       out (M, nblocks q) fp32 = blockdiag(x, w) + bias + residual (either may be NULL); q % 4 == 0
+ *   m2_split_glu_fwd          parts of gelu(h[:, :I]) * h[:, I:], h = blockdiag(x, w), I = nblocks q / 2; q % 64 == 0
+ * ------------------------------------------------------------------------------------------- */
+size_t m2_split_bytes(int rows, int nblocks, int p);
+int m2_split_rows_fwd(const float* x, void* out, float* channel_major, int M, int nblocks, int p, void* stream);
+int m2_split_channels_fwd(const float* x, void* out, int M, int K, void* stream);
+int m2_split_to_channels_fwd(const void* xs, const void* ws, float* out, int M, int N, int K, void* stream);
+int m2_split_linear_fwd(const void* xs, const void* ws, const float* bias, const float* residual, float* out, int M, int nblocks,
+                        int p, int q, void* stream);
+int m2_split_glu_fwd(const void* xs, const void* ws, void* out, int M, int nblocks, int p, int q, void* stream);
+
+/* ---------------------------------------------------------------------------------------------
  * The fused schedule of a stack of encoder layers (BertEncoder.forward, bert/src/bert_layers.py:691-813, with
  * BertLayer :575-599), bf16 GEMMs, enqueued by one call.  `layers` is a HOST array of device pointers; `spectra` holds
  * the layers' filter spectra one after the other (m2_mixer_filters_fwd); `h16` (M, d) bf16 and `h_channel_major` (d, M) fp32

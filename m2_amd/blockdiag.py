@@ -60,6 +60,7 @@ class BlockdiagLinear(nn.Module):
             self.register_parameter("bias", None)
         self.reset_parameters()
         self._w16 = None
+        self._parts = ops.WeightParts()
 
     def reset_parameters(self) -> None:
         # first block-row of a dense Kaiming-uniform matrix, rescaled for the sparsity
@@ -96,7 +97,11 @@ class BlockdiagLinear(nn.Module):
                 bias = F.pad(bias, (0, self.out_features_extended - self.out_features))
             bias = bias.contiguous()
         nb, q, p = self.weight.shape
-        if _fp32_path(x) and p % 8 == 0:
+        M = x.numel() // x.shape[-1]
+        if _fp32_path(x) and p % 8 == 0 and ops.split_supported(M, nb, p, q):
+            parts, _ = ops.split_rows(x.reshape(-1, self.in_features_extended).contiguous(), nb)
+            out = ops.split_linear(parts, self._parts.get(self.weight), M, nb, p, q, bias)
+        elif _fp32_path(x) and p % 8 == 0:
             out = ops.blockdiag_linear_f32(x.reshape(-1, self.in_features_extended).contiguous(),
                                            self.weight.detach().float().contiguous(), bias)
         else:

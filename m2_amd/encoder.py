@@ -188,6 +188,17 @@ class BertGatedLinearUnitMLP(nn.Module):
             return ops.glu_stream(a16, wg, packed=self.packed_glu(wg))
         return ops.blockdiag_glu(a16, wg)
 
+    def _fp32_parts(self, x: torch.Tensor) -> bool:
+        """The fp32 MLP as two products by parts, the gated one with its GELU: blocks of whole 32-value chunks between the two,
+        nothing padded, and the submodules just what they are built as (no hooks, no other activation)."""
+        gl, wo, act = self.gated_layers, self.wo, self.act
+        (nb, q, p), M = gl.weight.shape, x.shape[0]
+        I, d = self.config.intermediate_size, x.shape[1]
+        if any(m._forward_hooks or m._forward_pre_hooks for m in (gl, wo, act)) or type(act) is not nn.GELU or act.approximate != "none":
+            return False
+        return (nb % 2 == 0 and p % 8 == 0 and q % 64 == 0 and nb * p == d and nb * q == 2 * I and tuple(wo.weight.shape) == (nb, d // nb, I // nb)
+                and gl.bias is None and wo.bias is not None and ops.split_supported(M, nb, p, q) and ops.split_supported(M, nb, I // nb, d // nb))
+
     def ln_params(self):
         return self.layernorm.weight.detach().float(), self.layernorm.bias.detach().float(), self.layernorm.eps
 
@@ -216,6 +227,15 @@ class BertGatedLinearUnitMLP(nn.Module):
         gamma, beta, eps = self.ln_params()
         if hidden_states.dtype == torch.float32 and not torch.is_autocast_enabled():
             x = hidden_states.reshape(-1, shape[-1]).contiguous()
+            if self._fp32_parts(x):
+                M, (nb, q, p), q2 = x.shape[0], self.gated_layers.weight.shape, self.wo.weight.shape[1]
+                if x.data_ptr() % 16:
+                    x = x.clone()
+                g = ops.split_glu(ops.split_rows(x, nb)[0], self.gated_layers._parts.get(self.gated_layers.weight), M, nb, p, q)
+                s = ops.split_linear(g, self.wo._parts.get(self.wo.weight), M, nb, q // 2, q2,
+                                     self.wo.bias.detach().float().contiguous(), x)
+                o32, _, _ = ops.layernorm(s, gamma, beta, eps, want_f32=True)
+                return o32.view(shape)
             h = self.gated_layers(x)                                   # fp32 block-diagonal kernel
             I = self.config.intermediate_size
             g = self.act(h[:, :I]) * h[:, I:]

@@ -8,6 +8,8 @@ Data flow of `forward(u)`, u (B, L, d):
     y (d, B*L)      = m2_mixer_core_fwd(xproj, u^T, short_filter, spec)
     out (B*L, d)    = y^T @ out_linear.weight^T + bias     own kernel or library GEMM, by size
 
+(fp32: own kernels on three bf16 parts per value; the pass that splits u also writes u^T)
+
 so the three `transpose` passes of the reference disappear into GEMM operand orientation.  With fp32
 input outside autocast everything is fp32; with bf16 input or under CUDA autocast the projections
 and the stored activations are bf16 while the FFT convolution stays fp32.
@@ -58,6 +60,7 @@ class MonarchMixerSequenceMixing(nn.Module):
         self.short_filter = nn.Conv1d(in_channels=total_width, out_channels=total_width, kernel_size=3,
                                       groups=total_width, padding=2)
         self._cast_cache = {}
+        self._in_parts, self._out_parts = ops.WeightParts(), ops.WeightParts()
         self.cache_filters = False
         self._spec_cache = None
         self._filter_table = None
@@ -137,7 +140,8 @@ class MonarchMixerSequenceMixing(nn.Module):
         """x (M, d) -> in_linear.weight @ x^T without the bias, (3d, M) channel-major, in x's dtype (bf16 or fp32)."""
         M, d = x.shape
         w = self._cast("in_w", self.in_linear.weight, x.dtype)
-        if x.dtype == torch.bfloat16 and x.data_ptr() % 16 == 0 and ops.own_to_channels(M, d):
+        own = not (x.requires_grad and torch.is_grad_enabled())          # (the library call refuses those)
+        if own and x.dtype == torch.bfloat16 and x.data_ptr() % 16 == 0 and ops.own_to_channels(M, d):
             return ops.dense_to_channels(x, w)
         # Written as x @ W^T into the transposed view of the output: the same product as W @ x^T, for which the library
         # picks a faster kernel (126 against 144 us at M = 32768, d = 768)
@@ -145,12 +149,18 @@ class MonarchMixerSequenceMixing(nn.Module):
         torch.mm(x, w.t(), out=out.t())
         return out
 
+    def _fp32_parts(self, M: int) -> bool:
+        return M % 4 == 0 and ops.split_supported(M, 1, self.d_model, 3 * self.d_model)
+
     def project_out(self, y: torch.Tensor) -> torch.Tensor:
         """y (d, M) channel-major -> y^T @ out_linear.weight^T + bias, (M, d), in y's dtype (bf16 or fp32)."""
         d, M = y.shape
         w = self._cast("out_w", self.out_linear.weight, y.dtype)
         if y.dtype == torch.bfloat16 and ops.own_from_channels(M, d):
             return ops.dense_from_channels(y, w, self._cast("out_b", self.out_linear.bias, torch.float32))
+        if y.dtype == torch.float32 and self._fp32_parts(M):
+            return ops.split_linear(ops.split_channels(y), self._out_parts.get(self.out_linear.weight), M, 1, d, d,
+                                    self._cast("out_b", self.out_linear.bias, torch.float32))
         return torch.addmm(self._cast("out_b", self.out_linear.bias, y.dtype), y.t(), w.t())
 
     # -- reference API -----------------------------------------------------------------------
@@ -171,7 +181,13 @@ class MonarchMixerSequenceMixing(nn.Module):
                 u2, u16, u_cm = self.pre_norm(u2.float().contiguous(), want_f32=not low, want_bf16=low)
                 if low:
                     u2 = u16
-            xproj = self.project_in(u2.to(act).contiguous())                             # (3d, B*L), bias added in the core
+            x = u2.to(act).contiguous()
+            if not low and self._fp32_parts(B * L) and not (x.requires_grad and torch.is_grad_enabled()):
+                parts, x_cm = ops.split_rows(x, channel_major=u_cm is None and self.residual_long_conv)
+                xproj = ops.split_to_channels(parts, self._in_parts.get(self.in_linear.weight), B * L, 3 * d, d)
+                u_cm = x_cm if u_cm is None else u_cm
+            else:
+                xproj = self.project_in(x)                                               # (3d, B*L), bias added in the core
             if u_cm is None and self.residual_long_conv:
                 u_cm = u2.float().t().contiguous()                                       # (d, B*L)
             if not self.residual_long_conv:

@@ -294,6 +294,91 @@ def dense_from_channels(x: Tensor, w: Tensor, bias: Optional[Tensor] = None) -> 
     return out
 
 
+def split_supported(M: int, nb: int, p: int, q: int) -> bool:
+    """fp32 products of x (M, nb p) with w (nb, q, p) by parts?"""
+    return (M > 0 and p % 4 == 0 and q % 4 == 0 and lib.m2_split_bytes(M, nb, p) > 0 and lib.m2_split_bytes(nb * q, 1, p) > 0)
+
+
+def split_rows(x: Tensor, nb: int = 1, channel_major: bool = False):
+    """x (M, nb p) fp32 -> (its three bf16 parts per value, operand of the fp32 products below; x^T (nb p, M) on request)."""
+    M, K = x.shape
+    _require(x, "x", torch.float32)
+    if x.data_ptr() % 16:
+        x = x.clone()
+    out = torch.empty(lib.m2_split_bytes(M, nb, K // nb) // 2, dtype=torch.bfloat16, device=x.device)
+    xt = torch.empty(K, M, dtype=torch.float32, device=x.device) if channel_major else None
+    check(lib.m2_split_rows_fwd(_ptr(x), _ptr(out), _ptr(xt), M, nb, K // nb, _stream()))
+    return out, xt
+
+
+def split_channels(x: Tensor) -> Tensor:
+    """x (K, M) fp32 -> the parts of x^T."""
+    K, M = x.shape
+    _require(x, "x", torch.float32)
+    out = torch.empty(lib.m2_split_bytes(M, 1, K) // 2, dtype=torch.bfloat16, device=x.device)
+    check(lib.m2_split_channels_fwd(_ptr(x), _ptr(out), M, K, _stream()))
+    return out
+
+
+class WeightParts:
+    """The parts of one weight, split again when it changes.  Made complete before it is kept (any stream may use it then),
+    not kept while a graph is captured, and left out of copies and pickles."""
+
+    def __init__(self):
+        self._hit = None
+
+    def __reduce__(self):
+        return WeightParts, ()
+
+    def get(self, w: Tensor) -> Tensor:
+        keep = not w.is_inference()
+        tag = (w.data_ptr(), w._version, w.device, w.shape) if keep else None
+        if keep and self._hit is not None and self._hit[0] == tag:
+            return self._hit[1]
+        parts, _ = split_rows(w.detach().float().reshape(-1, w.shape[-1]).contiguous())
+        if keep and not torch.cuda.is_current_stream_capturing():
+            # the old parts may still be read on other streams
+            torch.cuda.current_stream().synchronize() if self._hit is None else torch.cuda.synchronize(w.device)
+            self._hit = (tag, parts)
+        return parts
+
+
+def _require_parts(t: Tensor, name: str, rows: int, nb: int, p: int) -> None:
+    _require(t, name, torch.bfloat16, (lib.m2_split_bytes(rows, nb, p) // 2,))
+
+
+def split_to_channels(xs: Tensor, ws: Tensor, M: int, N: int, K: int) -> Tensor:
+    """w @ x^T in fp32, (N, M), from the parts of x (M, K) and w (N, K)."""
+    _require_parts(xs, "xs", M, 1, K)
+    _require_parts(ws, "ws", N, 1, K)
+    out = torch.empty(N, M, dtype=torch.float32, device=xs.device)
+    check(lib.m2_split_to_channels_fwd(_ptr(xs), _ptr(ws), _ptr(out), M, N, K, _stream()))
+    return out
+
+
+def split_linear(xs: Tensor, ws: Tensor, M: int, nb: int, p: int, q: int, bias: Optional[Tensor] = None,
+                 residual: Optional[Tensor] = None) -> Tensor:
+    """blockdiag_multiply(x, w) (+ bias) (+ residual) in fp32, (M, nb q), from the parts of x (M, nb p) and w (nb, q, p)."""
+    _require_parts(xs, "xs", M, nb, p)
+    _require_parts(ws, "ws", nb * q, 1, p)
+    if bias is not None:
+        _require(bias, "bias", torch.float32, (nb * q,))
+    if residual is not None:
+        _require(residual, "residual", torch.float32, (M, nb * q))
+    out = torch.empty(M, nb * q, dtype=torch.float32, device=xs.device)
+    check(lib.m2_split_linear_fwd(_ptr(xs), _ptr(ws), _ptr(bias), _ptr(residual), _ptr(out), M, nb, p, q, _stream()))
+    return out
+
+
+def split_glu(xs: Tensor, ws: Tensor, M: int, nb: int, p: int, q: int) -> Tensor:
+    """gelu(h[:, :I]) * h[:, I:] with h = blockdiag_multiply(x, w) in fp32, as the parts of the (M, I) result, I = nb q / 2."""
+    _require_parts(xs, "xs", M, nb, p)
+    _require_parts(ws, "ws", nb * q, 1, p)
+    out = torch.empty(lib.m2_split_bytes(M, 1, nb * q // 2) // 2, dtype=torch.bfloat16, device=xs.device)
+    check(lib.m2_split_glu_fwd(_ptr(xs), _ptr(ws), _ptr(out), M, nb, p, q, _stream()))
+    return out
+
+
 def blockdiag_glu(x: Tensor, w: Tensor, out: Optional[Tensor] = None) -> Tensor:
     """gelu_erf(h[:, :I]) * h[:, I:] with h = blockdiag_multiply(x, w); x (M, in) bf16, w (nb, 2I/nb, in/nb) bf16."""
     M, in_f = x.shape

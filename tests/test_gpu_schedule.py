@@ -1,6 +1,7 @@
 """The native schedule of an encoder (m2_amd/schedule.py) against the Python schedule: the same bits in every form, and plans
 that follow their modules."""
 import copy
+import weakref
 
 import pytest
 import torch
@@ -154,7 +155,7 @@ def test_a_graph_keeps_what_it_reads(gpu):
         first, _ = model(ids)
         table = next(iter(model.encoder._native_plans.values())).table if native else model.encoder._filter_table[1]
         held, address = table.table, table.table.data_ptr()
-        gone = __import__("weakref").ref(table)
+        gone = weakref.ref(table)
         del table, held
         model.encoder._native_plans.clear()
         model.encoder._filter_table = None
