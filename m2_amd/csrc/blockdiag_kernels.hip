@@ -1,5 +1,4 @@
-// Block-diagonal ("Monarch") linear layers of the M2-BERT GLU MLP on bf16 MFMA, and the LayerNorm
-// that closes the layer.
+// Block-diagonal ("Monarch") linear layers of the M2-BERT GLU MLP on bf16 MFMA.
 //
 //   out[m, k q + j] = sum_i x[m, k p + i] w[k, j, i]          (bert/src/mm/blockdiag_multiply.py:19-34,49-60)
 //
@@ -9,7 +8,6 @@
 // `blockdiag_kernel<GLU=true>` (longer K).
 // Plain form with bias and a residual (bert/src/bert_layers.py:504-506, bert/src/mm/structured_linear.py:65-69):
 // `blockdiag_wide_kernel` (192-column tiles: q a multiple of 192), `blockdiag_kernel<GLU=false>` (other widths).
-// `layernorm_kernel` normalises rows and writes the three forms the next layer reads.
 //
 // MFMA: v_mfma_f32_32x32x16_bf16.  Lane (i = lane % 32, h = lane / 32) supplies A[i][8h .. 8h+7] and
 // B[8h .. 8h+7][i]; both operands are K-contiguous in memory (x row-major, w[k] is (q, p)), so every
@@ -461,156 +459,6 @@ static int launch_blockdiag_wide(const void* x, const void* w, const float* bias
   return check_launch("blockdiag_wide");
 }
 
-// LayerNorm over the last dimension of x (M, d) fp32, eps inside the square root.
-// Workgroup = 8 waves handles R = 8 RW rows; each wave normalises RW rows at once (all loads in flight
-// together) and writes the row-major outputs from registers.  For the channel-major output the
-// normalised rows also go through an LDS tile, 384 columns at a time (row pitch 386 floats, so that 32
-// consecutive tokens of two neighbouring channels fall in 64 different banks; 49 KB, so that three
-// workgroups share a compute unit and one's loads overlap another's stores), and are written back with
-// lanes along the token axis: every store instruction covers R consecutive tokens of 64 / R channels.
-// The input is read once.  PER = d / 64 values per lane.
-template <int PER>
-struct LnShape {
-  static constexpr int RW = PER <= 16 ? 4 : 2;      // rows in flight per wave (register budget)
-  static constexpr int R = 8 * RW;                  // rows per workgroup: 32 or 16
-  static constexpr int PC = PER < 6 ? PER : 6;      // 64-column groups per tile pass
-  static constexpr int NPASS = (PER + PC - 1) / PC;
-  static constexpr int PITCH = 64 * PC + 2;
-  static constexpr size_t LDS_BYTES = (size_t)R * PITCH * sizeof(float);
-};
-// Where the rows come from when the kernel normalises embeddings instead of a matrix:
-// row m = word[ids[m]] + type[tt[m] or 0] (+ pos[pos_ids[m] or m % L]).
-// Every index is clamped into its table before it is used, so a bad id reads a valid row instead of
-// foreign memory; when that happens and `bad_index` is not null the kernel stores 1 there (plain vector
-// store; the caller cleared it before the launch and reads it afterwards to report the error).
-struct EmbedSource {
-  const long long* ids;     // (M)
-  const long long* tt;      // (M) or null: type 0
-  const long long* pos_ids; // (M) or null: m % L
-  const float* word;        // (vocab, d)
-  const float* type;        // (type_vocab, d)
-  const float* pos;         // (max_positions, d) or null: no position embeddings
-  int L;
-  int vocab, type_vocab, max_positions;      // rows of the three tables
-  int* bad_index;           // or null
-};
-__device__ __forceinline__ long long clamp_index(long long i, int rows, bool& bad) {
-  if (i < 0 || i >= rows) {
-    bad = true;
-    return i < 0 ? 0 : rows - 1;
-  }
-  return i;
-}
-// IN: float, or uint16_t for rows stored as bf16 (the sum the reference's autocast path feeds its LayerNorm).
-template <int PER, bool EMBED, typename IN = float>
-__global__ __launch_bounds__(512) void layernorm_kernel(const IN* __restrict__ x, EmbedSource src,
-                                                        const float* __restrict__ gamma,
-                                                        const float* __restrict__ beta, float eps,
-                                                        float* __restrict__ out_f32,       // (M, d) or null
-                                                        uint16_t* __restrict__ out_bf16,   // (M, d) or null
-                                                        float* __restrict__ out_t,         // (d, M) or null
-                                                        int M) {
-  constexpr int d = 64 * PER, RW = LnShape<PER>::RW, R = LnShape<PER>::R, PITCH = LnShape<PER>::PITCH;
-  constexpr int PC = LnShape<PER>::PC, NPASS = LnShape<PER>::NPASS;
-  extern __shared__ float tile[];                       // [R][PITCH], used only with out_t
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int m0 = blockIdx.x * R;
-  float g[PER], bt[PER];
-  static_for<0, PER>([&](auto ii) {
-    g[decltype(ii)::value] = gamma[lane + 64 * decltype(ii)::value];
-    bt[decltype(ii)::value] = beta[lane + 64 * decltype(ii)::value];
-  });
-  float v[RW][PER];
-  float sum[RW], sq[RW];
-  static_for<0, RW>([&](auto rr_) {
-    constexpr int rr = decltype(rr_)::value;
-    int m = m0 + wave * RW + rr;
-    m = m < M ? m : M - 1;
-    if constexpr (!EMBED) {
-      const IN* xr = x + (long)m * d;
-      static_for<0, PER>([&](auto ii) {
-        if constexpr (sizeof(IN) == 2) v[rr][decltype(ii)::value] = bf16_to_f32(xr[lane + 64 * decltype(ii)::value]);
-        else v[rr][decltype(ii)::value] = xr[lane + 64 * decltype(ii)::value];
-      });
-    } else {
-      bool bad = false;
-      const float* wr = src.word + clamp_index(src.ids[m], src.vocab, bad) * d;
-      const float* tr = src.type + (src.tt ? clamp_index(src.tt[m], src.type_vocab, bad) : 0) * d;
-      static_for<0, PER>([&](auto ii) {
-        constexpr int i = decltype(ii)::value;
-        v[rr][i] = wr[lane + 64 * i] + tr[lane + 64 * i];
-      });
-      if (src.pos) {
-        const float* pr = src.pos + (src.pos_ids ? clamp_index(src.pos_ids[m], src.max_positions, bad)
-                                                 : (long long)(m % src.L)) * d;
-        static_for<0, PER>([&](auto ii) {
-          constexpr int i = decltype(ii)::value;
-          v[rr][i] += pr[lane + 64 * i];
-        });
-      }
-      if (bad && src.bad_index && lane == 0) *src.bad_index = 1;
-    }
-  });
-  static_for<0, RW>([&](auto rr_) {
-    constexpr int rr = decltype(rr_)::value;
-    float s = 0.f;
-    static_for<0, PER>([&](auto ii) { s += v[rr][decltype(ii)::value]; });
-    sum[rr] = s;
-  });
-  for (int o = 32; o > 0; o >>= 1)
-    static_for<0, RW>([&](auto rr_) { sum[decltype(rr_)::value] += __shfl_xor(sum[decltype(rr_)::value], o); });
-  static_for<0, RW>([&](auto rr_) {
-    constexpr int rr = decltype(rr_)::value;
-    sum[rr] *= (1.0f / (float)d);
-    float s = 0.f;
-    static_for<0, PER>([&](auto ii) {
-      const float c = v[rr][decltype(ii)::value] - sum[rr];
-      s += c * c;
-    });
-    sq[rr] = s;
-  });
-  for (int o = 32; o > 0; o >>= 1)
-    static_for<0, RW>([&](auto rr_) { sq[decltype(rr_)::value] += __shfl_xor(sq[decltype(rr_)::value], o); });
-  static_for<0, RW>([&](auto rr_) {
-    constexpr int rr = decltype(rr_)::value;
-    const int m = m0 + wave * RW + rr;
-    const float mean = sum[rr];
-    const float rstd = rsqrtf(sq[rr] * (1.0f / (float)d) + eps);
-    static_for<0, PER>([&](auto ii) {
-      constexpr int i = decltype(ii)::value;
-      v[rr][i] = (v[rr][i] - mean) * rstd * g[i] + bt[i];
-      if (m < M) {
-        if (out_f32) out_f32[(long)m * d + lane + 64 * i] = v[rr][i];
-        if (out_bf16) out_bf16[(long)m * d + lane + 64 * i] = f32_to_bf16(v[rr][i]);
-      }
-    });
-  });
-  if (!out_t) return;
-  // lane = (token tk, channel offset h): R tokens x (64 / R) channels per store instruction
-  constexpr int CH = 64 / R;
-  const int tk = lane % R, h = lane / R;
-  const int mt = m0 + tk;
-  static_for<0, NPASS>([&](auto pp) {
-    constexpr int ps = decltype(pp)::value;
-    constexpr int i0 = ps * PC, i1 = (i0 + PC < PER) ? i0 + PC : PER;      // 64-column groups of this pass
-    if (ps > 0) __syncthreads();                                            // the previous pass has been read
-    static_for<0, RW>([&](auto rr_) {
-      constexpr int rr = decltype(rr_)::value;
-      static_for<i0, i1>([&](auto ii) {
-        constexpr int i = decltype(ii)::value;
-        tile[(wave * RW + rr) * PITCH + lane + 64 * (i - i0)] = v[rr][i];
-      });
-    });
-    __syncthreads();
-    if (mt < M) {
-      const float* src = tile + tk * PITCH + h;
-      float* dst = out_t + (long)(64 * i0 + h) * M + mt;
-#pragma unroll 4
-      for (int c0 = wave * CH; c0 < 64 * (i1 - i0); c0 += 8 * CH) dst[(long)c0 * M] = src[c0];
-    }
-  });
-}
-
 // ---------------------------------------------------------------------------------------------
 // Weight-stationary GLU kernel for short K (p = in_features / nblocks <= 256).
 //
@@ -1047,69 +895,4 @@ extern "C" int m2_blockdiag_linear_f32_fwd(const float* x, const float* w, const
   hipLaunchKernelGGL(blockdiag_f32_kernel, dim3((unsigned)((ntiles + 3) / 4)), dim3(256), 0, (hipStream_t)stream, x, w, bias,
                      out, M, nblocks, p, q);
   return check_launch("blockdiag_f32");
-}
-
-template <bool EMBED, typename IN = float>
-static int launch_layernorm(const IN* x, const EmbedSource& src, const float* gamma, const float* beta, float eps,
-                            float* out_f32, void* out_bf16, float* out_channel_major, int M, int d, void* stream) {
-  hipStream_t st = (hipStream_t)stream;
-  uint16_t* o16 = (uint16_t*)out_bf16;
-  switch (d / 64) {
-#define LN_CASE(P)                                                                                                      \
-  case P: {                                                                                                             \
-    const size_t lds = out_channel_major ? LnShape<P>::LDS_BYTES : 0;                                                   \
-    auto kern = layernorm_kernel<P, EMBED, IN>;                                                                           \
-    if (lds > 64 * 1024) {                                                                                              \
-      hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);     \
-      if (e != hipSuccess) return set_error(M2_ERR_LAUNCH, "hipFuncSetAttribute(layernorm): %s", hipGetErrorString(e)); \
-    }                                                                                                                   \
-    hipLaunchKernelGGL(kern, dim3((M + LnShape<P>::R - 1) / LnShape<P>::R), dim3(512), lds, st, x, src, gamma, beta,   \
-                       eps, out_f32, o16, out_channel_major, M);                                                        \
-    break;                                                                                                              \
-  }
-    LN_CASE(1) LN_CASE(2) LN_CASE(3) LN_CASE(4) LN_CASE(5) LN_CASE(6) LN_CASE(7) LN_CASE(8) LN_CASE(9) LN_CASE(10) LN_CASE(11)
-    LN_CASE(12) LN_CASE(13) LN_CASE(14) LN_CASE(15) LN_CASE(16) LN_CASE(17) LN_CASE(18) LN_CASE(19) LN_CASE(20) LN_CASE(21)
-    LN_CASE(22) LN_CASE(23) LN_CASE(24) LN_CASE(25) LN_CASE(26) LN_CASE(27) LN_CASE(28) LN_CASE(29) LN_CASE(30) LN_CASE(31)
-    LN_CASE(32)
-#undef LN_CASE
-  }
-  return check_launch("layernorm");
-}
-
-extern "C" int m2_layernorm_fwd(const float* x, const float* gamma, const float* beta, float eps, float* out_f32,
-                                void* out_bf16, float* out_channel_major, int M, int d, void* stream) {
-  if (!x || !gamma || !beta) return set_error(M2_ERR_ARG, "m2_layernorm_fwd: null pointer");
-  if (M <= 0 || d <= 0 || d % 64 != 0 || d > 2048)
-    return set_error(M2_ERR_UNSUPPORTED, "m2_layernorm_fwd: need M > 0 and d a multiple of 64 up to 2048 (M=%d d=%d)", M, d);
-  return launch_layernorm<false>(x, EmbedSource{}, gamma, beta, eps, out_f32, out_bf16, out_channel_major, M, d, stream);
-}
-
-extern "C" int m2_layernorm_bf16_fwd(const void* x, const float* gamma, const float* beta, float eps, float* out_f32,
-                                     void* out_bf16, float* out_channel_major, int M, int d, void* stream) {
-  if (!x || !gamma || !beta) return set_error(M2_ERR_ARG, "m2_layernorm_bf16_fwd: null pointer");
-  if (M <= 0 || d <= 0 || d % 64 != 0 || d > 2048)
-    return set_error(M2_ERR_UNSUPPORTED, "m2_layernorm_bf16_fwd: need M > 0 and d a multiple of 64 up to 2048 (M=%d d=%d)", M, d);
-  return launch_layernorm<false, uint16_t>((const uint16_t*)x, EmbedSource{}, gamma, beta, eps, out_f32, out_bf16,
-                                           out_channel_major, M, d, stream);
-}
-
-extern "C" int m2_embed_layernorm_fwd(const long long* input_ids, const long long* token_type_ids,
-                                      const long long* position_ids, const float* word_emb, const float* type_emb,
-                                      const float* pos_emb, int vocab_size, int type_vocab_size, int max_positions,
-                                      const float* gamma, const float* beta, float eps, float* out_f32, void* out_bf16,
-                                      float* out_channel_major, int* bad_index, int B, int L, int d, void* stream) {
-  if (!input_ids || !word_emb || !type_emb || !gamma || !beta)
-    return set_error(M2_ERR_ARG, "m2_embed_layernorm_fwd: null pointer");
-  if (B <= 0 || L <= 0 || d <= 0 || d % 64 != 0 || d > 2048)
-    return set_error(M2_ERR_UNSUPPORTED, "m2_embed_layernorm_fwd: need B, L > 0 and d a multiple of 64 up to 2048 (B=%d L=%d d=%d)", B, L, d);
-  if ((long)B * L > 0x7fffffffL) return set_error(M2_ERR_UNSUPPORTED, "m2_embed_layernorm_fwd: B * L = %ld does not fit an int", (long)B * L);
-  if (position_ids && !pos_emb) return set_error(M2_ERR_ARG, "m2_embed_layernorm_fwd: position_ids without a position table");
-  if (vocab_size <= 0 || type_vocab_size <= 0 || (pos_emb && max_positions <= 0))
-    return set_error(M2_ERR_ARG, "m2_embed_layernorm_fwd: table sizes must be positive (vocab=%d type_vocab=%d max_positions=%d)",
-                     vocab_size, type_vocab_size, max_positions);
-  if (pos_emb && !position_ids && L > max_positions)
-    return set_error(M2_ERR_ARG, "m2_embed_layernorm_fwd: sequence length %d exceeds the position table (%d rows)", L, max_positions);
-  const EmbedSource src{input_ids, token_type_ids, position_ids, word_emb, type_emb, pos_emb, L,
-                        vocab_size, type_vocab_size, max_positions, bad_index};
-  return launch_layernorm<true>((const float*)nullptr, src, gamma, beta, eps, out_f32, out_bf16, out_channel_major, B * L, d, stream);
 }
