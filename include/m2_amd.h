@@ -246,6 +246,10 @@ int m2_layernorm_fwd(const float* x, const float* gamma, const float* beta, floa
 int m2_layernorm_bf16_fwd(const void* x, const float* gamma, const float* beta, float eps, float* out_f32,
                           void* out_bf16, float* out_channel_major, int M, int d, void* stream);
 
+/* Two of those forms from rows as they are: x (M, d) fp32 -> out_bf16 (M, d) and out_channel_major (d, M) fp32, in one pass
+ * (hidden states given to a stack of layers).  Needs d % 64 == 0. */
+int m2_input_forms_fwd(const float* x, void* out_bf16, float* out_channel_major, int M, int d, void* stream);
+
 /* out = LayerNorm(blockdiag_multiply(x, w) + bias + residual) in one kernel: m2_blockdiag_linear_fwd followed by
  * m2_layernorm_fwd without the fp32 intermediate (bert/src/bert_layers.py:504-506: wo, dropout, residual,
  * layernorm).  Arguments as in those two; any of the three outputs may be NULL.

@@ -359,6 +359,9 @@ class BertEncoder(nn.Module):
         with torch.autocast("cuda", enabled=False):
             pre_norm = self.layer[0].attention.hyena_training_additions       # layers then start from the fp32 form
             if not pre_norm:
+                if (h16 is None and hT is None and h32.shape[0] > 0 and h32.shape[1] % 64 == 0
+                        and not (h32.requires_grad and torch.is_grad_enabled())):      # (those the projections refuse)
+                    h16, hT = ops.input_forms(h32)
                 if h16 is None:
                     h16 = h32.to(torch.bfloat16)
                 if hT is None:

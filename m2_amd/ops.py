@@ -541,6 +541,16 @@ def layernorm(x: Tensor, gamma: Tensor, beta: Tensor, eps: float, want_f32: bool
     return o32, o16, ot
 
 
+def input_forms(x: Tensor):
+    """x (M, d) fp32, d a multiple of 64 -> (bf16 (M, d), f32 (d, M)) in one pass."""
+    _require(x, "x", torch.float32)
+    M, d = x.shape
+    o16 = torch.empty(M, d, dtype=torch.bfloat16, device=x.device)
+    ot = torch.empty(d, M, dtype=torch.float32, device=x.device)
+    check(lib.m2_input_forms_fwd(_ptr(x), _ptr(o16), _ptr(ot), M, d, _stream()))
+    return o16, ot
+
+
 def embed_layernorm(input_ids: Tensor, token_type_ids: Optional[Tensor], position_ids: Optional[Tensor], word_emb: Tensor,
                     type_emb: Tensor, pos_emb: Optional[Tensor], gamma: Tensor, beta: Tensor, eps: float,
                     want_f32: bool = True, want_bf16: bool = False, want_channel_major: bool = False,

@@ -45,3 +45,15 @@ def test_embed_layernorm_row_counts(B, L):
     ref = reference(rows, gamma, beta, 1e-12)
     assert ((o32.view(B * L, d).double() - ref).norm() / ref.norm()).item() < 2.5e-6
     assert torch.equal(ot.reshape(d, B * L).t(), o32.view(B * L, d)) and torch.equal(o16, o32.bfloat16())
+
+
+@pytest.mark.parametrize("M,d", [(1, 64), (63, 128), (64, 64), (65, 192), (300, 768), (4097, 960)])
+def test_input_forms(M, d):
+    from m2_amd import ops
+    base = torch.randn(M * d + 1, generator=torch.Generator(device="cuda").manual_seed(13), device="cuda")
+    base[0], base[1], base[M * d - 1] = float("inf"), float("nan"), -0.0
+    for x in (base[:-1].view(M, d), base[1:].view(M, d)):            # also rows that start off a 16-byte boundary
+        h16, hT = ops.input_forms(x)
+        ref = x.to(torch.bfloat16)
+        assert torch.equal(h16.isnan(), ref.isnan()) and torch.equal(h16.nan_to_num(), ref.nan_to_num())
+        assert torch.equal(hT.view(torch.int32), x.t().contiguous().view(torch.int32))
