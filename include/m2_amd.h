@@ -285,6 +285,7 @@ int m2_embed_layernorm_fwd(const long long* input_ids, const long long* token_ty
  * in fp32.  A split operand of `rows` rows of `nblocks` blocks of `p` values takes m2_split_bytes (0: unsupported): p a
  * multiple of 4, below 4 GB.
  *   m2_split_rows_fwd      x (M, nblocks p) fp32 -> parts; channel_major: NULL or (p, M) fp32, receives x^T (nblocks 1, M % 4 == 0)
+ *   m2_split_jobs_fwd      one to four such operands in one launch (`jobs`: a HOST array)
  *   m2_split_channels_fwd  x (K, M) fp32 -> parts of x^T; M % 4 == 0
  * Weights (nblocks, q, p) are split as nblocks q rows of one block.
  *   m2_split_to_channels_fwd  out (N, M) fp32 = w x^T; M % 4 == 0
@@ -293,6 +294,13 @@ int m2_embed_layernorm_fwd(const long long* input_ids, const long long* token_ty
  * ------------------------------------------------------------------------------------------- */
 size_t m2_split_bytes(int rows, int nblocks, int p);
 int m2_split_rows_fwd(const float* x, void* out, float* channel_major, int M, int nblocks, int p, void* stream);
+typedef struct m2_split_job {
+  const float* x;
+  void* out;
+  float* channel_major;    /* or NULL */
+  int rows, nblocks, p;
+} m2_split_job;
+int m2_split_jobs_fwd(const m2_split_job* jobs, int njobs, void* stream);
 int m2_split_channels_fwd(const float* x, void* out, int M, int K, void* stream);
 int m2_split_to_channels_fwd(const void* xs, const void* ws, float* out, int M, int N, int K, void* stream);
 int m2_split_linear_fwd(const void* xs, const void* ws, const float* bias, const float* residual, float* out, int M, int nblocks,

@@ -31,6 +31,11 @@ class LayerParams(ctypes.Structure):
                                         "mlp_packed", "glu_packed", "wo_b", "ln_gamma", "ln_beta")] + [("residual", c_int)]
 
 
+class SplitJob(ctypes.Structure):
+    """Mirror of `m2_split_job`."""
+    _fields_ = [(n, c_void_p) for n in ("x", "out", "channel_major")] + [(n, c_int) for n in ("rows", "nblocks", "p")]
+
+
 def _load() -> ctypes.CDLL:
     if not os.path.exists(LIB_PATH):
         raise ImportError(
@@ -111,6 +116,8 @@ def _load() -> ctypes.CDLL:
     lib.m2_split_bytes.argtypes = [c_int] * 3
     lib.m2_split_rows_fwd.restype = c_int
     lib.m2_split_rows_fwd.argtypes = [c_void_p] * 3 + [c_int] * 3 + [c_void_p]
+    lib.m2_split_jobs_fwd.restype = c_int
+    lib.m2_split_jobs_fwd.argtypes = [c_void_p, c_int, c_void_p]
     lib.m2_split_channels_fwd.restype = c_int
     lib.m2_split_channels_fwd.argtypes = [c_void_p] * 2 + [c_int] * 2 + [c_void_p]
     lib.m2_split_to_channels_fwd.restype = c_int
@@ -132,7 +139,7 @@ EXPORTS = ["m2_version", "m2_last_error", "m2_hyena_filter_workspace_bytes", "m2
            "m2_fftconv_supported_seqlen", "m2_filter_spectrum_bytes", "m2_filter_spectrum_fwd", "m2_mixer_core_fwd",
            "m2_fftconv_fwd", "m2_dense_supported", "m2_dense_to_channels_fwd", "m2_dense_from_channels_fwd", "m2_blockdiag_glu_fwd", "m2_blockdiag_linear_fwd", "m2_blockdiag_linear_f32_fwd", "m2_mlp_fused_supported", "m2_mlp_fused_packed_bytes", "m2_mlp_fused_pack", "m2_mlp_fused_fwd", "m2_glu_stream_supported", "m2_glu_stream_packed_bytes", "m2_glu_stream_pack", "m2_glu_stream_fwd", "m2_layernorm_fwd", "m2_layernorm_bf16_fwd", "m2_input_forms_fwd",
            "m2_embed_layernorm_fwd", "m2_blockdiag_linear_layernorm_supported", "m2_blockdiag_linear_layernorm_fwd", "m2_encoder_layers_workspace_bytes", "m2_encoder_layers_fwd",
-           "m2_split_bytes", "m2_split_rows_fwd", "m2_split_channels_fwd", "m2_split_to_channels_fwd", "m2_split_linear_fwd", "m2_split_glu_fwd"]
+           "m2_split_bytes", "m2_split_rows_fwd", "m2_split_jobs_fwd", "m2_split_channels_fwd", "m2_split_to_channels_fwd", "m2_split_linear_fwd", "m2_split_glu_fwd"]
 
 
 def check(rc: int) -> None:

@@ -60,7 +60,6 @@ class BlockdiagLinear(nn.Module):
             self.register_parameter("bias", None)
         self.reset_parameters()
         self._w16 = None
-        self._parts = ops.WeightParts()
 
     def reset_parameters(self) -> None:
         # first block-row of a dense Kaiming-uniform matrix, rescaled for the sparsity
@@ -99,8 +98,8 @@ class BlockdiagLinear(nn.Module):
         nb, q, p = self.weight.shape
         M = x.numel() // x.shape[-1]
         if _fp32_path(x) and p % 8 == 0 and ops.split_supported(M, nb, p, q):
-            parts, _ = ops.split_rows(x.reshape(-1, self.in_features_extended).contiguous(), nb)
-            out = ops.split_linear(parts, self._parts.get(self.weight), M, nb, p, q, bias)
+            parts, _, w = ops.split_rows(x.reshape(-1, self.in_features_extended).contiguous(), nb, weights=(self.weight,))
+            out = ops.split_linear(parts, w, M, nb, p, q, bias)
         elif _fp32_path(x) and p % 8 == 0:
             out = ops.blockdiag_linear_f32(x.reshape(-1, self.in_features_extended).contiguous(),
                                            self.weight.detach().float().contiguous(), bias)

@@ -37,11 +37,11 @@ __device__ __forceinline__ void store_parts(uint16_t* dst, const float* v) {
 // ---- splitting passes: a workgroup takes 32 rows x 64 k of one block (memory-bound: 4 bytes read, 6 written per value).
 // CM: the input is channel-major (K, M), nb = 1; else row-major (M, nb p), with a channel-major fp32 copy on request (nb = 1).
 template <bool CM>
-__global__ __launch_bounds__(256) void split_kernel(const float* __restrict__ x, uint16_t* __restrict__ out,
-                                                    float* __restrict__ xt, int M, int nb, int p) {
+__device__ __forceinline__ void split_tile(const float* __restrict__ x, uint16_t* __restrict__ out, float* __restrict__ xt,
+                                           int M, int nb, int p, int kx, int m0) {
   __shared__ float tile[64][33];
   const int t = threadIdx.x, pc = (p + 31) / 32, pairs = (pc + 1) / 2;
-  const int blk = blockIdx.x / pairs, k0 = (blockIdx.x % pairs) * 64, m0 = blockIdx.y * 32;
+  const int blk = kx / pairs, k0 = (kx % pairs) * 64;
   const int r = t >> 3, kl = 4 * (t & 7), row = m0 + r;
   const int ck = t >> 2, cm = 8 * (t & 3);           // channel-major side: one k, eight rows
   if constexpr (CM) {
@@ -76,6 +76,32 @@ __global__ __launch_bounds__(256) void split_kernel(const float* __restrict__ x,
         *reinterpret_cast<float4*>(xt + (long)(k0 + ck) * M + m0 + m) = float4{tile[ck][m], tile[ck][m + 1], tile[ck][m + 2], tile[ck][m + 3]};
     });
   }
+}
+
+__global__ __launch_bounds__(256) void split_channels_kernel(const float* __restrict__ x, uint16_t* __restrict__ out, int M, int K) {
+  split_tile<true>(x, out, nullptr, M, 1, K, blockIdx.x, blockIdx.y * 32);
+}
+
+// Up to four row-major operands in one launch: an activation and the weights it meets, which are split in every call (nothing
+// derived from a weight outlives the call, so a weight may be changed in any way between two calls).  The weights' share, measured
+// by itself: 8 us for the 2.4 M values of one mixer's two projections at d = 768.
+struct SplitJob {
+  const float* x;
+  uint16_t* out;
+  float* xt;
+  int M, nb, p, gx;         // gx: pairs of chunks of a row
+  unsigned first;           // of its workgroups
+};
+struct SplitJobs {
+  SplitJob job[4];
+};
+__global__ __launch_bounds__(256) void split_rows_kernel(SplitJobs jobs, int n) {
+  int j = 0;
+  for (int i = 1; i < n; ++i)
+    if (blockIdx.x >= jobs.job[i].first) j = i;
+  const SplitJob& s = jobs.job[j];
+  const unsigned b = blockIdx.x - s.first;
+  split_tile<false>(s.x, s.out, s.xt, s.M, s.nb, s.p, (int)(b % (unsigned)s.gx), (int)(b / (unsigned)s.gx) * 32);
 }
 
 // a pointer that is the same in all lanes, kept in scalar registers
@@ -338,20 +364,30 @@ extern "C" size_t m2_split_bytes(int rows, int nblocks, int p) {
   return split_ok(rows, nblocks, p) ? (size_t)rows * nblocks * ((p + 31) / 32) * kRowBytes : 0;
 }
 
-extern "C" int m2_split_rows_fwd(const float* x, void* out, float* channel_major, int M, int nblocks, int p, void* stream) {
-  const char* who = "m2_split_rows_fwd";
-  if (!x || !out) return set_error(M2_ERR_ARG, "%s: null pointer", who);
-  if (!split_ok(M, nblocks, p)) return set_error(M2_ERR_UNSUPPORTED, "%s: needs p a multiple of 4 and operands below 4 GB (M=%d nb=%d p=%d)", who, M, nblocks, p);
-  if (channel_major && (nblocks != 1 || M % 4)) return set_error(M2_ERR_UNSUPPORTED, "%s: a channel-major copy needs one block and M a multiple of 4 (M=%d nb=%d)", who, M, nblocks);
-  const int pc = (p + 31) / 32, gx = nblocks * ((pc + 1) / 2);
-  // rows beyond a launch's 65535 groups of 32 go into launches of their own
-  for (long m = 0; m < M; m += 65535l * 32) {
-    if (m && channel_major) return set_error(M2_ERR_UNSUPPORTED, "%s: a channel-major copy needs M up to 2097120 (M=%d)", who, M);
-    const int rows = (int)(M - m < 65535l * 32 ? M - m : 65535l * 32);
-    hipLaunchKernelGGL(split_kernel<false>, dim3(gx, (rows + 31) / 32), dim3(256), 0, (hipStream_t)stream, x + m * nblocks * p,
-                       (uint16_t*)out + m * nblocks * pc * 96, channel_major, rows, nblocks, p);
+extern "C" int m2_split_jobs_fwd(const m2_split_job* jobs, int njobs, void* stream) {
+  const char* who = "m2_split_jobs_fwd";
+  if (!jobs) return set_error(M2_ERR_ARG, "%s: null pointer", who);
+  if (njobs < 1 || njobs > 4) return set_error(M2_ERR_ARG, "%s: takes one to four operands, got %d", who, njobs);
+  SplitJobs sj;
+  long groups = 0;
+  for (int i = 0; i < njobs; ++i) {
+    const m2_split_job& j = jobs[i];
+    if (!j.x || !j.out) return set_error(M2_ERR_ARG, "%s: null pointer", who);
+    if (!split_ok(j.rows, j.nblocks, j.p)) return set_error(M2_ERR_UNSUPPORTED, "%s: needs p a multiple of 4 and operands below 4 GB (M=%d nb=%d p=%d)", who, j.rows, j.nblocks, j.p);
+    if (j.channel_major && (j.nblocks != 1 || j.rows % 4)) return set_error(M2_ERR_UNSUPPORTED, "%s: a channel-major copy needs one block and M a multiple of 4 (M=%d nb=%d)", who, j.rows, j.nblocks);
+    const int gx = j.nblocks * (((j.p + 31) / 32 + 1) / 2);
+    sj.job[i] = SplitJob{j.x, (uint16_t*)j.out, j.channel_major, j.rows, j.nblocks, j.p, gx, (unsigned)groups};
+    groups += (long)gx * ((j.rows + 31l) / 32);
   }
+  for (int i = njobs; i < 4; ++i) sj.job[i] = sj.job[0];
+  // (operands below 4 GB have fewer than 2^25 rows of 192 bytes, hence fewer than 2^21 groups each)
+  hipLaunchKernelGGL(split_rows_kernel, dim3((unsigned)groups), dim3(256), 0, (hipStream_t)stream, sj, njobs);
   return check_launch("split_rows");
+}
+
+extern "C" int m2_split_rows_fwd(const float* x, void* out, float* channel_major, int M, int nblocks, int p, void* stream) {
+  const m2_split_job job{x, out, channel_major, M, nblocks, p};
+  return m2_split_jobs_fwd(&job, 1, stream);
 }
 
 extern "C" int m2_split_channels_fwd(const float* x, void* out, int M, int K, void* stream) {
@@ -360,8 +396,7 @@ extern "C" int m2_split_channels_fwd(const float* x, void* out, int M, int K, vo
   if (!split_ok(M, 1, K) || M % 4 || M > 65535 * 32)
     return set_error(M2_ERR_UNSUPPORTED, "%s: needs M up to 2097120 and K multiples of 4 and operands below 4 GB (M=%d K=%d)", who, M, K);
   const int pc = (K + 31) / 32;
-  hipLaunchKernelGGL(split_kernel<true>, dim3((pc + 1) / 2, (M + 31) / 32), dim3(256), 0, (hipStream_t)stream, x, (uint16_t*)out,
-                     (float*)nullptr, M, 1, K);
+  hipLaunchKernelGGL(split_channels_kernel, dim3((pc + 1) / 2, (M + 31) / 32), dim3(256), 0, (hipStream_t)stream, x, (uint16_t*)out, M, K);
   return check_launch("split_channels");
 }
 

@@ -231,9 +231,9 @@ class BertGatedLinearUnitMLP(nn.Module):
                 M, (nb, q, p), q2 = x.shape[0], self.gated_layers.weight.shape, self.wo.weight.shape[1]
                 if x.data_ptr() % 16:
                     x = x.clone()
-                g = ops.split_glu(ops.split_rows(x, nb)[0], self.gated_layers._parts.get(self.gated_layers.weight), M, nb, p, q)
-                s = ops.split_linear(g, self.wo._parts.get(self.wo.weight), M, nb, q // 2, q2,
-                                     self.wo.bias.detach().float().contiguous(), x)
+                parts, _, w_gated, w_out = ops.split_rows(x, nb, weights=(self.gated_layers.weight, self.wo.weight))
+                g = ops.split_glu(parts, w_gated, M, nb, p, q)
+                s = ops.split_linear(g, w_out, M, nb, q // 2, q2, self.wo.bias.detach().float().contiguous(), x)
                 o32, _, _ = ops.layernorm(s, gamma, beta, eps, want_f32=True)
                 return o32.view(shape)
             h = self.gated_layers(x)                                   # fp32 block-diagonal kernel

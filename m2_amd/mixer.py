@@ -60,7 +60,6 @@ class MonarchMixerSequenceMixing(nn.Module):
         self.short_filter = nn.Conv1d(in_channels=total_width, out_channels=total_width, kernel_size=3,
                                       groups=total_width, padding=2)
         self._cast_cache = {}
-        self._in_parts, self._out_parts = ops.WeightParts(), ops.WeightParts()
         self.cache_filters = False
         self._spec_cache = None
         self._filter_table = None
@@ -149,18 +148,20 @@ class MonarchMixerSequenceMixing(nn.Module):
         torch.mm(x, w.t(), out=out.t())
         return out
 
-    def _fp32_parts(self, M: int) -> bool:
-        return M % 4 == 0 and ops.split_supported(M, 1, self.d_model, 3 * self.d_model)
+    def _fp32_parts(self, M: int, w_in: torch.Tensor, w_out: torch.Tensor) -> bool:
+        d = self.d_model
+        return M % 4 == 0 and w_in.shape == (3 * d, d) and w_out.shape == (d, d) and ops.split_supported(M, 1, d, 3 * d)
 
-    def project_out(self, y: torch.Tensor) -> torch.Tensor:
-        """y (d, M) channel-major -> y^T @ out_linear.weight^T + bias, (M, d), in y's dtype (bf16 or fp32)."""
+    def project_out(self, y: torch.Tensor, w_parts: Optional[torch.Tensor] = None) -> torch.Tensor:
+        """y (d, M) channel-major -> y^T @ out_linear.weight^T + bias, (M, d), in y's dtype (bf16 or fp32).  `w_parts`: the parts
+        of an fp32 weight when the caller has them."""
         d, M = y.shape
+        if w_parts is not None:
+            return ops.split_linear(ops.split_channels(y), w_parts, M, 1, d, d,
+                                    self._cast("out_b", self.out_linear.bias, torch.float32))
         w = self._cast("out_w", self.out_linear.weight, y.dtype)
         if y.dtype == torch.bfloat16 and ops.own_from_channels(M, d):
             return ops.dense_from_channels(y, w, self._cast("out_b", self.out_linear.bias, torch.float32))
-        if y.dtype == torch.float32 and self._fp32_parts(M):
-            return ops.split_linear(ops.split_channels(y), self._out_parts.get(self.out_linear.weight), M, 1, d, d,
-                                    self._cast("out_b", self.out_linear.bias, torch.float32))
         return torch.addmm(self._cast("out_b", self.out_linear.bias, y.dtype), y.t(), w.t())
 
     # -- reference API -----------------------------------------------------------------------
@@ -174,7 +175,7 @@ class MonarchMixerSequenceMixing(nn.Module):
         act = torch.bfloat16 if low else torch.float32
         u2 = u.reshape(B * L, d)
         with torch.autocast("cuda", enabled=False):
-            u_cm = None
+            u_cm, w_out = None, None
             if self.hyena_training_additions:
                 if self.training and self.drop.p > 0:
                     raise NotImplementedError("m2_amd is a forward/inference path: call .eval() first")
@@ -182,9 +183,10 @@ class MonarchMixerSequenceMixing(nn.Module):
                 if low:
                     u2 = u16
             x = u2.to(act).contiguous()
-            if not low and self._fp32_parts(B * L) and not (x.requires_grad and torch.is_grad_enabled()):
-                parts, x_cm = ops.split_rows(x, channel_major=u_cm is None and self.residual_long_conv)
-                xproj = ops.split_to_channels(parts, self._in_parts.get(self.in_linear.weight), B * L, 3 * d, d)
+            weights = None if low else (self.in_linear.weight, self.out_linear.weight)
+            if weights and self._fp32_parts(B * L, *weights) and not (x.requires_grad and torch.is_grad_enabled()):
+                parts, x_cm, w_in, w_out = ops.split_rows(x, channel_major=u_cm is None and self.residual_long_conv, weights=weights)
+                xproj = ops.split_to_channels(parts, w_in, B * L, 3 * d, d)
                 u_cm = x_cm if u_cm is None else u_cm
             else:
                 xproj = self.project_in(x)                                               # (3d, B*L), bias added in the core
@@ -193,5 +195,5 @@ class MonarchMixerSequenceMixing(nn.Module):
             if not self.residual_long_conv:
                 u_cm = None
             y = self.core(xproj.view(3 * d, B, L), None if u_cm is None else u_cm.view(d, B, L), B, L)
-            out = self.project_out(y.view(d, B * L))                                    # (B*L, d)
+            out = self.project_out(y.view(d, B * L), w_out)                             # (B*L, d)
         return out.view(B, L, d), None

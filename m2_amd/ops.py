@@ -13,7 +13,7 @@ from typing import Optional, Sequence
 import torch
 
 from . import _lib
-from ._lib import HyenaFilterParams, M2_DTYPE_BF16, M2_DTYPE_F32, check, lib
+from ._lib import HyenaFilterParams, SplitJob, M2_DTYPE_BF16, M2_DTYPE_F32, check, lib
 
 Tensor = torch.Tensor
 
@@ -299,52 +299,46 @@ def split_supported(M: int, nb: int, p: int, q: int) -> bool:
     return (M > 0 and p % 4 == 0 and q % 4 == 0 and lib.m2_split_bytes(M, nb, p) > 0 and lib.m2_split_bytes(nb * q, 1, p) > 0)
 
 
-def split_rows(x: Tensor, nb: int = 1, channel_major: bool = False):
-    """x (M, nb p) fp32 -> (its three bf16 parts per value, operand of the fp32 products below; x^T (nb p, M) on request)."""
+def _parts_elements(rows: int, nb: int, p: int) -> int:
+    """bf16 elements of a split operand (m2_split_bytes, which is twice this, where the size is supported)."""
+    return rows * nb * ((p + 31) // 32) * 96
+
+
+def split_rows(x: Tensor, nb: int = 1, channel_major: bool = False, weights: Sequence[Tensor] = ()):
+    """x (M, nb p) fp32 -> (its three bf16 parts per value, operand of the fp32 products below; x^T (nb p, M) on request), and
+    behind them the parts of up to three weights (..., p), split by the same launch.  Weights are split in every call: an address and
+    a version counter do not tell whether a weight is still the same (writes through `.data`, tensors made anew per access), and
+    a captured graph has to see the weight of the day."""
     M, K = x.shape
     _require(x, "x", torch.float32)
-    if x.data_ptr() % 16:
-        x = x.clone()
-    out = torch.empty(lib.m2_split_bytes(M, nb, K // nb) // 2, dtype=torch.bfloat16, device=x.device)
+    keep = [x.clone() if x.data_ptr() % 16 else x]
+    for w in weights:
+        if w.dtype != torch.float32 or not w.is_contiguous():
+            w = w.detach().float().contiguous()
+        _require(w, "weight", torch.float32)
+        keep.append(w.detach().clone() if w.data_ptr() % 16 else w)
     xt = torch.empty(K, M, dtype=torch.float32, device=x.device) if channel_major else None
-    check(lib.m2_split_rows_fwd(_ptr(x), _ptr(out), _ptr(xt), M, nb, K // nb, _stream()))
-    return out, xt
+    outs, jobs = [], (SplitJob * len(keep))()
+    for i, t in enumerate(keep):
+        n, p = (nb, K // nb) if i == 0 else (1, t.shape[-1])
+        rows = M if i == 0 else t.numel() // p
+        outs.append(torch.empty(_parts_elements(rows, n, p), dtype=torch.bfloat16, device=t.device))
+        jobs[i] = (t.data_ptr(), outs[i].data_ptr(), xt.data_ptr() if i == 0 and channel_major else None, rows, n, p)
+    check(lib.m2_split_jobs_fwd(jobs, len(jobs), _stream()))
+    return (outs[0], xt, *outs[1:])
 
 
 def split_channels(x: Tensor) -> Tensor:
     """x (K, M) fp32 -> the parts of x^T."""
     K, M = x.shape
     _require(x, "x", torch.float32)
-    out = torch.empty(lib.m2_split_bytes(M, 1, K) // 2, dtype=torch.bfloat16, device=x.device)
+    out = torch.empty(_parts_elements(M, 1, K), dtype=torch.bfloat16, device=x.device)
     check(lib.m2_split_channels_fwd(_ptr(x), _ptr(out), M, K, _stream()))
     return out
 
 
-class WeightParts:
-    """The parts of one weight, split again when it changes.  Made complete before it is kept (any stream may use it then),
-    not kept while a graph is captured, and left out of copies and pickles."""
-
-    def __init__(self):
-        self._hit = None
-
-    def __reduce__(self):
-        return WeightParts, ()
-
-    def get(self, w: Tensor) -> Tensor:
-        keep = not w.is_inference()
-        tag = (w.data_ptr(), w._version, w.device, w.shape) if keep else None
-        if keep and self._hit is not None and self._hit[0] == tag:
-            return self._hit[1]
-        parts, _ = split_rows(w.detach().float().reshape(-1, w.shape[-1]).contiguous())
-        if keep and not torch.cuda.is_current_stream_capturing():
-            # the old parts may still be read on other streams
-            torch.cuda.current_stream().synchronize() if self._hit is None else torch.cuda.synchronize(w.device)
-            self._hit = (tag, parts)
-        return parts
-
-
 def _require_parts(t: Tensor, name: str, rows: int, nb: int, p: int) -> None:
-    _require(t, name, torch.bfloat16, (lib.m2_split_bytes(rows, nb, p) // 2,))
+    _require(t, name, torch.bfloat16, (_parts_elements(rows, nb, p),))
 
 
 def split_to_channels(xs: Tensor, ws: Tensor, M: int, N: int, K: int) -> Tensor:
@@ -374,7 +368,7 @@ def split_glu(xs: Tensor, ws: Tensor, M: int, nb: int, p: int, q: int) -> Tensor
     """gelu(h[:, :I]) * h[:, I:] with h = blockdiag_multiply(x, w) in fp32, as the parts of the (M, I) result, I = nb q / 2."""
     _require_parts(xs, "xs", M, nb, p)
     _require_parts(ws, "ws", nb * q, 1, p)
-    out = torch.empty(lib.m2_split_bytes(M, 1, nb * q // 2) // 2, dtype=torch.bfloat16, device=xs.device)
+    out = torch.empty(_parts_elements(M, 1, nb * q // 2), dtype=torch.bfloat16, device=xs.device)
     check(lib.m2_split_glu_fwd(_ptr(xs), _ptr(ws), _ptr(out), M, nb, p, q, _stream()))
     return out
 

@@ -133,3 +133,78 @@ def test_fp32_modules_follow_their_weights(gpu):
         assert seen and (got - hooked).abs().max() < 1e-5
         mlp.wo.weight.add_(0.01)
         assert (mlp(x) - got).abs().max() > 1e-4
+
+
+# rows and chunks off the groups of 32 and 64, several blocks, one to three weights behind the activation
+@pytest.mark.parametrize("M,nb,p,shapes", [(4, 1, 4, [(4, 4)]), (33, 4, 24, [(4, 40, 24), (2, 100)]), (2052, 1, 768, [(2304, 768), (768, 768), (1, 36)])])
+def test_split_of_several_operands_at_once(gpu, M, nb, p, shapes):
+    from m2_amd import ops
+    g = torch.Generator().manual_seed(M)
+    x, ws = _rand(g, M, nb * p).to(gpu), [_rand(g, *s).to(gpu) for s in shapes]
+    one, _ = ops.split_rows(x, nb)
+    parts, xt, *wparts = ops.split_rows(x, nb, channel_major=nb == 1, weights=ws)
+    assert torch.equal(parts, one) and (xt is None or torch.equal(xt, x.t()))
+    for w, got in zip(ws, wparts, strict=True):
+        K = w.shape[-1]
+        assert torch.equal(got, ops.split_rows(w.view(-1, K))[0])
+        whole = got.view(-1, (K + 31) // 32, 3, 32).float().sum(2).view(w.numel() // K, -1)
+        assert torch.equal(whole[:, :K], w.view(-1, K)) and not whole[:, K:].any()
+
+
+def test_fp32_modules_read_the_weights_of_the_call(gpu):
+    """Weights written through `.data`, computed anew per access, replaced at an old address, or changed between two replays of
+    a captured graph: a result is always that of the weights as they are."""
+    import copy
+
+    import m2_amd
+    from torch.nn.utils import parametrize
+    cfg = m2_amd.m2_bert_80m(128)
+    layer = m2_amd.BertLayer(cfg).to(gpu).eval()
+    u = torch.randn(2, 128, 768, generator=torch.Generator().manual_seed(6)).to(gpu)
+    linears = [layer.attention.in_linear, layer.attention.out_linear, layer.mlp.gated_layers, layer.mlp.wo]
+
+    class Scaled(torch.nn.Module):
+        factor = 1.0
+
+        def forward(self, w):
+            return w * self.factor
+
+    def fresh():
+        other = m2_amd.BertLayer(cfg).to(gpu).eval()
+        other.load_state_dict({k: v.clone() for k, v in layer.state_dict().items()})
+        return other(u)
+
+    with torch.no_grad():
+        got = layer(u)
+        for lin in linears:
+            lin.weight.data.mul_(1.25)
+            before, got = got, layer(u)
+            assert torch.equal(got, fresh()) and not torch.equal(got, before)
+        for lin in linears:                                    # freed and made again: the address may come back
+            for _ in range(2):
+                old = lin.weight.detach()
+                lin.weight = None
+                values = (old * 0.9).cpu()
+                del old
+                lin.weight = torch.nn.Parameter(values.to(gpu))
+            before, got = got, layer(u)
+            assert torch.equal(got, fresh()) and not torch.equal(got, before)
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            held = layer(u)
+        for factor in (1.1, 0.8, 1.3):
+            for lin in linears:
+                lin.weight.mul_(factor)
+            torch.randn(512, 512, device=gpu) @ torch.randn(512, 512, device=gpu)
+            want = fresh()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(held, want), factor
+        want = copy.deepcopy(layer)
+        for lin in linears:
+            parametrize.register_parametrization(lin, "weight", Scaled())
+        for factor in (1.0, 1.5, 0.5, 2.0, 0.75):
+            for lin, other in zip(linears, (want.attention.in_linear, want.attention.out_linear, want.mlp.gated_layers, want.mlp.wo)):
+                lin.parametrizations.weight[0].factor = factor
+                other.weight.copy_(lin.parametrizations.weight.original * factor)
+            assert torch.equal(layer(u), want(u)), factor
