@@ -23,6 +23,14 @@ def _fp32_path(x: torch.Tensor) -> bool:
     return x.dtype == torch.float32 and not torch.is_autocast_enabled()
 
 
+def _parts_pay(M: int, nb: int, q: int, p: int) -> bool:
+    """One fp32 product by parts (two launches, the weight split in the first) or by the fp32-MFMA kernel?  us per call, parts /
+    fp32 kernel: 768 -> 6144 (four blocks) M = 512 30 / 23, 1024 30 / 42; 3072 -> 768 M = 512 30 / 31, 2048 37 / 53;
+    1536 -> 12288 M = 128 31 / 28, 256 33 / 39; 1792 -> 14336 M = 128 31 / 32; the fp32 kernel's chain over a long K:
+    6144 -> 1536 M = 8 36 / 42, 7168 -> 1792 M = 8 42 / 49."""
+    return p >= 1024 or M * nb * q * p >= 800_000_000
+
+
 def blockdiag_multiply(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
     """x (..., nblocks*p), weight (nblocks, q, p) -> (..., nblocks*q)."""
     if not x.is_cuda:
@@ -97,7 +105,7 @@ class BlockdiagLinear(nn.Module):
             bias = bias.contiguous()
         nb, q, p = self.weight.shape
         M = x.numel() // x.shape[-1]
-        if _fp32_path(x) and p % 8 == 0 and ops.split_supported(M, nb, p, q):
+        if _fp32_path(x) and p % 8 == 0 and _parts_pay(M, nb, q, p) and ops.split_supported(M, nb, p, q):
             parts, _, w = ops.split_rows(x.reshape(-1, self.in_features_extended).contiguous(), nb, weights=(self.weight,))
             out = ops.split_linear(parts, w, M, nb, p, q, bias)
         elif _fp32_path(x) and p % 8 == 0:

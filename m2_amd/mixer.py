@@ -148,9 +148,16 @@ class MonarchMixerSequenceMixing(nn.Module):
         torch.mm(x, w.t(), out=out.t())
         return out
 
-    def _fp32_parts(self, M: int, w_in: torch.Tensor, w_out: torch.Tensor) -> bool:
+    def _fp32_parts(self, M: int):
+        """The weights of both projections where these go by parts, else None.  They pay for splitting the weights, and few rows leave their tiles idle: us for both with
+        the copies around them, by parts / library fp32: d = 768 M = 128 48 / 24, 512 49 / 35, 1024 61 / 54, 2048 75 / 107;
+        d = 960 M = 512 62 / 47, 1024 74 / 76, 2048 101 / 136; d = 1536 M = 512 118 / 91, 1024 135 / 179; d = 1792 M = 512
+        143 / 126, 1024 165 / 247.  The lines cross where M d is about 2^20."""
         d = self.d_model
-        return M % 4 == 0 and w_in.shape == (3 * d, d) and w_out.shape == (d, d) and ops.split_supported(M, 1, d, 3 * d)
+        if M * d < 1 << 20 or M % 4 or not ops.split_supported(M, 1, d, 3 * d):
+            return None
+        w_in, w_out = self.in_linear.weight, self.out_linear.weight
+        return (w_in, w_out) if w_in.shape == (3 * d, d) and w_out.shape == (d, d) else None
 
     def project_out(self, y: torch.Tensor, w_parts: Optional[torch.Tensor] = None) -> torch.Tensor:
         """y (d, M) channel-major -> y^T @ out_linear.weight^T + bias, (M, d), in y's dtype (bf16 or fp32).  `w_parts`: the parts
@@ -183,8 +190,8 @@ class MonarchMixerSequenceMixing(nn.Module):
                 if low:
                     u2 = u16
             x = u2.to(act).contiguous()
-            weights = None if low else (self.in_linear.weight, self.out_linear.weight)
-            if weights and self._fp32_parts(B * L, *weights) and not (x.requires_grad and torch.is_grad_enabled()):
+            weights = None if low or (x.requires_grad and torch.is_grad_enabled()) else self._fp32_parts(B * L)
+            if weights is not None:
                 parts, x_cm, w_in, w_out = ops.split_rows(x, channel_major=u_cm is None and self.residual_long_conv, weights=weights)
                 xproj = ops.split_to_channels(parts, w_in, B * L, 3 * d, d)
                 u_cm = x_cm if u_cm is None else u_cm

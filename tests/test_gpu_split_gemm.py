@@ -151,7 +151,8 @@ def test_split_of_several_operands_at_once(gpu, M, nb, p, shapes):
         assert torch.equal(whole[:, :K], w.view(-1, K)) and not whole[:, K:].any()
 
 
-def test_fp32_modules_read_the_weights_of_the_call(gpu):
+@pytest.mark.parametrize("B", [2, 11])              # the mixer's projections by the library and by parts
+def test_fp32_modules_read_the_weights_of_the_call(gpu, B):
     """Weights written through `.data`, computed anew per access, replaced at an old address, or changed between two replays of
     a captured graph: a result is always that of the weights as they are."""
     import copy
@@ -160,7 +161,7 @@ def test_fp32_modules_read_the_weights_of_the_call(gpu):
     from torch.nn.utils import parametrize
     cfg = m2_amd.m2_bert_80m(128)
     layer = m2_amd.BertLayer(cfg).to(gpu).eval()
-    u = torch.randn(2, 128, 768, generator=torch.Generator().manual_seed(6)).to(gpu)
+    u = torch.randn(B, 128, 768, generator=torch.Generator().manual_seed(6)).to(gpu)
     linears = [layer.attention.in_linear, layer.attention.out_linear, layer.mlp.gated_layers, layer.mlp.wo]
 
     class Scaled(torch.nn.Module):
@@ -208,3 +209,38 @@ def test_fp32_modules_read_the_weights_of_the_call(gpu):
                 lin.parametrizations.weight[0].factor = factor
                 other.weight.copy_(lin.parametrizations.weight.original * factor)
             assert torch.equal(layer(u), want(u)), factor
+
+
+# either side of the rules that choose between parts and the fp32 kernels
+@pytest.mark.parametrize("i,o,M", [(768, 6144, 677), (768, 6144, 679), (6144, 1536, 3), (3072, 768, 1357)])
+def test_fp32_blockdiag_linear_by_size(gpu, i, o, M):
+    import m2_amd
+    from m2_amd import blockdiag
+    lin = m2_amd.BlockdiagLinear(i, o, nblocks=4)
+    nb, q, p = lin.weight.shape
+    assert blockdiag._parts_pay(M, nb, q, p) == (M != 677)
+    x = _rand(torch.Generator().manual_seed(M), M, i)
+    w, b = lin.weight.detach().double(), lin.bias.detach().double()
+    ref, absref = _blockdiag(x.double(), w) + b, _blockdiag(x.double().abs(), w.abs()) + b.abs()
+    with torch.no_grad():
+        got = lin.to(gpu)(x.to(gpu))
+    # (the fp32 kernel: K / 4 additions of four products each)
+    assert ((got.double().cpu() - ref).abs() <= absref * (p / 2 + 8) * 2.0 ** -24).all()
+
+
+@pytest.mark.parametrize("L,B", [(128, 10), (128, 11)])
+def test_fp32_mixer_by_size(gpu, L, B):
+    import m2_amd
+    from oracle import m2_oracle as O
+    cfg = m2_amd.m2_bert_80m(L)
+    sd = m2_amd.seeded_state_dict(cfg, 3, what="mixer")
+    mix = m2_amd.MonarchMixerSequenceMixing(768, l_max=L, bidirectional=True, hyena_emb_dim=5, hyena_filter_order=128,
+                                            residual_long_conv=True, hyena_w=10)
+    mix.load_state_dict(sd)
+    mix = mix.to(gpu).eval()
+    assert (mix._fp32_parts(B * L) is not None) == (B == 11)
+    u = torch.randn(B, L, 768, generator=torch.Generator().manual_seed(4))
+    with torch.no_grad():
+        want = O.mixer_forward(O.cast_state_dict(sd, torch.float64), "", u.double())
+        got = mix(u.to(gpu))[0].double().cpu()
+    assert (got - want).norm() <= 1.6e-5 * want.norm()          # fp32 sums, four times what is measured
