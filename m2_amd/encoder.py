@@ -192,10 +192,12 @@ class BertGatedLinearUnitMLP(nn.Module):
         """The fp32 MLP as two products by parts, the gated one with its GELU: blocks of whole 32-value chunks between the two,
         nothing padded, and the submodules just what they are built as (no hooks, no other activation)."""
         gl, wo, act = self.gated_layers, self.wo, self.act
+        if type(gl) is not BlockdiagLinear or type(wo) is not BlockdiagLinear or type(act) is not nn.GELU or act.approximate != "none":
+            return False
+        if any(m._forward_hooks or m._forward_pre_hooks or "forward" in m.__dict__ for m in (gl, wo, act)):
+            return False
         (nb, q, p), M = gl.weight.shape, x.shape[0]
         I, d = self.config.intermediate_size, x.shape[1]
-        if any(m._forward_hooks or m._forward_pre_hooks for m in (gl, wo, act)) or type(act) is not nn.GELU or act.approximate != "none":
-            return False
         return (nb % 2 == 0 and p % 8 == 0 and q % 64 == 0 and nb * p == d and nb * q == 2 * I and tuple(wo.weight.shape) == (nb, d // nb, I // nb)
                 and gl.bias is None and wo.bias is not None and ops.split_supported(M, nb, p, q) and ops.split_supported(M, nb, I // nb, d // nb))
 

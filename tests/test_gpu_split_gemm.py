@@ -202,6 +202,8 @@ def test_fp32_modules_read_the_weights_of_the_call(gpu, B):
             torch.cuda.synchronize()
             assert torch.equal(held, want), factor
         want = copy.deepcopy(layer)
+        for m in (want.mlp.gated_layers, want.mlp.wo):          # a subclass, as parametrised modules are: the same way through the MLP
+            m.__class__ = type("Other", (m2_amd.BlockdiagLinear,), {})
         for lin in linears:
             parametrize.register_parametrization(lin, "weight", Scaled())
         for factor in (1.0, 1.5, 0.5, 2.0, 0.75):
@@ -244,3 +246,50 @@ def test_fp32_mixer_by_size(gpu, L, B):
         want = O.mixer_forward(O.cast_state_dict(sd, torch.float64), "", u.double())
         got = mix(u.to(gpu))[0].double().cpu()
     assert (got - want).norm() <= 1.6e-5 * want.norm()          # fp32 sums, four times what is measured
+
+
+def test_fp32_mlp_calls_what_stands_in_for_its_linears(gpu):
+    """A dense layer, a module without a weight, a subclass and an instance with a forward of their own in the place of
+    gated_layers or wo: called, as with any other nn.Module."""
+    import m2_amd
+    mlp = m2_amd.BertLayer(m2_amd.m2_bert_80m(128)).to(gpu).eval().mlp
+    x = _rand(torch.Generator().manual_seed(9), 40, 768).to(gpu)
+
+    class Doubled(m2_amd.BlockdiagLinear):
+        def forward(self, v):
+            return 2 * super().forward(v)
+
+    class Wrapped(torch.nn.Module):
+        def __init__(self, inner):
+            super().__init__()
+            self.inner = inner
+
+        def forward(self, v):
+            return 2 * self.inner(v)
+
+    with torch.no_grad():
+        plain = mlp(x)
+        w, b = mlp.wo.weight.clone(), mlp.wo.bias.clone()
+        mlp.wo.weight.mul_(2)
+        mlp.wo.bias.mul_(2)
+        doubled = mlp(x)
+        mlp.wo.weight.copy_(w)
+        mlp.wo.bias.copy_(b)
+        assert (plain - doubled).abs().max() > 1e-2
+        inner = mlp.wo
+        mlp.wo = Wrapped(inner)
+        assert (mlp(x) - doubled).abs().max() < 1e-5
+        mlp.wo = inner
+        inner.__class__ = Doubled
+        assert (mlp(x) - doubled).abs().max() < 1e-5
+        inner.__class__ = m2_amd.BlockdiagLinear
+        inner.forward = lambda v: 2 * m2_amd.BlockdiagLinear.forward(inner, v)
+        assert (mlp(x) - doubled).abs().max() < 1e-5
+        del inner.forward
+        assert torch.equal(mlp(x), plain)
+        dense = torch.nn.Linear(768, 6144, bias=False).to(gpu)
+        for k in range(4):
+            dense.weight.zero_() if k == 0 else None
+            dense.weight[k * 1536:(k + 1) * 1536, k * 192:(k + 1) * 192] = mlp.gated_layers.weight[k]
+        mlp.gated_layers = dense
+        assert (mlp(x) - plain).abs().max() < 1e-4
