@@ -368,7 +368,9 @@ class BertEncoder(nn.Module):
                     h16 = h32.to(torch.bfloat16)
                 if hT is None:
                     hT = h32.t().contiguous()
-                plan = schedule.stack_plan(self, None, B, L)
+                # (an input that requires grad goes to the projections, which refuse it)
+                graded = torch.is_grad_enabled() and (h16.requires_grad or hT.requires_grad)
+                plan = None if graded else schedule.stack_plan(self, None, B, L)
                 if plan is not None:
                     return plan.run(B, all_layers, h16, hT)
             outs = []

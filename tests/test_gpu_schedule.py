@@ -168,3 +168,20 @@ def test_a_graph_keeps_what_it_reads(gpu):
         model.encoder._native_plans.clear()
         model.encoder._filter_table = None
         assert gone() is None
+
+
+@pytest.mark.parametrize("native", [True, False])
+def test_an_input_that_requires_grad_is_refused(gpu, native):
+    """There is no backward: hidden states that require grad raise instead of coming back detached."""
+    import m2_amd
+    cfg = m2_amd.m2_bert_80m(128)
+    cfg.num_hidden_layers = 1
+    enc = m2_amd.BertEncoder(cfg).to(gpu).eval()
+    enc.native_schedule = native
+    h = torch.randn(2, 128, 768, generator=torch.Generator().manual_seed(1)).to(gpu)
+    want = enc(h)[-1]
+    h.requires_grad_()
+    with pytest.raises(RuntimeError):
+        enc(h)
+    with torch.no_grad():
+        assert torch.equal(enc(h)[-1], want)
