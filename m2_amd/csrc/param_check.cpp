@@ -1,9 +1,11 @@
 // CPython extension m2_amd._param_check: "are these still the tensors a plan was made from?"
 //
 // A plan of the native schedule (m2_amd/schedule.py) holds device addresses of some fifty tensors per layer and copies
-// derived from four of them.  Before every use each tensor is looked up again where the modules keep it and its address
-// (and, for those that copies were made from, its version counter) compared; so is every module on the way there.  For
-// 12 layers that is about 1,100 look-ups: 0.1 ms in Python, 15 us here.
+// derived from four of them.  Before every use each tensor is looked up again where the modules keep it and its storage and
+// address (and, for those that copies were made from, its version counter) compared; so is every module on the way there.  For
+// 12 layers that is about 1,100 look-ups: 0.1 ms in Python, 15 us here.  An address alone says little: the allocator gives it out
+// again, and assigning to `.data` leaves the version counter where it was.  The weak reference keeps no memory alive but the
+// storage's own record, so that no other storage can take its place.
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
 #include <torch/csrc/autograd/python_variable.h>
@@ -17,6 +19,7 @@ struct ModuleSlot {
 };
 struct TensorSlot {
   PyObject *dict, *key;
+  c10::weak_intrusive_ptr<c10::StorageImpl> storage;
   const void* data;
   int64_t version;      // -1: not compared
 };
@@ -26,14 +29,18 @@ struct Checker {
   std::vector<TensorSlot>* tensors;
 };
 
-bool read_tensor(PyObject* dict, PyObject* key, const void** data, int64_t* version) {
+// The tensor at dict[key], or null (with or without a Python error).
+const at::Tensor* look_up(PyObject* dict, PyObject* key) {
   PyObject* o = PyDict_GetItemWithError(dict, key);
-  if (!o || !THPVariable_Check(o)) return false;
+  if (!o || !THPVariable_Check(o)) return nullptr;
   const at::Tensor& t = THPVariable_Unpack(o);
-  if (!t.defined()) return false;
-  *data = t.const_data_ptr();
-  if (*version >= 0) *version = t.is_inference() ? 0 : t._version();
-  return true;
+  return t.defined() && t.has_storage() ? &t : nullptr;
+}
+int64_t version_of(const at::Tensor& t) { return t.is_inference() ? 0 : t._version(); }
+
+bool same(const TensorSlot& s, const at::Tensor& t) {
+  return t.storage().unsafeGetStorageImpl() == s.storage._unsafe_get_target() && t.const_data_ptr() == s.data &&
+         (s.version < 0 || version_of(t) == s.version);
 }
 
 void checker_dealloc(PyObject* self) {
@@ -73,14 +80,14 @@ PyObject* checker_new(PyTypeObject* type, PyObject* args, PyObject*) {
     PyObject *dict, *key;
     int ver;
     if (!PyArg_ParseTuple(PyList_GET_ITEM(tens, i), "O!Op", &PyDict_Type, &dict, &key, &ver)) { Py_DECREF(c); return nullptr; }
-    TensorSlot s{dict, key, nullptr, ver ? 0 : -1};
-    if (!read_tensor(dict, key, &s.data, &s.version)) {
+    const at::Tensor* t = look_up(dict, key);
+    if (!t) {
       if (!PyErr_Occurred()) PyErr_SetObject(PyExc_KeyError, key);
       Py_DECREF(c);
       return nullptr;
     }
+    c->tensors->push_back({dict, key, t->storage().getWeakStorageImpl(), t->const_data_ptr(), ver ? version_of(*t) : -1});
     Py_INCREF(dict); Py_INCREF(key);
-    c->tensors->push_back(s);
   }
   return reinterpret_cast<PyObject*>(c);
 }
@@ -93,10 +100,9 @@ PyObject* checker_unchanged(PyObject* self, PyObject*) {
       if (PyErr_Occurred()) return nullptr;
       Py_RETURN_FALSE;
     }
-  for (const auto& t : *c->tensors) {
-    const void* data;
-    int64_t version = t.version < 0 ? -1 : 0;
-    if (!read_tensor(t.dict, t.key, &data, &version) || data != t.data || version != t.version) {
+  for (const auto& s : *c->tensors) {
+    const at::Tensor* t = look_up(s.dict, s.key);
+    if (!t || !same(s, *t)) {
       if (PyErr_Occurred()) return nullptr;
       Py_RETURN_FALSE;
     }

@@ -185,3 +185,26 @@ def test_an_input_that_requires_grad_is_refused(gpu, native):
         enc(h)
     with torch.no_grad():
         assert torch.equal(enc(h)[-1], want)
+
+
+def test_a_weight_at_the_address_of_an_earlier_one(gpu):
+    """Plans outlive weights that are replaced while forwards of another length run; an address comes back (as the allocator
+    gives it out again) and `.data` keeps the version counter: the plan must not take the new weight for the old one."""
+    import m2_amd
+    cfg = m2_amd.m2_bert_80m(256)
+    cfg.num_hidden_layers = 1
+    model = _model(cfg, gpu, 21)
+    short, long = _ids(cfg, 1, 128, 22, gpu), _ids(cfg, 1, 256, 23, gpu)
+    at, mlp = model.encoder.layer[0].attention, model.encoder.layer[0].mlp
+    for lin in (at.in_linear, at.out_linear, mlp.gated_layers, mlp.wo):
+        memory = lin.weight.detach().clone()
+        lin.weight.data = torch.from_dlpack(memory)             # a storage of its own on that memory
+        (before, _), _ = _both(model, short)
+        address, version = lin.weight.data_ptr(), lin.weight._version
+        lin.weight.data = memory * 1.5
+        model(long)                                             # the module's own copy is made anew here
+        memory.mul_(2.0)
+        lin.weight.data = torch.from_dlpack(memory)
+        assert (lin.weight.data_ptr(), lin.weight._version) == (address, version)
+        (got, _), (want, _) = _both(model, short)
+        assert torch.equal(got, want) and not torch.equal(got, before)

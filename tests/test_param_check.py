@@ -1,0 +1,50 @@
+"""The check behind the plans of the native schedule (m2_amd/csrc/param_check.cpp), on CPU tensors: what a plan depends on is
+recognised as changed whichever way it was changed."""
+import numpy as np
+import torch
+
+from m2_amd import _param_check
+
+
+def _checker(mod, key="weight", version=True):
+    return _param_check.Checker([], [(mod._parameters, key, version)])
+
+
+def test_another_tensor_at_the_same_address_is_another():
+    """As when the allocator gives the address of a freed weight out again: same address, same version, another storage."""
+    memory = np.zeros((8, 8), dtype=np.float32)
+    lin = torch.nn.Linear(8, 8)
+    lin.weight = torch.nn.Parameter(torch.from_numpy(memory))
+    check, address, version = _checker(lin), lin.weight.data_ptr(), lin.weight._version
+    assert check.unchanged()
+    lin.weight = None
+    assert not check.unchanged()
+    lin.weight = torch.nn.Parameter(torch.from_numpy(memory))
+    assert (lin.weight.data_ptr(), lin.weight._version) == (address, version)
+    assert not check.unchanged()
+
+
+def test_a_view_of_the_recorded_storage_is_the_recorded_tensor():
+    lin = torch.nn.Linear(8, 8)
+    check = _checker(lin)
+    lin.weight = torch.nn.Parameter(lin.weight.detach())
+    assert check.unchanged()
+
+
+def test_data_assigned_twice_is_noticed():
+    lin = torch.nn.Linear(8, 8)
+    check, version = _checker(lin), lin.weight._version
+    lin.weight.data = lin.weight.data * 2
+    assert lin.weight._version == version and not check.unchanged()
+    check = _checker(lin)
+    lin.weight.data = lin.weight.data * 2
+    lin.weight.data = lin.weight.data * 2
+    assert not check.unchanged()
+
+
+def test_versions_count_where_a_copy_was_made():
+    lin = torch.nn.Linear(8, 8)
+    copied, in_place = _checker(lin), _checker(lin, version=False)
+    with torch.no_grad():
+        lin.weight.add_(1)
+    assert not copied.unchanged() and in_place.unchanged()
