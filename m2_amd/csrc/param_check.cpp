@@ -2,8 +2,8 @@
 //
 // A plan of the native schedule (m2_amd/schedule.py) holds device addresses of some fifty tensors per layer and copies
 // derived from four of them.  Before every use each tensor is looked up again where the modules keep it and its storage and
-// address (and, for those that copies were made from, its version counter) compared; so is every module on the way there.  For
-// 12 layers that is about 1,100 look-ups: 0.1 ms in Python, 15 us here.  An address alone says little: the allocator gives it out
+// address (and, for those that copies were made from, its version counter) compared; so is every module on the way there, and
+// every plain number that went into the plan (epsilons, filter constants, options).  For 12 layers that is about 1,300 look-ups: 0.1 ms in Python, 15 us here.  An address alone says little: the allocator gives it out
 // again, and assigning to `.data` leaves the version counter where it was.  The weak reference keeps no memory alive but the
 // storage's own record, so that no other storage can take its place.
 #define PY_SSIZE_T_CLEAN
@@ -23,10 +23,14 @@ struct TensorSlot {
   const void* data;
   int64_t version;      // -1: not compared
 };
+struct ValueSlot {
+  PyObject *dict, *key, *expected;
+};
 struct Checker {
   PyObject_HEAD
   std::vector<ModuleSlot>* modules;
   std::vector<TensorSlot>* tensors;
+  std::vector<ValueSlot>* values;
 };
 
 // The tensor at dict[key], or null (with or without a Python error).
@@ -35,6 +39,12 @@ const at::Tensor* look_up(PyObject* dict, PyObject* key) {
   if (!o || !THPVariable_Check(o)) return nullptr;
   const at::Tensor& t = THPVariable_Unpack(o);
   return t.defined() && t.has_storage() ? &t : nullptr;
+}
+// Equal plain values: the object itself, or a number or text of the same type that compares equal.
+bool same_value(PyObject* a, PyObject* b) {
+  if (a == b) return true;
+  if (!a || Py_TYPE(a) != Py_TYPE(b) || !(PyFloat_CheckExact(a) || PyLong_CheckExact(a) || PyUnicode_CheckExact(a))) return false;
+  return PyObject_RichCompareBool(a, b, Py_EQ) == 1;
 }
 int64_t version_of(const at::Tensor& t) { return t.is_inference() ? 0 : t._version(); }
 
@@ -53,29 +63,41 @@ void checker_dealloc(PyObject* self) {
     for (auto& t : *c->tensors) { Py_DECREF(t.dict); Py_DECREF(t.key); }
     delete c->tensors;
   }
+  if (c->values) {
+    for (auto& v : *c->values) { Py_DECREF(v.dict); Py_DECREF(v.key); Py_DECREF(v.expected); }
+    delete c->values;
+  }
   Py_TYPE(self)->tp_free(self);
 }
 
-// Checker(modules, tensors): sequences of (dict, key) and (dict, key, compare_version); the present state is recorded.
+// (dict, key) pairs and the object at each of them
+template <typename Slot>
+bool record(PyObject* list, std::vector<Slot>* slots) {
+  for (Py_ssize_t i = 0; i < PyList_GET_SIZE(list); ++i) {
+    PyObject *dict, *key;
+    if (!PyArg_ParseTuple(PyList_GET_ITEM(list, i), "O!O", &PyDict_Type, &dict, &key)) return false;
+    PyObject* o = PyDict_GetItemWithError(dict, key);
+    if (!o) {
+      if (!PyErr_Occurred()) PyErr_SetObject(PyExc_KeyError, key);
+      return false;
+    }
+    slots->push_back({dict, key, o});
+    Py_INCREF(dict); Py_INCREF(key); Py_INCREF(o);
+  }
+  return true;
+}
+
+// Checker(modules, tensors, values): lists of (dict, key), (dict, key, compare_version) and (dict, key); the present state is
+// recorded.
 PyObject* checker_new(PyTypeObject* type, PyObject* args, PyObject*) {
-  PyObject *mods, *tens;
-  if (!PyArg_ParseTuple(args, "O!O!", &PyList_Type, &mods, &PyList_Type, &tens)) return nullptr;
+  PyObject *mods, *tens, *vals;
+  if (!PyArg_ParseTuple(args, "O!O!O!", &PyList_Type, &mods, &PyList_Type, &tens, &PyList_Type, &vals)) return nullptr;
   Checker* c = reinterpret_cast<Checker*>(type->tp_alloc(type, 0));
   if (!c) return nullptr;
   c->modules = new std::vector<ModuleSlot>();
   c->tensors = new std::vector<TensorSlot>();
-  for (Py_ssize_t i = 0; i < PyList_GET_SIZE(mods); ++i) {
-    PyObject *dict, *key;
-    if (!PyArg_ParseTuple(PyList_GET_ITEM(mods, i), "O!O", &PyDict_Type, &dict, &key)) { Py_DECREF(c); return nullptr; }
-    PyObject* o = PyDict_GetItemWithError(dict, key);
-    if (!o) {
-      if (!PyErr_Occurred()) PyErr_SetObject(PyExc_KeyError, key);
-      Py_DECREF(c);
-      return nullptr;
-    }
-    Py_INCREF(dict); Py_INCREF(key); Py_INCREF(o);
-    c->modules->push_back({dict, key, o});
-  }
+  c->values = new std::vector<ValueSlot>();
+  if (!record(mods, c->modules) || !record(vals, c->values)) { Py_DECREF(c); return nullptr; }
   for (Py_ssize_t i = 0; i < PyList_GET_SIZE(tens); ++i) {
     PyObject *dict, *key;
     int ver;
@@ -100,6 +122,11 @@ PyObject* checker_unchanged(PyObject* self, PyObject*) {
       if (PyErr_Occurred()) return nullptr;
       Py_RETURN_FALSE;
     }
+  for (const auto& v : *c->values)
+    if (!same_value(PyDict_GetItemWithError(v.dict, v.key), v.expected)) {
+      if (PyErr_Occurred()) return nullptr;
+      Py_RETURN_FALSE;
+    }
   for (const auto& s : *c->tensors) {
     const at::Tensor* t = look_up(s.dict, s.key);
     if (!t || !same(s, *t)) {
@@ -110,7 +137,7 @@ PyObject* checker_unchanged(PyObject* self, PyObject*) {
   Py_RETURN_TRUE;
 }
 
-PyMethodDef checker_methods[] = {{"unchanged", checker_unchanged, METH_NOARGS, "True if every module and tensor is as recorded."},
+PyMethodDef checker_methods[] = {{"unchanged", checker_unchanged, METH_NOARGS, "True if every module, tensor and value is as recorded."},
                                  {nullptr, nullptr, 0, nullptr}};
 PyTypeObject CheckerType = {PyVarObject_HEAD_INIT(nullptr, 0) "m2_amd._param_check.Checker"};
 PyModuleDef module_def = {PyModuleDef_HEAD_INIT, "_param_check", nullptr, -1, nullptr};

@@ -3,8 +3,9 @@
 `BertEncoder._run_layers` walks over its layers in Python, about 170 us of host time per layer and 0.2 ms more for the
 filter table, which is what a short forward then costs whatever the GPU does (L = 128, B = 1: 2.4 ms for 0.75 ms of
 kernels).  A `StackPlan` holds what the calls need: the layers' device pointers, the bf16 and packed copies of the
-weights, the filter pointer table.  It is made once and, before each use, compared tensor by tensor with what the modules
-hold now (address, and version counter for the weights that copies were made from): `_param_check.Checker`.
+weights, the filter pointer table.  It is made once and, before each use, compared with what the modules hold now, tensor
+by tensor (storage and address, and version counter for the weights that copies were made from) and value by value:
+`_param_check.Checker`.
 
 Same kernels in the same order on the current stream as the Python schedule, hence the same bits.  It serves row counts
 whose projections run on the library's own kernels; larger forwards, whose host time hides behind the GPU's, and encoders
@@ -33,8 +34,9 @@ class StackPlan:
     """Device pointers of an encoder's layers (and of the embeddings in front of it) for one length and MLP route."""
 
     def __init__(self, encoder, embeddings, L: int, fused_mlp: bool, few_rows: bool):
-        # (dict, key) of every module and (dict, key, compare the version) of every tensor the plan depends on
-        mods, tens = [(encoder._modules, "layer")], []
+        # (dict, key) of every module, (dict, key, compare the version) of every tensor and (dict, key) of every plain value that
+        # the plan depends on
+        mods, tens, vals = [(encoder._modules, "layer")], [], []
 
         def child(mod, key):
             mods.append((mod._modules, key))
@@ -48,6 +50,12 @@ class StackPlan:
                 raise ValueError("parameters that are not plain fp32")
             return t
 
+        def value(obj, key):
+            if key not in obj.__dict__:
+                raise ValueError(f"no plain attribute {key}")
+            vals.append((obj.__dict__, key))
+            return obj.__dict__[key]
+
         stack = encoder._modules["layer"]
         n = len(stack._modules)
         self.layers = n
@@ -57,13 +65,17 @@ class StackPlan:
         for i, key in enumerate(stack._modules):
             lay = child(stack, key)
             at, mlp = child(lay, "attention"), child(lay, "mlp")
-            for name in ("filter_fn", "filter_fn2")[:2 if at.residual_long_conv else 1]:
+            for name in ("filter_fn", "filter_fn2")[:2 if value(at, "residual_long_conv") else 1]:
                 f = child(at, name)
                 skips.append(tensor(f, "bias"))
                 emb = child(f, "pos_emb")
                 fwd = child(f, "implicit_filter")
-                row = [tensor(emb, "z"), tensor(emb, "t"), tensor(child(fwd, "1"), "freq"), tensor(child(f, "modulation"), "deltas")]
-                for seq in (fwd, child(f, "implicit_filter_rev") if at.bidirectional else None):
+                mod = child(f, "modulation")
+                for key_ in ("order", "emb_dim", "w_mod"):
+                    value(f, key_)
+                value(mod, "shift")
+                row = [tensor(emb, "z"), tensor(emb, "t"), tensor(child(fwd, "1"), "freq"), tensor(mod, "deltas")]
+                for seq in (fwd, child(f, "implicit_filter_rev") if value(f, "bidirectional") else None):
                     if seq is None:
                         row += [None] * 7
                         continue
@@ -85,13 +97,17 @@ class StackPlan:
             p.in_w, p.out_w, p.w_gated, p.w_out = w_in.data_ptr(), w_out.data_ptr(), wg16.data_ptr(), wo16.data_ptr()
             (p.in_b, p.out_b, p.short_w, p.short_b, p.wo_b, p.ln_gamma, p.ln_beta) = [t.data_ptr() for t in in_place]
             p.residual = 1 if at.residual_long_conv else 0
+            value(at, "d_model")
+            value(at, "bidirectional")
+            cfg = value(mlp, "config")
+            sizes = (value(cfg, "intermediate_size"), value(cfg, "monarch_mlp_nblocks"), float(value(ln, "eps")))
             if i == 0:
                 f0 = at.filter_fn
-                self.d, self.I, self.nb = at.d_model, mlp.config.intermediate_size, mlp.config.monarch_mlp_nblocks
-                self.eps = float(ln.eps)
+                self.d = at.d_model
+                self.I, self.nb, self.eps = sizes
                 self.w_mod, self.shift = float(f0.w_mod), float(f0.modulation.shift)
                 stream_glu = not fused_mlp and not few_rows and ops.glu_stream_supported(self.d, self.I, self.nb)
-            elif (mlp.config.intermediate_size, mlp.config.monarch_mlp_nblocks, float(ln.eps)) != (self.I, self.nb, self.eps):
+            elif sizes != (self.I, self.nb, self.eps):
                 raise ValueError("layers that differ")
             if fused_mlp:
                 self.keep.append(mlp.packed_mlp(wg16, wo16))
@@ -104,16 +120,16 @@ class StackPlan:
         if embeddings is not None:
             e = embeddings
             word, typ = tensor(child(e, "word_embeddings"), "weight"), tensor(child(e, "token_type_embeddings"), "weight")
-            pos = tensor(child(e, "position_embeddings"), "weight") if e.use_positional_encodings else None
+            pos = tensor(child(e, "position_embeddings"), "weight") if value(e, "use_positional_encodings") else None
             ln = child(e, "LayerNorm")
             g, b = tensor(ln, "weight"), tensor(ln, "bias")
             tens.append((e._buffers, "_bad_index", _IN_PLACE))
             if any(t is not None and (t.dim() != 2 or t.shape[1] != self.d) for t in (word, typ, pos)) or g.shape != (self.d,):
                 raise ValueError("embedding tables of another width")
             self.embed = (word.data_ptr(), typ.data_ptr(), None if pos is None else pos.data_ptr(), word.shape[0], typ.shape[0],
-                          0 if pos is None else pos.shape[0], g.data_ptr(), b.data_ptr(), float(ln.eps))
+                          0 if pos is None else pos.shape[0], g.data_ptr(), b.data_ptr(), float(value(ln, "eps")))
             self.bad_index = e._bad_index.data_ptr()
-        self.checker = _param_check.Checker(mods, tens)
+        self.checker = _param_check.Checker(mods, tens, vals)
         self.L = L
         self.spec_bytes = lib.m2_filter_spectrum_bytes(self.d, L)
         self.filter_ws = lib.m2_mixer_filters_workspace_bytes(n, self.table.fpm, L, self.d, self.table.order)

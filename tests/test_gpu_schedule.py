@@ -208,3 +208,43 @@ def test_a_weight_at_the_address_of_an_earlier_one(gpu):
         assert (lin.weight.data_ptr(), lin.weight._version) == (address, version)
         (got, _), (want, _) = _both(model, short)
         assert torch.equal(got, want) and not torch.equal(got, before)
+
+
+def test_plans_follow_plain_values(gpu):
+    """Epsilons, filter constants and options are read by every forward: a plan made before they were changed is not used."""
+    import m2_amd
+    cfg = m2_amd.m2_bert_80m(128)
+    cfg.num_hidden_layers = 2
+    model = _model(cfg, gpu, 24)
+    ids = _ids(cfg, 2, 128, 25, gpu)
+    (prev, _), _ = _both(model, ids)
+    lays = model.encoder.layer
+
+    def changed(what):
+        nonlocal prev
+        model.encoder.native_schedule = True
+        got, _ = model(ids)
+        model.encoder.native_schedule = False
+        want, _ = model(ids)
+        assert torch.equal(got, want) and not torch.equal(got, prev), what
+        prev = got
+
+    lays[1].mlp.layernorm.eps = 0.3
+    changed("one layer's epsilon")
+    lays[0].mlp.layernorm.eps = 0.3
+    changed("both layers' epsilon")
+    model.embeddings.LayerNorm.eps = 0.2
+    changed("epsilon of the embeddings")
+    for lay in lays:
+        for f in (lay.attention.filter_fn, lay.attention.filter_fn2):
+            f.modulation.shift = 0.1
+    changed("shift")
+    for lay in lays:
+        for f in (lay.attention.filter_fn, lay.attention.filter_fn2):
+            f.w_mod = 2
+    changed("w_mod")
+    for lay in lays:
+        lay.attention.residual_long_conv = False
+    changed("without the residual convolution")
+    model.embeddings.use_positional_encodings = False
+    changed("without positions")

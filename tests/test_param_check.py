@@ -1,13 +1,14 @@
 """The check behind the plans of the native schedule (m2_amd/csrc/param_check.cpp), on CPU tensors: what a plan depends on is
 recognised as changed whichever way it was changed."""
 import numpy as np
+import pytest
 import torch
 
 from m2_amd import _param_check
 
 
 def _checker(mod, key="weight", version=True):
-    return _param_check.Checker([], [(mod._parameters, key, version)])
+    return _param_check.Checker([], [(mod._parameters, key, version)], [])
 
 
 def test_another_tensor_at_the_same_address_is_another():
@@ -48,3 +49,19 @@ def test_versions_count_where_a_copy_was_made():
     with torch.no_grad():
         lin.weight.add_(1)
     assert not copied.unchanged() and in_place.unchanged()
+
+
+@pytest.mark.parametrize("value,others", [(1e-12, (1e-5, 1, None)), (3, (4, 3.0, True)), (None, (0, 0.0)), (True, (False, 1)),
+                                          (float(2.5), (2.25,)), ("a", ("b", 1))])
+def test_plain_values_are_compared(value, others):
+    lin = torch.nn.LayerNorm(8)
+    lin.eps = value
+    check = _param_check.Checker([], [], [(lin.__dict__, "eps")])
+    assert check.unchanged()
+    for other in others:
+        lin.eps = other
+        assert not check.unchanged(), other
+    lin.eps = float(str(value)) if isinstance(value, float) else value          # an equal number, another object
+    assert check.unchanged()
+    del lin.eps
+    assert not check.unchanged()
