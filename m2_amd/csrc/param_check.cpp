@@ -1,8 +1,8 @@
 // CPython extension m2_amd._param_check: "are these still the tensors a plan was made from?"
 //
 // A plan of the native schedule (m2_amd/schedule.py) holds device addresses of some fifty tensors per layer and copies
-// derived from four of them.  Before every use each tensor is looked up again where the modules keep it and its storage and
-// address (and, for those that copies were made from, its version counter) compared; so is every module on the way there, and
+// derived from four of them.  Before every use each tensor is looked up again where the modules keep it and its storage, address,
+// type and shape (and, for those that copies were made from, its version counter) compared; so is every module on the way there, and
 // every plain number that went into the plan (epsilons, filter constants, options).  For 12 layers that is about 1,300 look-ups: 0.1 ms in Python, 15 us here.  An address alone says little: the allocator gives it out
 // again, and assigning to `.data` leaves the version counter where it was.  The weak reference keeps no memory alive but the
 // storage's own record, so that no other storage can take its place.
@@ -22,6 +22,8 @@ struct TensorSlot {
   c10::weak_intrusive_ptr<c10::StorageImpl> storage;
   const void* data;
   int64_t version;      // -1: not compared
+  at::ScalarType dtype;
+  c10::SmallVector<int64_t, 4> sizes, strides;
 };
 struct ValueSlot {
   PyObject *dict, *key, *expected;
@@ -50,7 +52,7 @@ int64_t version_of(const at::Tensor& t) { return t.is_inference() ? 0 : t._versi
 
 bool same(const TensorSlot& s, const at::Tensor& t) {
   return t.storage().unsafeGetStorageImpl() == s.storage._unsafe_get_target() && t.const_data_ptr() == s.data &&
-         (s.version < 0 || version_of(t) == s.version);
+         t.scalar_type() == s.dtype && t.sizes().equals(s.sizes) && t.strides().equals(s.strides) && (s.version < 0 || version_of(t) == s.version);
 }
 
 void checker_dealloc(PyObject* self) {
@@ -108,7 +110,8 @@ PyObject* checker_new(PyTypeObject* type, PyObject* args, PyObject*) {
       Py_DECREF(c);
       return nullptr;
     }
-    c->tensors->push_back({dict, key, t->storage().getWeakStorageImpl(), t->const_data_ptr(), ver ? version_of(*t) : -1});
+    c->tensors->push_back({dict, key, t->storage().getWeakStorageImpl(), t->const_data_ptr(), ver ? version_of(*t) : -1, t->scalar_type(),
+                          {t->sizes().begin(), t->sizes().end()}, {t->strides().begin(), t->strides().end()}});
     Py_INCREF(dict); Py_INCREF(key);
   }
   return reinterpret_cast<PyObject*>(c);

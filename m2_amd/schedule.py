@@ -4,7 +4,7 @@
 filter table, which is what a short forward then costs whatever the GPU does (L = 128, B = 1: 2.4 ms for 0.75 ms of
 kernels).  A `StackPlan` holds what the calls need: the layers' device pointers, the bf16 and packed copies of the
 weights, the filter pointer table.  It is made once and, before each use, compared with what the modules hold now, tensor
-by tensor (storage and address, and version counter for the weights that copies were made from) and value by value:
+by tensor (storage, address and shape, and version counter for the weights that copies were made from) and value by value:
 `_param_check.Checker`.
 
 Same kernels in the same order on the current stream as the Python schedule, hence the same bits.  It serves row counts
@@ -42,12 +42,14 @@ class StackPlan:
             mods.append((mod._modules, key))
             return mod._modules[key]
 
-        def tensor(mod, key, how=_IN_PLACE):
+        def tensor(mod, key, how=_IN_PLACE, shape=None):
             where = mod._parameters if key in mod._parameters else mod._buffers
             tens.append((where, key, how))
             t = where[key]
             if not (t.is_cuda and t.dtype == torch.float32 and t.is_contiguous()):
                 raise ValueError("parameters that are not plain fp32")
+            if shape is not None and t.shape != shape:      # the kernels take sizes, not shapes: never read beyond a tensor
+                raise ValueError(f"{key} of shape {tuple(t.shape)} where {shape} is expected")
             return t
 
         def value(obj, key):
@@ -86,10 +88,15 @@ class StackPlan:
                 rows.append(row)
             lin_in, lin_out, short = child(at, "in_linear"), child(at, "out_linear"), child(at, "short_filter")
             gated, wo, ln = child(mlp, "gated_layers"), child(mlp, "wo"), child(mlp, "layernorm")
-            in_place = [tensor(lin_in, "bias"), tensor(lin_out, "bias"), tensor(short, "weight"), tensor(short, "bias"),
-                        tensor(wo, "bias"), tensor(ln, "weight"), tensor(ln, "bias")]
-            for m in (lin_in, lin_out, gated, wo):
-                tensor(m, "weight", _COPIED)
+            cfg = value(mlp, "config")
+            d, I, nb = value(at, "d_model"), value(cfg, "intermediate_size"), value(cfg, "monarch_mlp_nblocks")
+            if d % nb or I % nb:
+                raise ValueError("padded blocks")
+            in_place = [tensor(lin_in, "bias", shape=(3 * d,)), tensor(lin_out, "bias", shape=(d,)),
+                        tensor(short, "weight", shape=(3 * d, 1, 3)), tensor(short, "bias", shape=(3 * d,)),
+                        tensor(wo, "bias", shape=(d,)), tensor(ln, "weight", shape=(d,)), tensor(ln, "bias", shape=(d,))]
+            for m, shape in ((lin_in, (3 * d, d)), (lin_out, (d, d)), (gated, (nb, 2 * I // nb, d // nb)), (wo, (nb, d // nb, I // nb))):
+                tensor(m, "weight", _COPIED, shape)
             w_in, w_out = at._cast("in_w", lin_in.weight, torch.bfloat16), at._cast("out_w", lin_out.weight, torch.bfloat16)
             wg16, wo16 = gated.weight_bf16(), wo.weight_bf16()
             self.keep += [w_in, w_out, wg16, wo16]
@@ -97,17 +104,14 @@ class StackPlan:
             p.in_w, p.out_w, p.w_gated, p.w_out = w_in.data_ptr(), w_out.data_ptr(), wg16.data_ptr(), wo16.data_ptr()
             (p.in_b, p.out_b, p.short_w, p.short_b, p.wo_b, p.ln_gamma, p.ln_beta) = [t.data_ptr() for t in in_place]
             p.residual = 1 if at.residual_long_conv else 0
-            value(at, "d_model")
             value(at, "bidirectional")
-            cfg = value(mlp, "config")
-            sizes = (value(cfg, "intermediate_size"), value(cfg, "monarch_mlp_nblocks"), float(value(ln, "eps")))
+            sizes = (d, I, nb, float(value(ln, "eps")))
             if i == 0:
                 f0 = at.filter_fn
-                self.d = at.d_model
-                self.I, self.nb, self.eps = sizes
+                self.d, self.I, self.nb, self.eps = sizes
                 self.w_mod, self.shift = float(f0.w_mod), float(f0.modulation.shift)
                 stream_glu = not fused_mlp and not few_rows and ops.glu_stream_supported(self.d, self.I, self.nb)
-            elif sizes != (self.I, self.nb, self.eps):
+            elif sizes != (self.d, self.I, self.nb, self.eps):
                 raise ValueError("layers that differ")
             if fused_mlp:
                 self.keep.append(mlp.packed_mlp(wg16, wo16))
@@ -124,7 +128,7 @@ class StackPlan:
             ln = child(e, "LayerNorm")
             g, b = tensor(ln, "weight"), tensor(ln, "bias")
             tens.append((e._buffers, "_bad_index", _IN_PLACE))
-            if any(t is not None and (t.dim() != 2 or t.shape[1] != self.d) for t in (word, typ, pos)) or g.shape != (self.d,):
+            if any(t is not None and (t.dim() != 2 or t.shape[1] != self.d) for t in (word, typ, pos)) or g.shape != (self.d,) or b.shape != (self.d,):
                 raise ValueError("embedding tables of another width")
             self.embed = (word.data_ptr(), typ.data_ptr(), None if pos is None else pos.data_ptr(), word.shape[0], typ.shape[0],
                           0 if pos is None else pos.shape[0], g.data_ptr(), b.data_ptr(), float(value(ln, "eps")))

@@ -248,3 +248,32 @@ def test_plans_follow_plain_values(gpu):
     changed("without the residual convolution")
     model.embeddings.use_positional_encodings = False
     changed("without positions")
+
+
+def test_a_narrowed_table_and_wrong_shapes(gpu):
+    """Rows cut off a table after a plan was made are rows no id may name; a parameter of another shape is refused, not read past its
+    end."""
+    import m2_amd
+    cfg = m2_amd.m2_bert_80m(128)
+    cfg.num_hidden_layers = 1
+    model = _model(cfg, gpu, 26)
+    ids = _ids(cfg, 1, 128, 27, gpu) % 1000
+    ids[0, 3] = 2000
+    before, _ = model(ids)
+    word = model.embeddings.word_embeddings
+    word.weight.data = word.weight.data[:1000]
+    with pytest.raises(IndexError):
+        model(ids)
+    ids[0, 3] = 999
+    (got, _), (want, _) = _both(model, ids)
+    assert torch.equal(got, want)
+    mlp, at = model.encoder.layer[0].mlp, model.encoder.layer[0].attention
+    for mod, key, shape in ((mlp.layernorm, "weight", (512,)), (mlp.layernorm, "bias", (512,)), (mlp.wo, "bias", (700,)),
+                            (at.in_linear, "weight", (2304, 512)), (at.out_linear, "weight", (512, 768)), (at.short_filter, "bias", (768,))):
+        was = mod._parameters[key]
+        mod._parameters[key] = torch.nn.Parameter(torch.zeros(shape, device=gpu))
+        with pytest.raises((ValueError, RuntimeError)):
+            model(ids)
+        mod._parameters[key] = was
+    again, _ = model(ids)
+    assert torch.equal(again, got)

@@ -65,3 +65,13 @@ def test_plain_values_are_compared(value, others):
     assert check.unchanged()
     del lin.eps
     assert not check.unchanged()
+
+
+def test_a_part_of_the_recorded_tensor_is_another():
+    """Same storage, same address, fewer rows, other strides or another type."""
+    for change in (lambda w: w[:4], lambda w: w.t(), lambda w: w.view(64), lambda w: w.view(torch.int32)):
+        lin = torch.nn.Linear(8, 8)
+        check, address = _checker(lin, version=False), lin.weight.data_ptr()
+        new = change(lin.weight.detach())
+        lin.weight = torch.nn.Parameter(new, requires_grad=new.is_floating_point())
+        assert lin.weight.data_ptr() == address and not check.unchanged()
