@@ -10,6 +10,7 @@
 #include <Python.h>
 #include <torch/csrc/autograd/python_variable.h>
 
+#include <exception>
 #include <vector>
 
 namespace {
@@ -104,15 +105,20 @@ PyObject* checker_new(PyTypeObject* type, PyObject* args, PyObject*) {
     PyObject *dict, *key;
     int ver;
     if (!PyArg_ParseTuple(PyList_GET_ITEM(tens, i), "O!Op", &PyDict_Type, &dict, &key, &ver)) { Py_DECREF(c); return nullptr; }
-    const at::Tensor* t = look_up(dict, key);
-    if (!t) {
+    try {                            // a tensor without memory behind it (fake, functional) throws: no exception may leave this entry
+      const at::Tensor* t = look_up(dict, key);
+      if (t) {
+        c->tensors->push_back({dict, key, t->storage().getWeakStorageImpl(), t->const_data_ptr(), ver ? version_of(*t) : -1, t->scalar_type(),
+                               {t->sizes().begin(), t->sizes().end()}, {t->strides().begin(), t->strides().end()}});
+        Py_INCREF(dict); Py_INCREF(key);
+        continue;
+      }
       if (!PyErr_Occurred()) PyErr_SetObject(PyExc_KeyError, key);
-      Py_DECREF(c);
-      return nullptr;
+    } catch (const std::exception& e) {
+      PyErr_SetString(PyExc_ValueError, e.what());
     }
-    c->tensors->push_back({dict, key, t->storage().getWeakStorageImpl(), t->const_data_ptr(), ver ? version_of(*t) : -1, t->scalar_type(),
-                          {t->sizes().begin(), t->sizes().end()}, {t->strides().begin(), t->strides().end()}});
-    Py_INCREF(dict); Py_INCREF(key);
+    Py_DECREF(c);
+    return nullptr;
   }
   return reinterpret_cast<PyObject*>(c);
 }
@@ -131,8 +137,13 @@ PyObject* checker_unchanged(PyObject* self, PyObject*) {
       Py_RETURN_FALSE;
     }
   for (const auto& s : *c->tensors) {
-    const at::Tensor* t = look_up(s.dict, s.key);
-    if (!t || !same(s, *t)) {
+    bool unchanged = false;
+    try {
+      const at::Tensor* t = look_up(s.dict, s.key);
+      unchanged = t && same(s, *t);
+    } catch (const std::exception&) {      // not a tensor with memory any more
+    }
+    if (!unchanged) {
       if (PyErr_Occurred()) return nullptr;
       Py_RETURN_FALSE;
     }

@@ -75,3 +75,23 @@ def test_a_part_of_the_recorded_tensor_is_another():
         new = change(lin.weight.detach())
         lin.weight = torch.nn.Parameter(new, requires_grad=new.is_floating_point())
         assert lin.weight.data_ptr() == address and not check.unchanged()
+
+
+def test_tensors_without_memory_are_errors_and_changes():
+    """Sparse and fake tensors have no address: a change before a plan is used, an error when one is made, never an exception out of
+    the C entry."""
+    from torch._subclasses.fake_tensor import FakeTensorMode
+    with FakeTensorMode():
+        fake = torch.empty(8, 8)
+    lin = torch.nn.Linear(8, 8)
+    check = _checker(lin)
+    where = lin._parameters
+    was, where["weight"] = where["weight"], fake
+    assert not check.unchanged()
+    for other in (None, 3, torch.ones(8, 8).to_sparse(), torch.ones(8, 8).to_sparse_csr(), torch.ones(8, 8).to_mkldnn()):
+        where["weight"] = other
+        assert not check.unchanged()
+        with pytest.raises((KeyError, ValueError)):
+            _checker(lin)
+    where["weight"] = was
+    assert check.unchanged()
