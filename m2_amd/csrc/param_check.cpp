@@ -11,12 +11,14 @@
 #include <torch/csrc/autograd/python_variable.h>
 
 #include <exception>
+#include <type_traits>
 #include <vector>
 
 namespace {
 
 struct ModuleSlot {
   PyObject *dict, *key, *expected;
+  PyTypeObject* type;   // (a parametrisation changes the class of the module in its place)
 };
 struct TensorSlot {
   PyObject *dict, *key;
@@ -59,7 +61,7 @@ bool same(const TensorSlot& s, const at::Tensor& t) {
 void checker_dealloc(PyObject* self) {
   Checker* c = reinterpret_cast<Checker*>(self);
   if (c->modules) {
-    for (auto& m : *c->modules) { Py_DECREF(m.dict); Py_DECREF(m.key); Py_DECREF(m.expected); }
+    for (auto& m : *c->modules) { Py_DECREF(m.dict); Py_DECREF(m.key); Py_DECREF(m.expected); Py_DECREF(m.type); }
     delete c->modules;
   }
   if (c->tensors) {
@@ -84,7 +86,12 @@ bool record(PyObject* list, std::vector<Slot>* slots) {
       if (!PyErr_Occurred()) PyErr_SetObject(PyExc_KeyError, key);
       return false;
     }
-    slots->push_back({dict, key, o});
+    if constexpr (std::is_same<Slot, ModuleSlot>::value) {
+      slots->push_back({dict, key, o, Py_TYPE(o)});
+      Py_INCREF(Py_TYPE(o));
+    } else {
+      slots->push_back({dict, key, o});
+    }
     Py_INCREF(dict); Py_INCREF(key); Py_INCREF(o);
   }
   return true;
@@ -127,7 +134,7 @@ PyObject* checker_new(PyTypeObject* type, PyObject* args, PyObject*) {
 PyObject* checker_unchanged(PyObject* self, PyObject*) {
   Checker* c = reinterpret_cast<Checker*>(self);
   for (const auto& m : *c->modules)
-    if (PyDict_GetItemWithError(m.dict, m.key) != m.expected) {
+    if (PyDict_GetItemWithError(m.dict, m.key) != m.expected || Py_TYPE(m.expected) != m.type) {
       if (PyErr_Occurred()) return nullptr;
       Py_RETURN_FALSE;
     }

@@ -9,7 +9,7 @@ by tensor (storage, address and shape, and version counter for the weights that 
 
 Same kernels in the same order on the current stream as the Python schedule, hence the same bits.  It serves row counts
 whose projections run on the library's own kernels; larger forwards, whose host time hides behind the GPU's, and encoders
-with per-layer options stay with the Python schedule.
+with per-layer options, modules of other classes or computed weights stay with the Python schedule.
 """
 from __future__ import annotations
 
@@ -18,8 +18,11 @@ from typing import List, Optional
 
 import torch
 
-from . import ops
+from . import encoder as _encoder, ops
 from ._lib import LayerParams, check, lib
+from .blockdiag import BlockdiagLinear
+from .hyena import HyenaFilter
+from .mixer import MonarchMixerSequenceMixing
 
 try:
     from . import _param_check
@@ -38,14 +41,20 @@ class StackPlan:
         # the plan depends on
         mods, tens, vals = [(encoder._modules, "layer")], [], []
 
-        def child(mod, key):
+        # What is not there, or not what the modules are built with, is a ValueError: the Python schedule asks the modules themselves.
+        def child(mod, key, kind=None):
+            found = mod._modules.get(key)
+            if found is None or (kind is not None and type(found) is not kind):
+                raise ValueError(f"{key} is not the module it was built as")
             mods.append((mod._modules, key))
-            return mod._modules[key]
+            return found
 
         def tensor(mod, key, how=_IN_PLACE, shape=None):
             where = mod._parameters if key in mod._parameters else mod._buffers
+            t = where.get(key)
+            if t is None:                                  # absent, or computed (a parametrisation, weight_norm, pruning)
+                raise ValueError(f"{key} is not a plain parameter")
             tens.append((where, key, how))
-            t = where[key]
             if not (t.is_cuda and t.dtype == torch.float32 and t.is_contiguous()):
                 raise ValueError("parameters that are not plain fp32")
             if shape is not None and t.shape != shape:      # the kernels take sizes, not shapes: never read beyond a tensor
@@ -68,7 +77,7 @@ class StackPlan:
             lay = child(stack, key)
             at, mlp = child(lay, "attention"), child(lay, "mlp")
             for name in ("filter_fn", "filter_fn2")[:2 if value(at, "residual_long_conv") else 1]:
-                f = child(at, name)
+                f = child(at, name, HyenaFilter)
                 skips.append(tensor(f, "bias"))
                 emb = child(f, "pos_emb")
                 fwd = child(f, "implicit_filter")
@@ -87,7 +96,7 @@ class StackPlan:
                     row.append(tensor(child(seq, "6"), "weight"))
                 rows.append(row)
             lin_in, lin_out, short = child(at, "in_linear"), child(at, "out_linear"), child(at, "short_filter")
-            gated, wo, ln = child(mlp, "gated_layers"), child(mlp, "wo"), child(mlp, "layernorm")
+            gated, wo, ln = child(mlp, "gated_layers", BlockdiagLinear), child(mlp, "wo", BlockdiagLinear), child(mlp, "layernorm")
             cfg = value(mlp, "config")
             d, I, nb = value(at, "d_model"), value(cfg, "intermediate_size"), value(cfg, "monarch_mlp_nblocks")
             if d % nb or I % nb:
@@ -178,12 +187,18 @@ def stack_plan(encoder, embeddings, B: int, L: int) -> Optional[StackPlan]:
     layers = encoder._modules["layer"]._modules.values()
     M = B * L
     for lay in layers:
-        at, mlp = lay._modules["attention"], lay._modules["mlp"]
+        if type(lay) is not _encoder.BertLayer:
+            return None
+        at, mlp = lay._modules.get("attention"), lay._modules.get("mlp")
+        # classes of a caller's own run their own methods
+        if type(at) is not MonarchMixerSequenceMixing or type(mlp) is not _encoder.BertGatedLinearUnitMLP:
+            return None
         if (at.cache_filters or at.hyena_training_additions or mlp.fuse_wo_layernorm or not mlp.fuse_mlp or not mlp.bf16_presum
                 or not mlp.stream_glu):
             return None
     d = at.d_model
-    if at.in_linear.weight.dtype != torch.float32 or not at.in_linear.weight.is_cuda:
+    w = at.in_linear.weight
+    if w.dtype != torch.float32 or not w.is_cuda:
         return None
     if not ops.own_to_channels(M, d) or not ops.own_from_channels(M, d):
         return None

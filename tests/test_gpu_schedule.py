@@ -277,3 +277,61 @@ def test_a_narrowed_table_and_wrong_shapes(gpu):
         mod._parameters[key] = was
     again, _ = model(ids)
     assert torch.equal(again, got)
+
+
+def test_computed_weights_and_other_classes_take_the_python_schedule(gpu):
+    """Parametrised, weight-normed and pruned weights, subclasses and modules without a plan's parameters: a forward runs as with
+    the native schedule off."""
+    import m2_amd
+    from m2_amd import encoder as enc, mixer
+    from torch.nn.utils import parametrize, prune
+    cfg = m2_amd.m2_bert_80m(128)
+    cfg.num_hidden_layers = 2
+    ids = _ids(cfg, 1, 128, 28, gpu)
+
+    class Halved(torch.nn.Module):
+        def forward(self, w):
+            return w * 0.5
+
+    class OwnLayer(enc.BertLayer):
+        def fused(self, *args, **kw):
+            o32, h16, hT = super().fused(*args, **kw)
+            return None if o32 is None else o32 + 1, h16, hT
+
+    class OwnMixer(mixer.MonarchMixerSequenceMixing):
+        def project_out(self, y, *args):
+            return super().project_out(y, *args) * 2
+
+    class OwnMLP(enc.BertGatedLinearUnitMLP):
+        def normed(self, a16, *args):
+            return super().normed(a16 * 2, *args)
+
+    class OwnLinear(m2_amd.BlockdiagLinear):
+        def weight_bf16(self):
+            return super().weight_bf16() * 2
+
+    def retype(mod, cls):
+        mod.__class__ = cls
+
+    changes = {
+        "parametrised": lambda lay: parametrize.register_parametrization(lay.attention.in_linear, "weight", Halved()),
+        "block-diagonal parametrised": lambda lay: parametrize.register_parametrization(lay.mlp.wo, "weight", Halved()),
+        "filter parametrised": lambda lay: parametrize.register_parametrization(lay.attention.filter_fn.implicit_filter[4], "weight", Halved()),
+        "weight norm": lambda lay: torch.nn.utils.parametrizations.weight_norm(lay.attention.out_linear),
+        "pruned": lambda lay: prune.random_unstructured(lay.attention.out_linear, "weight", 0.5),
+        "layer": lambda lay: retype(lay, OwnLayer), "mixer": lambda lay: retype(lay.attention, OwnMixer),
+        "mlp": lambda lay: retype(lay.mlp, OwnMLP), "linear": lambda lay: retype(lay.mlp.gated_layers, OwnLinear)}
+    for what, change in changes.items():
+        for first in (False, True):                  # changed before any plan, and after one was made
+            model = _model(cfg, gpu, 29)
+            before, _ = model(ids)
+            if first:
+                model.encoder._native_plans.clear()
+            torch.manual_seed(1)
+            change(model.encoder.layer[1])
+            got, _ = model(ids)
+            model.encoder.native_schedule = False
+            want, _ = model(ids)
+            assert torch.equal(got, want), what
+            if what != "weight norm":                # (that one keeps the values)
+                assert not torch.equal(got, before), what

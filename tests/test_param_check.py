@@ -95,3 +95,15 @@ def test_tensors_without_memory_are_errors_and_changes():
             _checker(lin)
     where["weight"] = was
     assert check.unchanged()
+
+
+def test_another_module_or_another_class_in_its_place():
+    seq = torch.nn.Sequential(torch.nn.Linear(8, 8))
+    check = _param_check.Checker([(seq._modules, "0")], [], [])
+    assert check.unchanged()
+    seq[0].__class__ = type("Other", (torch.nn.Linear,), {})
+    assert not check.unchanged()
+    seq[0].__class__ = torch.nn.Linear
+    assert check.unchanged()
+    seq[0] = torch.nn.Linear(8, 8)
+    assert not check.unchanged()
