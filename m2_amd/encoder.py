@@ -450,8 +450,10 @@ class BertEncoder(nn.Module):
                             ev = torch.cuda.Event()
                             ev.record(cur)
                             generate(i + 1, ev)
+                # (a `fused` of a caller's own need not know `last`: it then writes two forms that nobody reads)
+                last = {"last": True} if i == n - 1 and type(layer).fused is BertLayer.fused else {}
                 o32, h16, hT = layer.fused(h16, hT, B, L, want_f32=keep32, spec=spec, spec_ready=ready,
-                                           after_core=hook, h32=o32, last=i == n - 1)
+                                           after_core=hook, h32=o32, **last)
                 if want:
                     outs.append(o32)
             if overlap and overlap != "inline-batched":

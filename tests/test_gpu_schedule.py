@@ -335,3 +335,22 @@ def test_computed_weights_and_other_classes_take_the_python_schedule(gpu):
             assert torch.equal(got, want), what
             if what != "weight norm":                # (that one keeps the values)
                 assert not torch.equal(got, before), what
+
+
+def test_a_layer_class_with_the_plain_signature(gpu):
+    import m2_amd
+    from m2_amd import encoder as enc
+
+    class Plain(enc.BertLayer):
+        def fused(self, h16, hT, B, L, want_f32, spec=None, spec_ready=None, after_core=None, h32=None):
+            return super().fused(h16, hT, B, L, want_f32, spec=spec, spec_ready=spec_ready, after_core=after_core, h32=h32)
+
+    cfg = m2_amd.m2_bert_80m(128)
+    cfg.num_hidden_layers = 2
+    ids = _ids(cfg, 1, 128, 30, gpu)
+    model = _model(cfg, gpu, 31)
+    want, _ = model(ids)
+    for lay in model.encoder.layer:
+        lay.__class__ = Plain
+    got, _ = model(ids)
+    assert torch.equal(got, want)
