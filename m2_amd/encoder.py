@@ -659,11 +659,14 @@ class BertModel(nn.Module):
             outs = [o.clone() for o in static_out]
         enc = [o.view(B, L, -1) for o in outs]
         pooled = None
-        if self.pooler is not None:
-            if attention_mask is None:
-                attention_mask = torch.ones_like(input_ids)
-            pooled = self.pooler(enc[-1], mask=attention_mask)
-        # last, behind everything that is to be enqueued: it waits for the stream
-        if self.validate_ids and not torch.cuda.is_current_stream_capturing():
-            self.embeddings.check_indices()
+        try:
+            if self.pooler is not None:
+                if attention_mask is None:
+                    attention_mask = torch.ones_like(input_ids)
+                pooled = self.pooler(enc[-1], mask=attention_mask)
+        finally:
+            # last, behind everything that is to be enqueued: it waits for the stream.  Also when the pooler raises: a bad id is
+            # this forward's error and not the next one's
+            if self.validate_ids and not torch.cuda.is_current_stream_capturing():
+                self.embeddings.check_indices()
         return (enc if output_all_encoded_layers else enc[-1]), pooled

@@ -354,3 +354,27 @@ def test_a_layer_class_with_the_plain_signature(gpu):
         lay.__class__ = Plain
     got, _ = model(ids)
     assert torch.equal(got, want)
+
+
+def test_a_bad_index_is_reported_before_a_failing_pooler(gpu):
+    """The flag of a forward with a bad id is read in that forward, whatever becomes of its pooler."""
+    import m2_amd
+    cfg = m2_amd.m2_bert_80m(128)
+    cfg.num_hidden_layers = 1
+    model = _model(cfg, gpu, 32)
+    ids = _ids(cfg, 1, 128, 33, gpu)
+    want, _ = model(ids)
+    bad = ids.clone()
+    bad[0, 5] = cfg.vocab_size
+
+    def fail(module, args):
+        raise ArithmeticError("pooler")
+
+    handle = model.pooler.register_forward_pre_hook(fail)
+    with pytest.raises(IndexError):
+        model(bad)
+    with pytest.raises(ArithmeticError):
+        model(ids)
+    handle.remove()
+    got, _ = model(ids)                                     # nothing is left of the bad id
+    assert torch.equal(got, want)
