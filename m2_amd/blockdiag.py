@@ -88,9 +88,12 @@ class BlockdiagLinear(nn.Module):
 
     def weight_bf16(self) -> torch.Tensor:
         tag = (self.weight.data_ptr(), self.weight._version, self.weight.device)
-        if self._w16 is None or self._w16[0] != tag:
-            self._w16 = (tag, self.weight.detach().to(torch.bfloat16).contiguous())
-        return self._w16[1]
+        hit = self._w16
+        if hit is None or hit[0] != tag:
+            hit = (tag, self.weight.detach().to(torch.bfloat16).contiguous())
+            if not torch.cuda.is_current_stream_capturing():       # (what a capture makes holds nothing before a replay)
+                self._w16 = hit
+        return hit[1]
 
     def forward(self, x):
         if not x.is_cuda:

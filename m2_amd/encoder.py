@@ -153,15 +153,22 @@ class BertGatedLinearUnitMLP(nn.Module):
         return fused, M * d <= 245760
 
     def packed_mlp(self, wg: torch.Tensor, wo: torch.Tensor) -> torch.Tensor:
-        """The packed copy the one-kernel MLP streams: rebuilt whenever one of the bf16 copies has been rebuilt."""
-        if self._packed is None or self._packed[0] is not wg or self._packed[1] is not wo:
-            self._packed = (wg, wo, ops.mlp_fused_pack(wg, wo))
-        return self._packed[2]
+        """The packed copy the one-kernel MLP streams: rebuilt whenever one of the bf16 copies has been rebuilt.  (What a stream
+        capture makes holds nothing before a replay, and is not kept.)"""
+        hit = self._packed
+        if hit is None or hit[0] is not wg or hit[1] is not wo:
+            hit = (wg, wo, ops.mlp_fused_pack(wg, wo))
+            if not torch.cuda.is_current_stream_capturing():
+                self._packed = hit
+        return hit[2]
 
     def packed_glu(self, wg: torch.Tensor) -> torch.Tensor:
-        if self._packed_glu is None or self._packed_glu[0] is not wg:      # rebuilt with the bf16 copy
-            self._packed_glu = (wg, ops.glu_stream_pack(wg))
-        return self._packed_glu[1]
+        hit = self._packed_glu
+        if hit is None or hit[0] is not wg:      # rebuilt with the bf16 copy
+            hit = (wg, ops.glu_stream_pack(wg))
+            if not torch.cuda.is_current_stream_capturing():
+                self._packed_glu = hit
+        return hit[1]
 
     def presum(self, a16: torch.Tensor) -> torch.Tensor:
         """a16 (M, d) bf16 -> wo(glu(a16)) + bias + a16, (M, d) fp32 (the LayerNorm input; bf16 with `bf16_presum`)."""

@@ -72,7 +72,8 @@ class MonarchMixerSequenceMixing(nn.Module):
         hit = self._cast_cache.get(key)
         if hit is None or hit[0] != tag:
             hit = (tag, p.detach().to(dtype).contiguous())
-            self._cast_cache[key] = hit
+            if not torch.cuda.is_current_stream_capturing():       # (what a capture makes holds nothing before a replay)
+                self._cast_cache[key] = hit
         return hit[1]
 
     def filter_spectrum(self, L: int) -> torch.Tensor:

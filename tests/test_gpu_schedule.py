@@ -378,3 +378,51 @@ def test_a_bad_index_is_reported_before_a_failing_pooler(gpu):
     handle.remove()
     got, _ = model(ids)                                     # nothing is left of the bad id
     assert torch.equal(got, want)
+
+
+def _captured(call):
+    """(result tensors of a captured call, its graph); the call's Python side has run once, its kernels not at all."""
+    graph = torch.cuda.CUDAGraph()
+    with torch.no_grad(), torch.cuda.graph(graph):
+        held = call()
+    return held, graph
+
+
+# the one-kernel MLP's and the streaming product's packed weights, first wanted by a capture after a forward of few rows
+@pytest.mark.parametrize("helper,B", [("m2_bert_80m", 8), ("m2_bert_large", 3), ("m2_bert_large", 17)])
+def test_copies_made_during_a_capture_are_not_kept(gpu, helper, B):
+    import m2_amd
+    cfg = getattr(m2_amd, helper)(128)
+    cfg.num_hidden_layers = 2
+    one, many = _ids(cfg, 1, 128, 34, gpu), _ids(cfg, B, 128, 35, gpu)
+    want, _ = _model(cfg, gpu, 36)(many)
+    model = _model(cfg, gpu, 36)
+    model.encoder.native_schedule = False
+    model.validate_ids = False
+    first, _ = model(one)
+    (held, _), graph = _captured(lambda: model(many))
+    eager, _ = model(many)                                  # before any replay
+    assert torch.equal(eager, want)
+    for _ in range(3):
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(held, want)
+        assert torch.equal(model(one)[0], first)
+
+
+def test_casts_made_during_a_capture_are_not_kept(gpu):
+    import m2_amd
+    cfg = m2_amd.m2_bert_80m(128)
+    layer = m2_amd.BertLayer(cfg).to(gpu).eval()
+    u = torch.randn(2, 128, 768, generator=torch.Generator().manual_seed(37)).to(gpu)
+    u16 = u.bfloat16()
+    with torch.no_grad():
+        layer(u)                                            # the filters' table; no bf16 copy yet
+        held, graph = _captured(lambda: layer(u16))
+        eager = layer(u16)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(held, eager)
+        other = m2_amd.BertLayer(cfg).to(gpu).eval()
+        other.load_state_dict(layer.state_dict())
+        assert torch.equal(other(u16), eager)
