@@ -58,20 +58,41 @@ bool same(const TensorSlot& s, const at::Tensor& t) {
          t.scalar_type() == s.dtype && t.sizes().equals(s.sizes) && t.strides().equals(s.strides) && (s.version < 0 || version_of(t) == s.version);
 }
 
-void checker_dealloc(PyObject* self) {
+// The dicts lead to modules, and those may lead back to the plan that holds this object: the garbage collector has to see them.
+int checker_traverse(PyObject* self, visitproc visit, void* arg) {
   Checker* c = reinterpret_cast<Checker*>(self);
-  if (c->modules) {
-    for (auto& m : *c->modules) { Py_DECREF(m.dict); Py_DECREF(m.key); Py_DECREF(m.expected); Py_DECREF(m.type); }
-    delete c->modules;
-  }
-  if (c->tensors) {
-    for (auto& t : *c->tensors) { Py_DECREF(t.dict); Py_DECREF(t.key); }
-    delete c->tensors;
-  }
-  if (c->values) {
-    for (auto& v : *c->values) { Py_DECREF(v.dict); Py_DECREF(v.key); Py_DECREF(v.expected); }
-    delete c->values;
-  }
+  if (c->modules)
+    for (auto& m : *c->modules) { Py_VISIT(m.dict); Py_VISIT(m.key); Py_VISIT(m.expected); Py_VISIT(m.type); }
+  if (c->tensors)
+    for (auto& t : *c->tensors) { Py_VISIT(t.dict); Py_VISIT(t.key); }
+  if (c->values)
+    for (auto& v : *c->values) { Py_VISIT(v.dict); Py_VISIT(v.key); Py_VISIT(v.expected); }
+  return 0;
+}
+
+// An emptied checker compares nothing: only the collector may call this.
+int checker_clear(PyObject* self) {
+  Checker* c = reinterpret_cast<Checker*>(self);
+  std::vector<PyObject*> drop;                 // released when the slots are gone: a destructor may come back here
+  if (c->modules)
+    for (auto& m : *c->modules) drop.insert(drop.end(), {m.dict, m.key, m.expected, reinterpret_cast<PyObject*>(m.type)});
+  if (c->tensors)
+    for (auto& t : *c->tensors) drop.insert(drop.end(), {t.dict, t.key});
+  if (c->values)
+    for (auto& v : *c->values) drop.insert(drop.end(), {v.dict, v.key, v.expected});
+  delete c->modules;
+  delete c->tensors;
+  delete c->values;
+  c->modules = nullptr;
+  c->tensors = nullptr;
+  c->values = nullptr;
+  for (PyObject* o : drop) Py_DECREF(o);
+  return 0;
+}
+
+void checker_dealloc(PyObject* self) {
+  PyObject_GC_UnTrack(self);
+  checker_clear(self);
   Py_TYPE(self)->tp_free(self);
 }
 
@@ -133,6 +154,7 @@ PyObject* checker_new(PyTypeObject* type, PyObject* args, PyObject*) {
 // unchanged() -> bool
 PyObject* checker_unchanged(PyObject* self, PyObject*) {
   Checker* c = reinterpret_cast<Checker*>(self);
+  if (!c->modules || !c->tensors || !c->values) Py_RETURN_FALSE;
   for (const auto& m : *c->modules)
     if (PyDict_GetItemWithError(m.dict, m.key) != m.expected || Py_TYPE(m.expected) != m.type) {
       if (PyErr_Occurred()) return nullptr;
@@ -167,7 +189,9 @@ PyModuleDef module_def = {PyModuleDef_HEAD_INIT, "_param_check", nullptr, -1, nu
 
 PyMODINIT_FUNC PyInit__param_check() {
   CheckerType.tp_basicsize = sizeof(Checker);
-  CheckerType.tp_flags = Py_TPFLAGS_DEFAULT;
+  CheckerType.tp_flags = Py_TPFLAGS_DEFAULT | Py_TPFLAGS_HAVE_GC;
+  CheckerType.tp_traverse = checker_traverse;
+  CheckerType.tp_clear = checker_clear;
   CheckerType.tp_new = checker_new;
   CheckerType.tp_dealloc = checker_dealloc;
   CheckerType.tp_methods = checker_methods;

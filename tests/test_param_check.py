@@ -107,3 +107,18 @@ def test_another_module_or_another_class_in_its_place():
     assert check.unchanged()
     seq[0] = torch.nn.Linear(8, 8)
     assert not check.unchanged()
+
+
+def test_a_cycle_through_the_check_is_collected():
+    import gc
+    import weakref
+    for slots in (lambda m: ([(m._modules, "0")], [], []), lambda m: ([], [(m[0]._parameters, "weight", True)], []),
+                  lambda m: ([], [], [(m.__dict__, "training")])):
+        seq = torch.nn.Sequential(torch.nn.Linear(8, 8))
+        seq[0].__dict__["_parameters"]["weight"].owner = seq       # and back
+        seq[0].owner_dict = {"owner": seq}
+        seq.check = _param_check.Checker(*slots(seq))
+        gone = weakref.ref(seq)
+        del seq
+        gc.collect()
+        assert gone() is None
