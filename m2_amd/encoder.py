@@ -377,9 +377,10 @@ class BertEncoder(nn.Module):
                     hT = h32.t().contiguous()
                 # (an input that requires grad goes to the projections, which refuse it)
                 graded = torch.is_grad_enabled() and (h16.requires_grad or hT.requires_grad)
-                plan = None if graded else schedule.stack_plan(self, None, B, L)
-                if plan is not None:
-                    return plan.run(B, all_layers, h16, hT)
+                found = None if graded else schedule.stack_plan(self, B, L, h16.device)
+                if found is not None:
+                    plan, which = found
+                    return plan.run(which, B, all_layers, h16, hT)
             outs = []
             n = len(self.layer)
             o32 = h32
@@ -501,14 +502,17 @@ class BertEncoder(nn.Module):
                              for t in (v if isinstance(v, list) else [v])) + tuple(b.data_ptr() for _, skips in entries
                                                                                    for b in skips)
         if self._filter_table is None or self._filter_table[0] != probe:
+            plan = self._native_plans.get(L)
+            if plan is not None and plan.current(self):      # (its table is this one; a stream capture could not make another)
+                return plan.table, groups
             self._filter_table = (probe, ops.FilterTable([e[0] for e in entries], [e[1] for e in entries], L, m0.d_model,
                                                          m0.filter_fn.order, m0.filter_fn.emb_dim))
         return self._filter_table[1], groups
 
-    def _graph_reads(self) -> tuple:
-        """What a graph captured just now reads beside parameters: pointer tables and packed weights, which forwards of
-        other lengths replace here and which therefore have to live as long as the graph."""
-        return self._filter_table, tuple(self._native_plans.values())
+    def _graph_reads(self, L: int) -> tuple:
+        """What a graph captured just now for length L reads beside parameters: pointer tables and packed weights, which
+        forwards of other lengths replace here and which therefore have to live as long as the graph."""
+        return self._filter_table, self._native_plans.get(L)
 
     def _run_graphed(self, h32: Optional[torch.Tensor], B: int, L: int, all_layers: bool,
                      h16: Optional[torch.Tensor] = None, hT: Optional[torch.Tensor] = None) -> List[torch.Tensor]:
@@ -526,7 +530,7 @@ class BertEncoder(nn.Module):
             graph = torch.cuda.CUDAGraph()
             with torch.cuda.graph(graph):
                 static_out = self._run_layers(static[0], B, L, all_layers, h16=static[1], hT=static[2])
-            entry = (graph, static, static_out, self._graph_reads())
+            entry = (graph, static, static_out, self._graph_reads(L))
             self._graphs[key] = entry
         graph, static, static_out, _ = entry
         for dst, src in zip(static, (h32, h16, hT)):
@@ -593,6 +597,7 @@ class BertModel(nn.Module):
         # synchronisation) and raises IndexError like nn.Embedding would; False leaves the flag to
         # `embeddings.check_indices()`.  The embedding tables are part of the captured graph too:
         self.validate_ids = True
+        self._embed_part = None      # of the native schedule
         self.register_load_state_dict_post_hook(lambda module, keys: module.encoder.reset_graphs())
 
     def _run_native(self, ids, tt, pos, all_layers: bool):
@@ -600,6 +605,8 @@ class BertModel(nn.Module):
         embedding call would refuse, ...: the Python schedule then runs, or reports the error)."""
         B, L = ids.shape
         emb = self.embeddings
+        if type(emb) is not BertEmbeddings or type(self.encoder)._run_layers is not BertEncoder._run_layers:
+            return None
         if (emb.training and emb.dropout.p > 0) or ids.dtype != torch.int64 or not ids.is_cuda:
             return None
         if tt is not None or pos is not None:
@@ -611,8 +618,12 @@ class BertModel(nn.Module):
             return None
         if pos is None and emb.use_positional_encodings and emb.position_embeddings.weight.shape[0] < L:
             return None
-        plan = schedule.stack_plan(self.encoder, emb, B, L)
-        return None if plan is None else plan.run(B, all_layers, None, None, ids.contiguous(), tt, pos)
+        found = schedule.stack_plan(self.encoder, B, L, ids.device)
+        part = None if found is None else schedule.embed_part(self, found[0].d)
+        if part is None:
+            return None
+        plan, which = found
+        return plan.run(which, B, all_layers, None, None, part, ids.contiguous(), tt, pos)
 
     def get_input_embeddings(self):
         return self.embeddings.word_embeddings
@@ -656,7 +667,7 @@ class BertModel(nn.Module):
                 graph = torch.cuda.CUDAGraph()
                 with torch.cuda.graph(graph):
                     static_out = run(*static)
-                entry = (graph, static, static_out, self.encoder._graph_reads())
+                entry = (graph, static, static_out, self.encoder._graph_reads(L))
                 self.encoder._graphs[key] = entry
             graph, static, static_out, _ = entry
             for dst, src in zip(static, given):

@@ -426,3 +426,49 @@ def test_casts_made_during_a_capture_are_not_kept(gpu):
         other = m2_amd.BertLayer(cfg).to(gpu).eval()
         other.load_state_dict(layer.state_dict())
         assert torch.equal(other(u16), eager)
+
+
+# after an eager forward of one sequence: a capture at another row count of the native schedule (with other MLP kernels), and one
+# that the Python schedule serves; through the model and through the encoder
+@pytest.mark.parametrize("helper,L,B", [("m2_bert_80m", 128, 2), ("m2_bert_80m", 128, 8), ("m2_bert_large", 128, 3), ("m2_bert_80m", 1024, 9),
+                                        ("m2_bert_large", 128, 17)])
+def test_capture_at_another_batch_size(gpu, helper, L, B):
+    import m2_amd
+    cfg = getattr(m2_amd, helper)(L)
+    cfg.num_hidden_layers = 2
+    one, many = _ids(cfg, 1, L, 38, gpu), _ids(cfg, B, L, 39, gpu)
+    h = torch.randn(B, L, cfg.hidden_size, generator=torch.Generator().manual_seed(40)).to(gpu)
+    ref = _model(cfg, gpu, 41)
+    want, wenc = ref(many)[0], ref.encoder(h)[-1]
+    model = _model(cfg, gpu, 41)
+    model.validate_ids = False
+    model.pooler = None
+    first, _ = model(one)
+    (held, _), graph = _captured(lambda: model(many))
+    held_enc, graph_enc = _captured(lambda: model.encoder(h)[-1])
+    assert torch.equal(model(many)[0], want)
+    for _ in range(3):
+        graph.replay()
+        graph_enc.replay()
+        torch.randn(512, 512, device=gpu) @ torch.randn(512, 512, device=gpu)
+        torch.cuda.synchronize()
+        assert torch.equal(held, want) and torch.equal(held_enc, wenc)
+        assert torch.equal(model(one)[0], first)
+
+
+def test_embeddings_replaced_as_a_module(gpu):
+    """Another embeddings module in front of the same encoder, there and back, and two models that share an encoder."""
+    import m2_amd
+    cfg = m2_amd.m2_bert_80m(128)
+    cfg.num_hidden_layers = 1
+    a, b = _model(cfg, gpu, 42), _model(cfg, gpu, 43)
+    ids = _ids(cfg, 1, 128, 44, gpu)
+    first, _ = a(ids)
+    b.encoder = a.encoder
+    other, _ = b(ids)
+    assert torch.equal(a(ids)[0], first) and not torch.equal(other, first)
+    mine, a.embeddings = a.embeddings, b.embeddings
+    (got, _), (want, _) = _both(a, ids)
+    assert torch.equal(got, want) and torch.equal(got, other)
+    a.embeddings = mine
+    assert torch.equal(a(ids)[0], first)
