@@ -512,7 +512,8 @@ class BertEncoder(nn.Module):
     def _graph_reads(self, L: int) -> tuple:
         """What a graph captured just now for length L reads beside parameters: pointer tables and packed weights, which
         forwards of other lengths replace here and which therefore have to live as long as the graph."""
-        return self._filter_table, self._native_plans.get(L)
+        table, plan = self._filter_table, self._native_plans.get(L)
+        return tuple(r for r in (None if table is None else table[1], plan) if r is not None)
 
     def _run_graphed(self, h32: Optional[torch.Tensor], B: int, L: int, all_layers: bool,
                      h16: Optional[torch.Tensor] = None, hT: Optional[torch.Tensor] = None) -> List[torch.Tensor]:
@@ -532,10 +533,12 @@ class BertEncoder(nn.Module):
                 static_out = self._run_layers(static[0], B, L, all_layers, h16=static[1], hT=static[2])
             entry = (graph, static, static_out, self._graph_reads(L))
             self._graphs[key] = entry
-        graph, static, static_out, _ = entry
+        graph, static, static_out, reads = entry
         for dst, src in zip(static, (h32, h16, hT)):
             if dst is not None:
                 dst.copy_(src)
+        for held in reads:
+            held.use_on_current_stream()
         graph.replay()
         return [o.clone() for o in static_out]
 
@@ -669,10 +672,12 @@ class BertModel(nn.Module):
                     static_out = run(*static)
                 entry = (graph, static, static_out, self.encoder._graph_reads(L))
                 self.encoder._graphs[key] = entry
-            graph, static, static_out, _ = entry
+            graph, static, static_out, reads = entry
             for dst, src in zip(static, given):
                 if dst is not None:
                     dst.copy_(src)
+            for held in reads:
+                held.use_on_current_stream()
             graph.replay()
             outs = [o.clone() for o in static_out]
         enc = [o.view(B, L, -1) for o in outs]

@@ -106,6 +106,28 @@ def hyena_filter_taps(filters: Sequence[dict], L: int, d: int, order: int, emb_d
     return taps
 
 
+class StreamUse:
+    """Device memory that is made once on one stream and read on any, then dropped at any time.  `use_on_current_stream` comes
+    before each launch that reads it: a stream met for the first time waits for `ready`, the event behind what made the memory
+    (None: it was complete when the host went on), and the allocator keeps the memory back, once it is dropped, until that stream
+    has come past its last use."""
+
+    def __init__(self, tensors: Sequence[Tensor], ready: Optional["torch.cuda.Event"] = None):
+        self.tensors, self.ready = list(tensors), ready
+        self.streams = {torch.cuda.current_stream().cuda_stream}
+
+    def use_on_current_stream(self) -> None:
+        stream = torch.cuda.current_stream()
+        if stream.cuda_stream in self.streams:
+            return
+        for t in self.tensors:
+            t.record_stream(stream)
+        if not torch.cuda.is_current_stream_capturing():     # (a capture cannot wait for what lies outside; its replays come later)
+            if self.ready is not None:
+                stream.wait_event(self.ready)
+            self.streams.add(stream.cuda_stream)
+
+
 class FilterTable:
     """Pointer table, in device memory, of the implicit filters of a batch of mixers (what `m2_mixer_filters_fwd`
     reads), with the tensors it points to kept alive.  Built once per set of parameter tensors (`key` = their
@@ -156,6 +178,10 @@ class FilterTable:
                                "with these parameter tensors before capturing")
         self.table = torch.tensor(rows, dtype=torch.int64).to(dev)
         self.skip = torch.tensor(skip_row, dtype=torch.int64).to(dev)
+        self._use = StreamUse((self.table, self.skip))
+
+    def use_on_current_stream(self) -> None:
+        self._use.use_on_current_stream()
 
     @classmethod
     def of_rows(cls, rows: Sequence[Sequence[Optional[Tensor]]], skips: Sequence[Tensor], fpm: int, L: int, d: int, order: int,
@@ -177,6 +203,7 @@ class FilterTable:
         dev = rows[0][0].device
         self.table = torch.tensor([[0 if t is None else t.data_ptr() for t in row] for row in rows], dtype=torch.int64).to(dev)
         self.skip = torch.tensor([b.data_ptr() for b in skips], dtype=torch.int64).to(dev)
+        self._use = StreamUse((self.table, self.skip))
         return self
 
     def spectrum_floats(self) -> int:
@@ -191,6 +218,7 @@ def mixer_filter_spectra(table: FilterTable, w_mod: float = 1.0, shift: float = 
     if first < 0 or count < 1 or first + count > table.nmixers:
         raise ValueError(f"mixers [{first}, {first + count}) outside the table of {table.nmixers}")
     dev = table.table.device
+    table.use_on_current_stream()
     n = table.spectrum_floats()
     if out is None:
         out = torch.empty(count, n, dtype=torch.float32, device=dev)

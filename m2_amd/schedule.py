@@ -182,10 +182,17 @@ class StackPlan:
         self.table = ops.FilterTable.of_rows(rows, skips, len(rows) // n, L, self.d, f0.order, f0.emb_dim)
         self.checker = slots.checker()
         self.device = self.table.table.device
+        ready = torch.cuda.Event()
+        ready.record()
+        self._use = ops.StreamUse(self.keep, ready)
         self.L = L
         self.spec_bytes = lib.m2_filter_spectrum_bytes(self.d, L)
         self.filter_ws = lib.m2_mixer_filters_workspace_bytes(n, self.table.fpm, L, self.d, self.table.order)
         self.filter_ws_layer = max(1, lib.m2_mixer_filters_workspace_bytes(1, self.table.fpm, L, self.d, self.table.order))
+
+    def use_on_current_stream(self) -> None:
+        self.table.use_on_current_stream()
+        self._use.use_on_current_stream()
 
     def route(self, mlp, M: int) -> Optional[int]:
         """Which of `arrays` serves M rows."""
@@ -206,6 +213,7 @@ class StackPlan:
         M = B * L
         dev = ids.device if ids is not None else h16.device
         stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+        self.use_on_current_stream()
         up = lambda v: (v + 255) & ~255      # noqa: E731
         o_spec = up(self.filter_ws)
         o_act = o_spec + up(n * self.spec_bytes)
@@ -261,8 +269,6 @@ def stack_plan(encoder, B: int, L: int, device: torch.device):
             plan = StackPlan(encoder, L)
         except ValueError:
             return None
-        if len(encoder._native_plans) >= 16:         # lengths: drop the oldest
-            encoder._native_plans.pop(next(iter(encoder._native_plans)))
         encoder._native_plans[L] = plan
     elif (plan.layers * plan.spec_bytes > encoder.UPFRONT_MAX_BYTES                     # (limits that were lowered since)
           or encoder.FILTER_WORKSPACE_BYTES // plan.filter_ws_layer < plan.layers):

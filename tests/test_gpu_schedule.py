@@ -472,3 +472,33 @@ def test_embeddings_replaced_as_a_module(gpu):
     assert torch.equal(got, want) and torch.equal(got, other)
     a.embeddings = mine
     assert torch.equal(a(ids)[0], first)
+
+
+def test_a_dropped_plan_outlives_its_use_on_another_stream(gpu):
+    """The memory of a plan that is dropped while another stream still reads it is not given out again before that stream is done."""
+    import m2_amd
+    cfg = m2_amd.m2_bert_80m(128)
+    cfg.num_hidden_layers = 2
+    model = _model(cfg, gpu, 45)
+    model.validate_ids = False
+    ids = _ids(cfg, 1, 128, 46, gpu)
+    want = model(ids)[0].clone()
+    a = torch.randn(8192, 8192, device=gpu, dtype=torch.bfloat16)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    torch.cuda.synchronize()
+    with torch.cuda.stream(side):
+        for _ in range(200):
+            b = a @ a
+        got = model(ids)[0]
+    plan = model.encoder._native_plans[128]
+    address, like = plan.table.table.data_ptr(), plan.table.table.shape
+    assert plan._use.streams >= {side.cuda_stream} and plan.table._use.streams >= {side.cuda_stream}
+    del plan
+    model.encoder._native_plans.clear()
+    new = [torch.full(like, 1, dtype=torch.int64, device=gpu) for _ in range(32)]
+    assert not side.query(), "the other stream was done too early for this test to say anything"
+    assert all(t.data_ptr() != address for t in new)
+    torch.cuda.synchronize()
+    assert torch.equal(got, want)
+    del b
