@@ -358,6 +358,7 @@ class BertEncoder(nn.Module):
     @staticmethod
     def _drop_graphs_after_load(module, incompatible_keys) -> None:
         module._graphs = {}
+        module._native_plans = {}
 
     # -- the fused schedule --------------------------------------------------------------------
     def _run_layers(self, h32: Optional[torch.Tensor], B: int, L: int, all_layers: bool,

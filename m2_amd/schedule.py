@@ -269,6 +269,11 @@ def stack_plan(encoder, B: int, L: int, device: torch.device):
             plan = StackPlan(encoder, L)
         except ValueError:
             return None
+        # What changed for one length changed for others: none of them keeps copies of replaced weights.  (At most one plan for
+        # each of the nine lengths.)
+        for other, p in list(encoder._native_plans.items()):
+            if p is None or not p.current(encoder):
+                encoder._native_plans.pop(other, None)
         encoder._native_plans[L] = plan
     elif (plan.layers * plan.spec_bytes > encoder.UPFRONT_MAX_BYTES                     # (limits that were lowered since)
           or encoder.FILTER_WORKSPACE_BYTES // plan.filter_ws_layer < plan.layers):

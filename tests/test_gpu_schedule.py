@@ -502,3 +502,24 @@ def test_a_dropped_plan_outlives_its_use_on_another_stream(gpu):
     torch.cuda.synchronize()
     assert torch.equal(got, want)
     del b
+
+
+def test_plans_keep_no_replaced_weights(gpu):
+    import m2_amd
+    cfg = m2_amd.m2_bert_80m(256)
+    cfg.num_hidden_layers = 1
+    model = _model(cfg, gpu, 47)
+    short, long = _ids(cfg, 1, 128, 48, gpu), _ids(cfg, 1, 256, 49, gpu)
+    model(short), model(long)
+    old = [weakref.ref(t) for p in model.encoder._native_plans.values() for t in p.keep]
+    assert len(model.encoder._native_plans) == 2 and all(r() is not None for r in old)
+    with torch.no_grad():
+        for lin in (model.encoder.layer[0].attention.in_linear, model.encoder.layer[0].attention.out_linear,
+                    model.encoder.layer[0].mlp.gated_layers, model.encoder.layer[0].mlp.wo):
+            lin.weight.mul_(2)
+    model(short)
+    assert list(model.encoder._native_plans) == [128] and all(r() is None for r in old)
+    model(long)
+    assert len(model.encoder._native_plans) == 2
+    model.load_state_dict(m2_amd.seeded_state_dict(cfg, 50))
+    assert not model.encoder._native_plans
