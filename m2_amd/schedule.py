@@ -14,6 +14,7 @@ with per-layer options, modules of other classes or computed weights stay with t
 from __future__ import annotations
 
 import ctypes
+import warnings
 from typing import List, Optional
 
 import torch
@@ -27,7 +28,11 @@ from .mixer import MonarchMixerSequenceMixing
 try:
     from . import _param_check
 except ImportError as e:
-    raise ImportError("m2_amd/_param_check.so is missing or does not fit this torch: build it with `python m2_amd/build.py`") from e
+    # built against torch's internals, unlike the library with its plain C interface: without it everything runs, short forwards
+    # with the Python schedule's host time
+    _param_check = None
+    warnings.warn(f"m2_amd/_param_check.so is missing or does not fit this torch ({e}): short forwards take the slower Python schedule; "
+                  "build it with `python m2_amd/build.py`", RuntimeWarning)
 
 
 _IN_PLACE, _COPIED = False, True       # read at its address / a copy was made from it: compare the version too
@@ -239,7 +244,7 @@ class StackPlan:
 
 def stack_plan(encoder, B: int, L: int, device: torch.device):
     """(the plan for L, made or re-used, and which of its arrays serves B L rows), or None where the Python schedule serves."""
-    if not encoder.native_schedule or not encoder.batch_filters or encoder.overlap_filters not in (None, False):
+    if _param_check is None or not encoder.native_schedule or not encoder.batch_filters or encoder.overlap_filters not in (None, False):
         return None
     M = B * L
     for lay in encoder._modules["layer"]._modules.values():

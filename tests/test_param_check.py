@@ -1,5 +1,7 @@
 """The check behind the plans of the native schedule (m2_amd/csrc/param_check.cpp), on CPU tensors: what a plan depends on is
 recognised as changed whichever way it was changed."""
+import os
+
 import numpy as np
 import pytest
 import torch
@@ -122,3 +124,21 @@ def test_a_cycle_through_the_check_is_collected():
         del seq
         gc.collect()
         assert gone() is None
+
+
+def test_the_package_works_without_the_extension():
+    """Only plans need it: a package without it (or with one that does not fit torch) imports with a warning and makes no plans."""
+    import subprocess
+    import sys
+    code = ("import sys, warnings\n"
+            "sys.modules['m2_amd._param_check'] = None\n"
+            "with warnings.catch_warnings(record=True) as seen:\n"
+            "    warnings.simplefilter('always')\n"
+            "    import m2_amd\n"
+            "assert any('_param_check' in str(w.message) for w in seen)\n"
+            "from m2_amd import schedule\n"
+            "assert schedule._param_check is None\n"
+            "assert schedule.stack_plan(m2_amd.BertEncoder(m2_amd.m2_bert_80m(128)), 1, 128, None) is None\n")
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    r = subprocess.run([sys.executable, "-c", code], cwd=root, capture_output=True, text=True)
+    assert r.returncode == 0, r.stderr
