@@ -346,6 +346,11 @@ class BertEncoder(nn.Module):
         # post hooks of every module it recursed into: new weights drop the captured graphs
         self.register_load_state_dict_post_hook(BertEncoder._drop_graphs_after_load)
 
+    def __setstate__(self, state):
+        super().__setstate__(state)
+        self.__dict__.setdefault("native_schedule", True)          # encoders pickled before there were plans
+        self.__dict__.setdefault("_native_plans", {})
+
     # -- graph bookkeeping -------------------------------------------------------------------
     def reset_graphs(self) -> None:
         self._graphs = {}
@@ -589,6 +594,8 @@ class BertModel(nn.Module):
     """Embeddings + encoder + pooler; returns (sequence output or list of layer outputs, pooled output or None)
     like the reference (bert/src/bert_layers.py:880-1010)."""
 
+    _embed_part = None      # of the native schedule
+
     def __init__(self, config: M2BertConfig, add_pooling_layer: bool = True, use_hip_graph: bool = False):
         super().__init__()
         if getattr(config, "attention_pooling", False):
@@ -601,7 +608,6 @@ class BertModel(nn.Module):
         # synchronisation) and raises IndexError like nn.Embedding would; False leaves the flag to
         # `embeddings.check_indices()`.  The embedding tables are part of the captured graph too:
         self.validate_ids = True
-        self._embed_part = None      # of the native schedule
         self.register_load_state_dict_post_hook(lambda module, keys: module.encoder.reset_graphs())
 
     def _run_native(self, ids, tt, pos, all_layers: bool):

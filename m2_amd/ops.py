@@ -365,6 +365,10 @@ def split_channels(x: Tensor) -> Tensor:
     return out
 
 
+def WeightParts() -> None:
+    """What pickles of modules from when the parts of a weight were kept call by this name: nothing is kept now."""
+
+
 def _require_parts(t: Tensor, name: str, rows: int, nb: int, p: int) -> None:
     _require(t, name, torch.bfloat16, (_parts_elements(rows, nb, p),))
 
