@@ -160,7 +160,7 @@ int m2_fftconv_fwd(const void* x, const float* spec, void* y, int B, int L, int 
  * activations and the channel-major ones the core reads and writes:
  *   to_channels    out (N, M) = w (N, K) x (M, K)^T
  *   from_channels  out (M, N) = x (K, M)^T w (N, K)^T + bias (N, fp32 or NULL)
- * m2_dense_supported: M and N multiples of 8, K a multiple of 64, either operand below 4 GB.
+ * m2_dense_supported: M and N multiples of 8, K a multiple of 64, either operand below 4 GB.  All of them 16-byte aligned.
  * ------------------------------------------------------------------------------------------- */
 int m2_dense_supported(int M, int N, int K);
 int m2_dense_to_channels_fwd(const void* x, const void* w, void* out, int M, int N, int K, void* stream);
@@ -283,7 +283,7 @@ int m2_embed_layernorm_fwd(const long long* input_ids, const long long* token_ty
  * autocast: bert/src/mm/monarch_mixer_sequence_mixer.py:108,152, bert/src/mm/blockdiag_multiply.py:19-60).  An operand is
  * split into three bf16 parts per value, x = hi + mid + lo; the products use all terms down to 2^-24 relative and accumulate
  * in fp32.  A split operand of `rows` rows of `nblocks` blocks of `p` values takes m2_split_bytes (0: unsupported): p a
- * multiple of 4, below 4 GB.
+ * multiple of 4, below 4 GB.  Split operands are 16-byte aligned.
  *   m2_split_rows_fwd      x (M, nblocks p) fp32 -> parts; channel_major: NULL or (p, M) fp32, receives x^T (nblocks 1, M % 4 == 0)
  *   m2_split_jobs_fwd      one to four such operands in one launch (`jobs`: a HOST array)
  *   m2_split_channels_fwd  x (K, M) fp32 -> parts of x^T; M % 4 == 0
@@ -312,7 +312,7 @@ int m2_split_glu_fwd(const void* xs, const void* ws, void* out, int M, int nbloc
  * BertLayer :575-599), bf16 GEMMs, enqueued by one call.  `layers` is a HOST array of device pointers; `spectra` holds
  * the layers' filter spectra one after the other (m2_mixer_filters_fwd); `h16` (M, d) bf16 and `h_channel_major` (d, M) fp32
  * are the two forms of the input; out_f32[i] receives layer i's output (M, d) fp32 or is NULL.  The workspace holds
- * m2_encoder_layers_workspace_bytes.  Sizes: m2_dense_supported for both projections and what the other entry points
+ * m2_encoder_layers_workspace_bytes, 16-byte aligned.  Sizes: m2_dense_supported for both projections and what the other entry points
  * take.  `mlp_packed` (m2_mlp_fused_pack) selects the one-kernel MLP, else `glu_packed` (m2_glu_stream_pack) the streaming
  * gated product, else m2_blockdiag_glu_fwd.
  * ------------------------------------------------------------------------------------------- */

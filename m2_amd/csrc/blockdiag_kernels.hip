@@ -865,8 +865,9 @@ extern "C" int m2_blockdiag_linear_fwd(const void* x, const void* w, const float
   if (rc) return rc;
   hipStream_t st = (hipStream_t)stream;
   if (out_dtype == M2_DTYPE_BF16) {
-    // the row offsets of the tile engine's direct loads are 32 bits wide
-    if (p % 64 == 0 && (long)M * in_features * 2 < (1l << 32) && (long)nblocks * q * p * 2 < (1l << 32))
+    // the tile engine's direct loads take 16-byte aligned operands (the masked kernel loads through registers, which any address
+    // suits) and row offsets of 32 bits
+    if (p % 64 == 0 && aligned16(x, w, residual, out) && (long)M * in_features * 2 < (1l << 32) && (long)nblocks * q * p * 2 < (1l << 32))
       return blockdiag_linear_engine(x, w, bias, residual, out, M, nblocks, p, q, st);
     return q >= 128 ? launch_blockdiag<2, 2, false, uint16_t, 1, true>(x, w, bias, residual, out, M, nblocks, p, q, out_features, st)
                     : launch_blockdiag<4, 1, false, uint16_t, 1, true>(x, w, bias, residual, out, M, nblocks, p, q, out_features, st);

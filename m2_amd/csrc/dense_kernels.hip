@@ -281,6 +281,7 @@ static int check_dense(const char* who, const void* x, const void* w, const void
   if (M <= 0 || N <= 0 || K <= 0) return set_error(M2_ERR_ARG, "%s: sizes must be positive (M=%d N=%d K=%d)", who, M, N, K);
   if (!m2_dense_supported(M, N, K))
     return set_error(M2_ERR_UNSUPPORTED, "%s: needs M and N multiples of 8, K a multiple of 64 and operands below 4 GB (M=%d N=%d K=%d)", who, M, N, K);
+  if (!aligned16(x, w, out)) return set_error(M2_ERR_UNSUPPORTED, "%s: operands must be 16-byte aligned", who);
   return M2_OK;
 }
 

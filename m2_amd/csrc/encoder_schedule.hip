@@ -4,7 +4,7 @@
 //   y     (d, M)  = mixer core(xproj, hT, spec)    fftconv*_kernels.hip
 //   a     (M, d)  = y^T W_out^T + b                dense_kernels.hip
 //   s     (M, d)  = wo(glu(a)) + b + a, bf16       mlp_fused / glu_stream / dense / blockdiag kernels
-//   h16 | hT | out32 = LayerNorm(s)                blockdiag_kernels.hip
+//   h16 | hT | out32 = LayerNorm(s)                layernorm_kernels.hip
 //
 // Host code only: what it saves is the host's time per launch.  Issued module by module from Python a layer takes about
 // 170 us of host time whatever its size; here five or six launches of about 3 us each.
@@ -45,6 +45,7 @@ extern "C" int m2_encoder_layers_fwd(const m2_layer_params* layers, int nlayers,
     return set_error(M2_ERR_ARG, "%s: sizes must be positive (layers=%d B=%d L=%d d=%d I=%d)", who, nlayers, B, L, d, intermediate);
   if ((long)B * L > 0x7fffffffL) return set_error(M2_ERR_UNSUPPORTED, "%s: B * L = %ld does not fit an int", who, (long)B * L);
   const int M = B * L;
+  if (!aligned16(workspace)) return set_error(M2_ERR_UNSUPPORTED, "%s: the workspace must be 16-byte aligned", who);
   for (int i = 0; i < nlayers; ++i) {
     const m2_layer_params& p = layers[i];
     if (!p.in_w || !p.short_w || !p.short_b || !p.out_w || !p.w_gated || !p.w_out || !p.ln_gamma || !p.ln_beta)

@@ -11,6 +11,11 @@ namespace m2 {
 int set_error(int code, const char* fmt, ...) __attribute__((format(printf, 2, 3)));
 // hipGetLastError() after a launch -> 0 or M2_ERR_LAUNCH (message recorded).
 int check_launch(const char* what);
+// The direct global -> LDS loads take whole 16-byte pieces at 16-byte addresses.
+inline bool aligned16(const void* a, const void* b = nullptr, const void* c = nullptr, const void* d = nullptr) {
+  return (((uintptr_t)a | (uintptr_t)b | (uintptr_t)c | (uintptr_t)d) & 15) == 0;
+}
+
 // Compute units of the current device (cached per device).
 int num_cus();
 

@@ -327,6 +327,7 @@ static int launch_split(SplitArgs g, hipStream_t st) {
 // small ones fill the last round.  The gated product's epilogue takes 0.42 us per 1024 results.
 template <bool GLU>
 static int split_launch(const SplitArgs& g, hipStream_t st) {
+  if (!aligned16(g.p, g.q, g.parts)) return set_error(M2_ERR_UNSUPPORTED, "split_gemm: split operands must be 16-byte aligned");
   static const struct { int bi, bj; float first, step; } kTiles[5] = {
       {64, 64, 0.43f, 0.43f}, {128, 64, 1.0f, 0.69f}, {128, 128, 1.29f, 1.29f}, {192, 128, 1.65f, 1.65f}, {128, 192, 1.65f, 1.65f}};
   int best = 0;
@@ -373,6 +374,7 @@ extern "C" int m2_split_jobs_fwd(const m2_split_job* jobs, int njobs, void* stre
   for (int i = 0; i < njobs; ++i) {
     const m2_split_job& j = jobs[i];
     if (!j.x || !j.out) return set_error(M2_ERR_ARG, "%s: null pointer", who);
+    if (!aligned16(j.out)) return set_error(M2_ERR_UNSUPPORTED, "%s: split operands must be 16-byte aligned", who);
     if (!split_ok(j.rows, j.nblocks, j.p)) return set_error(M2_ERR_UNSUPPORTED, "%s: needs p a multiple of 4 and operands below 4 GB (M=%d nb=%d p=%d)", who, j.rows, j.nblocks, j.p);
     if (j.channel_major && (j.nblocks != 1 || j.rows % 4)) return set_error(M2_ERR_UNSUPPORTED, "%s: a channel-major copy needs one block and M a multiple of 4 (M=%d nb=%d)", who, j.rows, j.nblocks);
     const int gx = j.nblocks * (((j.p + 31) / 32 + 1) / 2);
@@ -395,6 +397,7 @@ extern "C" int m2_split_channels_fwd(const float* x, void* out, int M, int K, vo
   if (!x || !out) return set_error(M2_ERR_ARG, "%s: null pointer", who);
   if (!split_ok(M, 1, K) || M % 4 || M > 65535 * 32)
     return set_error(M2_ERR_UNSUPPORTED, "%s: needs M up to 2097120 and K multiples of 4 and operands below 4 GB (M=%d K=%d)", who, M, K);
+  if (!aligned16(out)) return set_error(M2_ERR_UNSUPPORTED, "%s: split operands must be 16-byte aligned", who);
   const int pc = (K + 31) / 32;
   hipLaunchKernelGGL(split_channels_kernel, dim3((pc + 1) / 2, (M + 31) / 32), dim3(256), 0, (hipStream_t)stream, x, (uint16_t*)out, M, K);
   return check_launch("split_channels");

@@ -141,7 +141,7 @@ class MonarchMixerSequenceMixing(nn.Module):
         M, d = x.shape
         w = self._cast("in_w", self.in_linear.weight, x.dtype)
         own = not (x.requires_grad and torch.is_grad_enabled())          # (the library call refuses those)
-        if own and x.dtype == torch.bfloat16 and x.data_ptr() % 16 == 0 and ops.own_to_channels(M, d):
+        if own and x.dtype == torch.bfloat16 and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0 and ops.own_to_channels(M, d):
             return ops.dense_to_channels(x, w)
         # Written as x @ W^T into the transposed view of the output: the same product as W @ x^T, for which the library
         # picks a faster kernel (126 against 144 us at M = 32768, d = 768)
@@ -168,7 +168,7 @@ class MonarchMixerSequenceMixing(nn.Module):
             return ops.split_linear(ops.split_channels(y), w_parts, M, 1, d, d,
                                     self._cast("out_b", self.out_linear.bias, torch.float32))
         w = self._cast("out_w", self.out_linear.weight, y.dtype)
-        if y.dtype == torch.bfloat16 and ops.own_from_channels(M, d):
+        if y.dtype == torch.bfloat16 and w.data_ptr() % 16 == 0 and ops.own_from_channels(M, d):
             return ops.dense_from_channels(y, w, self._cast("out_b", self.out_linear.bias, torch.float32))
         return torch.addmm(self._cast("out_b", self.out_linear.bias, y.dtype), y.t(), w.t())
 

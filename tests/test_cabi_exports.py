@@ -132,3 +132,23 @@ def test_static_scratch_covers_what_its_documentation_promises():
         for d in (768, 1536):
             assert lib.m2_hyena_filter_workspace_bytes(nf, L, d, 128) <= M2_HYENA_FILTER_STATIC_SCRATCH_BYTES, (nf, L, d)
     assert lib.m2_hyena_filter_workspace_bytes(2, 16384, 768, 128) > M2_HYENA_FILTER_STATIC_SCRATCH_BYTES
+
+
+def test_unaligned_operands_are_refused():
+    """What goes through direct 16-byte loads has to lie at a multiple of 16; nothing is launched otherwise."""
+    from m2_amd._lib import LayerParams, SplitJob, lib
+    ok, off = ctypes.c_void_p(4096), ctypes.c_void_p(4098)
+    for args in ((off, ok, ok), (ok, off, ok), (ok, ok, off)):
+        assert lib.m2_dense_to_channels_fwd(*args, 64, 64, 64, None) == -2 and b"aligned" in lib.m2_last_error()
+        x, w, out = args
+        assert lib.m2_dense_from_channels_fwd(x, w, None, out, 64, 64, 64, None) == -2 and b"aligned" in lib.m2_last_error()
+    job = (SplitJob * 1)((4096, 4098, None, 32, 1, 32))
+    assert lib.m2_split_jobs_fwd(job, 1, None) == -2 and b"aligned" in lib.m2_last_error()
+    assert lib.m2_split_jobs_fwd(job, 5, None) == -1 and lib.m2_split_jobs_fwd(job, 0, None) == -1
+    assert lib.m2_split_channels_fwd(ok, off, 32, 32, None) == -2 and b"aligned" in lib.m2_last_error()
+    assert lib.m2_split_to_channels_fwd(off, ok, ok, 32, 32, 32, None) == -2 and b"aligned" in lib.m2_last_error()
+    assert lib.m2_split_linear_fwd(ok, off, None, None, ok, 32, 2, 32, 32, None) == -2 and b"aligned" in lib.m2_last_error()
+    assert lib.m2_split_glu_fwd(ok, off, ok, 32, 2, 32, 64, None) == -2 and b"aligned" in lib.m2_last_error()
+    layers, outs = (LayerParams * 1)(), (ctypes.c_void_p * 1)()
+    assert lib.m2_encoder_layers_fwd(layers, 1, ok, ok, ok, outs, off, 1, 128, 768, 3072, 4, 1e-12, None) == -2
+    assert b"aligned" in lib.m2_last_error()

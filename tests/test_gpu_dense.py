@@ -99,3 +99,37 @@ def test_glu_stream_split_chunks(gpu, M, d):
     rows = torch.cat([torch.arange(min(M, 40)), torch.arange(max(0, M - 140), M)]).unique()
     _within_glu(got[rows.to(gpu)], *_glu(x[rows], w))
     assert (got.float() - tiled.float()).abs().max() <= 2.0 ** -6 * tiled.float().abs().max()
+
+
+def _unaligned(t):
+    """The same values two bytes off a 16-byte address."""
+    buf = torch.empty(t.numel() + 8, dtype=t.dtype, device=t.device)
+    off = next(k for k in range(8) if (buf.data_ptr() + k * t.element_size()) % 16 == t.element_size())
+    return buf[off:off + t.numel()].view_as(t).copy_(t)
+
+
+def test_unaligned_bf16_operands(gpu):
+    """Weights that are views into a flat bf16 buffer, and inputs, residuals and outputs at any address: kernels that load 16 bytes at a
+    time through LDS are not used for them, the results are those of aligned ones."""
+    import m2_amd
+    from m2_amd import ops
+    g = torch.Generator().manual_seed(5)
+    for M, nb, q, p in ((33, 4, 192, 768), (1000, 4, 384, 1536), (2049, 2, 448, 1792)):
+        x, w, res, bias = _bf16(g, M, nb * p), _bf16(g, nb, q, p) * 0.05, _bf16(g, M, nb * q), torch.randn(nb * q, generator=g)
+        ref, absref = _blockdiag(x.double(), w.double()), _blockdiag(x.double().abs(), w.double().abs())
+        ref, absref = ref + bias.double() + res.double(), absref + bias.double().abs() + res.double().abs()
+        xg, wg, rg, bg = x.to(gpu), w.to(gpu), res.to(gpu), bias.to(gpu)
+        _within_bf16(ops.blockdiag_linear(_unaligned(xg), wg, bg, rg), ref, absref)
+        _within_bf16(ops.blockdiag_linear(xg, _unaligned(wg), bg, rg), ref, absref)
+        _within_bf16(ops.blockdiag_linear(xg, wg, bg, _unaligned(rg)), ref, absref)
+        out = _unaligned(torch.empty(M, nb * q, dtype=torch.bfloat16, device=gpu))
+        _within_bf16(ops.blockdiag_linear(xg, wg, bg, rg, out=out), ref, absref)
+    layer = m2_amd.BertLayer(m2_amd.m2_bert_80m(128)).to(gpu).eval()
+    u = torch.randn(2, 128, 768, generator=g).to(gpu).bfloat16()
+    with torch.no_grad():
+        want = layer(u).float()
+        for lin in (layer.attention.in_linear, layer.attention.out_linear, layer.mlp.gated_layers, layer.mlp.wo):
+            lin.weight = torch.nn.Parameter(_unaligned(lin.weight.detach().bfloat16()))
+            assert lin.weight.data_ptr() % 16 == 2
+        for got in (layer(u), layer(_unaligned(u))):
+            assert (got.float() - want).norm() <= 1e-2 * want.norm()
