@@ -181,6 +181,8 @@ int m2_dense_from_channels_fwd(const void* x, const void* w, const float* bias, 
  * reference's 960-wide model, run on a masked variant of the general kernel). */
 int m2_blockdiag_glu_fwd(const void* x, const void* w, void* out, int M, int in_features, int intermediate,
                          int nblocks, void* stream);
+/* 1: m2_blockdiag_glu_fwd has a kernel for so few rows that beats m2_glu_stream_fwd (host code). */
+int m2_blockdiag_glu_few_rows(int M, int in_features, int nblocks);
 
 /* out = blockdiag_multiply(x, w) (+ bias) (+ residual).
  * x (M, in_features) bf16; w (nblocks, out/nblocks, in/nblocks) bf16; bias (out_features) fp32 or NULL;

@@ -289,6 +289,11 @@ static int check_dense(const char* who, const void* x, const void* w, const void
 
 using namespace m2;
 
+extern "C" int m2_blockdiag_glu_few_rows(int M, int in_features, int nblocks) {
+  if (M <= 0 || nblocks <= 0 || in_features <= 0 || in_features % nblocks) return 0;
+  return glu_few_rows_pays(M, nblocks, in_features / nblocks) ? 1 : 0;
+}
+
 extern "C" int m2_dense_supported(int M, int N, int K) {
   if (M < 8 || N < 8 || K < 64 || M % 8 || N % 8 || K % 64) return 0;
   // the direct loads of the tile engine take 32-bit byte offsets

@@ -148,9 +148,9 @@ class BertGatedLinearUnitMLP(nn.Module):
         """(one-kernel MLP?, few rows?) for M rows.  Up to 512 rows the one-kernel MLP leaves most compute units idle
         (21.5 us whatever the row count) and the two products as kernels of their own take 11 us at M = 128, 12.5 at 256,
         19 at 512, 20 at 1024.  For few rows m2_blockdiag_glu_fwd has a kernel that beats the streaming one."""
-        d = self.config.hidden_size
-        fused = M > 512 and ops.mlp_fused_supported(d, self.config.intermediate_size, self.config.monarch_mlp_nblocks)
-        return fused, M * d <= 245760
+        d, nb = self.config.hidden_size, self.config.monarch_mlp_nblocks
+        fused = M > 512 and ops.mlp_fused_supported(d, self.config.intermediate_size, nb)
+        return fused, bool(ops.lib.m2_blockdiag_glu_few_rows(M, d, nb))
 
     def packed_mlp(self, wg: torch.Tensor, wo: torch.Tensor) -> torch.Tensor:
         """The packed copy the one-kernel MLP streams: rebuilt whenever one of the bf16 copies has been rebuilt.  (What a stream

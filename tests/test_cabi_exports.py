@@ -152,3 +152,17 @@ def test_unaligned_operands_are_refused():
     layers, outs = (LayerParams * 1)(), (ctypes.c_void_p * 1)()
     assert lib.m2_encoder_layers_fwd(layers, 1, ok, ok, ok, outs, off, 1, 128, 768, 3072, 4, 1e-12, None) == -2
     assert b"aligned" in lib.m2_last_error()
+
+
+def test_few_rows_rule_is_the_library_s():
+    """The modules ask the library which gated product serves a row count, at every width."""
+    import m2_amd
+    from m2_amd._lib import lib
+    for helper, rows in (("m2_bert_80m", 320), ("m2_bert_110m", 256), ("m2_bert_large", 160), ("m2_bert_341m", 137)):
+        cfg = getattr(m2_amd, helper)(128)
+        mlp = m2_amd.BertLayer(cfg).mlp
+        d, nb = cfg.hidden_size, cfg.monarch_mlp_nblocks
+        assert [lib.m2_blockdiag_glu_few_rows(M, d, nb) for M in (1, rows, rows + 1)] == [1, 1, 0]
+        assert mlp.mlp_route(rows)[1] is True and mlp.mlp_route(rows + 1)[1] is False
+    assert lib.m2_blockdiag_glu_few_rows(8, 4096, 4) == 0 and lib.m2_blockdiag_glu_few_rows(0, 768, 4) == 0
+    assert lib.m2_blockdiag_glu_few_rows(8, 770, 4) == 0 and lib.m2_blockdiag_glu_few_rows(8, 768, 0) == 0
