@@ -29,7 +29,7 @@ struct TensorSlot {
   c10::SmallVector<int64_t, 4> sizes, strides;
 };
 struct ValueSlot {
-  PyObject *dict, *key, *expected;
+  PyObject *dict, *key, *expected;      // expected: null where the dict has no such key
 };
 struct Checker {
   PyObject_HEAD
@@ -48,7 +48,7 @@ const at::Tensor* look_up(PyObject* dict, PyObject* key) {
 // Equal plain values: the object itself, or a number or text of the same type that compares equal.
 bool same_value(PyObject* a, PyObject* b) {
   if (a == b) return true;
-  if (!a || Py_TYPE(a) != Py_TYPE(b) || !(PyFloat_CheckExact(a) || PyLong_CheckExact(a) || PyUnicode_CheckExact(a))) return false;
+  if (!a || !b || Py_TYPE(a) != Py_TYPE(b) || !(PyFloat_CheckExact(a) || PyLong_CheckExact(a) || PyUnicode_CheckExact(a))) return false;
   return PyObject_RichCompareBool(a, b, Py_EQ) == 1;
 }
 int64_t version_of(const at::Tensor& t) { return t.is_inference() ? 0 : t._version(); }
@@ -86,7 +86,7 @@ int checker_clear(PyObject* self) {
   c->modules = nullptr;
   c->tensors = nullptr;
   c->values = nullptr;
-  for (PyObject* o : drop) Py_DECREF(o);
+  for (PyObject* o : drop) Py_XDECREF(o);
   return 0;
 }
 
@@ -96,14 +96,14 @@ void checker_dealloc(PyObject* self) {
   Py_TYPE(self)->tp_free(self);
 }
 
-// (dict, key) pairs and the object at each of them
+// (dict, key) pairs and the object at each of them (a value may be absent)
 template <typename Slot>
 bool record(PyObject* list, std::vector<Slot>* slots) {
   for (Py_ssize_t i = 0; i < PyList_GET_SIZE(list); ++i) {
     PyObject *dict, *key;
     if (!PyArg_ParseTuple(PyList_GET_ITEM(list, i), "O!O", &PyDict_Type, &dict, &key)) return false;
     PyObject* o = PyDict_GetItemWithError(dict, key);
-    if (!o) {
+    if (!o && (PyErr_Occurred() || std::is_same<Slot, ModuleSlot>::value)) {
       if (!PyErr_Occurred()) PyErr_SetObject(PyExc_KeyError, key);
       return false;
     }
@@ -113,7 +113,7 @@ bool record(PyObject* list, std::vector<Slot>* slots) {
     } else {
       slots->push_back({dict, key, o});
     }
-    Py_INCREF(dict); Py_INCREF(key); Py_INCREF(o);
+    Py_INCREF(dict); Py_INCREF(key); Py_XINCREF(o);
   }
   return true;
 }

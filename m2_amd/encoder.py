@@ -385,8 +385,8 @@ class BertEncoder(nn.Module):
                 graded = torch.is_grad_enabled() and (h16.requires_grad or hT.requires_grad)
                 found = None if graded else schedule.stack_plan(self, B, L, h16.device)
                 if found is not None:
-                    plan, which = found
-                    return plan.run(which, B, all_layers, h16, hT)
+                    plan, route = found
+                    return plan.run(route, B, all_layers, h16, hT)
             outs = []
             n = len(self.layer)
             o32 = h32
@@ -509,7 +509,7 @@ class BertEncoder(nn.Module):
                                                                                    for b in skips)
         if self._filter_table is None or self._filter_table[0] != probe:
             plan = self._native_plans.get(L)
-            if plan is not None and plan.current(self):      # (its table is this one; a stream capture could not make another)
+            if plan is not None and plan.usable and plan.current(self):      # (its table is this one; a stream capture could not make another)
                 return plan.table, groups
             self._filter_table = (probe, ops.FilterTable([e[0] for e in entries], [e[1] for e in entries], L, m0.d_model,
                                                          m0.filter_fn.order, m0.filter_fn.emb_dim))
@@ -519,7 +519,7 @@ class BertEncoder(nn.Module):
         """What a graph captured just now for length L reads beside parameters: pointer tables and packed weights, which
         forwards of other lengths replace here and which therefore have to live as long as the graph."""
         table, plan = self._filter_table, self._native_plans.get(L)
-        return tuple(r for r in (None if table is None else table[1], plan) if r is not None)
+        return tuple(([] if table is None else [table[1]]) + ([plan] if plan is not None and plan.usable else []))
 
     def _run_graphed(self, h32: Optional[torch.Tensor], B: int, L: int, all_layers: bool,
                      h16: Optional[torch.Tensor] = None, hT: Optional[torch.Tensor] = None) -> List[torch.Tensor]:
@@ -544,7 +544,7 @@ class BertEncoder(nn.Module):
             if dst is not None:
                 dst.copy_(src)
         for held in reads:
-            held.use_on_current_stream()
+            held.use_on(torch.cuda.current_stream())
         graph.replay()
         return [o.clone() for o in static_out]
 
@@ -632,8 +632,8 @@ class BertModel(nn.Module):
         part = None if found is None else schedule.embed_part(self, found[0].d)
         if part is None:
             return None
-        plan, which = found
-        return plan.run(which, B, all_layers, None, None, part, ids.contiguous(), tt, pos)
+        plan, route = found
+        return plan.run(route, B, all_layers, None, None, part, ids.contiguous(), tt, pos)
 
     def get_input_embeddings(self):
         return self.embeddings.word_embeddings
@@ -684,7 +684,7 @@ class BertModel(nn.Module):
                 if dst is not None:
                     dst.copy_(src)
             for held in reads:
-                held.use_on_current_stream()
+                held.use_on(torch.cuda.current_stream())
             graph.replay()
             outs = [o.clone() for o in static_out]
         enc = [o.view(B, L, -1) for o in outs]

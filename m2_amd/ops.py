@@ -107,8 +107,8 @@ def hyena_filter_taps(filters: Sequence[dict], L: int, d: int, order: int, emb_d
 
 
 class StreamUse:
-    """Device memory that is made once on one stream and read on any, then dropped at any time.  `use_on_current_stream` comes
-    before each launch that reads it: a stream met for the first time waits for `ready`, the event behind what made the memory
+    """Device memory that is made once on one stream and read on any, then dropped at any time.  `use_on` comes before each
+    launch that reads it: a stream met for the first time waits for `ready`, the event behind what made the memory
     (None: it was complete when the host went on), and the allocator keeps the memory back, once it is dropped, until that stream
     has come past its last use."""
 
@@ -116,8 +116,7 @@ class StreamUse:
         self.tensors, self.ready = list(tensors), ready
         self.streams = {torch.cuda.current_stream().cuda_stream}
 
-    def use_on_current_stream(self) -> None:
-        stream = torch.cuda.current_stream()
+    def use_on(self, stream: "torch.cuda.Stream") -> None:
         if stream.cuda_stream in self.streams:
             return
         for t in self.tensors:
@@ -180,8 +179,8 @@ class FilterTable:
         self.skip = torch.tensor(skip_row, dtype=torch.int64).to(dev)
         self._use = StreamUse((self.table, self.skip))
 
-    def use_on_current_stream(self) -> None:
-        self._use.use_on_current_stream()
+    def use_on(self, stream: "torch.cuda.Stream") -> None:
+        self._use.use_on(stream)
 
     @classmethod
     def of_rows(cls, rows: Sequence[Sequence[Optional[Tensor]]], skips: Sequence[Tensor], fpm: int, L: int, d: int, order: int,
@@ -218,7 +217,7 @@ def mixer_filter_spectra(table: FilterTable, w_mod: float = 1.0, shift: float = 
     if first < 0 or count < 1 or first + count > table.nmixers:
         raise ValueError(f"mixers [{first}, {first + count}) outside the table of {table.nmixers}")
     dev = table.table.device
-    table.use_on_current_stream()
+    table.use_on(torch.cuda.current_stream())
     n = table.spectrum_floats()
     if out is None:
         out = torch.empty(count, n, dtype=torch.float32, device=dev)

@@ -48,15 +48,19 @@ class _Slots:
 
     def child(self, mod, key, kind=None):
         found = mod._modules.get(key)
-        if found is None or (kind is not None and type(found) is not kind):
-            raise ValueError(f"{key} is not the module it was built as")
+        if found is None:
+            self.values.append((mod._modules, key))
+            raise ValueError(f"no module {key}")
         self.modules.append((mod._modules, key))
+        if kind is not None and type(found) is not kind:
+            raise ValueError(f"{key} is not the module it was built as")
         return found
 
     def tensor(self, mod, key, how=_IN_PLACE, shape=None):
         where = mod._parameters if key in mod._parameters else mod._buffers
         t = where.get(key)
         if t is None:                                  # absent, or computed (a parametrisation, weight_norm, pruning)
+            self.values += [(mod._parameters, key), (mod._buffers, key)]
             raise ValueError(f"{key} is not a plain parameter")
         self.tensors.append((where, key, how))
         if not (t.is_cuda and t.dtype == torch.float32 and t.is_contiguous()):
@@ -66,10 +70,15 @@ class _Slots:
         return t
 
     def value(self, obj, key):
+        self.values.append((obj.__dict__, key))
         if key not in obj.__dict__:
             raise ValueError(f"no plain attribute {key}")
-        self.values.append((obj.__dict__, key))
         return obj.__dict__[key]
+
+    def option(self, obj, key):
+        """An attribute of the object, or of its class where the object has none of its own."""
+        self.values.append((obj.__dict__, key))
+        return getattr(obj, key)
 
     def checker(self):
         return _param_check.Checker(self.modules, self.tensors, self.values)
@@ -110,23 +119,53 @@ def embed_part(model, d: int) -> Optional[EmbedPart]:
     return part
 
 
-class StackPlan:
-    """Device pointers of an encoder's layers for one length, for every row count: what any of them reads is made with the plan, so
-    that a forward of another batch size needs nothing that a stream capture could not make."""
+# (options of the MLP that the native schedule has a path for)
+_MLP_OPTIONS = {"fuse_wo_layernorm": False, "fuse_mlp": True, "bf16_presum": True, "stream_glu": True}
 
-    def __init__(self, encoder, L: int):
-        slots = _Slots()
-        slots.modules.append((encoder._modules, "layer"))
+
+def _class_options() -> tuple:
+    return tuple(bool(getattr(_encoder.BertGatedLinearUnitMLP, key)) for key in _MLP_OPTIONS)
+
+
+class NoPlan:
+    """That an encoder as it is has no plan: what was looked at before that was clear, so as not to look at it again each time."""
+
+    usable, keep = False, ()
+
+    def __init__(self, encoder, slots: _Slots):
+        self.layers = len(encoder._modules["layer"]._modules)
+        self.class_options = _class_options()
+        self.checker = slots.checker()
+
+    def current(self, encoder) -> bool:
+        return (self.layers == len(encoder._modules["layer"]._modules) and self.class_options == _class_options()
+                and self.checker.unchanged())
+
+    def __reduce__(self):                    # a plan belongs to its modules: copies and pickles of them make their own
+        return type(None), ()
+
+
+class StackPlan(NoPlan):
+    """Device pointers of an encoder's layers for one length, for every row count.  The packed weights of a route come with its first
+    use outside a stream capture; a capture that wants them earlier takes the Python schedule, and the table from here."""
+
+    usable = True
+
+    def __init__(self, encoder, L: int, slots: _Slots):
         child, tensor, value = slots.child, slots.tensor, slots.value
         stack = encoder._modules["layer"]
         n = len(stack._modules)
-        self.layers = n
-        self.arrays = [(LayerParams * n)(), None, None]        # plain; with the streaming product's packed weights; with the MLP's
+        plain = (LayerParams * n)()
         self.keep: List[torch.Tensor] = []
+        self.mlps = []
         rows, skips = [], []
         for i, key in enumerate(stack._modules):
-            lay = child(stack, key)
-            at, mlp = child(lay, "attention"), child(lay, "mlp")
+            lay = child(stack, key, _encoder.BertLayer)
+            # classes of a caller's own run their own methods
+            at, mlp = child(lay, "attention", MonarchMixerSequenceMixing), child(lay, "mlp", _encoder.BertGatedLinearUnitMLP)
+            if (slots.option(at, "cache_filters") or slots.option(at, "hyena_training_additions")
+                    or any(bool(slots.option(mlp, k)) is not v for k, v in _MLP_OPTIONS.items())):
+                raise ValueError("options of the Python schedule")
             for name in ("filter_fn", "filter_fn2")[:2 if value(at, "residual_long_conv") else 1]:
                 f = child(at, name, HyenaFilter)
                 skips.append(tensor(f, "bias"))
@@ -160,7 +199,7 @@ class StackPlan:
             w_in, w_out = at._cast("in_w", lin_in.weight, torch.bfloat16), at._cast("out_w", lin_out.weight, torch.bfloat16)
             wg16, wo16 = gated.weight_bf16(), wo.weight_bf16()
             self.keep += [w_in, w_out, wg16, wo16]
-            p = self.arrays[0][i]
+            p = plain[i]
             p.in_w, p.out_w, p.w_gated, p.w_out = w_in.data_ptr(), w_out.data_ptr(), wg16.data_ptr(), wo16.data_ptr()
             (p.in_b, p.out_b, p.short_w, p.short_b, p.wo_b, p.ln_gamma, p.ln_beta) = [t.data_ptr() for t in in_place]
             p.residual = 1 if at.residual_long_conv else 0
@@ -170,55 +209,59 @@ class StackPlan:
                 f0 = at.filter_fn
                 self.d, self.I, self.nb, self.eps = sizes
                 self.w_mod, self.shift = float(f0.w_mod), float(f0.modulation.shift)
-                if ops.glu_stream_supported(self.d, self.I, self.nb):
-                    self.arrays[1] = (LayerParams * n)()
-                if ops.mlp_fused_supported(self.d, self.I, self.nb):
-                    self.arrays[2] = (LayerParams * n)()
+                self.supported = (True, ops.glu_stream_supported(self.d, self.I, self.nb), ops.mlp_fused_supported(self.d, self.I, self.nb))
             elif sizes != (self.d, self.I, self.nb, self.eps):
                 raise ValueError("layers that differ")
-            if self.arrays[1] is not None:
-                self.arrays[1][i] = p
-                self.keep.append(mlp.packed_glu(wg16))
-                self.arrays[1][i].glu_packed = self.keep[-1].data_ptr()
-            if self.arrays[2] is not None:
-                self.arrays[2][i] = p
-                self.keep.append(mlp.packed_mlp(wg16, wo16))
-                self.arrays[2][i].mlp_packed = self.keep[-1].data_ptr()
+            self.mlps.append(mlp)
         self.table = ops.FilterTable.of_rows(rows, skips, len(rows) // n, L, self.d, f0.order, f0.emb_dim)
-        self.checker = slots.checker()
+        super().__init__(encoder, slots)
         self.device = self.table.table.device
-        ready = torch.cuda.Event()
-        ready.record()
-        self._use = ops.StreamUse(self.keep, ready)
+        # the layers' pointers with the memory they need: plain, with the streaming product's packed weights, with the one-kernel MLP's
+        self.routes: list = [(plain, self._made_here(self.keep)), None, None]
         self.L = L
         self.spec_bytes = lib.m2_filter_spectrum_bytes(self.d, L)
         self.filter_ws = lib.m2_mixer_filters_workspace_bytes(n, self.table.fpm, L, self.d, self.table.order)
         self.filter_ws_layer = max(1, lib.m2_mixer_filters_workspace_bytes(1, self.table.fpm, L, self.d, self.table.order))
 
-    def use_on_current_stream(self) -> None:
-        self.table.use_on_current_stream()
-        self._use.use_on_current_stream()
+    @staticmethod
+    def _made_here(tensors) -> ops.StreamUse:
+        ready = torch.cuda.Event()
+        ready.record()
+        return ops.StreamUse(tensors, ready)
 
-    def route(self, mlp, M: int) -> Optional[int]:
-        """Which of `arrays` serves M rows."""
-        fused, few = mlp.mlp_route(M)
-        which = 2 if fused else 1 if not few and self.arrays[1] is not None else 0
-        return which if self.arrays[which] is not None else None
+    def use_on(self, stream: torch.cuda.Stream) -> None:
+        self.table.use_on(stream)
+        for route in self.routes:
+            if route is not None:
+                route[1].use_on(stream)
 
-    def current(self, encoder) -> bool:
-        return self.layers == len(encoder._modules["layer"]._modules) and self.checker.unchanged()
+    def route(self, M: int):
+        """The one of `routes` that serves M rows, or None where it would have to be made during a stream capture."""
+        fused, few = self.mlps[-1].mlp_route(M)
+        which = 2 if fused else 1 if not few and self.supported[1] else 0
+        found = self.routes[which]
+        if found is None and self.supported[which] and not torch.cuda.is_current_stream_capturing():
+            packs, array = [], (LayerParams * self.layers)()
+            for i, mlp in enumerate(self.mlps):
+                array[i] = self.routes[0][0][i]
+                wg16, wo16 = self.keep[4 * i + 2], self.keep[4 * i + 3]
+                packs.append(mlp.packed_glu(wg16) if which == 1 else mlp.packed_mlp(wg16, wo16))
+                setattr(array[i], "glu_packed" if which == 1 else "mlp_packed", packs[-1].data_ptr())
+            self.routes[which] = found = (array, self._made_here(packs))
+        return found
 
-    def __reduce__(self):                    # a plan belongs to its modules: copies and pickles of them make their own
-        return type(None), ()
-
-    def run(self, which: int, B: int, all_layers: bool, h16: Optional[torch.Tensor], hT: Optional[torch.Tensor],
+    def run(self, route, B: int, all_layers: bool, h16: Optional[torch.Tensor], hT: Optional[torch.Tensor],
             part: Optional[EmbedPart] = None, ids=None, tt=None, pos=None):
         """Enqueues the stack on the current stream; input either as h16 / hT or as token ids for the embeddings (`part`)."""
         n, L, d = self.layers, self.L, self.d
         M = B * L
         dev = ids.device if ids is not None else h16.device
-        stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
-        self.use_on_current_stream()
+        current = torch.cuda.current_stream()
+        t = self.table
+        t.use_on(current)
+        self.routes[0][1].use_on(current)
+        route[1].use_on(current)
+        stream = ctypes.c_void_p(current.cuda_stream)
         up = lambda v: (v + 255) & ~255      # noqa: E731
         o_spec = up(self.filter_ws)
         o_act = o_spec + up(n * self.spec_bytes)
@@ -229,7 +272,6 @@ class StackPlan:
         ptrs = (ctypes.c_void_p * n)()
         for i, o in enumerate(outs):
             ptrs[n - len(outs) + i] = o.data_ptr()
-        t = self.table
         check(lib.m2_mixer_filters_fwd(t.table.data_ptr(), t.skip.data_ptr(), n, t.fpm, L, d, t.order, t.emb_dim, self.w_mod, self.shift,
                                        base, base + o_spec, stream))
         if ids is not None:
@@ -238,42 +280,42 @@ class StackPlan:
                                              *part.args, None, p16, pT, part.bad_index, B, L, d, stream))
         else:
             p16, pT = h16.data_ptr(), hT.data_ptr()
-        check(lib.m2_encoder_layers_fwd(self.arrays[which], n, base + o_spec, p16, pT, ptrs, base + o_act, B, L, d, self.I, self.nb, self.eps, stream))
+        check(lib.m2_encoder_layers_fwd(route[0], n, base + o_spec, p16, pT, ptrs, base + o_act, B, L, d, self.I, self.nb, self.eps, stream))
         return outs
 
 
 def stack_plan(encoder, B: int, L: int, device: torch.device):
-    """(the plan for L, made or re-used, and which of its arrays serves B L rows), or None where the Python schedule serves."""
+    """(the plan for L, made or re-used, and the route of it that serves B L rows), or None where the Python schedule serves."""
     if _param_check is None or not encoder.native_schedule or not encoder.batch_filters or encoder.overlap_filters not in (None, False):
         return None
     M = B * L
-    for lay in encoder._modules["layer"]._modules.values():
-        if type(lay) is not _encoder.BertLayer:
+    plan = encoder._native_plans.get(L)
+    if plan is not None and plan.current(encoder):
+        if not plan.usable:
             return None
-        at, mlp = lay._modules.get("attention"), lay._modules.get("mlp")
-        # classes of a caller's own run their own methods
-        if type(at) is not MonarchMixerSequenceMixing or type(mlp) is not _encoder.BertGatedLinearUnitMLP:
+        d = plan.d
+    else:
+        plan, first = None, next(iter(encoder._modules["layer"]._modules.values()), None)
+        if type(first) is not _encoder.BertLayer or type(first.attention) is not MonarchMixerSequenceMixing:
             return None
-        if (at.cache_filters or at.hyena_training_additions or mlp.fuse_wo_layernorm or not mlp.fuse_mlp or not mlp.bf16_presum
-                or not mlp.stream_glu):
-            return None
-    d = at.d_model
-    w = at.in_linear.weight
-    if w.dtype != torch.float32 or not w.is_cuda:
-        return None
+        d = first.attention.d_model
     if not ops.own_to_channels(M, d) or not ops.own_from_channels(M, d):
         return None
-    plan = encoder._native_plans.get(L)
-    if plan is None or not plan.current(encoder):
+    if plan is None:
         if torch.cuda.is_current_stream_capturing():
             return None                              # the filter table is copied from the host: not inside a capture
         groups = encoder._batched_filter_groups(L)   # the same rule: layers alike, spectra small enough, ...
         if groups is None or len(groups) != 1:
             return None
+        slots = _Slots()
+        slots.modules.append((encoder._modules, "layer"))
         try:
-            plan = StackPlan(encoder, L)
+            plan = StackPlan(encoder, L, slots)
         except ValueError:
-            return None
+            try:
+                plan = NoPlan(encoder, slots)
+            except (KeyError, ValueError):
+                return None
         # What changed for one length changed for others: none of them keeps copies of replaced weights.  (At most one plan for
         # each of the nine lengths.)
         for other, p in list(encoder._native_plans.items()):
@@ -283,5 +325,7 @@ def stack_plan(encoder, B: int, L: int, device: torch.device):
     elif (plan.layers * plan.spec_bytes > encoder.UPFRONT_MAX_BYTES                     # (limits that were lowered since)
           or encoder.FILTER_WORKSPACE_BYTES // plan.filter_ws_layer < plan.layers):
         return None
-    which = plan.route(mlp, M)
-    return None if which is None or plan.device != device else (plan, which)
+    if not plan.usable or plan.device != device:
+        return None
+    route = plan.route(M)
+    return None if route is None else (plan, route)

@@ -320,7 +320,7 @@ def test_computed_weights_and_other_classes_take_the_python_schedule(gpu):
         "weight norm": lambda lay: torch.nn.utils.parametrizations.weight_norm(lay.attention.out_linear),
         "pruned": lambda lay: prune.random_unstructured(lay.attention.out_linear, "weight", 0.5),
         "layer": lambda lay: retype(lay, OwnLayer), "mixer": lambda lay: retype(lay.attention, OwnMixer),
-        "mlp": lambda lay: retype(lay.mlp, OwnMLP), "linear": lambda lay: retype(lay.mlp.gated_layers, OwnLinear)}
+        "option": lambda lay: setattr(lay.mlp, "bf16_presum", False), "mlp": lambda lay: retype(lay.mlp, OwnMLP), "linear": lambda lay: retype(lay.mlp.gated_layers, OwnLinear)}
     for what, change in changes.items():
         for first in (False, True):                  # changed before any plan, and after one was made
             model = _model(cfg, gpu, 29)
@@ -335,6 +335,11 @@ def test_computed_weights_and_other_classes_take_the_python_schedule(gpu):
             assert torch.equal(got, want), what
             if what != "weight norm":                # (that one keeps the values)
                 assert not torch.equal(got, before), what
+            model.encoder.native_schedule = True     # that there is no plan is remembered, until something changes
+            none = model.encoder._native_plans[128]
+            assert torch.equal(model(ids)[0], want) and not none.usable and model.encoder._native_plans[128] is none, what
+            model.encoder.layer[1] = _model(cfg, gpu, 29).encoder.layer[1]
+            assert torch.equal(model(ids)[0], before) and model.encoder._native_plans[128].usable, what
 
 
 def test_a_layer_class_with_the_plain_signature(gpu):
@@ -493,7 +498,7 @@ def test_a_dropped_plan_outlives_its_use_on_another_stream(gpu):
         got = model(ids)[0]
     plan = model.encoder._native_plans[128]
     address, like = plan.table.table.data_ptr(), plan.table.table.shape
-    assert plan._use.streams >= {side.cuda_stream} and plan.table._use.streams >= {side.cuda_stream}
+    assert plan.routes[0][1].streams >= {side.cuda_stream} and plan.table._use.streams >= {side.cuda_stream}
     del plan
     model.encoder._native_plans.clear()
     new = [torch.full(like, 1, dtype=torch.int64, device=gpu) for _ in range(32)]

@@ -67,6 +67,10 @@ def test_plain_values_are_compared(value, others):
     assert check.unchanged()
     del lin.eps
     assert not check.unchanged()
+    absent = _param_check.Checker([], [], [(lin.__dict__, "eps")])          # and the absence of one
+    assert absent.unchanged()
+    lin.eps = None
+    assert not absent.unchanged()
 
 
 def test_a_part_of_the_recorded_tensor_is_another():
