@@ -1,5 +1,5 @@
-// fp32 matrix products on the bf16 matrix cores: every fp32 operand as three bf16 parts (x = hi + mid + lo exactly, 8 + 8 + 8
-// mantissa bits) and the six products down to 2^-24 relative (hi hi, hi mid, mid hi, mid mid, hi lo, lo hi), fp32
+// fp32 matrix products on the bf16 matrix cores: every fp32 operand as three bf16 parts (x = hi + mid + lo, 8 + 8 + 8 mantissa
+// bits: exact down to |x| = 2^-110; bf16 ends at 2^-133, so smaller values lose low bits) and the six products down to 2^-24 relative (hi hi, hi mid, mid hi, mid mid, hi lo, lo hi), fp32
 // accumulation.  The dense projections and the block-diagonal MLP of fp32 callers outside autocast.
 //
 // What bounds an fp32 product here is the matrix pipe: 157 TFLOP/s for fp32 operands, 2.5 PFLOP/s for bf16 ones, i.e. 415
@@ -17,7 +17,7 @@
 namespace m2 {
 
 // x = h + m + l.  The rest after an infinite h is 0, and a finite x whose rounded h is infinite is truncated instead: finite
-// inputs have finite parts, and the sum of the parts is the input in every case.
+// inputs have finite parts, and the sum of the parts is the input wherever bf16 reaches 24 bits below it (|x| >= 2^-110).
 __device__ __forceinline__ void split_parts(float x, float& h, float& m, float& l) {
   h = __uint_as_float(pack_bf16x2(x, 0.f) << 16);
   if (fabsf(h) == INFINITY) h = __uint_as_float(__float_as_uint(x) & 0xffff0000u);

@@ -16,14 +16,31 @@ def _model(cfg, gpu, seed, **kw):
     return model.to(gpu).eval()
 
 
-def _both(model, *args, **kw):
-    """(native result, Python-schedule result); the native one must really have run."""
+def _counted(call):
+    """(result, how often a plan ran for it)"""
+    from m2_amd import schedule
+    run, calls = schedule.StackPlan.run, []
+
+    def counting(self, *args, **kw):
+        calls.append(self)
+        return run(self, *args, **kw)
+
+    schedule.StackPlan.run = counting
+    try:
+        return call(), len(calls)
+    finally:
+        schedule.StackPlan.run = run
+
+
+def _both(model, *args, encoder_only=False, **kw):
+    """(native result, Python-schedule result); a plan must have run for the first and none for the second."""
+    call = model.encoder if encoder_only else model
     model.encoder.native_schedule = True
-    got = model(*args, **kw)
-    assert any(p.checker.unchanged() for p in model.encoder._native_plans.values())
+    got, runs = _counted(lambda: call(*args, **kw))
     model.encoder.native_schedule = False
-    want = model(*args, **kw)
+    want, none = _counted(lambda: call(*args, **kw))
     model.encoder.native_schedule = True
+    assert (runs, none) == (1, 0)
     return got, want
 
 
@@ -50,9 +67,7 @@ def test_native_schedule_matches_python_schedule(gpu, helper, l_max, B, L):
     (a, _), (b, _) = _both(model, ids, token_type_ids=tt, position_ids=pos)
     assert torch.equal(a, b) and not torch.equal(a, seq)
     h = torch.randn(B, L, cfg.hidden_size, generator=torch.Generator().manual_seed(7)).to(gpu)
-    outs = model.encoder(h)
-    model.encoder.native_schedule = False
-    want = model.encoder(h)
+    outs, want = _both(model, h, encoder_only=True)
     assert len(outs) == 3 and all(torch.equal(a, b) for a, b in zip(outs, want))
 
 
@@ -223,7 +238,8 @@ def test_plans_follow_plain_values(gpu):
     def changed(what):
         nonlocal prev
         model.encoder.native_schedule = True
-        got, _ = model(ids)
+        (got, _), runs = _counted(lambda: model(ids))
+        assert runs == (0 if what == "one layer's epsilon" else 1), what        # (layers that differ: the Python schedule)
         model.encoder.native_schedule = False
         want, _ = model(ids)
         assert torch.equal(got, want) and not torch.equal(got, prev), what
@@ -329,7 +345,8 @@ def test_computed_weights_and_other_classes_take_the_python_schedule(gpu):
                 model.encoder._native_plans.clear()
             torch.manual_seed(1)
             change(model.encoder.layer[1])
-            got, _ = model(ids)
+            (got, _), runs = _counted(lambda: model(ids))
+            assert runs == 0, what
             model.encoder.native_schedule = False
             want, _ = model(ids)
             assert torch.equal(got, want), what

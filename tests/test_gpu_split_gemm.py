@@ -96,7 +96,7 @@ def test_split_infinities_and_nan(gpu):
 
 
 def test_fp32_modules_follow_their_weights(gpu):
-    """Parts are split again when a weight changes; hooks and unaligned or non-contiguous inputs take their way."""
+    """A changed weight is the one used; hooks and unaligned or non-contiguous inputs take their way."""
     import copy
 
     import m2_amd
