@@ -544,7 +544,7 @@ class BertEncoder(nn.Module):
             if dst is not None:
                 dst.copy_(src)
         for held in reads:
-            held.use_on(torch.cuda.current_stream())
+            held.use_on(ops._stream())
         graph.replay()
         return [o.clone() for o in static_out]
 
@@ -684,7 +684,7 @@ class BertModel(nn.Module):
                 if dst is not None:
                     dst.copy_(src)
             for held in reads:
-                held.use_on(torch.cuda.current_stream())
+                held.use_on(ops._stream())
             graph.replay()
             outs = [o.clone() for o in static_out]
         enc = [o.view(B, L, -1) for o in outs]

@@ -18,8 +18,14 @@ from ._lib import HyenaFilterParams, SplitJob, M2_DTYPE_BF16, M2_DTYPE_F32, chec
 Tensor = torch.Tensor
 
 
+# handle of the current stream of a device: 0.3 us, where torch.cuda.current_stream() makes an object in 3 us
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def _stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
+    if _raw_stream is None or not torch.cuda.is_initialized():
+        return torch.cuda.current_stream().cuda_stream
+    return _raw_stream(torch._C._cuda_getDevice())
 
 
 def _require(t: Tensor, name: str, dtype=None, shape=None) -> None:
@@ -114,17 +120,19 @@ class StreamUse:
 
     def __init__(self, tensors: Sequence[Tensor], ready: Optional["torch.cuda.Event"] = None):
         self.tensors, self.ready = list(tensors), ready
-        self.streams = {torch.cuda.current_stream().cuda_stream}
+        self.streams = {_stream()}
 
-    def use_on(self, stream: "torch.cuda.Stream") -> None:
-        if stream.cuda_stream in self.streams:
+    def use_on(self, handle: int) -> None:
+        """`handle`: of the current stream."""
+        if handle in self.streams:
             return
+        stream = torch.cuda.current_stream()
         for t in self.tensors:
             t.record_stream(stream)
         if not torch.cuda.is_current_stream_capturing():     # (a capture cannot wait for what lies outside; its replays come later)
             if self.ready is not None:
                 stream.wait_event(self.ready)
-            self.streams.add(stream.cuda_stream)
+            self.streams.add(handle)
 
 
 class FilterTable:
@@ -179,8 +187,8 @@ class FilterTable:
         self.skip = torch.tensor(skip_row, dtype=torch.int64).to(dev)
         self._use = StreamUse((self.table, self.skip))
 
-    def use_on(self, stream: "torch.cuda.Stream") -> None:
-        self._use.use_on(stream)
+    def use_on(self, handle: int) -> None:
+        self._use.use_on(handle)
 
     @classmethod
     def of_rows(cls, rows: Sequence[Sequence[Optional[Tensor]]], skips: Sequence[Tensor], fpm: int, L: int, d: int, order: int,
@@ -217,7 +225,8 @@ def mixer_filter_spectra(table: FilterTable, w_mod: float = 1.0, shift: float = 
     if first < 0 or count < 1 or first + count > table.nmixers:
         raise ValueError(f"mixers [{first}, {first + count}) outside the table of {table.nmixers}")
     dev = table.table.device
-    table.use_on(torch.cuda.current_stream())
+    stream = _stream()
+    table.use_on(stream)
     n = table.spectrum_floats()
     if out is None:
         out = torch.empty(count, n, dtype=torch.float32, device=dev)
@@ -228,7 +237,7 @@ def mixer_filter_spectra(table: FilterTable, w_mod: float = 1.0, shift: float = 
     check(lib.m2_mixer_filters_fwd(ctypes.c_void_p(table.table.data_ptr() + first * table.fpm * 18 * 8),
                                    ctypes.c_void_p(table.skip.data_ptr() + first * table.fpm * 8), count, table.fpm,
                                    table.L, table.d, table.order, table.emb_dim, float(w_mod), float(shift),
-                                   _ptr(workspace), _ptr(out), _stream()))
+                                   _ptr(workspace), _ptr(out), stream))
     return out
 
 
@@ -285,7 +294,11 @@ def fftconv(x: Tensor, spec: Tensor, B: int, L: int, d: int) -> Tensor:
 #                  4096 91 / 72.  Below that torch's call costs 19 us whatever the size (its host side), own 8 .. 20.
 #   from_channels  d = 768: 4096 13 / 20, 16384 25 / 27, 32768 45 / 49; d = 960: 8192 23 / 29, 16384 36 / 48, 32768 69 / 74;
 #                  d = 1536: 2048 22 / 20, 4096 30 / 27, 8192 41 / 41, 16384 84 / 77; d = 1792: 4096 35 / 32, 8192 58 / 51.
-# So the own kernels serve products of up to about 29 GFLOP (to_channels), and every one of d <= 1024 (from_channels).
+# So the own kernels serve products of up to about 29 GFLOP (to_channels), and every one of d <= 1024 (from_channels).  At d >= 960 a
+# single product near that line is up to 20 % faster in the library; own ones serve it all the same, because a forward that uses them
+# for both projections is enqueued natively, and with them the streaming GLU and wo of few rows.  Whole forwards as captured graphs,
+# where the host costs nothing, all steps before / these (ms): 24 x 1536 M = 1024 3.98 / 2.70, 2048 4.37 / 3.74; 12 x 960 M = 2048
+# 1.57 / 1.13, 4096 1.97 / 1.79; 12 x 1792 M = 2048 3.14 / 2.22.
 _OWN_DENSE_FLOPS = 2.95e10
 
 

@@ -229,11 +229,11 @@ class StackPlan(NoPlan):
         ready.record()
         return ops.StreamUse(tensors, ready)
 
-    def use_on(self, stream: torch.cuda.Stream) -> None:
-        self.table.use_on(stream)
+    def use_on(self, handle: int) -> None:
+        self.table.use_on(handle)
         for route in self.routes:
             if route is not None:
-                route[1].use_on(stream)
+                route[1].use_on(handle)
 
     def route(self, M: int):
         """The one of `routes` that serves M rows, or None where it would have to be made during a stream capture."""
@@ -256,12 +256,12 @@ class StackPlan(NoPlan):
         n, L, d = self.layers, self.L, self.d
         M = B * L
         dev = ids.device if ids is not None else h16.device
-        current = torch.cuda.current_stream()
+        current = ops._stream()
         t = self.table
         t.use_on(current)
         self.routes[0][1].use_on(current)
         route[1].use_on(current)
-        stream = ctypes.c_void_p(current.cuda_stream)
+        stream = ctypes.c_void_p(current)
         up = lambda v: (v + 255) & ~255      # noqa: E731
         o_spec = up(self.filter_ws)
         o_act = o_spec + up(n * self.spec_bytes)
