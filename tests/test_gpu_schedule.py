@@ -374,8 +374,10 @@ def test_a_layer_class_with_the_plain_signature(gpu):
     want, _ = model(ids)
     for lay in model.encoder.layer:
         lay.__class__ = Plain
-    got, _ = model(ids)
-    assert torch.equal(got, want)
+    for native in (True, False):
+        model.encoder.native_schedule = native
+        got, _ = model(ids)
+        assert torch.equal(got, want)
 
 
 def test_a_bad_index_is_reported_before_a_failing_pooler(gpu):
