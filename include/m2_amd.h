@@ -117,9 +117,8 @@ int m2_mixer_filters_fwd(const m2_hyena_filter_params* params_dev, const float* 
  * native counterpart in the reference: flashmm.mm_block_fwd (csrc/flashmm/flash_mm.cpp:70-226).
  * ------------------------------------------------------------------------------------------- */
 
-/* 1 if sequence length L is supported: a power of two in [128, 32768] (one LDS-resident transform per
- * row up to 1024, two half-length transforms per row for 2048 .. 16384; at 32768 each of the two real signals
- * of a row is convolved on its own in polyphase form, again as two LDS-resident half transforms). */
+/* 1 if sequence length L is supported: a power of two in [128, 32768] (one LDS-resident transform of L points
+ * per real signal of a row, at 32768 two of L / 2 points). */
 int m2_fftconv_supported_seqlen(int L);
 
 /* Bytes of the opaque spectrum buffer for d channels and sequence length L (both filters): 16 d L, the size of
@@ -129,9 +128,8 @@ size_t m2_filter_spectrum_bytes(int d, int L);
 /* taps1, taps2: (d, 2L) fp32 bidirectional taps of filter_fn and filter_fn2 (taps2 may be NULL:
  * treated as zero).  D1, D2: (d) fp32 skip weights (`filter_fn.bias`, `filter_fn2.bias`; either
  * may be NULL = 0): the reference's "+ u * D" term (hyena_utils.py:35) equals adding D to tap 0,
- * which is done here.  spec: m2_filter_spectrum_bytes(d, L) bytes; receives
- * rfft(taps + D e0, 2L)/(2L) of both filters (at L = 32768: of their even and odd samples) in the order
- * m2_mixer_core_fwd reads them. */
+ * which is done here.  spec: m2_filter_spectrum_bytes(d, L) bytes; receives, of both filters, the transform
+ * of (first half + i second half of the taps) at the points z^L = -i over L, in the order m2_mixer_core_fwd reads it. */
 int m2_filter_spectrum_fwd(const float* taps1, const float* taps2, const float* D1, const float* D2, float* spec,
                            int d, int L, void* stream);
 

@@ -1,219 +1,107 @@
-// L = 32768: the fused mixer core and the filter-spectrum kernel with every real signal of a row transformed
-// on its own, as H = L complex points, through the half-transform machinery of fft_split.h.
+// L = 32768: the fused mixer core and the filter-spectrum kernel.  One transform of L points does not fit the 160 KB of LDS;
+// the ring of fft_twist.h splits once more,
 //
-// A row of the N = 2L point convolution does not fit the 160 KB of LDS as one complex transform, nor as the
-// two half transforms that serve L <= 16384.  Here the two real signals of the mixer (the gated short-conv
-// product a, and the layer input u) are not packed into one complex row; each is convolved separately in
-// polyphase form:
+//   z^L + i = (z^H - r)(z^H + r),  H = L / 2 = 16384,  r = exp(-i pi / 4)
 //
-//   c[m] = s[2m] + i s[2m+1]  (m < L/2; the zero padding makes the upper half of the H = L points zero)
-//   C = FFT_H(c) = Ce + i Co,   Ce = FFT_H(even samples) = (C[k] + conj C[H-k]) / 2,
-//                               Co = FFT_H(odd samples)  = (C[k] - conj C[H-k]) / 2i
-//   Ye = Ce Ke + w_H^k Co Ko,   Yo = Ce Ko + Co Ke        (Ke, Ko: the filter's even / odd taps, FFT_H)
-//   d = IFFT_H(Ye + i Yo):      y[2m] = Re d[m], y[2m+1] = Im d[m], m < L/2
+// and every real signal s = s0 + z^H s1 goes through two transforms of H points, of s0 + r s1 at shift 1/8 and of s0 - r s1 at
+// shift 5/8.  With P and Q the two products the result is y0 = Re(P + Q), y1 = Re((P - Q) / r) (the factor 1/2 is in the spectra).
 //
-// The H-point transform with a zero upper half is exactly what fft_split.h runs as two half transforms of
-// NS = H/2 = 16384 points (even and odd frequencies), and the pairing k <-> H - k is the mirror / complement
-// pairing of its last pass, so a thread holds both members of every pair.  Per pair the spectrum buffer
-// stores Ke and Ko (16 bytes) in the order the multiply consumes them; the root w_H^k is rebuilt in the multiply
-// from one per-thread constant per half transform and compile-time constants:
+//   spec[channel][signal][half][register pair 0 .. 15][T]  float4, as in fftconv_kernels.hip
 //
-//   spec[channel][filter 0..1][half 0..1] float4 (Ke, Ko)[slot 0..15][T]
+// One workgroup of 512 threads fills a compute unit.  A thread holds 32 samples of either half of the row in the layout of the first
+// pass (positions t + 512 j and H + t + 512 j), which u is read in directly, consecutive lanes consecutive floats.  The product of
+// the short convolutions, the gate and the results are staged through the transform's buffer (32768 floats are the 16384 complex
+// slots), 64 consecutive time steps per thread on the global side.
 //
-// The filter kernel gets Ke and Ko from ONE transform per filter: the (d, 2L) taps row read as H complex
-// numbers is k_even + i k_odd.
-//
-// A row is processed without staging through LDS: threads load and store global memory directly in the
-// layout of the first pass (complex slot m = t + T j holds time steps 2m, 2m+1), where consecutive lanes
-// touch consecutive 4- or 8-byte pieces.  Order per row: a -> y1 (two half transforms with filter 1),
-// acc = y1 * gate, then the two half transforms of u with filter 2 are added to acc one after the other
-// (u is loaded again for the second one instead of being kept in registers).
+// 268 us at B = 1, d = 768 in bf16 (318 in fp32), against 338 (405) with the polyphase form that this took over from, whose product
+// paired mirrored frequencies at nine times the multiplications: 124 us of vector instructions, 700 MB of memory traffic, and with one
+// workgroup per unit the two hardly overlap.  Requesting the next row's inputs or u ahead needs more registers than there are: with
+// 100 of them spilled the kernel took 305 us.
 //
 // Stands in for the same reference code as fftconv_kernels.hip (bert/src/mm/hyena_utils.py:16-42,
 // 231-236; bert/src/mm/monarch_mixer_sequence_mixer.py:112-147).
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
-#include "fft_engine.h"
-#include "fft_split.h"
+#include "fft_twist.h"
 #include "hyena_filter.h"
 #include "row_io.h"
 
 namespace m2 {
 
-// One pair of the polyphase multiply: za = C[k], zb = C[H - k]; returns D[k] in za and D[H - k] in zb.
-// K = (Ke, Ko) at frequency k, with the scale 1 / 4H folded in; the third factor w_H^k Ko is formed here: the root is
-// beta (this thread's group, one per half transform, the same for every row) times the constant w_64^S.
-template <int S>
-__device__ __forceinline__ void pair_multiply_real(cf& za, cf& zb, float4 K, cf beta) {
-  const cf A = {za.re + zb.re, za.im - zb.im};         // 2 Ce
-  const cf Bq = {za.im + zb.im, zb.re - za.re};        // 2 Co
-  const cf ke = {K.x, K.y}, ko = {K.z, K.w};
-  const cf kw = cmul(beta, mul_w64<S, false>(ko));
-  const cf Ye = cadd(cmul(A, ke), cmul(Bq, kw));
-  const cf Yo = cadd(cmul(A, ko), cmul(Bq, ke));
-  za = {Ye.re - Yo.im, Ye.im + Yo.re};                 // Ye + i Yo
-  zb = {Ye.re + Yo.im, Yo.re - Ye.im};                 // conj(Ye) + i conj(Yo)
-}
-// self-paired frequency (k = 0 or H/2): everything is real; kw = +ko at k = 0 and -ko at k = H/2
-__device__ __forceinline__ cf self_multiply_real(cf z, float ke, float ko, float kw) {
-  return {z.re * ke + z.im * kw, z.re * ko + z.im * ke};
-}
+typedef Twist16384 RealPlan;      // half transforms
+static_assert(twist_offsets_ok<RealPlan>(), "LDS offsets of the plan");
+constexpr float kRho = 0.70710678118654752440f;      // r = kRho (1 - i)
 
-// spectral multiply of the 16 + 16 points a thread holds after fwd_groups, slots 4 HB .. 4 HB + 3 (same
-// pairing as multiply_batch in fft_split.h)
-// beta: root of the thread's group (slot s of it adds w_16^s); in the special work item of the even half the slots
-// 1 .. 7 belong to group 0 (root 1) and the slots 8 .. 15 to group R2 / 2 (root beta_sp, slot s - 8 of it).
-template <bool EVEN_SPECIAL, int HB>
-__device__ __forceinline__ void multiply_batch_real(cf (&x)[32], const float4 (&K)[4], cf beta, cf beta_sp) {
-  static_for<0, 4>([&](auto ss) {
-    constexpr int s = 4 * HB + decltype(ss)::value;
-    const float4 k = K[decltype(ss)::value];
-    if constexpr (!EVEN_SPECIAL) {
-      pair_multiply_real<4 * s>(x[bitrev(s, 4)], x[16 + bitrev(15 - s, 4)], k, beta);
-    } else if constexpr (s == 0) {
-      // K = (Ke(0), Ko(0), Ke(H/2), Ko(H/2))
-      x[bitrev(0, 4)] = self_multiply_real(x[bitrev(0, 4)], k.x, k.y, k.y);
-      x[bitrev(8, 4)] = self_multiply_real(x[bitrev(8, 4)], k.z, k.w, -k.w);
-    } else if constexpr (s < 8) {
-      pair_multiply_real<4 * s>(x[bitrev(s, 4)], x[bitrev(16 - s, 4)], k, cf{1.f, 0.f});
-    } else {
-      pair_multiply_real<4 * (s - 8)>(x[16 + bitrev(s - 8, 4)], x[16 + bitrev(23 - s, 4)], k, beta_sp);
-    }
+// floats of the spectrum buffer per (channel, signal, half)
+template <class P>
+constexpr long real_spec_block() { return 2L * P::H; }
+
+// Staging of 2 H floats through the transform's buffer: thread t owns the time steps 64 t .. 64 t + 63.  The rows of 64 floats are
+// padded by 4 so that the 16-byte accesses of consecutive threads spread over the banks.
+constexpr int stage_phys(int n) { return n + 4 * (n >> 6); }
+
+// Causal 3-tap convolution of 8 time steps in registers, w folded as in fftconv_kernels.hip
+__device__ __forceinline__ void short_conv8(const float (&in)[10], const float (&w)[3], float f, float (&out)[8]) {
+  static_for<0, 8>([&](auto ee) {
+    constexpr int e = decltype(ee)::value;
+    out[e] = f + w[0] * in[e] + w[1] * in[e + 1] + w[2] * in[e + 2];
   });
 }
-template <int HB>
-__device__ __forceinline__ void load_spectrum_batch_real(float4 (&K)[4], const float4* __restrict__ sp4, int T) {
-  static_for<0, 4>([&](auto s) { K[decltype(s)::value] = sp4[(4 * HB + decltype(s)::value) * T]; });
-}
 
-// One half transform of one real signal: forward passes from registers (first-pass layout), polyphase multiply,
-// inverse passes back to registers.  Same barrier structure as half_convolution in fft_split.h; the spectrum
-// comes in four batches, each loaded while the one before it is multiplied.
-template <class P, bool ODD>
-__device__ __forceinline__ void half_convolution_real(cf (&x)[32], int t, float2* row, const float2* tab2,
-                                                      const cf (&b)[P::NB1], const float4* __restrict__ sp4, cf beta,
-                                                      cf beta_sp, int ga, int gb, bool special) {
-  fwd_pass1<P, ODD>(x, t, row, b);
-  phase_barrier();
-  fwd_pass2<P>(x, t, row, tab2);
-  phase_barrier();
-  float4 Ka[4], Kb[4];
-  load_spectrum_batch_real<0>(Ka, sp4, P::T);
-  fwd_groups<P>(x, row, ga, gb);
-  __builtin_amdgcn_sched_barrier(0);
-  auto multiply = [&](auto sp) __attribute__((always_inline)) {
-    constexpr bool S = decltype(sp)::value == 1;
-    load_spectrum_batch_real<1>(Kb, sp4, P::T);
-    multiply_batch_real<S, 0>(x, Ka, beta, beta_sp);
-    load_spectrum_batch_real<2>(Ka, sp4, P::T);
-    multiply_batch_real<S, 1>(x, Kb, beta, beta_sp);
-    load_spectrum_batch_real<3>(Kb, sp4, P::T);
-    multiply_batch_real<S, 2>(x, Ka, beta, beta_sp);
-    multiply_batch_real<S, 3>(x, Kb, beta, beta_sp);
-  };
-  if (!ODD && special) multiply(ic<1>{});
-  else multiply(ic<0>{});
-  __builtin_amdgcn_sched_barrier(0);
-  inv_groups<P>(x, row, ga, gb);
-  phase_barrier();
-  inv_pass2<P>(x, t, row, tab2);
-  phase_barrier();
-  inv_pass1<P, ODD>(x, t, row, b);
-}
-
-// floats of the spectrum buffer per (channel, filter, half): 16 slots x T work items x float4
+// the factors at shift 5/8 from those at 1/8
 template <class P>
-constexpr long real_spec_block() { return 16L * P::T * 4; }
-
-// ------------------------------------------------------------------------------------------
-// global memory in first-pass layout: complex slot m <-> time steps 2m, 2m + 1
-// ------------------------------------------------------------------------------------------
-// raw bits of time steps (2m, 2m+1); m = -1 reads slot 0 instead (the caller discards it)
-__device__ __forceinline__ uint32_t fetch_pair(const uint16_t* p, int m) {
-  return reinterpret_cast<const uint32_t*>(p)[m < 0 ? 0 : m];
-}
-__device__ __forceinline__ f32x2_t fetch_pair(const float* p, int m) {
-  return reinterpret_cast<const f32x2_t*>(p)[m < 0 ? 0 : m];
-}
-__device__ __forceinline__ float2 expand_pair(uint32_t r) {
-  return make_float2(__uint_as_float(r << 16), __uint_as_float(r & 0xffff0000u));
-}
-__device__ __forceinline__ float2 expand_pair(f32x2_t r) { return make_float2(r.x, r.y); }
-__device__ __forceinline__ void store_pair(uint16_t* p, int m, float a, float b) {
-  reinterpret_cast<uint32_t*>(p)[m] = pack_bf16x2(a, b);
-}
-__device__ __forceinline__ void store_pair(float* p, int m, float a, float b) {
-  reinterpret_cast<float2*>(p)[m] = make_float2(a, b);
-}
-template <typename ACT> struct PairBits;
-template <> struct PairBits<uint16_t> { typedef uint32_t type; };
-template <> struct PairBits<float> { typedef f32x2_t type; };
-
-// slot of register x[i R1 + j] of thread t in the first-pass layout
-template <class P>
-__device__ __forceinline__ int slot_of(int t, int i, int j) { return t + P::T * i + P::S1 * j; }
-
-// Causal 3-tap convolution of one (3d, B, L) channel at the time steps of this thread's 32 slots:
-// out[r] = (sc(2m), sc(2m+1)) with sc(n) = bias + w0 in[n-2] + w1 in[n-1] + w2 in[n], in = stored value + add
-// (time steps before 0 are the convolution's zero padding).  All 64 loads of a bf16 row are put in flight at once
-// (64 registers); an fp32 row goes in two batches.
-template <class P, typename ACT>
-__device__ __forceinline__ void short_conv_slots(const ACT* __restrict__ p, int t, const float (&w)[3], float bias,
-                                                 float add, cf (&out)[32]) {
-  typedef typename PairBits<ACT>::type bits;
-  constexpr int NB = sizeof(ACT) == 2 ? 32 : 16;      // slots per batch
-  const float fbias = bias + add * (w[0] + w[1] + w[2]);
-  static_for<0, 32 / NB>([&](auto hh) {
-    constexpr int h0 = decltype(hh)::value * NB;
-    bits prev[NB], cur[NB];
-    static_for<0, NB>([&](auto rr) {
-      constexpr int r = h0 + decltype(rr)::value;
-      const int m = slot_of<P>(t, r / P::R1, r % P::R1);
-      cur[r - h0] = fetch_pair(p, m);
-      prev[r - h0] = fetch_pair(p, m - 1);
-    });
-    __builtin_amdgcn_sched_barrier(0);
-    static_for<0, NB>([&](auto rr) {
-      constexpr int r = h0 + decltype(rr)::value;
-      const int m = slot_of<P>(t, r / P::R1, r % P::R1);
-      const float2 c = expand_pair(cur[r - h0]);
-      float2 q = expand_pair(prev[r - h0]);
-      if constexpr (r == 0) {      // only slot m = t of register 0 can be slot 0
-        q.x = m > 0 ? q.x : 0.f;
-        q.y = m > 0 ? q.y : 0.f;
-      }
-      // `add` (the in-projection's bias) is folded into the convolution's bias: conv(x + add) = conv(x) + add (w0 + w1 +
-      // w2), except at time steps 0 and 1, where taps fall on the zero padding outside the biased signal
-      out[r] = {fbias + w[0] * q.x + w[1] * q.y + w[2] * c.x, fbias + w[0] * q.y + w[1] * c.x + w[2] * c.y};
-      if constexpr (r == 0) {
-        if (m == 0) {
-          out[r].re -= add * (w[0] + w[1]);
-          out[r].im -= add * w[0];
-        }
-      }
-    });
+__device__ __forceinline__ TwistForward<P, 5> shifted(const TwistForward<P, 1>& a) {
+  TwistForward<P, 5> b;
+  static_for<0, P::NG>([&](auto ii) {
+    constexpr int i = decltype(ii)::value;
+    b.last[i].fine = mul_root<4, 8 * P::H>(a.last[i].fine);
+    b.last[i].mid = mul_root<4, 2 * P::H>(a.last[i].mid);
   });
+  return b;
 }
-// the signal itself (no short convolution) at this thread's slots
-template <class P, typename ACT>
-__device__ __forceinline__ void load_slots(const ACT* __restrict__ p, int t, cf (&out)[32]) {
-  typedef typename PairBits<ACT>::type bits;
-  bits cur[32];
+
+// acc += the convolution of (lo, hi) held in first-pass layout; sp: the signal's two blocks.  `again` provides lo and hi for the
+// second half (registers or memory).
+template <class P, class A>
+__device__ __forceinline__ void convolve_halves(float (&lo)[32], float (&hi)[32], A&& again, cf (&acc)[32], int t, float2* row, const float2* tab1,
+                                                const float2* tab5, const TwistForward<P, 1>& tf1,
+                                                const TwistInverse<P>& ti, const TwistEnd<P, 1>& te1, const TwistEnd<P, 5>& te5,
+                                                const float4* __restrict__ sp) {
+  cf x[32];
   static_for<0, 32>([&](auto rr) {
     constexpr int r = decltype(rr)::value;
-    cur[r] = fetch_pair(p, slot_of<P>(t, r / P::R1, r % P::R1));
+    const float v = kRho * hi[r];
+    x[r] = {lo[r] + v, -v};
+  });
+  convolve<P, 1, false>(x, t, row, tab1, tf1, ti, sp);
+  // acc.re: first half of the row, acc.im: second.  P without its shift is f v; P / r = f v exp(i pi / 4)
+  static_for<0, 32>([&](auto rr) {
+    constexpr int r = decltype(rr)::value, i = r / P::R1, j = r % P::R1;
+    const cf v = mul_root<j, 8 * P::R1, true>(x[r]);
+    const float re = te1.f[i].re * v.re - te1.f[i].im * v.im, im = te1.f[i].re * v.im + te1.f[i].im * v.re;
+    acc[r].re += re;
+    acc[r].im = fmaf(kRho, re - im, acc[r].im);
   });
   __builtin_amdgcn_sched_barrier(0);
+  again(lo, hi);
   static_for<0, 32>([&](auto rr) {
     constexpr int r = decltype(rr)::value;
-    const float2 c = expand_pair(cur[r]);
-    out[r] = {c.x, c.y};
+    const float v = kRho * hi[r];
+    x[r] = {lo[r] - v, v};
+  });
+  convolve<P, 5, false>(x, t, row, tab5, shifted(tf1), ti, sp + real_spec_block<P>() / 4);
+  static_for<0, 32>([&](auto rr) {
+    constexpr int r = decltype(rr)::value, i = r / P::R1, j = r % P::R1;
+    const cf v = mul_root<5 * j, 8 * P::R1, true>(x[r]);
+    const float re = te5.f[i].re * v.re - te5.f[i].im * v.im, im = te5.f[i].re * v.im + te5.f[i].im * v.re;
+    acc[r].re += re;
+    acc[r].im = fmaf(-kRho, re - im, acc[r].im);
   });
 }
 
 // ------------------------------------------------------------------------------------------
-// the fused mixer core, sequence length 2 P::L
+// the fused mixer core, sequence length 2 P::H
 // ------------------------------------------------------------------------------------------
 // FULL: short convolutions and gates (sw, sb non-null); otherwise a plain long convolution of one input.
 // HAS_U: the residual long convolution of the layer input u (uin non-null).
@@ -227,249 +115,262 @@ __global__ __launch_bounds__(P::T) __attribute__((amdgpu_waves_per_eu(2, 2))) vo
     const float* __restrict__ spec,     // (d, 2, 2) blocks of real_spec_block<P>() floats
     ACT* __restrict__ y,                // (d, B, LS)
     int B, int d) {
-  constexpr int T = P::T;
-  constexpr long LS = 2L * P::L;
-  constexpr long BLK = real_spec_block<P>();
+  constexpr int T = P::T, H = P::H;
+  constexpr long LS = 2L * H, BLK = real_spec_block<P>();
+  static_assert(T == 512 && P::E == 32 && P::NB1 == 1 && stage_phys(2 * H) <= 2 * P::ROW, "512 threads, 64 time steps each");
   extern __shared__ float2 lds[];
   float2* row = lds;
-  float2* tab2 = lds + P::ROW_LDS;
-  const int t = threadIdx.x;
+  float* stage = reinterpret_cast<float*>(lds);
+  const float2 *tab1 = lds + P::ROW, *tab5 = tab1 + P::TAB;
+  const int t = threadIdx.x, n0 = 64 * t;
 
-  tab2_init<P>(tab2);
-  cf b[P::NB1];
-  static_for<0, P::NB1>([&](auto ii) { b[decltype(ii)::value] = unit_root(t + T * decltype(ii)::value, P::N); });
-  const SplitGroups<P> grp = split_groups<P>(t);
-  // roots of the polyphase multiply: frequency k = k0 + R1 R2 s for slot s of group g, k0 = g / R2 + R1 (g % R2), and
-  // the pair at k of the half transform sits at 2 k + ODD of the H-point transform
-  const cf beta_e = unit_root(2 * (grp.ge / P::R2 + P::R1 * (grp.ge % P::R2)), P::N);
-  const cf beta_o = unit_root(2 * (grp.go / P::R2 + P::R1 * (grp.go % P::R2)) + 1, P::N);
-  const cf beta_sp = unit_root(2 * (P::R1 * (P::R2 / 2)), P::N);
-  phase_barrier();
+  tables_init<P, 1>(lds + P::ROW);
+  tables_init<P, 5>(lds + P::ROW + P::TAB);
+  TwistForward<P, 1> tf1;
+  TwistInverse<P> ti;
+  TwistEnd<P, 1> te1;
+  TwistEnd<P, 5> te5;
+  tf1.init(t);
+  ti.init(t);
+  te1.init(t);
+  te5.init(t);
+  sync_threads<T>();
 
-  // workgroup -> (channel, batch row) as in mixer_split_kernel: XCD e takes the channels c = e (mod 8)
+  // workgroup -> (channel, batch row) as in mixer_pair_kernel: XCD e takes the channels c = e (mod 8)
   const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3, slots = gridDim.x >> 3;
   const int rows_per_xcd = (d >> 3) * B;
   for (int j = slot; j < rows_per_xcd; j += slots) {
     // the same for every lane: say so, so that row base addresses live in scalar registers
     const int c = __builtin_amdgcn_readfirstlane((j / B) * 8 + xcd), bb = __builtin_amdgcn_readfirstlane(j % B);
-    const float* spc = spec + (long)c * 4 * BLK;
-    cf x[32], acc[32];
+    const float4* sp = reinterpret_cast<const float4*>(spec + (long)c * 4 * BLK);
+    float lo[32], hi[32];
+    cf acc[32];
+    static_for<0, 32>([&](auto rr) { acc[decltype(rr)::value] = {0.f, 0.f}; });
 
     // ---- first signal: a = sc(x1) sc(v)  (or the plain input), convolved with filter 1
-    if constexpr (FULL) {
-      float w1[3], wv[3];
+    {
+      RawRow<ACT, 8, true> r1, rv;
+      const ACT* px = FULL ? xproj + ((long)(0 * d + c) * B + bb) * LS : xproj + ((long)c * B + bb) * LS;
+      const ACT* pv = xproj + ((long)(2 * d + c) * B + bb) * LS;
+      static_for<0, 8>([&](auto qq) {
+        constexpr int q = decltype(qq)::value;
+        r1.template fetch<q>(px, n0 + 8 * q);
+        if constexpr (FULL) rv.template fetch<q>(pv, n0 + 8 * q);
+      });
+      float w1[3], wv[3], p1 = 0.f, pbv = 0.f, f1 = 0.f, fv = 0.f;
+      if constexpr (FULL) {
 #pragma unroll
-      for (int k = 0; k < 3; ++k) {
-        w1[k] = sw[(long)c * 3 + k];
-        wv[k] = sw[((long)2 * d + c) * 3 + k];
+        for (int k = 0; k < 3; ++k) {
+          w1[k] = sw[(long)c * 3 + k];
+          wv[k] = sw[((long)2 * d + c) * 3 + k];
+        }
+        if (pbias) { p1 = pbias[c]; pbv = pbias[2 * d + c]; }
+        f1 = sb[c] + p1 * (w1[0] + w1[1] + w1[2]);
+        fv = sb[2 * d + c] + pbv * (wv[0] + wv[1] + wv[2]);
       }
-      const float p1 = pbias ? pbias[c] : 0.f, pv = pbias ? pbias[2 * d + c] : 0.f;
-      short_conv_slots<P, ACT>(xproj + ((long)(0 * d + c) * B + bb) * LS, t, w1, sb[c], p1, x);
-      short_conv_slots<P, ACT>(xproj + ((long)(2 * d + c) * B + bb) * LS, t, wv, sb[2 * d + c], pv, acc);
+      __builtin_amdgcn_sched_barrier(0);
+      static_for<0, 8>([&](auto qq) {
+        constexpr int q = decltype(qq)::value;
+        const int n = n0 + 8 * q;
+        float in[10], a[8], v[8];
+        r1.template expand<q>(n, in);
+        if constexpr (FULL) {
+          short_conv8(in, w1, f1, a);
+          rv.template expand<q>(n, in);
+          short_conv8(in, wv, fv, v);
+          if constexpr (q == 0) {
+            if (t == 0) {      // time steps 0 and 1: taps that fall on the zero padding, outside the biased signal
+              a[0] -= p1 * (w1[0] + w1[1]); a[1] -= p1 * w1[0];
+              v[0] -= pbv * (wv[0] + wv[1]); v[1] -= pbv * wv[0];
+            }
+          }
+          static_for<0, 8>([&](auto ee) { a[decltype(ee)::value] *= v[decltype(ee)::value]; });
+        } else {
+          static_for<0, 8>([&](auto ee) { a[decltype(ee)::value] = in[decltype(ee)::value + 2]; });
+        }
+        float4* dst = reinterpret_cast<float4*>(stage + stage_phys(n0) + 8 * q);
+        dst[0] = make_float4(a[0], a[1], a[2], a[3]);
+        dst[1] = make_float4(a[4], a[5], a[6], a[7]);
+        __builtin_amdgcn_sched_barrier(0);
+      });
+    }
+    sync_threads<T>();
+    auto from_stage = [&](auto&& put) __attribute__((always_inline)) {
+      const float* pl = stage + stage_phys(t);
       static_for<0, 32>([&](auto rr) {
         constexpr int r = decltype(rr)::value;
-        x[r] = {x[r].re * acc[r].re, x[r].im * acc[r].im};
+        put(rr, pl[stage_phys(512 * r)], pl[stage_phys(H + 512 * r)]);
       });
-    } else {
-      load_slots<P, ACT>(xproj + ((long)c * B + bb) * LS, t, x);
-    }
-    static_for<0, 32>([&](auto rr) { acc[decltype(rr)::value] = x[decltype(rr)::value]; });     // a, for the odd half
-    {
-      const float4* sp4 = reinterpret_cast<const float4*>(spc) + t;
-      half_convolution_real<P, false>(x, t, row, tab2, b, sp4, beta_e, beta_sp, grp.ge, grp.gm, grp.special);
-    }
-    static_for<0, 32>([&](auto rr) {       // x <- a for the odd half, acc <- the even half's result
-      constexpr int r = decltype(rr)::value;
-      const cf e = x[r];
-      x[r] = acc[r];
-      acc[r] = e;
+    };
+    from_stage([&](auto rr, float l, float h) __attribute__((always_inline)) {
+      lo[decltype(rr)::value] = l;
+      hi[decltype(rr)::value] = h;
     });
-    {
-      const float4* sp4 = reinterpret_cast<const float4*>(spc + BLK) + t;
-      half_convolution_real<P, true>(x, t, row, tab2, b, sp4, beta_o, beta_sp, grp.go, grp.gc, false);
-    }
-    static_for<0, 32>([&](auto rr) {
-      constexpr int r = decltype(rr)::value;
-      acc[r] = cadd(acc[r], x[r]);
-    });
+    sync_threads<T>();                     // the transform's slots overlap the staged row
+    convolve_halves<P>(lo, hi, [](float (&)[32], float (&)[32]) {}, acc, t, row, tab1, tab5, tf1, ti, te1, te5, sp);
 
-    // ---- gate: acc = y1 * sc(x2)
-    __builtin_amdgcn_sched_barrier(0);
+    // u, read twice rather than kept across the first half transform
+    const float* pu = HAS_U ? uin + ((long)c * B + bb) * LS : nullptr;
+    auto load_u = [&](float (&l)[32], float (&h)[32]) __attribute__((always_inline)) {
+      int again = 0;
+      asm volatile("" : "+s"(again));      // a second load, not the first one's registers kept across the half transform
+      const float* p = pu + again;
+      static_for<0, 32>([&](auto rr) {
+        constexpr int r = decltype(rr)::value;
+        l[r] = (p + 512 * r)[(unsigned)t];
+        h[r] = (p + H + 512 * r)[(unsigned)t];
+      });
+    };
+
+    // ---- gate: acc = y1 * sc(x2), by way of the stage
     if constexpr (FULL) {
-      float w2[3];
+      RawRow<ACT, 8, true> r2;
+      const ACT* p2 = xproj + ((long)(1 * d + c) * B + bb) * LS;
+      static_for<0, 8>([&](auto qq) { r2.template fetch<decltype(qq)::value>(p2, n0 + 8 * decltype(qq)::value); });
+      float w2[3], pb2 = 0.f;
 #pragma unroll
       for (int k = 0; k < 3; ++k) w2[k] = sw[((long)d + c) * 3 + k];
-      const float p2 = pbias ? pbias[d + c] : 0.f;
-      short_conv_slots<P, ACT>(xproj + ((long)(1 * d + c) * B + bb) * LS, t, w2, sb[d + c], p2, x);
+      if (pbias) pb2 = pbias[d + c];
+      const float f2 = sb[d + c] + pb2 * (w2[0] + w2[1] + w2[2]);
+      sync_threads<T>();                   // everybody has read the last pass's slots
+      float* ps = stage + stage_phys(t);
       static_for<0, 32>([&](auto rr) {
         constexpr int r = decltype(rr)::value;
-        acc[r] = {acc[r].re * x[r].re, acc[r].im * x[r].im};
+        ps[stage_phys(512 * r)] = acc[r].re;
+        ps[stage_phys(H + 512 * r)] = acc[r].im;
       });
+      sync_threads<T>();
+      static_for<0, 8>([&](auto qq) {
+        constexpr int q = decltype(qq)::value;
+        float in[10], g[8];
+        r2.template expand<q>(n0 + 8 * q, in);
+        short_conv8(in, w2, f2, g);
+        if constexpr (q == 0) {
+          if (t == 0) { g[0] -= pb2 * (w2[0] + w2[1]); g[1] -= pb2 * w2[0]; }
+        }
+        float4* at = reinterpret_cast<float4*>(stage + stage_phys(n0) + 8 * q);
+        const float4 v0 = at[0], v1 = at[1];
+        const float o[8] = {v0.x * g[0], v0.y * g[1], v0.z * g[2], v0.w * g[3], v1.x * g[4], v1.y * g[5], v1.z * g[6], v1.w * g[7]};
+        if constexpr (HAS_U) {
+          at[0] = make_float4(o[0], o[1], o[2], o[3]);
+          at[1] = make_float4(o[4], o[5], o[6], o[7]);
+        } else {
+          store8(y + ((long)c * B + bb) * LS, n0 + 8 * q, o);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      });
+      sync_threads<T>();
+      if constexpr (HAS_U) {
+        from_stage([&](auto rr, float l, float h) __attribute__((always_inline)) { acc[decltype(rr)::value] = {l, h}; });
+        sync_threads<T>();
+      }
     }
 
-    // ---- second signal: the layer input u, convolved with filter 2; its two half transforms are added to acc
-    __builtin_amdgcn_sched_barrier(0);
+    // ---- second signal: the layer input u, convolved with filter 2 on top of it
     if constexpr (HAS_U) {
-      const float* pu = uin + ((long)c * B + bb) * LS;
-      load_slots<P, float>(pu, t, x);
-      {
-        const float4* sp4 = reinterpret_cast<const float4*>(spc + 2 * BLK) + t;
-        half_convolution_real<P, false>(x, t, row, tab2, b, sp4, beta_e, beta_sp, grp.ge, grp.gm, grp.special);
-      }
-      static_for<0, 32>([&](auto rr) {
-        constexpr int r = decltype(rr)::value;
-        acc[r] = cadd(acc[r], x[r]);
-      });
-      __builtin_amdgcn_sched_barrier(0);
-      int again = 0;
-      asm volatile("" : "+v"(again));    // a second load, not the first one's registers kept across the half transform
-      load_slots<P, float>(pu + again, t, x);
-      {
-        const float4* sp4 = reinterpret_cast<const float4*>(spc + 3 * BLK) + t;
-        half_convolution_real<P, true>(x, t, row, tab2, b, sp4, beta_o, beta_sp, grp.go, grp.gc, false);
-      }
-      static_for<0, 32>([&](auto rr) {
-        constexpr int r = decltype(rr)::value;
-        acc[r] = cadd(acc[r], x[r]);
-      });
+      load_u(lo, hi);
+      convolve_halves<P>(lo, hi, load_u, acc, t, row, tab1, tab5, tf1, ti, te1, te5, sp + BLK / 2);
     }
-
-    ACT* py = y + ((long)c * B + bb) * LS;
-    static_for<0, 32>([&](auto rr) {
-      constexpr int r = decltype(rr)::value;
-      store_pair(py, slot_of<P>(t, r / P::R1, r % P::R1), acc[r].re, acc[r].im);
-    });
-    // every half transform starts and ends in LDS slots this thread owns: no barrier between rows
+    if constexpr (HAS_U || !FULL) {        // results to 64 consecutive time steps per thread
+      sync_threads<T>();
+      float* ps = stage + stage_phys(t);
+      static_for<0, 32>([&](auto rr) {
+        constexpr int r = decltype(rr)::value;
+        ps[stage_phys(512 * r)] = acc[r].re;
+        ps[stage_phys(H + 512 * r)] = acc[r].im;
+      });
+      sync_threads<T>();
+      static_for<0, 8>([&](auto qq) {
+        constexpr int q = decltype(qq)::value;
+        const float4* at = reinterpret_cast<const float4*>(stage + stage_phys(n0) + 8 * q);
+        const float4 v0 = at[0], v1 = at[1];
+        const float o[8] = {v0.x, v0.y, v0.z, v0.w, v1.x, v1.y, v1.z, v1.w};
+        store8(y + ((long)c * B + bb) * LS, n0 + 8 * q, o);
+      });
+      sync_threads<T>();                   // the next row's prologue overwrites what has just been read
+    }
   }
 }
 
 // ------------------------------------------------------------------------------------------
-// filter taps -> (Ke, Ko) in the layout above; work item = (channel, filter), both half transforms
+// filter taps -> spectra; work item = (channel, filter), both half transforms
 // ------------------------------------------------------------------------------------------
 template <class P>
-__global__ __launch_bounds__(P::T) void filter_spectrum_real_kernel(
+__global__ __launch_bounds__(P::T) __attribute__((amdgpu_waves_per_eu(2, 2))) void filter_spectrum_real_kernel(
     const float* taps1,    // (d, 2 LS) bidirectional taps of filter_fn
     const float* taps2,    // (d, 2 LS) bidirectional taps of filter_fn2 (null: its blocks are zeroed)
     const float* D1,       // (d) skip weight of filter_fn, added to tap 0 (may be null)
     const float* D2,       // (d) skip weight of filter_fn2 (may be null)
     float* __restrict__ spec, int d, SpectrumBatch sb) {
-  constexpr int NS = P::L, H = P::N, T = P::T, R1 = P::R1, R2 = P::R2;
+  constexpr int H = P::H, T = P::T;
+  constexpr long LS = 2L * H, BLK = real_spec_block<P>();
   {
     float* sp = spec;
-    select_mixer(sb, d, 2 * H, taps1, taps2, D1, D2, sp);
+    select_mixer(sb, d, 2 * LS, taps1, taps2, D1, D2, sp);
     spec = sp;
   }
-  constexpr long BLK = real_spec_block<P>();
   extern __shared__ float2 lds[];
   float2* row = lds;
-  float2* tab2 = lds + P::ROW_LDS;
+  const float2 *tab1 = lds + P::ROW, *tab5 = tab1 + P::TAB;
   const int t = threadIdx.x;
 
-  tab2_init<P>(tab2);
-  cf b[P::NB1];
-  static_for<0, P::NB1>([&](auto ii) { b[decltype(ii)::value] = unit_root(t + T * decltype(ii)::value, P::N); });
-  const SplitGroups<P> grp = split_groups<P>(t);
-  // 1/H of the inverse, 1/2 of Ke / Ko from the packed transform, 1/2 of Ce / Co in the mixer kernel
-  const float scale = 0.25f / (float)H;
-  __syncthreads();
+  tables_init<P, 1>(lds + P::ROW);
+  tables_init<P, 5>(lds + P::ROW + P::TAB);
+  TwistForward<P, 1> tf1;
+  TwistForward<P, 5> tf5;
+  tf1.init(t);
+  tf5.init(t);
+  sync_threads<T>();
+  const float scale = 1.f / (float)LS;      // 1/H of the inverse, 1/2 of the two halves
 
-  // work item = (channel, filter): the taps row is read once; its even-half combination goes to LDS at once, the
-  // odd-half combination waits in registers (64) while the even half is transformed
+  // the taps row is read once: both halves' inputs are formed, the second waits in registers
   for (int item = blockIdx.x; item < 2 * d; item += gridDim.x) {
-    const int c = item >> 1, f = item & 1;
-    const float* taps = f ? taps2 : taps1;
-    const float* D = f ? D2 : D1;
-    float* blk = spec + (long)item * 2 * BLK;
+    const int c = item >> 1;
+    const float* taps = item & 1 ? taps2 : taps1;
+    const float* D = item & 1 ? D2 : D1;
+    float4* blk = reinterpret_cast<float4*>(spec + (long)item * 2 * BLK) + t;
     if (!taps) {
       static_for<0, 2>([&](auto hh) {
-        float4* z4 = reinterpret_cast<float4*>(blk + decltype(hh)::value * BLK) + t;
-        static_for<0, 16>([&](auto ss) { z4[decltype(ss)::value * T] = make_float4(0.f, 0.f, 0.f, 0.f); });
+        static_for<0, 16>([&](auto ss) { blk[decltype(hh)::value * (BLK / 4) + decltype(ss)::value * T] = make_float4(0.f, 0.f, 0.f, 0.f); });
       });
       continue;
     }
-    // g[m] = taps[2m] + i taps[2m+1], m < H; even half: g_lo + g_hi, odd half: g_lo - g_hi
-    constexpr int Q = NS / 2 / T;
-    f32x4_t od[Q];
+    // k = lo + i hi over the two halves of the window, k = k0 + z^H k1: k0 +- r k1
+    cf x[32], q[32];
     {
-      f32x4_t lo[Q], hi[Q];
-      static_for<0, Q>([&](auto qq) {
-        constexpr int q = decltype(qq)::value;
-        const float* p = taps + (long)c * 2 * H + 4 * (q * T + t);
-        lo[q] = *reinterpret_cast<const f32x4_t*>(p);
-        hi[q] = *reinterpret_cast<const f32x4_t*>(p + 2 * NS);
+      const float* p = taps + (long)c * 2 * LS;
+      const float dd = (D && t == 0) ? D[c] : 0.f;      // the skip weight is one more tap at lag 0
+      static_for<0, 32>([&](auto rr) {
+        constexpr int r = decltype(rr)::value;
+        x[r] = {(p + 512 * r)[(unsigned)t], (p + LS + 512 * r)[(unsigned)t]};
+        q[r] = {(p + H + 512 * r)[(unsigned)t], (p + LS + H + 512 * r)[(unsigned)t]};
       });
-      if (D && t == 0) lo[0].x += D[c];      // the skip weight is one more tap at lag 0
-      static_for<0, Q>([&](auto qq) {
-        constexpr int q = decltype(qq)::value;
-        float2* dst = row + sphys(2 * (q * T + t));     // 2 consecutive slots never straddle a pad
-        dst[0] = make_float2(lo[q].x + hi[q].x, lo[q].y + hi[q].y);
-        dst[1] = make_float2(lo[q].z + hi[q].z, lo[q].w + hi[q].w);
-        od[q] = lo[q] - hi[q];
+      x[0].re += dd;
+      static_for<0, 32>([&](auto rr) {
+        constexpr int r = decltype(rr)::value;
+        const cf v = {kRho * (q[r].re + q[r].im), kRho * (q[r].im - q[r].re)};
+        q[r] = {x[r].re - v.re, x[r].im - v.im};
+        x[r] = {x[r].re + v.re, x[r].im + v.im};
       });
     }
-    auto one_half = [&](auto hh) __attribute__((always_inline)) {
-      constexpr bool ODD = decltype(hh)::value == 1;
-      float4* sp4 = reinterpret_cast<float4*>(blk + (ODD ? BLK : 0)) + t;
-      if constexpr (ODD) {
-        static_for<0, Q>([&](auto qq) {
-          constexpr int q = decltype(qq)::value;
-          float2* dst = row + sphys(2 * (q * T + t));
-          dst[0] = make_float2(od[q].x, od[q].y);
-          dst[1] = make_float2(od[q].z, od[q].w);
-        });
-      }
-      __syncthreads();
-      cf x[32];
-      pass1_load<P>(x, t, row);
-      fwd_pass1<P, ODD>(x, t, row, b);
-      __syncthreads();
-      fwd_pass2<P>(x, t, row, tab2);
-      __syncthreads();
-      const int ga = ODD ? grp.go : grp.ge, gb = ODD ? grp.gc : grp.gm;
-      fwd_groups<P>(x, row, ga, gb);
-      __syncthreads();      // LDS is restaged by the next half / item
-
-      // (Ke, Ko) of the pair (za at frequency k of this half transform, zb at its partner)
-      auto emit = [&](auto slot, cf za, cf zb) __attribute__((always_inline)) {
-        sp4[decltype(slot)::value * T] = make_float4(scale * (za.re + zb.re), scale * (za.im - zb.im),
-                                                     scale * (za.im + zb.im), scale * (zb.re - za.re));
-      };
-      if (!ODD && grp.special) {
-        const cf z0 = x[bitrev(0, 4)], zn = x[bitrev(8, 4)];
-        sp4[0] = make_float4(4.f * scale * z0.re, 4.f * scale * z0.im, 4.f * scale * zn.re, 4.f * scale * zn.im);
-        static_for<1, 8>([&](auto ss) {
-          constexpr int s = decltype(ss)::value;
-          emit(ss, x[bitrev(s, 4)], x[bitrev(16 - s, 4)]);
-        });
-        static_for<0, 8>([&](auto ss) {
-          constexpr int s = decltype(ss)::value;
-          emit(ic<8 + s>{}, x[16 + bitrev(s, 4)], x[16 + bitrev(15 - s, 4)]);
-        });
-      } else {
-        static_for<0, 16>([&](auto ss) {
-          constexpr int s = decltype(ss)::value;
-          emit(ss, x[bitrev(s, 4)], x[16 + bitrev(15 - s, 4)]);
-        });
-      }
-    };
-    one_half(ic<0>{});
-    one_half(ic<1>{});
+    sync_threads<T>();                      // the item before has been read
+    transform<P, 1>(x, t, row, tab1, tf1);
+    store_spectrum<P>(x, scale, blk);
+    sync_threads<T>();
+    static_for<0, 32>([&](auto rr) { x[decltype(rr)::value] = q[decltype(rr)::value]; });
+    transform<P, 5>(x, t, row, tab5, tf5);
+    store_spectrum<P>(x, scale, blk + BLK / 4);
   }
 }
 
 // ------------------------------------------------------------------------------------------
 // host-side launchers
 // ------------------------------------------------------------------------------------------
-typedef SplitPlan<14, 32, 32> RealPlan;      // half transforms of 16384 points: sequence length 32768
-static_assert(split_offsets_ok<RealPlan>(), "LDS offsets of the split plan");
-
-size_t real_spectrum_bytes(int d) { return (size_t)d * 4 * real_spec_block<RealPlan>() * sizeof(float); }
-
 template <typename ACT>
 static int launch_mixer_real(const void* xproj, const float* u, const float* sw, const float* sb, const float* pbias,
                              const float* spec, void* y, int B, int d, hipStream_t stream) {
   typedef RealPlan P;
-  const size_t lds_bytes = (size_t)P::WG_LDS * sizeof(float2);
+  const size_t lds_bytes = (size_t)(P::ROW + 2 * P::TAB) * sizeof(float2);
   auto kern = sw ? (u ? mixer_real_kernel<P, ACT, true, true> : mixer_real_kernel<P, ACT, true, false>)
                  : mixer_real_kernel<P, ACT, false, false>;
   if (!sw && u) return set_error(M2_ERR_ARG, "mixer_real: a plain convolution takes no second input");
@@ -494,7 +395,7 @@ int launch_mixer_real_dispatch(const void* xproj, const float* u, const float* s
 int launch_filter_spectrum_real(const float* taps1, const float* taps2, const float* D1, const float* D2, float* spec,
                                 int d, const SpectrumBatch& sb, int nmixers, hipStream_t stream) {
   typedef RealPlan P;
-  const size_t lds_bytes = (size_t)P::WG_LDS * sizeof(float2);
+  const size_t lds_bytes = (size_t)(P::ROW + 2 * P::TAB) * sizeof(float2);
   auto kern = filter_spectrum_real_kernel<P>;
   hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes);
   if (e != hipSuccess) return set_error(M2_ERR_LAUNCH, "hipFuncSetAttribute(filter_spectrum_real): %s", hipGetErrorString(e));

@@ -3,6 +3,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+#include <type_traits>
 
 #include "m2_internal.h"
 
@@ -38,6 +39,10 @@ template <typename ACT, int Q, bool CHAINED = false> struct RawRow;
 template <int Q, bool CHAINED> struct RawRow<float, Q, CHAINED> {
   f32x4_t a[Q], b[Q];
   f32x2_t h[Q];
+  template <int I> __device__ __forceinline__ void clear(std::integral_constant<int, I>) {
+    a[I] = b[I] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    h[I] = f32x2_t{0.f, 0.f};
+  }
   template <int I> __device__ __forceinline__ void fetch(const float* p, int n0) {
     a[I] = *reinterpret_cast<const f32x4_t*>(p + n0);
     b[I] = *reinterpret_cast<const f32x4_t*>(p + n0 + 4);
@@ -67,6 +72,10 @@ template <int Q, bool CHAINED> struct RawRow<float, Q, CHAINED> {
 template <int Q, bool CHAINED> struct RawRow<uint16_t, Q, CHAINED> {
   u32x4_t a[Q];
   uint32_t h[Q];
+  template <int I> __device__ __forceinline__ void clear(std::integral_constant<int, I>) {
+    a[I] = u32x4_t{0u, 0u, 0u, 0u};
+    h[I] = 0u;
+  }
   template <int I> __device__ __forceinline__ void fetch(const uint16_t* p, int n0) {
     a[I] = *reinterpret_cast<const u32x4_t*>(p + n0);
     if constexpr (!(CHAINED && I > 0))

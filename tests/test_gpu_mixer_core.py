@@ -1,0 +1,39 @@
+"""The mixer core and the plain long convolution against fp64 transforms, at row counts that leave row batches, workgroups and rounds
+partly filled, and on either side of the rule that chooses a kernel at L = 8192."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _conv(a, k, D):
+    k = k.double().clone()
+    k[:, 0] += D.double()
+    n = k.shape[-1]
+    return torch.fft.irfft(torch.fft.rfft(a, n=n) * torch.fft.rfft(k, n=n)[:, None], n=n)[..., :a.shape[-1]]
+
+
+@pytest.mark.parametrize("L,d,B", [(128, 8, 1), (128, 24, 7), (128, 768, 33), (256, 8, 9), (512, 16, 5), (1024, 8, 3), (2048, 8, 3), (4096, 8, 1),
+                                   (8192, 8, 1), (8192, 256, 2), (8192, 256, 3), (16384, 8, 2), (32768, 8, 1)])
+@pytest.mark.parametrize("act", [torch.float32, torch.bfloat16])
+def test_mixer_core_rows(gpu, L, d, B, act):
+    from m2_amd import ops
+    g = torch.Generator().manual_seed(L + d + B)
+    taps = [torch.randn(d, 2 * L, generator=g) / L ** 0.5 for _ in range(2)]
+    D = [torch.randn(d, generator=g) for _ in range(2)]
+    xproj, u = torch.randn(3 * d, B, L, generator=g).to(act), torch.randn(d, B, L, generator=g)
+    sw, sb, pb = (torch.randn(3 * d, *s, generator=g) for s in ((3,), (), ()))
+    spec = ops.filter_spectrum(taps[0].to(gpu), taps[1].to(gpu), D[0].to(gpu), D[1].to(gpu))
+    x = torch.nn.functional.pad(xproj.double() + pb.double()[:, None, None], (2, 0))
+    s = sb.double()[:, None, None] + sum(sw.double()[:, k, None, None] * x[..., k:k + L] for k in range(3))
+    first, second = _conv(s[:d] * s[2 * d:], taps[0], D[0]) * s[d:2 * d], _conv(u.double(), taps[1], D[1])
+    # fp32: two roundings of 2^-24 per stage of either transform, a few in the convolutions and the gate.  bf16: the gate and the
+    # result are rounded to 2^-9, here relative to a result of which they are a part
+    tol = (4 * (L.bit_length() - 1) + 12) * 2.0 ** -24 if act == torch.float32 else 2.0 ** -8
+    for second_signal in (True, False):
+        y = ops.mixer_core(xproj.to(gpu), u.to(gpu) if second_signal else None, sw.to(gpu), sb.to(gpu), spec, B, L, d, proj_bias=pb.to(gpu))
+        ref = first + second if second_signal else first
+        assert (y.double().cpu() - ref).norm() <= tol * ref.norm()
+    plain = ops.fftconv(u.to(act).to(gpu), spec, B, L, d).double().cpu()
+    ref = _conv(u.to(act).double(), taps[0], D[0])
+    assert (plain - ref).norm() <= tol * ref.norm()
