@@ -7,9 +7,9 @@
 //
 // A workgroup owns 16 channels of one mixer: 32 rows of L complex points in LDS (one per channel and filter; re = the first half
 // of the 2L window, im = the second: fft_twist.h), exactly one batch of rows for its 32 T threads.  Phase 1: wave w projects the positions of
-// MLP w mod nmlp (forward / reverse MLP of either filter) for the 16 channels on v_mfma_f32_16x16x32_bf16
-// (W3 rows as the A operand, split into bf16 hi / lo parts in registers; the last hidden layer's activations,
-// which the hidden kernel left as bf16 hi / lo parts, as the B operand; three products: fp32-grade accuracy),
+// MLP w mod nmlp (forward / reverse MLP of either filter) for the 16 channels on v_mfma_f32_16x16x32_f16
+// (W3 rows as the A operand, split into fp16 hi / lo parts in registers; the last hidden layer's activations,
+// which the hidden kernel left in the same form, as the B operand; three products, hyena_filter.h),
 // multiplies by exp(-t |delta|) + shift and drops each value at its place in the window.  Phase 2: every row is
 // transformed by its T threads (same passes as the stand-alone spectrum kernel) and stored in the mixer core's
 // order.  All mixers of a model go in one launch (blockIdx.y).
@@ -28,7 +28,7 @@ __global__ __launch_bounds__(2 * kFusedRows * P::T) void project_spectrum_kernel
     const FilterPtrs* __restrict__ tab,         // fpm entries per mixer
     const float* const* __restrict__ skip,      // fpm skip-weight pointers per mixer (entries, or the table, may be null)
     int fpm, int d, float shift,
-    const uint16_t* __restrict__ h_hi,          // (2 nfilters, L, 128) bf16: high parts of the last hidden layer
+    const uint16_t* __restrict__ h_hi,          // (2 nfilters, L, 128) fp16: high parts of the last hidden layer
     const uint16_t* __restrict__ h_lo,          // low parts
     float4* __restrict__ spec, long spec_stride4) {
   constexpr int L = P::H, T = P::T, NT = 2 * kFusedRows * T, NW = NT / 64;
@@ -54,25 +54,38 @@ __global__ __launch_bounds__(2 * kFusedRows * P::T) void project_spectrum_kernel
     const FilterPtrs& F = tab[f];
     const float* W3 = F.mlp[dir].w3;
     if (W3 != nullptr) {
-      bf16x8 ahi[kOrder / 32], alo[kOrder / 32];
+      f16x8 ahi[kOrder / 32], alo[kOrder / 32];
+      float rs[4];                     // reciprocal scales of the lane's four channels
       {
         const float* wrow = W3 + (long)(c0 + i16) * kOrder + 8 * q4;
+        float v[kOrder / 4], top = 0.f;
 #pragma unroll
         for (int ks = 0; ks < kOrder / 32; ++ks) {
           const float4 v0 = *reinterpret_cast<const float4*>(wrow + 32 * ks);
           const float4 v1 = *reinterpret_cast<const float4*>(wrow + 32 * ks + 4);
-          const float v[8] = {v0.x, v0.y, v0.z, v0.w, v1.x, v1.y, v1.z, v1.w};
-          float h[8], l[8];
-#pragma unroll
-          for (int j = 0; j < 8; ++j) {
-            h[j] = bf16_to_f32(f32_to_bf16(v[j]));
-            l[j] = v[j] - h[j];
-          }
-          const u32x4 vh = {pack_bf16x2(h[0], h[1]), pack_bf16x2(h[2], h[3]), pack_bf16x2(h[4], h[5]), pack_bf16x2(h[6], h[7])};
-          const u32x4 vl = {pack_bf16x2(l[0], l[1]), pack_bf16x2(l[2], l[3]), pack_bf16x2(l[4], l[5]), pack_bf16x2(l[6], l[7])};
-          ahi[ks] = __builtin_bit_cast(bf16x8, vh);
-          alo[ks] = __builtin_bit_cast(bf16x8, vl);
+          v[8 * ks] = v0.x; v[8 * ks + 1] = v0.y; v[8 * ks + 2] = v0.z; v[8 * ks + 3] = v0.w;
+          v[8 * ks + 4] = v1.x; v[8 * ks + 5] = v1.y; v[8 * ks + 6] = v1.z; v[8 * ks + 7] = v1.w;
         }
+#pragma unroll
+        for (int j = 0; j < kOrder / 4; ++j) top = fmaxf(top, fabsf(v[j]));
+        top = fmaxf(top, __shfl_xor(top, 16));
+        top = fmaxf(top, __shfl_xor(top, 32));
+        const float scale = row_scale(top), back = 1.f / (scale * kActScale);
+#pragma unroll
+        for (int ks = 0; ks < kOrder / 32; ++ks) {
+          u32x4 vh, vl;
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            uint32_t h, l;
+            split2(v[8 * ks + 2 * j] * scale, v[8 * ks + 2 * j + 1] * scale, h, l);
+            vh[j] = h;
+            vl[j] = l;
+          }
+          ahi[ks] = __builtin_bit_cast(f16x8, vh);
+          alo[ks] = __builtin_bit_cast(f16x8, vl);
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j) rs[j] = __shfl(back, 4 * q4 + j);
       }
       float adelta[4];
 #pragma unroll
@@ -92,20 +105,20 @@ __global__ __launch_bounds__(2 * kFusedRows * P::T) void project_spectrum_kernel
         floatx4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int ks = 0; ks < kOrder / 32; ++ks) {      // smallest terms first
-          acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(alo[ks], __builtin_bit_cast(bf16x8, bh[ks]), acc, 0, 0, 0);
-          acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ahi[ks], __builtin_bit_cast(bf16x8, bl[ks]), acc, 0, 0, 0);
+          acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(alo[ks], __builtin_bit_cast(f16x8, bh[ks]), acc, 0, 0, 0);
+          acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(ahi[ks], __builtin_bit_cast(f16x8, bl[ks]), acc, 0, 0, 0);
         }
 #pragma unroll
         for (int ks = 0; ks < kOrder / 32; ++ks)
-          acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ahi[ks], __builtin_bit_cast(bf16x8, bh[ks]), acc, 0, 0, 0);
+          acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(ahi[ks], __builtin_bit_cast(f16x8, bh[ks]), acc, 0, 0, 0);
         // accumulator element j of lane (i16, q4): channel c0 + 4 q4 + j, position p
         // forward taps fill the first half of the window, reverse taps the second from its end
         float* dst = reinterpret_cast<float*>(lds + (8 * q4 + which) * P::ROW + P::phys(dir == 0 ? p : L - 1 - p)) + dir;
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-          // exp(-t |delta|); the bare hardware exp2 flushes results below 2^-126 to zero, which is the value to
+          // (exp(-t |delta|) + shift) r; the bare hardware exp2 flushes results below 2^-126 to zero, which is the value to
           // 1e-38 absolute
-          const float decay = __builtin_amdgcn_exp2f(tl * adelta[j]) + shift;
+          const float decay = fmaf(__builtin_amdgcn_exp2f(tl * adelta[j]), rs[j], shift * rs[j]);
           dst[(long)j * P::ROW * 4] = acc[j] * decay;
         }
       }

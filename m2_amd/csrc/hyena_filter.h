@@ -1,5 +1,5 @@
 // Types shared by the filter-generation translation units (hyena_filter_kernels.hip, filter_fused_kernels.hip):
-// the pointer table of a batch of implicit filters and the helpers that turn fp32 values into bf16 parts for
+// the pointer table of a batch of implicit filters and the helpers that turn fp32 values into fp16 parts for
 // the matrix cores.
 #pragma once
 #include <hip/hip_runtime.h>
@@ -40,15 +40,31 @@ struct TabByPointer {
 
 typedef float floatx16 __attribute__((ext_vector_type(16)));
 typedef float floatx4 __attribute__((ext_vector_type(4)));
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
-// x = hi + mid + lo with three bf16 terms: 24 mantissa bits, i.e. all of an fp32 value
-__device__ __forceinline__ void split3(float x, float& hi, float& mid, float& lo) {
-  hi = bf16_to_f32(f32_to_bf16(x));
-  const float r = x - hi;
-  mid = bf16_to_f32(f32_to_bf16(r));
-  lo = r - mid;                      // the conversion of lo to bf16 happens where it is packed
+// The matrix products of the filter MLPs: either operand as two fp16 parts, x 2^e = hi + lo, three products (hi lo, lo hi, hi hi),
+// fp32 accumulation.  Two parts hold 23 - 24 bits and the product left out is below 2^-24 of the whole one, so a product is good to
+// what fp32 arithmetic gives.  fp16 has five bits of exponent: e scales activations (|h| <= 1) by 2^13 and every row of a weight
+// so that its largest entry lies in [2^12, 2^13), which keeps entries down to 2^-16 of the largest exact to 2^-24 of themselves and
+// all others to 2^-38 of the largest.  (Three bf16 parts and six products, which this took over from, are exact and cost twice the
+// matrix instructions, half as many conversions again and half as many registers for stationary weights again.)
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+constexpr float kActScale = 8192.f;      // 2^13
+
+// two values -> their high and low parts, packed
+__device__ __forceinline__ void split2(float a, float b, uint32_t& hi, uint32_t& lo) {
+  const f16x2 h = __builtin_convertvector(f32x2{a, b}, f16x2);
+  const f32x2 back = __builtin_convertvector(h, f32x2);
+  hi = __builtin_bit_cast(uint32_t, h);
+  lo = __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{a - back.x, b - back.y}, f16x2));
+}
+// Scale of a row whose largest magnitude is m: 2^e.  (A row below 2^-47 is scaled by 2^60, no more: its reciprocal multiplies biases.)
+__device__ __forceinline__ float row_scale(float m) {
+  int e = 12 - (int)((__float_as_uint(m) >> 23) & 0xff) + 127;      // -116 (infinity) ...
+  e = e > 60 ? 60 : e;
+  return __uint_as_float((uint32_t)(127 + e) << 23);
 }
 
 // Spectrum kernels of a batch of mixers: blockIdx.y selects the mixer.  taps: filter f of mixer m at

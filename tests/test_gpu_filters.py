@@ -1,0 +1,54 @@
+"""Filter taps where the split weights and the tiles of their products can go wrong: rows of very different sizes, zero rows, widths
+with fewer channel tiles than waves and with a remainder, lengths on either side of each kernel, against fp64."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("L,d", [(128, 64), (1024, 64), (1088, 192), (1024, 320), (2048, 192)])
+def test_taps_of_rows_of_any_size(gpu, L, d):
+    import m2_amd
+    from oracle import m2_oracle as O
+    g = torch.Generator().manual_seed(L + d)
+    fn = m2_amd.HyenaFilter(d, emb_dim=5, order=128, seq_len=L, bidirectional=True, w=10)
+    with torch.no_grad():
+        for name, p in fn.named_parameters():
+            leaf = name.rsplit(".", 1)[-1]
+            if "implicit_filter" not in name or leaf == "freq":
+                continue
+            p.normal_(0.0, 0.1, generator=g)
+            if leaf == "weight" and p.shape[1] == 128:
+                last = p.shape[0] == d
+                # inner rows down to nothing, output rows over most of fp32's range, single large entries in both
+                p.mul_(2.0 ** torch.randint(-50 if last else -20, 50 if last else 1, (p.shape[0], 1), generator=g))
+                p[3] = 0.0
+                p[5, 7] *= 64.0
+                if not last:
+                    p[9] *= 2.0 ** -60
+    sd = {k: v.detach().clone().double() for k, v in fn.state_dict().items()}
+    taps = fn.to(gpu).bidirectional_taps(L).double().cpu()
+    ref = O.bidirectional_kernel(*(O.hyena_filter_taps(sd, "", L, rev=r)[0].T for r in (False, True)), L)
+    sd32 = {k: v.float() for k, v in sd.items()}
+    ref32 = O.bidirectional_kernel(*(O.hyena_filter_taps(sd32, "", L, rev=r)[0].T for r in (False, True)), L).double()
+    assert torch.isfinite(taps).all()
+    # channel by channel: products good to a few 2^-24 each, and what fp32 arithmetic itself makes of sin(10 x)
+    norm = ref.norm(dim=1)
+    err, err32 = (taps - ref).norm(dim=1), (ref32 - ref).norm(dim=1)
+    assert (err <= 8 * 2.0 ** -24 * norm + 4 * err32).all(), (err / norm.clamp_min(1e-300)).max()
+    assert not taps[3].any()
+
+
+def test_taps_of_infinite_and_large_weights(gpu):
+    """Finite weights of any size give finite taps, infinite ones poison their channel only."""
+    import m2_amd
+    L, d = 1024, 64
+    fn = m2_amd.HyenaFilter(d, emb_dim=5, order=128, seq_len=L, bidirectional=True, w=10)
+    with torch.no_grad():
+        for w in (fn.implicit_filter[6].weight,):
+            w[1] = 1e36
+            w[2, 4] = float("inf")
+            w[6, 8] = float("nan")
+    taps = fn.to(gpu).bidirectional_taps(L).cpu()[:, :L]
+    bad = ~torch.isfinite(taps).all(dim=1)
+    assert bad[2] and bad[6] and int(bad.sum()) == 2
