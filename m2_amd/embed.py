@@ -8,6 +8,7 @@ token ids directly to `encode_token_ids`.
 """
 from __future__ import annotations
 
+from array import array
 from typing import Callable, Dict, Iterable, List, Optional, Sequence
 
 import numpy as np
@@ -31,6 +32,19 @@ def pad_or_truncate(ids: torch.Tensor, length: int) -> torch.Tensor:
     return ids[:, :length]
 
 
+def _host_row(row) -> Optional[np.ndarray]:
+    """A list or tuple of whole numbers, or an integer CPU tensor, as a flat int64 array; None for anything else, which torch.as_tensor
+    is asked about (floats, empty and nested lists, strings, ...)."""
+    if isinstance(row, torch.Tensor):
+        return row.detach().reshape(-1).numpy() if row.dtype == torch.int64 and row.device.type == "cpu" else None
+    if type(row) in (list, tuple) and len(row) > 0:
+        try:
+            return np.frombuffer(array("q", row), np.int64)
+        except (TypeError, OverflowError):
+            return None
+    return None
+
+
 class M2BertTextEncoder:
     """`model`: a BertModel with a pooler, on the GPU, in eval mode.  Every text is padded or cut to
     `max_seq_len` tokens (the reference's `evaluation_max_seq_len`), texts are run `batch_size` at a time and the
@@ -50,25 +64,47 @@ class M2BertTextEncoder:
                          attention_masks: Optional[Sequence] = None) -> np.ndarray:
         """token_ids: one 1-D sequence of ids per text (any lengths, may be empty); returns (len(token_ids), d)
         fp32.  Without attention_masks every given token counts as real and the padding as masked."""
-        out = torch.empty(0, self.model.config.hidden_size)
+        out = [torch.empty(0, self.model.config.hidden_size)]
         for lo in range(0, len(token_ids), batch_size):
-            ids_rows, mask_rows = [], []
-            for k in range(lo, min(lo + batch_size, len(token_ids))):
-                ids = torch.as_tensor(token_ids[k], dtype=torch.long).reshape(1, -1)
-                mask = torch.ones_like(ids) if attention_masks is None else \
-                    torch.as_tensor(attention_masks[k], dtype=torch.long).reshape(1, -1)
-                if mask.shape != ids.shape:
-                    raise ValueError(f"text {k}: {ids.shape[1]} token ids but {mask.shape[1]} mask entries")
-                ids_rows.append(pad_or_truncate(ids, self.max_seq_len))
-                mask_rows.append(pad_or_truncate(mask, self.max_seq_len))
-            ids_b = torch.cat(ids_rows, 0).to(self.device)
-            mask_b = torch.cat(mask_rows, 0).to(self.device)
+            hi = min(lo + batch_size, len(token_ids))
+            ids_b, mask_b = self._assemble(token_ids, attention_masks, lo, hi)
             with torch.no_grad():
-                _, pooled = self.model(input_ids=ids_b, attention_mask=mask_b)
-            out = torch.cat((out, pooled.detach().float().cpu()), 0)
+                _, pooled = self.model(input_ids=ids_b.to(self.device), attention_mask=mask_b.to(self.device))
+            out.append(pooled.detach().float().cpu())
+        out = torch.cat(out, 0)
         if torch.isnan(out).any():
             raise ValueError("NaNs in the encoded texts")
         return out.numpy()
+
+    def _assemble(self, token_ids: Sequence, attention_masks: Optional[Sequence], lo: int, hi: int):
+        """Texts [lo, hi) as padded or cut (hi - lo, max_seq_len) ids and mask.  Rows are written into two arrays; a torch tensor
+        per text, its mask, both padded and all of them concatenated took 60 us a text, 3 ms of the 12 of 75 texts of up to 512 tokens."""
+        L = self.max_seq_len
+        ids_b, mask_b = np.zeros((hi - lo, L), np.int64), np.zeros((hi - lo, L), np.int64)
+        for k in range(lo, hi):
+            ids = _host_row(token_ids[k])
+            mask = None if attention_masks is None else _host_row(attention_masks[k])
+            if ids is None or (mask is None and attention_masks is not None):
+                return self._assemble_tensors(token_ids, attention_masks, lo, hi)
+            if mask is not None and mask.shape != ids.shape:
+                raise ValueError(f"text {k}: {ids.shape[0]} token ids but {mask.shape[0]} mask entries")
+            n = min(ids.shape[0], L)
+            ids_b[k - lo, :n] = ids[:n]
+            mask_b[k - lo, :n] = 1 if mask is None else mask[:n]
+        return torch.from_numpy(ids_b), torch.from_numpy(mask_b)
+
+    def _assemble_tensors(self, token_ids: Sequence, attention_masks: Optional[Sequence], lo: int, hi: int):
+        """The same for whatever torch.as_tensor takes."""
+        ids_rows, mask_rows = [], []
+        for k in range(lo, hi):
+            ids = torch.as_tensor(token_ids[k], dtype=torch.long).reshape(1, -1)
+            mask = torch.ones_like(ids) if attention_masks is None else \
+                torch.as_tensor(attention_masks[k], dtype=torch.long).reshape(1, -1)
+            if mask.shape != ids.shape:
+                raise ValueError(f"text {k}: {ids.shape[1]} token ids but {mask.shape[1]} mask entries")
+            ids_rows.append(pad_or_truncate(ids, self.max_seq_len))
+            mask_rows.append(pad_or_truncate(mask, self.max_seq_len))
+        return torch.cat(ids_rows, 0), torch.cat(mask_rows, 0)
 
     def _encode_texts(self, texts: List[str], batch_size: int) -> np.ndarray:
         if self.tokenizer is None:
