@@ -303,6 +303,7 @@ extern "C" int m2_dense_supported(int M, int N, int K) {
 extern "C" int m2_dense_to_channels_fwd(const void* x, const void* w, void* out, int M, int N, int K, void* stream) {
   const int rc = check_dense("m2_dense_to_channels_fwd", x, w, out, M, N, K);
   if (rc) return rc;
+  if (dense_ws_serves(M, N, K)) return dense_ws_launch(x, w, out, M, N, M, (hipStream_t)stream);
   GemmArgs g{(const uint16_t*)x, (const uint16_t*)w, (uint16_t*)out, nullptr, nullptr, K, K, M, M, N, K, 1, 0, 0, 0, 1};
   return dense_launch<false>(pick_variant(g, false), g, (hipStream_t)stream);
 }

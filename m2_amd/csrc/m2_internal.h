@@ -25,6 +25,10 @@ int glu_few_rows(const void* x, const void* w, void* out, int M, int nb, int p, 
 int blockdiag_linear_engine(const void* x, const void* w, const float* bias, const void* resid, void* out, int M, int nb, int p,
                             int q, hipStream_t stream);
 
+// OUT (N, M) = W (N, K) X (M, K)^T with the weights in registers (dense_ws_kernels.hip), rows of OUT ldo elements apart.
+bool dense_ws_serves(int M, int N, int K);
+int dense_ws_launch(const void* x, const void* w, void* out, int M, int N, long ldo, hipStream_t stream);
+
 // round-to-nearest-even float -> bfloat16 bits (NaN stays NaN)
 // float -> bf16 bits, round to nearest even (host restatement of what v_cvt_pk_bf16_f32 does)
 __host__ __device__ __forceinline__ uint16_t f32_to_bf16_bits(float f) {

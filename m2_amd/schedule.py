@@ -299,7 +299,7 @@ def stack_plan(encoder, B: int, L: int, device: torch.device):
         if type(first) is not _encoder.BertLayer or type(first.attention) is not MonarchMixerSequenceMixing:
             return None
         d = first.attention.d_model
-    if not ops.own_to_channels(M, d) or not ops.own_from_channels(M, d):
+    if not ops.native_rows(M, d):
         return None
     if plan is None:
         if torch.cuda.is_current_stream_capturing():

@@ -37,6 +37,21 @@ def test_dense_projections(gpu, M, N, K):
     _within_bf16(ops.dense_from_channels(xt, w.to(gpu), bias.to(gpu)), ref + bias.double(), absref + bias.double().abs())
 
 
+# the product with its weights in registers: the fewest rows it takes, fewer and more slabs of 32 rows than row ranges, a last slab of
+# 8, 16 and 24 rows, one group of channels and so many that an XCD holds no whole row range, one to three and many slabs per range
+@pytest.mark.parametrize("M,N", [(512, 2304), (520, 2304), (904, 2304), (1800, 2304), (2712, 768), (5632, 2304), (3000, 256), (8200, 256),
+                                 (1000, 9216), (31744, 2304), (16376, 2304)])
+def test_dense_weights_in_registers(gpu, M, N):
+    from m2_amd import ops
+    g = torch.Generator(device=gpu).manual_seed(M + N)
+    x, w = torch.randn(M, 768, generator=g, device=gpu).bfloat16(), torch.randn(N, 768, generator=g, device=gpu).bfloat16()
+    n = torch.cat([torch.arange(min(N, 300)), torch.arange(N - 128, N)]).unique().to(gpu)      # every row of x against these channels
+    got = ops.dense_to_channels(x, w)
+    _within_bf16(got[n].t(), x.cpu().double() @ w[n].cpu().double().T, x.cpu().double().abs() @ w[n].cpu().double().abs().T)
+    m = torch.cat([torch.arange(0, M, max(1, M // 70)), torch.arange(M - 40, M)]).unique().to(gpu)   # and every channel on these rows
+    _within_bf16(got[:, m].t(), x[m].cpu().double() @ w.cpu().double().T, x[m].cpu().double().abs() @ w.cpu().double().abs().T)
+
+
 def test_dense_unsupported_sizes_are_refused(gpu):
     from m2_amd import ops
     for M, N, K in ((12, 64, 64), (64, 20, 64), (64, 64, 96)):
