@@ -146,6 +146,9 @@ int m2_filter_spectrum_fwd(const float* taps1, const float* taps2, const float* 
 int m2_mixer_core_fwd(const void* xproj, const float* proj_bias, const float* u, const float* short_w,
                       const float* short_b, const float* spec, void* y, int B, int L, int d, int act_dtype,
                       void* stream);
+/* The same with the rows of xproj (channels) xproj_row >= B * L elements apart, a multiple of 8. */
+int m2_mixer_core_rows_fwd(const void* xproj, long xproj_row, const float* proj_bias, const float* u, const float* short_w,
+                           const float* short_b, const float* spec, void* y, int B, int L, int d, int act_dtype, void* stream);
 
 /* Plain long convolution y[c,b,:] = fftconv(x[c,b,:]; k1)[:L] + D1[c] x[c,b,:] with the first filter
  * of `spec` (HyenaFilter.forward on its own, bert/src/mm/hyena_utils.py:219-248).
@@ -162,6 +165,10 @@ int m2_fftconv_fwd(const void* x, const float* spec, void* y, int B, int L, int 
  * ------------------------------------------------------------------------------------------- */
 int m2_dense_supported(int M, int N, int K);
 int m2_dense_to_channels_fwd(const void* x, const void* w, void* out, int M, int N, int K, void* stream);
+/* The same with the rows of `out` (channels) out_row >= M elements apart, a multiple of 8, and the distance at which this product is
+ * fastest (M for most sizes; the core reads such rows through m2_mixer_core_rows_fwd). */
+int m2_dense_to_channels_rows_fwd(const void* x, const void* w, void* out, long out_row, int M, int N, int K, void* stream);
+long m2_dense_channels_row(int M, int N, int K);
 int m2_dense_from_channels_fwd(const void* x, const void* w, const float* bias, void* out, int M, int N, int K,
                                void* stream);
 

@@ -7,7 +7,7 @@ from __future__ import annotations
 
 import ctypes
 import os
-from ctypes import POINTER, c_char_p, c_float, c_int, c_size_t, c_void_p
+from ctypes import POINTER, c_char_p, c_float, c_int, c_long, c_size_t, c_void_p
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libm2_amd.so")
@@ -61,6 +61,8 @@ def _load() -> ctypes.CDLL:
     lib.m2_mixer_core_fwd.restype = c_int
     lib.m2_mixer_core_fwd.argtypes = [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int,
                                       c_int, c_int, c_void_p]
+    lib.m2_mixer_core_rows_fwd.restype = c_int
+    lib.m2_mixer_core_rows_fwd.argtypes = [c_void_p, c_long] + lib.m2_mixer_core_fwd.argtypes[1:]
     lib.m2_fftconv_fwd.restype = c_int
     lib.m2_fftconv_fwd.argtypes = [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_void_p]
     lib.m2_mixer_filters_workspace_bytes.restype = ctypes.c_size_t
@@ -72,6 +74,10 @@ def _load() -> ctypes.CDLL:
     lib.m2_dense_supported.argtypes = [c_int] * 3
     lib.m2_dense_to_channels_fwd.restype = c_int
     lib.m2_dense_to_channels_fwd.argtypes = [c_void_p] * 3 + [c_int] * 3 + [c_void_p]
+    lib.m2_dense_to_channels_rows_fwd.restype = c_int
+    lib.m2_dense_to_channels_rows_fwd.argtypes = [c_void_p] * 3 + [c_long] + [c_int] * 3 + [c_void_p]
+    lib.m2_dense_channels_row.restype = c_long
+    lib.m2_dense_channels_row.argtypes = [c_int] * 3
     lib.m2_dense_from_channels_fwd.restype = c_int
     lib.m2_dense_from_channels_fwd.argtypes = [c_void_p] * 4 + [c_int] * 3 + [c_void_p]
     lib.m2_blockdiag_glu_fwd.restype = c_int
@@ -138,8 +144,8 @@ def _load() -> ctypes.CDLL:
 lib = _load()
 
 EXPORTS = ["m2_version", "m2_last_error", "m2_hyena_filter_workspace_bytes", "m2_hyena_filter_fwd", "m2_hyena_filter_fwd_static", "m2_mixer_filters_workspace_bytes", "m2_mixer_filters_fwd",
-           "m2_fftconv_supported_seqlen", "m2_filter_spectrum_bytes", "m2_filter_spectrum_fwd", "m2_mixer_core_fwd",
-           "m2_fftconv_fwd", "m2_dense_supported", "m2_dense_to_channels_fwd", "m2_dense_from_channels_fwd", "m2_blockdiag_glu_fwd", "m2_blockdiag_glu_few_rows", "m2_blockdiag_linear_fwd", "m2_blockdiag_linear_f32_fwd", "m2_mlp_fused_supported", "m2_mlp_fused_packed_bytes", "m2_mlp_fused_pack", "m2_mlp_fused_fwd", "m2_glu_stream_supported", "m2_glu_stream_packed_bytes", "m2_glu_stream_pack", "m2_glu_stream_fwd", "m2_layernorm_fwd", "m2_layernorm_bf16_fwd", "m2_input_forms_fwd",
+           "m2_fftconv_supported_seqlen", "m2_filter_spectrum_bytes", "m2_filter_spectrum_fwd", "m2_mixer_core_fwd", "m2_mixer_core_rows_fwd",
+           "m2_fftconv_fwd", "m2_dense_supported", "m2_dense_to_channels_fwd", "m2_dense_to_channels_rows_fwd", "m2_dense_channels_row", "m2_dense_from_channels_fwd", "m2_blockdiag_glu_fwd", "m2_blockdiag_glu_few_rows", "m2_blockdiag_linear_fwd", "m2_blockdiag_linear_f32_fwd", "m2_mlp_fused_supported", "m2_mlp_fused_packed_bytes", "m2_mlp_fused_pack", "m2_mlp_fused_fwd", "m2_glu_stream_supported", "m2_glu_stream_packed_bytes", "m2_glu_stream_pack", "m2_glu_stream_fwd", "m2_layernorm_fwd", "m2_layernorm_bf16_fwd", "m2_input_forms_fwd",
            "m2_embed_layernorm_fwd", "m2_blockdiag_linear_layernorm_supported", "m2_blockdiag_linear_layernorm_fwd", "m2_encoder_layers_workspace_bytes", "m2_encoder_layers_fwd",
            "m2_split_bytes", "m2_split_rows_fwd", "m2_split_jobs_fwd", "m2_split_channels_fwd", "m2_split_to_channels_fwd", "m2_split_linear_fwd", "m2_split_glu_fwd"]
 

@@ -300,12 +300,28 @@ extern "C" int m2_dense_supported(int M, int N, int K) {
   return ((long)M * K * 2 < (1l << 32) && (long)N * K * 2 < (1l << 32)) ? 1 : 0;
 }
 
-extern "C" int m2_dense_to_channels_fwd(const void* x, const void* w, void* out, int M, int N, int K, void* stream) {
-  const int rc = check_dense("m2_dense_to_channels_fwd", x, w, out, M, N, K);
+static int dense_to_channels(const char* who, const void* x, const void* w, void* out, int M, int N, int K, long ldo, void* stream) {
+  const int rc = check_dense(who, x, w, out, M, N, K);
   if (rc) return rc;
-  if (dense_ws_serves(M, N, K)) return dense_ws_launch(x, w, out, M, N, M, (hipStream_t)stream);
-  GemmArgs g{(const uint16_t*)x, (const uint16_t*)w, (uint16_t*)out, nullptr, nullptr, K, K, M, M, N, K, 1, 0, 0, 0, 1};
+  if (ldo < M || ldo % 8) return set_error(M2_ERR_ARG, "%s: rows of the output %ld apart, need a multiple of 8 from M = %d on", who, ldo, M);
+  if (dense_ws_serves(M, N, K)) return dense_ws_launch(x, w, out, M, N, ldo, (hipStream_t)stream);
+  GemmArgs g{(const uint16_t*)x, (const uint16_t*)w, (uint16_t*)out, nullptr, nullptr, K, K, ldo, M, N, K, 1, 0, 0, 0, 1};
   return dense_launch<false>(pick_variant(g, false), g, (hipStream_t)stream);
+}
+
+extern "C" int m2_dense_to_channels_fwd(const void* x, const void* w, void* out, int M, int N, int K, void* stream) {
+  return dense_to_channels("m2_dense_to_channels_fwd", x, w, out, M, N, K, M, stream);
+}
+
+extern "C" int m2_dense_to_channels_rows_fwd(const void* x, const void* w, void* out, long out_row, int M, int N, int K, void* stream) {
+  return dense_to_channels("m2_dense_to_channels_rows_fwd", x, w, out, M, N, K, out_row, stream);
+}
+
+// Rows a multiple of 16 KB apart put everything that the weight-stationary kernel stores at a time into one or few of an XCD's 16 L2
+// channels; a line more between them spreads it.  us without / with: M = 32768 130 / 96, 24576 90 / 78, 16384 50.1 / 48.8, 8192 30.4 / 29.8;
+// other strides gain nothing (31744 93 / 95, 28672 87 / 87, 20480 60 / 59).
+extern "C" long m2_dense_channels_row(int M, int N, int K) {
+  return dense_ws_serves(M, N, K) && M % 8192 == 0 ? M + 64l : (long)M;
 }
 
 extern "C" int m2_dense_from_channels_fwd(const void* x, const void* w, const float* bias, void* out, int M, int N, int K,

@@ -14,13 +14,15 @@ using namespace m2;
 
 namespace {
 struct Layout {
+  long xrow;      // elements between two channels of xproj
   size_t xproj, y, a, g, s, h16, hT, total;
 };
 Layout layout(long M, long d, long I) {
   auto up = [](size_t v) { return (v + 255) & ~(size_t)255; };
   Layout l;
+  l.xrow = m2_dense_channels_row((int)M, (int)(3 * d), (int)d);
   l.xproj = 0;
-  l.y = up(l.xproj + (size_t)(3 * d * M) * 2);
+  l.y = up(l.xproj + (size_t)(3 * d * l.xrow) * 2);
   l.a = up(l.y + (size_t)(d * M) * 2);
   l.g = up(l.a + (size_t)(d * M) * 2);
   l.s = up(l.g + (size_t)(I * M) * 2);
@@ -58,10 +60,10 @@ extern "C" int m2_encoder_layers_fwd(const m2_layer_params* layers, int nlayers,
   const size_t spec_stride = m2_filter_spectrum_bytes(d, L) / sizeof(float);
   for (int i = 0; i < nlayers; ++i) {
     const m2_layer_params& p = layers[i];
-    int rc = m2_dense_to_channels_fwd(h16, p.in_w, xproj, M, 3 * d, d, stream);
+    int rc = m2_dense_to_channels_rows_fwd(h16, p.in_w, xproj, l.xrow, M, 3 * d, d, stream);
     if (rc) return rc;
-    rc = m2_mixer_core_fwd(xproj, p.in_b, p.residual ? h_channel_major : nullptr, p.short_w, p.short_b, spectra + i * spec_stride, y, B, L, d,
-                           M2_DTYPE_BF16, stream);
+    rc = m2_mixer_core_rows_fwd(xproj, l.xrow, p.in_b, p.residual ? h_channel_major : nullptr, p.short_w, p.short_b, spectra + i * spec_stride,
+                                y, B, L, d, M2_DTYPE_BF16, stream);
     if (rc) return rc;
     rc = m2_dense_from_channels_fwd(y, p.out_w, p.out_b, a, M, d, d, stream);
     if (rc) return rc;

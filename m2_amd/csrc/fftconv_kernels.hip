@@ -66,6 +66,7 @@ struct PairLayout {
 template <class P, typename ACT, bool FULL>
 __global__ __launch_bounds__(PairLayout<P>::WG) __attribute__((amdgpu_waves_per_eu(P::E == 16 ? 3 : 2, P::E == 16 ? 3 : 2))) void mixer_pair_kernel(
     const ACT* __restrict__ xproj,      // (3d, B, L): x1 | x2 | v, channel-major
+    long ldx,                           // elements between two channels of xproj, B L or more
     const float* __restrict__ uin,      // (d, B, L)   layer input, channel-major (may be null)
     const float* __restrict__ sw,       // (3d, 3)     short-conv taps
     const float* __restrict__ sb,       // (3d)        short-conv bias
@@ -117,11 +118,11 @@ __global__ __launch_bounds__(PairLayout<P>::WG) __attribute__((amdgpu_waves_per_
       constexpr int q = decltype(qq)::value;
       const int n = n0 + 8 * q;
       if constexpr (FULL) {
-        r1.template fetch<q>(xproj + ((long)(0 * d + c) * B + b) * L, n);
-        rv.template fetch<q>(xproj + ((long)(2 * d + c) * B + b) * L, n);
-        r2.template fetch<q>(xproj + ((long)(1 * d + c) * B + b) * L, n);
+        r1.template fetch<q>(xproj + (long)(0 * d + c) * ldx + (long)b * L, n);
+        rv.template fetch<q>(xproj + (long)(2 * d + c) * ldx + (long)b * L, n);
+        r2.template fetch<q>(xproj + (long)(1 * d + c) * ldx + (long)b * L, n);
       } else {
-        r1.template fetch<q>(xproj + ((long)c * B + b) * L, n);
+        r1.template fetch<q>(xproj + (long)c * ldx + (long)b * L, n);
       }
       if (uin) {
         const float* pu = uin + ((long)c * B + b) * L + n;
@@ -318,7 +319,7 @@ __global__ __launch_bounds__(SpectrumLayout<P>::WG) __attribute__((amdgpu_waves_
 // host-side dispatch
 // ------------------------------------------------------------------------------------------
 template <class P, typename ACT>
-static int launch_mixer_pair(const void* xproj, const float* u, const float* sw, const float* sb, const float* pbias,
+static int launch_mixer_pair(const void* xproj, long ldx, const float* u, const float* sw, const float* sb, const float* pbias,
                              const float* spec, void* y, int B, int d, hipStream_t stream) {
   typedef PairLayout<P> Lay;
   auto kern = sw ? mixer_pair_kernel<P, ACT, true> : mixer_pair_kernel<P, ACT, false>;
@@ -344,7 +345,7 @@ static int launch_mixer_pair(const void* xproj, const float* u, const float* sw,
   // every workgroup the same number of row batches: the fewest workgroups that need no extra round
   const int rounds = (slots_needed + slots - 1) / slots;
   slots = (slots_needed + rounds - 1) / rounds;
-  hipLaunchKernelGGL(kern, dim3(8 * slots), dim3(Lay::WG), Lay::lds_bytes, stream, (const ACT*)xproj, u, sw, sb, pbias,
+  hipLaunchKernelGGL(kern, dim3(8 * slots), dim3(Lay::WG), Lay::lds_bytes, stream, (const ACT*)xproj, ldx, u, sw, sb, pbias,
                      (const float4*)spec, (ACT*)y, B, d);
   return check_launch("mixer_pair");
 }
@@ -366,13 +367,13 @@ static int launch_filter_spectrum(const float* taps1, const float* taps2, const 
 }
 
 // L = 32768 (two half transforms of 16384 points per signal), defined in fftconv_real_kernels.hip
-int launch_mixer_real_dispatch(const void* xproj, const float* u, const float* sw, const float* sb, const float* pbias,
+int launch_mixer_real_dispatch(const void* xproj, long ldx, const float* u, const float* sw, const float* sb, const float* pbias,
                                const float* spec, void* y, int B, int d, int act_dtype, hipStream_t stream);
 int launch_filter_spectrum_real(const float* taps1, const float* taps2, const float* D1, const float* D2, float* spec,
                                 int d, const SpectrumBatch& sb, int nmixers, hipStream_t stream);
 
 // L = 8192 and 16384, one signal after the other: defined in fftconv_long_kernels.hip
-int launch_mixer_long_dispatch(const void* xproj, const float* u, const float* sw, const float* sb, const float* pbias,
+int launch_mixer_long_dispatch(const void* xproj, long ldx, const float* u, const float* sw, const float* sb, const float* pbias,
                                const float* spec, void* y, int B, int L, int d, int act_dtype, hipStream_t stream);
 
 // One mixer given by pointers (sb.taps null, nmixers 1) or a batch of mixers described by `sb`.
@@ -388,17 +389,17 @@ int launch_filter_spectrum_any(const float* taps1, const float* taps2, const flo
 }
 
 // sw null: plain convolution of a (d, B, L) input
-static int launch_mixer_any(const void* xproj, const float* u, const float* sw, const float* sb, const float* pbias,
+static int launch_mixer_any(const void* xproj, long ldx, const float* u, const float* sw, const float* sb, const float* pbias,
                             const float* spec, void* y, int B, int L, int d, int act_dtype, hipStream_t s) {
   // L = 8192: with both signals at once a compute unit holds one row, one after the other it holds two and each row takes 1.87 times as
   // long, their barriers hidden behind each other (B = 4: 172 us against 184).  Which of the two leaves fewer units idle in its
   // last round decides where that is more than they differ by (B = 1, d = 768, three rows per unit: 47 us against 56).
   const long rows = (long)d * B, cus = num_cus();
   const bool one_by_one = L == 8192 && (rows + cus - 1) / cus * 100 * cus > 93 * ((rows + 2 * cus - 1) / (2 * cus) * 2 * cus);
-  if (L == 16384 || one_by_one) return launch_mixer_long_dispatch(xproj, u, sw, sb, pbias, spec, y, B, L, d, act_dtype, s);
+  if (L == 16384 || one_by_one) return launch_mixer_long_dispatch(xproj, ldx, u, sw, sb, pbias, spec, y, B, L, d, act_dtype, s);
   switch (L) {
-    case 32768: return launch_mixer_real_dispatch(xproj, u, sw, sb, pbias, spec, y, B, d, act_dtype, s);
-#define X(LEN)                                                                                                     case LEN:                                                                                                          return act_dtype == M2_DTYPE_F32 ? launch_mixer_pair<Twist##LEN, float>(xproj, u, sw, sb, pbias, spec, y, B, d, s)                                      : launch_mixer_pair<Twist##LEN, uint16_t>(xproj, u, sw, sb, pbias, spec, y, B, d, s);
+    case 32768: return launch_mixer_real_dispatch(xproj, ldx, u, sw, sb, pbias, spec, y, B, d, act_dtype, s);
+#define X(LEN)                                                                                                     case LEN:                                                                                                          return act_dtype == M2_DTYPE_F32 ? launch_mixer_pair<Twist##LEN, float>(xproj, ldx, u, sw, sb, pbias, spec, y, B, d, s)                                      : launch_mixer_pair<Twist##LEN, uint16_t>(xproj, ldx, u, sw, sb, pbias, spec, y, B, d, s);
     M2_FOR_EACH_PAIR_LENGTH(X)
 #undef X
   }
@@ -427,17 +428,30 @@ extern "C" int m2_filter_spectrum_fwd(const float* taps1, const float* taps2, co
   return launch_filter_spectrum_any(taps1, taps2, D1, D2, spec, d, L, none, 1, (hipStream_t)stream);
 }
 
+static int mixer_core(const char* who, const void* xproj, long ldx, const float* proj_bias, const float* u, const float* short_w,
+                                 const float* short_b, const float* spec, void* y, int B, int L, int d, int act_dtype,
+                                 void* stream) {
+  if (!xproj || !short_w || !short_b || !spec || !y) return set_error(M2_ERR_ARG, "%s: null pointer", who);
+  if (B <= 0 || d <= 0 || d % 8 != 0) return set_error(M2_ERR_ARG, "%s: need B > 0 and d a positive multiple of 8 (B=%d d=%d)", who, B, d);
+  if ((long)B * 3 * d > 0x7fffffffL) return set_error(M2_ERR_UNSUPPORTED, "%s: B * 3 d = %ld rows do not fit an int", who, (long)B * 3 * d);
+  if (act_dtype != M2_DTYPE_F32 && act_dtype != M2_DTYPE_BF16)
+    return set_error(M2_ERR_ARG, "%s: act_dtype %d is neither M2_DTYPE_F32 nor M2_DTYPE_BF16", who, act_dtype);
+  if (!m2_fftconv_supported_seqlen(L))
+    return set_error(M2_ERR_UNSUPPORTED, "%s: L=%d unsupported (need L a power of two in [128, 32768])", who, L);
+  if (ldx < (long)B * L || ldx % 8) return set_error(M2_ERR_ARG, "%s: rows of xproj %ld apart, need a multiple of 8 from B * L = %ld on", who, ldx, (long)B * L);
+  return launch_mixer_any(xproj, ldx, u, short_w, short_b, proj_bias, spec, y, B, L, d, act_dtype, (hipStream_t)stream);
+}
+
 extern "C" int m2_mixer_core_fwd(const void* xproj, const float* proj_bias, const float* u, const float* short_w,
                                  const float* short_b, const float* spec, void* y, int B, int L, int d, int act_dtype,
                                  void* stream) {
-  if (!xproj || !short_w || !short_b || !spec || !y) return set_error(M2_ERR_ARG, "m2_mixer_core_fwd: null pointer");
-  if (B <= 0 || d <= 0 || d % 8 != 0) return set_error(M2_ERR_ARG, "m2_mixer_core_fwd: need B > 0 and d a positive multiple of 8 (B=%d d=%d)", B, d);
-  if ((long)B * 3 * d > 0x7fffffffL) return set_error(M2_ERR_UNSUPPORTED, "m2_mixer_core_fwd: B * 3 d = %ld rows do not fit an int", (long)B * 3 * d);
-  if (act_dtype != M2_DTYPE_F32 && act_dtype != M2_DTYPE_BF16)
-    return set_error(M2_ERR_ARG, "m2_mixer_core_fwd: act_dtype %d is neither M2_DTYPE_F32 nor M2_DTYPE_BF16", act_dtype);
-  if (!m2_fftconv_supported_seqlen(L))
-    return set_error(M2_ERR_UNSUPPORTED, "m2_mixer_core_fwd: L=%d unsupported (need L a power of two in [128, 32768])", L);
-  return launch_mixer_any(xproj, u, short_w, short_b, proj_bias, spec, y, B, L, d, act_dtype, (hipStream_t)stream);
+  return mixer_core("m2_mixer_core_fwd", xproj, (long)B * L, proj_bias, u, short_w, short_b, spec, y, B, L, d, act_dtype, stream);
+}
+
+extern "C" int m2_mixer_core_rows_fwd(const void* xproj, long xproj_row, const float* proj_bias, const float* u, const float* short_w,
+                                      const float* short_b, const float* spec, void* y, int B, int L, int d, int act_dtype,
+                                      void* stream) {
+  return mixer_core("m2_mixer_core_rows_fwd", xproj, xproj_row, proj_bias, u, short_w, short_b, spec, y, B, L, d, act_dtype, stream);
 }
 
 extern "C" int m2_fftconv_fwd(const void* x, const float* spec, void* y, int B, int L, int d, int act_dtype,
@@ -449,5 +463,5 @@ extern "C" int m2_fftconv_fwd(const void* x, const float* spec, void* y, int B, 
     return set_error(M2_ERR_ARG, "m2_fftconv_fwd: act_dtype %d is neither M2_DTYPE_F32 nor M2_DTYPE_BF16", act_dtype);
   if (!m2_fftconv_supported_seqlen(L))
     return set_error(M2_ERR_UNSUPPORTED, "m2_fftconv_fwd: L=%d unsupported (need L a power of two in [128, 32768])", L);
-  return launch_mixer_any(x, nullptr, nullptr, nullptr, nullptr, spec, y, B, L, d, act_dtype, (hipStream_t)stream);
+  return launch_mixer_any(x, (long)B * L, nullptr, nullptr, nullptr, nullptr, spec, y, B, L, d, act_dtype, (hipStream_t)stream);
 }

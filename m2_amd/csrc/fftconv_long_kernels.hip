@@ -27,6 +27,7 @@ static_assert(twist_offsets_ok<Twist8192>() && twist_offsets_ok<Twist16384>(), "
 template <class P, typename ACT, bool FULL, bool HAS_U>
 __global__ __launch_bounds__(P::T) __attribute__((amdgpu_waves_per_eu(2, 2))) void mixer_long_kernel(
     const ACT* __restrict__ xproj,      // (3d, B, L): x1 | x2 | v, channel-major
+    long ldx,                           // elements between two channels of xproj, B L or more
     const float* __restrict__ uin,      // (d, B, L)   layer input, channel-major (may be null)
     const float* __restrict__ sw,       // (3d, 3)     short-conv taps; null = plain convolution of a (d, B, L) input
     const float* __restrict__ sb,       // (3d)        short-conv bias
@@ -65,11 +66,11 @@ __global__ __launch_bounds__(P::T) __attribute__((amdgpu_waves_per_eu(2, 2))) vo
       constexpr int q = decltype(qq)::value;
       const int n = n0 + 8 * q;
       if constexpr (FULL) {
-        r1.template fetch<q>(xproj + ((long)(0 * d + c) * B + bb) * L, n);
-        rv.template fetch<q>(xproj + ((long)(2 * d + c) * B + bb) * L, n);
-        r2.template fetch<q>(xproj + ((long)(1 * d + c) * B + bb) * L, n);
+        r1.template fetch<q>(xproj + (long)(0 * d + c) * ldx + (long)bb * L, n);
+        rv.template fetch<q>(xproj + (long)(2 * d + c) * ldx + (long)bb * L, n);
+        r2.template fetch<q>(xproj + (long)(1 * d + c) * ldx + (long)bb * L, n);
       } else {
-        r1.template fetch<q>(xproj + ((long)c * B + bb) * L, n);
+        r1.template fetch<q>(xproj + (long)c * ldx + (long)bb * L, n);
       }
       if constexpr (HAS_U) {
         const float* pu = uin + ((long)c * B + bb) * L + n;
@@ -216,7 +217,7 @@ __global__ __launch_bounds__(P::T) __attribute__((amdgpu_waves_per_eu(2, 2))) vo
 }
 
 template <class P, typename ACT>
-static int launch_mixer_long(const void* xproj, const float* u, const float* sw, const float* sb, const float* pbias,
+static int launch_mixer_long(const void* xproj, long ldx, const float* u, const float* sw, const float* sb, const float* pbias,
                              const float* spec, void* y, int B, int d, hipStream_t stream) {
   const size_t lds_bytes = (size_t)(P::ROW + P::TAB) * sizeof(float2);
   auto kern = sw ? (u ? mixer_long_kernel<P, ACT, true, true> : mixer_long_kernel<P, ACT, true, false>)
@@ -232,20 +233,20 @@ static int launch_mixer_long(const void* xproj, const float* u, const float* sw,
   if (slots > rows_per_xcd) slots = rows_per_xcd;
   const int rounds = (rows_per_xcd + slots - 1) / slots;      // every workgroup the same number of rows
   slots = (rows_per_xcd + rounds - 1) / rounds;
-  hipLaunchKernelGGL(kern, dim3(8 * slots), dim3(P::T), lds_bytes, stream, (const ACT*)xproj, u, sw, sb, pbias,
+  hipLaunchKernelGGL(kern, dim3(8 * slots), dim3(P::T), lds_bytes, stream, (const ACT*)xproj, ldx, u, sw, sb, pbias,
                      (const float4*)spec, (ACT*)y, B, d);
   return check_launch("mixer_long");
 }
 
-int launch_mixer_long_dispatch(const void* xproj, const float* u, const float* sw, const float* sb, const float* pbias,
+int launch_mixer_long_dispatch(const void* xproj, long ldx, const float* u, const float* sw, const float* sb, const float* pbias,
                                const float* spec, void* y, int B, int L, int d, int act_dtype, hipStream_t stream) {
   const bool f32 = act_dtype == M2_DTYPE_F32;
   if (L == 8192)
-    return f32 ? launch_mixer_long<Twist8192, float>(xproj, u, sw, sb, pbias, spec, y, B, d, stream)
-               : launch_mixer_long<Twist8192, uint16_t>(xproj, u, sw, sb, pbias, spec, y, B, d, stream);
+    return f32 ? launch_mixer_long<Twist8192, float>(xproj, ldx, u, sw, sb, pbias, spec, y, B, d, stream)
+               : launch_mixer_long<Twist8192, uint16_t>(xproj, ldx, u, sw, sb, pbias, spec, y, B, d, stream);
   if (L == 16384)
-    return f32 ? launch_mixer_long<Twist16384, float>(xproj, u, sw, sb, pbias, spec, y, B, d, stream)
-               : launch_mixer_long<Twist16384, uint16_t>(xproj, u, sw, sb, pbias, spec, y, B, d, stream);
+    return f32 ? launch_mixer_long<Twist16384, float>(xproj, ldx, u, sw, sb, pbias, spec, y, B, d, stream)
+               : launch_mixer_long<Twist16384, uint16_t>(xproj, ldx, u, sw, sb, pbias, spec, y, B, d, stream);
   return set_error(M2_ERR_UNSUPPORTED, "mixer_long: no plan for L=%d", L);
 }
 

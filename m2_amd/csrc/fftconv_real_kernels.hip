@@ -108,6 +108,7 @@ __device__ __forceinline__ void convolve_halves(float (&lo)[32], float (&hi)[32]
 template <class P, typename ACT, bool FULL, bool HAS_U>
 __global__ __launch_bounds__(P::T) __attribute__((amdgpu_waves_per_eu(2, 2))) void mixer_real_kernel(
     const ACT* __restrict__ xproj,      // (3d, B, LS): x1 | x2 | v, channel-major
+    long ldx,                           // elements between two channels of xproj, B L or more
     const float* __restrict__ uin,      // (d, B, LS)  layer input, channel-major (may be null)
     const float* __restrict__ sw,       // (3d, 3)     short-conv taps
     const float* __restrict__ sb,       // (3d)        short-conv bias
@@ -150,8 +151,8 @@ __global__ __launch_bounds__(P::T) __attribute__((amdgpu_waves_per_eu(2, 2))) vo
     // ---- first signal: a = sc(x1) sc(v)  (or the plain input), convolved with filter 1
     {
       RawRow<ACT, 8, true> r1, rv;
-      const ACT* px = FULL ? xproj + ((long)(0 * d + c) * B + bb) * LS : xproj + ((long)c * B + bb) * LS;
-      const ACT* pv = xproj + ((long)(2 * d + c) * B + bb) * LS;
+      const ACT* px = FULL ? xproj + (long)(0 * d + c) * ldx + (long)bb * LS : xproj + (long)c * ldx + (long)bb * LS;
+      const ACT* pv = xproj + (long)(2 * d + c) * ldx + (long)bb * LS;
       static_for<0, 8>([&](auto qq) {
         constexpr int q = decltype(qq)::value;
         r1.template fetch<q>(px, n0 + 8 * q);
@@ -225,7 +226,7 @@ __global__ __launch_bounds__(P::T) __attribute__((amdgpu_waves_per_eu(2, 2))) vo
     // ---- gate: acc = y1 * sc(x2), by way of the stage
     if constexpr (FULL) {
       RawRow<ACT, 8, true> r2;
-      const ACT* p2 = xproj + ((long)(1 * d + c) * B + bb) * LS;
+      const ACT* p2 = xproj + (long)(1 * d + c) * ldx + (long)bb * LS;
       static_for<0, 8>([&](auto qq) { r2.template fetch<decltype(qq)::value>(p2, n0 + 8 * decltype(qq)::value); });
       float w2[3], pb2 = 0.f;
 #pragma unroll
@@ -367,7 +368,7 @@ __global__ __launch_bounds__(P::T) __attribute__((amdgpu_waves_per_eu(2, 2))) vo
 // host-side launchers
 // ------------------------------------------------------------------------------------------
 template <typename ACT>
-static int launch_mixer_real(const void* xproj, const float* u, const float* sw, const float* sb, const float* pbias,
+static int launch_mixer_real(const void* xproj, long ldx, const float* u, const float* sw, const float* sb, const float* pbias,
                              const float* spec, void* y, int B, int d, hipStream_t stream) {
   typedef RealPlan P;
   const size_t lds_bytes = (size_t)(P::ROW + 2 * P::TAB) * sizeof(float2);
@@ -381,15 +382,15 @@ static int launch_mixer_real(const void* xproj, const float* u, const float* sw,
   if (slots > rows_per_xcd) slots = rows_per_xcd;
   const int rounds = (rows_per_xcd + slots - 1) / slots;      // every workgroup the same number of rows
   slots = (rows_per_xcd + rounds - 1) / rounds;
-  hipLaunchKernelGGL(kern, dim3(8 * slots), dim3(P::T), lds_bytes, stream, (const ACT*)xproj, u, sw, sb, pbias, spec,
+  hipLaunchKernelGGL(kern, dim3(8 * slots), dim3(P::T), lds_bytes, stream, (const ACT*)xproj, ldx, u, sw, sb, pbias, spec,
                      (ACT*)y, B, d);
   return check_launch("mixer_real");
 }
 
-int launch_mixer_real_dispatch(const void* xproj, const float* u, const float* sw, const float* sb, const float* pbias,
+int launch_mixer_real_dispatch(const void* xproj, long ldx, const float* u, const float* sw, const float* sb, const float* pbias,
                                const float* spec, void* y, int B, int d, int act_dtype, hipStream_t stream) {
-  return act_dtype == M2_DTYPE_F32 ? launch_mixer_real<float>(xproj, u, sw, sb, pbias, spec, y, B, d, stream)
-                                   : launch_mixer_real<uint16_t>(xproj, u, sw, sb, pbias, spec, y, B, d, stream);
+  return act_dtype == M2_DTYPE_F32 ? launch_mixer_real<float>(xproj, ldx, u, sw, sb, pbias, spec, y, B, d, stream)
+                                   : launch_mixer_real<uint16_t>(xproj, ldx, u, sw, sb, pbias, spec, y, B, d, stream);
 }
 
 int launch_filter_spectrum_real(const float* taps1, const float* taps2, const float* D1, const float* D2, float* spec,

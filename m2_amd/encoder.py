@@ -290,10 +290,10 @@ class BertLayer(nn.Module):
         d = at.d_model
         if at.hyena_training_additions:      # extra input LayerNorm: needs the fp32 form, replaces h16 / hT
             _, h16, hT = at.pre_norm(h32, want_f32=False, want_bf16=True)
-        xproj = at.project_in(h16)                   # (3d, M) channel-major, bias added in the core
+        xproj = at.projected(h16, B, L)              # channel-major, bias added in the core
         if spec_ready is not None:
             torch.cuda.current_stream().wait_event(spec_ready)
-        y = at.core(xproj.view(3 * d, B, L), hT.view(d, B, L) if at.residual_long_conv else None, B, L, spec=spec)
+        y = at.core(xproj, hT.view(d, B, L) if at.residual_long_conv else None, B, L, spec=spec)
         if after_core is not None:
             after_core()
         a16 = at.project_out(y.view(d, B * L))                                       # (M, d)

@@ -121,13 +121,15 @@ class MonarchMixerSequenceMixing(nn.Module):
     def core(self, xproj: torch.Tensor, u_cm: Optional[torch.Tensor], B: int, L: int,
              spec: Optional[torch.Tensor] = None) -> torch.Tensor:
         """Channel-major core: xproj (3d, B, L) = in_linear.weight @ u^T WITHOUT the bias (the kernel adds
-        in_linear.bias as it loads), u_cm (d, B, L) fp32 -> y (d, B, L)."""
+        in_linear.bias as it loads), u_cm (d, B, L) fp32 -> y (d, B, L).  xproj may also be (3d, row), row >= B L, the values of a
+        channel at the start of its row."""
         if spec is None:
             spec = self.filter_spectrum(L)
         sw = self._cast("short_w", self.short_filter.weight, torch.float32).view(3 * self.d_model, 3)
         sb = self._cast("short_b", self.short_filter.bias, torch.float32)
         pb = self._cast("in_b32", self.in_linear.bias, torch.float32)
-        return ops.mixer_core(xproj, u_cm, sw, sb, spec, B, L, self.d_model, proj_bias=pb)
+        row = xproj.shape[1] if xproj.dim() == 2 else None
+        return ops.mixer_core(xproj, u_cm, sw, sb, spec, B, L, self.d_model, proj_bias=pb, row=row)
 
     def pre_norm(self, h32: torch.Tensor, want_f32: bool, want_bf16: bool):
         """The extra input LayerNorm of hyena_training_additions: (M, d) fp32 -> (f32 | None, bf16 | None,
@@ -136,13 +138,22 @@ class MonarchMixerSequenceMixing(nn.Module):
         return ops.layernorm(h32, ln.weight.detach().float(), ln.bias.detach().float(), ln.eps, want_f32=want_f32,
                              want_bf16=want_bf16, want_channel_major=self.residual_long_conv)
 
-    def project_in(self, x: torch.Tensor) -> torch.Tensor:
-        """x (M, d) -> in_linear.weight @ x^T without the bias, (3d, M) channel-major, in x's dtype (bf16 or fp32)."""
+    def projected(self, x: torch.Tensor, B: int, L: int) -> torch.Tensor:
+        """project_in as the core takes it: (3d, B, L), or (3d, row) where a row a little longer than B L is faster to write.  (A class
+        of a caller's own may have a core or a projection that knows no such rows.)"""
+        M, d = x.shape
+        if type(self) is MonarchMixerSequenceMixing and x.dtype == torch.bfloat16 and ops.channels_row(M, d) != M:
+            return self.project_in(x, wide=True)
+        return self.project_in(x).view(3 * d, B, L)
+
+    def project_in(self, x: torch.Tensor, wide: bool = False) -> torch.Tensor:
+        """x (M, d) -> in_linear.weight @ x^T without the bias, (3d, M) channel-major, in x's dtype (bf16 or fp32).  wide: (3d, row),
+        the M values of a channel at the start of its row, where ops.channels_row says that this is faster."""
         M, d = x.shape
         w = self._cast("in_w", self.in_linear.weight, x.dtype)
         own = not (x.requires_grad and torch.is_grad_enabled())          # (the library call refuses those)
         if own and x.dtype == torch.bfloat16 and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0 and ops.own_to_channels(M, d):
-            return ops.dense_to_channels(x, w)
+            return ops.dense_to_channels(x, w, ops.channels_row(M, d) if wide else None)
         # Written as x @ W^T into the transposed view of the output: the same product as W @ x^T, for which the library
         # picks a faster kernel (126 against 144 us at M = 32768, d = 768)
         out = torch.empty(3 * d, M, dtype=x.dtype, device=x.device)
@@ -194,14 +205,14 @@ class MonarchMixerSequenceMixing(nn.Module):
             weights = None if low or (x.requires_grad and torch.is_grad_enabled()) else self._fp32_parts(B * L)
             if weights is not None:
                 parts, x_cm, w_in, w_out = ops.split_rows(x, channel_major=u_cm is None and self.residual_long_conv, weights=weights)
-                xproj = ops.split_to_channels(parts, w_in, B * L, 3 * d, d)
+                xproj = ops.split_to_channels(parts, w_in, B * L, 3 * d, d).view(3 * d, B, L)
                 u_cm = x_cm if u_cm is None else u_cm
             else:
-                xproj = self.project_in(x)                                               # (3d, B*L), bias added in the core
+                xproj = self.projected(x, B, L)                                          # (3d, B, L), bias added in the core
             if u_cm is None and self.residual_long_conv:
                 u_cm = u2.float().t().contiguous()                                       # (d, B*L)
             if not self.residual_long_conv:
                 u_cm = None
-            y = self.core(xproj.view(3 * d, B, L), None if u_cm is None else u_cm.view(d, B, L), B, L)
+            y = self.core(xproj, None if u_cm is None else u_cm.view(d, B, L), B, L)
             out = self.project_out(y.view(d, B * L), w_out)                             # (B*L, d)
         return out.view(B, L, d), None

@@ -257,10 +257,11 @@ def filter_spectrum(taps1: Tensor, taps2: Optional[Tensor], D1: Optional[Tensor]
 
 
 def mixer_core(xproj: Tensor, u: Optional[Tensor], short_w: Tensor, short_b: Tensor, spec: Tensor, B: int, L: int,
-               d: int, out: Optional[Tensor] = None, proj_bias: Optional[Tensor] = None) -> Tensor:
+               d: int, out: Optional[Tensor] = None, proj_bias: Optional[Tensor] = None, row: Optional[int] = None) -> Tensor:
     """y (d, B, L) from the channel-major in-projection (3d, B, L) and layer input (d, B, L).
-    `proj_bias` (3d) fp32 is added to xproj on load (pass the in_linear bias when the GEMM ran without it)."""
-    _require(xproj, "xproj", None, (3 * d, B, L))
+    `proj_bias` (3d) fp32 is added to xproj on load (pass the in_linear bias when the GEMM ran without it).
+    `row`: xproj is (3d, row), the B L values of a channel at the start of its row."""
+    _require(xproj, "xproj", None, (3 * d, B, L) if row is None else (3 * d, row))
     code = _act_code(xproj.dtype)
     if proj_bias is not None:
         _require(proj_bias, "proj_bias", torch.float32, (3 * d,))
@@ -273,8 +274,8 @@ def mixer_core(xproj: Tensor, u: Optional[Tensor], short_w: Tensor, short_b: Ten
         out = torch.empty(d, B, L, dtype=xproj.dtype, device=xproj.device)
     else:
         _require(out, "out", xproj.dtype, (d, B, L))
-    check(lib.m2_mixer_core_fwd(_ptr(xproj), _ptr(proj_bias), _ptr(u), _ptr(short_w), _ptr(short_b), _ptr(spec),
-                                _ptr(out), B, L, d, code, _stream()))
+    check(lib.m2_mixer_core_rows_fwd(_ptr(xproj), B * L if row is None else row, _ptr(proj_bias), _ptr(u), _ptr(short_w),
+                                     _ptr(short_b), _ptr(spec), _ptr(out), B, L, d, code, _stream()))
     return out
 
 
@@ -316,14 +317,21 @@ def own_from_channels(M: int, d: int) -> bool:
     return (d <= 1024 or 6.0 * M * d * d <= _OWN_DENSE_FLOPS) and bool(lib.m2_dense_supported(M, d, d))
 
 
-def dense_to_channels(x: Tensor, w: Tensor) -> Tensor:
-    """w @ x^T: x (M, K) bf16, w (N, K) bf16 -> (N, M) bf16, fp32 accumulation."""
+def channels_row(M: int, d: int) -> int:
+    """The distance between two channels of in_linear's output at which writing it is fastest: M, or a line more."""
+    return lib.m2_dense_channels_row(M, 3 * d, d)
+
+
+def dense_to_channels(x: Tensor, w: Tensor, row: Optional[int] = None) -> Tensor:
+    """w @ x^T: x (M, K) bf16, w (N, K) bf16 -> (N, M) bf16, fp32 accumulation.  `row`: (N, row), whose columns from M on are left as
+    they are."""
     M, K = x.shape
     N = w.shape[0]
     _require(x, "x", torch.bfloat16)
     _require(w, "w", torch.bfloat16, (N, K))
-    out = torch.empty(N, M, dtype=torch.bfloat16, device=x.device)
-    check(lib.m2_dense_to_channels_fwd(_ptr(x), _ptr(w), _ptr(out), M, N, K, _stream()))
+    row = M if row is None else row
+    out = torch.empty(N, row, dtype=torch.bfloat16, device=x.device)
+    check(lib.m2_dense_to_channels_rows_fwd(_ptr(x), _ptr(w), _ptr(out), row, M, N, K, _stream()))
     return out
 
 

@@ -52,6 +52,31 @@ def test_dense_weights_in_registers(gpu, M, N):
     _within_bf16(got[:, m].t(), x[m].cpu().double() @ w.cpu().double().T, x[m].cpu().double().abs() @ w.cpu().double().abs().T)
 
 
+def test_channels_with_a_gap_between_them(gpu):
+    """The projection into rows further apart than their values, and the core reading such rows: bit for bit those of dense rows, on
+    each of the core's kernels and both kernels of the projection."""
+    from m2_amd import ops
+    g = torch.Generator(device=gpu).manual_seed(3)
+    assert ops.channels_row(32768, 768) == 32832 and ops.channels_row(16376, 768) == 16376 and ops.channels_row(8192, 960) == 8192
+    for L, B, d in ((128, 2, 768), (2048, 4, 768), (4096, 1, 64), (8192, 1, 768), (16384, 2, 64), (32768, 1, 8)):
+        M, row = B * L, B * L + 72
+        x, w = (torch.randn(n, 768, generator=g, device=gpu).bfloat16() for n in (M, 3 * d))
+        dense = ops.dense_to_channels(x, w)
+        wide = ops.dense_to_channels(x, w, row)
+        assert wide.shape == (3 * d, row) and torch.equal(wide[:, :M], dense)
+        sw, sb, pb = (torch.randn(3 * d, *s, generator=g, device=gpu) for s in ((3,), (), ()))
+        u = torch.randn(d, B, L, generator=g, device=gpu)
+        spec = ops.filter_spectrum(*(torch.randn(d, 2 * L, generator=g, device=gpu) * 0.02 for _ in range(2)), None, None)
+        gap = wide.clone()
+        gap[:, M:] = float("nan")
+        for dt in (torch.bfloat16, torch.float32):
+            want = ops.mixer_core(dense.to(dt).view(3 * d, B, L), u, sw, sb, spec, B, L, d, proj_bias=pb)
+            got = ops.mixer_core(gap.to(dt), u, sw, sb, spec, B, L, d, proj_bias=pb, row=row)
+            assert torch.equal(got, want), (L, dt)
+    with pytest.raises(RuntimeError, match="multiple of 8"):
+        ops.dense_to_channels(x, w, 32769)
+
+
 def test_dense_unsupported_sizes_are_refused(gpu):
     from m2_amd import ops
     for M, N, K in ((12, 64, 64), (64, 20, 64), (64, 64, 96)):
