@@ -446,8 +446,8 @@ def main():
                         "ms_per_step_median": ms, "ms_per_step_max": reps[-1] / args.steps * 1e3,
                         "timed_seconds_total": sum(reps)},
         "tokens_per_ms": B * L / ms,
-        "roofline": {"kernel": ("mixer_real_kernel" if L == 32768 else "mixer_split_kernel" if L >= 2048
-                                else "mixer_core_kernel") + " (short conv + gates + two FFT long convs + add)"
+        "roofline": {"kernel": ("mixer_real_kernel" if L == 32768 else "mixer_long_kernel" if L >= 8192
+                                else "mixer_pair_kernel") + " (short conv + gates + two FFT long convs + add)"
                                " with the filter-generation kernels of the layer",
                      "bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBPS, "unit": "GB/s",
                      "frac": achieved / HBM_PEAK_GBPS,
