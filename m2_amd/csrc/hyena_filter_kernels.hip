@@ -47,7 +47,7 @@ __device__ __forceinline__ float sin_reduced(float x) {
 // that hidden_kernel fetches them with coalesced 16-byte loads and no arithmetic:
 // wsplit[mlp][layer][part][wave w][K step ks][lane (i, h)] = 8 fp16 of row 32 w + i, K = 16 ks + 8 h .. + 7, and behind the parts the
 // reciprocal 2^-(e + 13) of each row's scale and the activations'.
-// The d x 128 output projection likewise, for project_kernel:
+// The d x 128 output projection likewise, for the hidden kernel that goes on to project:
 // w3split[mlp][part][32-channel tile][K step ks][lane (i, h)] = 8 fp16 of row 32 tile + i, K = 16 ks + 8 h .. + 7, then d reciprocals.
 // A workgroup of 512 threads takes the 32 rows of one (mlp, layer, wave) or one (mlp, tile).
 constexpr int kSplitPerLayer = 2 * kOrder * kOrder + 2 * kOrder;      // fp16-sized elements per (mlp, layer)
@@ -350,8 +350,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   }
 }
 
-// Workgroup = 4 waves = 128 channels; wave w owns channels [c0 + 32 w, + 32) with its weight rows split
-// in fp16 hi / lo parts held in registers.  The workgroup walks kPosPerWg positions in tiles of 32:
+// Workgroup = 4 waves = 128 channels; wave w owns channels [c0 + 32 w, + 32) and splits its weight rows itself into fp16 hi / lo
+// parts, which stay in registers.  The channels' decay rates and scales do not (with both in registers 34 of them went to scratch and
+// back for every tile): they are read from LDS where they are used.  The workgroup walks kPosPerWg positions in tiles of 32:
 // the h3 tile (hi and lo parts, 16 KB) is fetched with coalesced 16-byte loads one tile ahead, staged in
 // LDS (double buffered, rows padded to 272 bytes so that the 16-byte operand reads of 32 rows spread over
 // all banks) and shared by the four waves.
@@ -361,9 +362,9 @@ constexpr int kHRow = 2 * kOrder + 16;   // bytes per padded LDS row of one h3 p
 template <class TAB>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 4))) void project_kernel(TAB tab, int L, int d, float shift,
                                                       const uint16_t* __restrict__ h_hi, const uint16_t* __restrict__ h_lo,
-                                                      const uint16_t* __restrict__ w3split,
                                                       float* __restrict__ taps /* (nf, d, 2L) */) {
   __shared__ __attribute__((aligned(16))) unsigned char hbuf[2][2][32 * kHRow];     // [buffer][hi, lo][row]
+  __shared__ float4 rate[4][8], back[4][8];        // of a wave's 32 channels: -|delta| log2(e), reciprocal scale
   const int fi = blockIdx.z >> 1, dir = blockIdx.z & 1;
   const FilterPtrs& F = tab.at(fi);
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, i32 = lane & 31, half = lane >> 5;
@@ -406,23 +407,33 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 4))) voi
   fetch(0, ic<0>{});
   if (ntiles > 1) fetch(1, ic<1>{});
 
-  // A operand: rows c0 + i32, K = 16 ks + 8 half + {0..7}, hi / lo parts as split_weights_kernel laid them out
+  // A operand: rows c0 + i32, K = 16 ks + 8 half + {0..7}, read once for the scale and once for the parts
   f16x8 ahi[kOrder / 16], alo[kOrder / 16];
-  float adelta[16], rs[16];
   if (active) {
-    const uint16_t* w3 = w3split + blockIdx.z * w3_split_elems(d);
-    const u32x4* wp = reinterpret_cast<const u32x4*>(w3) + (c0 / 32) * 8 * 64 + lane;
-    const float* scales = reinterpret_cast<const float*>(w3 + 2l * d * kOrder);
+    const float* row = F.mlp[dir].w3 + (long)(c0 + i32) * kOrder + 8 * half;
+    float top = 0.f;
+#pragma unroll 2
+    for (int ks = 0; ks < kOrder / 16; ++ks)
+#pragma unroll
+      for (int j = 0; j < 8; ++j) top = fmaxf(top, fabsf(row[16 * ks + j]));
+    top = fmaxf(top, __shfl_xor(top, 32));
+    const float scale = row_scale(top);
 #pragma unroll
     for (int ks = 0; ks < kOrder / 16; ++ks) {
-      ahi[ks] = __builtin_bit_cast(f16x8, wp[ks * 64]);
-      alo[ks] = __builtin_bit_cast(f16x8, wp[ks * 64 + d * kOrder / 8]);
-    }
+      u32x4 vh, vl;
 #pragma unroll
-    for (int v = 0; v < 16; ++v) {
-      const int c = c0 + 8 * (v >> 2) + 4 * half + (v & 3);
-      adelta[v] = -fabsf(F.deltas[c]) * 1.44269504088896341f;
-      rs[v] = scales[c];
+      for (int j = 0; j < 4; ++j) {
+        uint32_t h, l;
+        split2(row[16 * ks + 2 * j] * scale, row[16 * ks + 2 * j + 1] * scale, h, l);
+        vh[j] = h;
+        vl[j] = l;
+      }
+      ahi[ks] = __builtin_bit_cast(f16x8, vh);
+      alo[ks] = __builtin_bit_cast(f16x8, vl);
+    }
+    if (half == 0) {
+      reinterpret_cast<float*>(rate[wave])[i32] = -fabsf(F.deltas[c0 + i32]) * 1.44269504088896341f;
+      reinterpret_cast<float*>(back[wave])[i32] = 1.f / (scale * kActScale);
     }
   }
   stage(0, ic<0>{});
@@ -452,12 +463,17 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 4))) voi
       const float tl = F.t[l];
       float* po = out + (long)(c0 + 4 * half) * 2 * L + (dir == 0 ? l : (2L * L - 1 - l));
 #pragma unroll
-      for (int v = 0; v < 16; ++v) {
-        // (exp(-t |delta|) + shift) r, r the reciprocal scale of the channel; the bare hardware exp2 flushes results below 2^-126
-        // to zero, which is the value to 1e-38 absolute
-        const float decay = fmaf(__builtin_amdgcn_exp2f(tl * adelta[v]), rs[v], shift * rs[v]);
-        // streaming store: the taps (100 MB per mixer at L = 8192) are read once, by a later kernel (-5 % for the call)
-        __builtin_nontemporal_store(acc[v] * decay, po + (long)(8 * (v >> 2) + (v & 3)) * 2 * L);
+      for (int vq = 0; vq < 4; ++vq) {
+        const float4 dq = rate[wave][2 * vq + half], rq = back[wave][2 * vq + half];
+        const float adelta[4] = {dq.x, dq.y, dq.z, dq.w}, rs[4] = {rq.x, rq.y, rq.z, rq.w};
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          // (exp(-t |delta|) + shift) r, r the reciprocal scale of the channel; the bare hardware exp2 flushes results below 2^-126
+          // to zero, which is the value to 1e-38 absolute
+          const float decay = fmaf(__builtin_amdgcn_exp2f(tl * adelta[j]), rs[j], shift * rs[j]);
+          // streaming store: the taps (100 MB per mixer at L = 8192) are read once, by a later kernel (-5 % for the call)
+          __builtin_nontemporal_store(acc[4 * vq + j] * decay, po + (long)(8 * vq + j) * 2 * L);
+        }
       }
     }
     if (pt + 1 < ntiles) stage(P ^ 1, ic<P ^ 1>{});
@@ -483,13 +499,14 @@ extern "C" size_t m2_hyena_filter_workspace_bytes(int nfilters, int L, int d, in
          (size_t)2 * nfilters * 2 * d * order * sizeof(uint16_t);
 }
 
-// The three launches of a batch of filters (weight re-split, hidden layers, projection + decay), the table coming
+// The two or three launches of a batch of filters (weight re-split, hidden layers, projection + decay), the table coming
 // either by value or from device memory.  `w3split` / `taps` null: the projection is left to the caller (the fused
-// projection + spectrum kernel of short sequences, which splits the projection weights itself).
+// projection + spectrum kernel of short sequences).  Kernels that keep a projection's weights in registers split them themselves.
 template <class TAB>
 static int filter_launches(TAB tab, int nfilters, int L, int d, int emb_dim, float w_mod, float shift, uint16_t* h_hi,
                            uint16_t* h_lo, uint16_t* wsplit, uint16_t* w3split, float* taps, hipStream_t s) {
-  const int split_blocks = 2 * nfilters * 2 * 4 + (w3split ? 2 * nfilters * (d / 32) : 0);
+  const bool one_kernel = taps && L >= 1024 && L % 64 == 0;      // hidden layers and projection
+  const int split_blocks = 2 * nfilters * 2 * 4 + (one_kernel ? 2 * nfilters * (d / 32) : 0);
   hipLaunchKernelGGL(split_weights_kernel<TAB>, dim3(split_blocks), dim3(512), 0, s, tab, 2 * nfilters, d, wsplit, w3split);
   int rc = check_launch("hyena split_weights_kernel");
   if (rc) return rc;
@@ -497,7 +514,7 @@ static int filter_launches(TAB tab, int nfilters, int L, int d, int emb_dim, flo
   // projection), short sequences need the workgroups spread over the chip.  From L = 1024 on hidden layers and projection are one
   // kernel, h3 never leaves the chip; us for hidden layers + projection + spectra of 12 mixers, d = 768, with 128 and with 64
   // positions: L = 1024 158 / 157, 4096 514 / 534, 8192 947 / 994; three bf16 parts and 64 positions: 190 / 587 / 1078.
-  if (taps && L >= 1024 && L % 64 == 0) {
+  if (one_kernel) {
     if (L % 128 == 0)
       hipLaunchKernelGGL((hidden_kernel<4, TAB, true>), dim3(L / 128, 2 * nfilters), dim3(256), 0, s, tab, L, emb_dim, w_mod, wsplit,
                          h_hi, h_lo, d, shift, w3split, taps);
@@ -511,7 +528,7 @@ static int filter_launches(TAB tab, int nfilters, int L, int d, int emb_dim, flo
   rc = check_launch("hyena hidden_kernel");
   if (rc || !taps) return rc;
   hipLaunchKernelGGL(project_kernel<TAB>, dim3((L + kPosPerWg - 1) / kPosPerWg, (d + 127) / 128, 2 * nfilters), dim3(256), 0, s, tab, L, d, shift,
-                     h_hi, h_lo, w3split, taps);
+                     h_hi, h_lo, taps);
   return check_launch("hyena project_kernel");
 }
 
