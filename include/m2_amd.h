@@ -63,7 +63,7 @@ typedef struct m2_hyena_filter_params {
 
 /* Bytes of workspace m2_hyena_filter_fwd needs for `nfilters` filters of length L and width d: the last hidden
  * layer's activations (2 nfilters L order fp32-sized values) and the weights re-split for the matrix cores
- * (2 nfilters x (2 layers x 3 16-bit values x order^2 + 2 16-bit parts x d x order); the room of a third part holds the scales). */
+ * (2 nfilters x (2 layers x 3 bf16 parts x order^2 + 2 fp16 parts x d x order)). */
 size_t m2_hyena_filter_workspace_bytes(int nfilters, int L, int d, int order);
 
 /* taps[f] (d, 2L) fp32, f < nfilters:  taps[f][c][l]      = k_fwd[c][l]       for l < L

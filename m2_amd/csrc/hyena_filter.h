@@ -1,5 +1,5 @@
 // Types shared by the filter-generation translation units (hyena_filter_kernels.hip, filter_fused_kernels.hip):
-// the pointer table of a batch of implicit filters and the helpers that turn fp32 values into fp16 parts for
+// the pointer table of a batch of implicit filters and the helpers that turn fp32 values into bf16 or fp16 parts for
 // the matrix cores.
 #pragma once
 #include <hip/hip_runtime.h>
@@ -42,12 +42,27 @@ typedef float floatx16 __attribute__((ext_vector_type(16)));
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
-// The matrix products of the filter MLPs: either operand as two fp16 parts, x 2^e = hi + lo, three products (hi lo, lo hi, hi hi),
-// fp32 accumulation.  Two parts hold 23 - 24 bits and the product left out is below 2^-24 of the whole one, so a product is good to
-// what fp32 arithmetic gives.  fp16 has five bits of exponent: e scales activations (|h| <= 1) by 2^13 and every row of a weight
-// so that its largest entry lies in [2^12, 2^13), which keeps entries down to 2^-16 of the largest exact to 2^-24 of themselves and
-// all others to 2^-38 of the largest.  (Three bf16 parts and six products, which this took over from, are exact and cost twice the
-// matrix instructions, half as many conversions again and half as many registers for stationary weights again.)
+// The matrix products of the filter MLPs, fp32 accumulation.
+//
+// The two 128 x 128 layers: either operand as three bf16 parts, x = hi + mid + lo, which hold all 24 bits of an fp32 value of any size,
+// and the six products down to 2^-24 of the whole one (mid lo, lo mid and lo lo, below 2^-24, are left out).  What such a layer loses,
+// sin(freq x) of the next one amplifies by its argument.  (Two fp16 parts and three products, as below, save half of the matrix
+// instructions, 5 to 10 % of filter generation, and with operands whose mantissas lie between two numbers of 11 bits they put every
+// argument off by 2.6e-7 of itself where fp32 products leave 0.6e-7.)
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+__device__ __forceinline__ void split3(float x, float& hi, float& mid, float& lo) {
+  hi = bf16_to_f32(f32_to_bf16(x));
+  const float r = x - hi;
+  mid = bf16_to_f32(f32_to_bf16(r));
+  lo = r - mid;                      // the conversion of lo to bf16 happens where it is packed
+}
+
+// The output projection, whose result nothing amplifies: two fp16 parts, x 2^e = hi + lo, three products (hi lo, lo hi, hi hi).  The
+// parts hold a value to 2^-23 of itself and the product left out is at most 2^-22 of the whole one (the error of a product is 2^-21
+// at most and 2^-23.7 in the root mean square).  fp16 has five bits of exponent: every row of the weight is scaled so that its largest
+// entry lies in [2^12, 2^13), activations by 2^13.  What is below 2^-13 of the largest has its low part among fp16's subnormal numbers
+// and is held to 2^-38 of the largest.  Two bf16 parts (16 bits, the same matrix instructions) left the taps at 4e-6 from fp64, these
+// leave them where fp32 arithmetic does, at 2e-7; a third part would double the instructions.
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));

@@ -6,14 +6,14 @@
 // (bert/src/mm/hyena_utils.py:168-175 the MLP, :50-63 Sin, :110-112 modulation, :201-217 filter /
 // filter_rev, :231-236 placement of the forward and the flipped reverse taps in a 2L window.)
 //
-// Three kernels.  `split_weights_kernel` re-splits the weights into two fp16 parts in MFMA operand layout (hyena_filter.h; a few
-// microseconds, once per call).  `hidden_kernel` evaluates the three sin layers for 32 or 128 positions per workgroup: the first
-// (emb -> 128) on the vector ALU, the two 128 x 128 layers as three-product split-fp16 MFMA GEMMs (v_mfma_f32_32x32x16_f16 on the
-// parts of weights and activations: products good to 2^-24, which matters because sin(freq * x) amplifies any rounding of
-// x) with the activations resident in LDS; it writes h3 in the same two parts.  `project_kernel` is the 128 -> d projection, again
-// three products, whose epilogue applies the decay and stores the taps channel-major, forward taps at [0, L) and reverse taps
-// mirrored into [L, 2L).  For L >= 1024 the last two are one launch (`hidden_kernel<4, ., PROJECT = true>`: the
-// workgroup that evaluated the hidden layers of 128 positions goes on to project them, h3 never leaves LDS); for
+// Three kernels.  `split_weights_kernel` re-splits the weights into parts in MFMA operand layout (hyena_filter.h; a few
+// microseconds, once per call).  `hidden_kernel` evaluates the three sin layers for 32 or 64 positions per workgroup: the first
+// (emb -> 128) on the vector ALU, the two 128 x 128 layers as six-product split-bf16 MFMA GEMMs (v_mfma_f32_32x32x16_bf16 on the
+// three parts of weights and activations: fp32 products, which matters because sin(freq * x) amplifies any rounding of
+// x) with the activations resident in LDS; it writes h3 in two fp16 parts.  `project_kernel` is the 128 -> d projection, three
+// products of two fp16 parts, whose epilogue applies the decay and stores the taps channel-major, forward taps at [0, L) and reverse taps
+// mirrored into [L, 2L).  For L >= 1024 the last two are one launch (`hidden_kernel<2, ., PROJECT = true>`: the
+// workgroup that evaluated the hidden layers of 64 positions goes on to project them, h3 never leaves LDS); for
 // L <= 512 the batched entry point hands h3 to the projection + spectrum kernel of filter_fused_kernels.hip instead.
 #include <hip/hip_runtime.h>
 
@@ -43,45 +43,45 @@ __device__ __forceinline__ float sin_reduced(float x) {
   return __uint_as_float(__float_as_uint(s) ^ ((uint32_t)static_cast<int>(n) << 31));      // odd n: the other sign
 }
 
-// The 128 x 128 weights of the two inner layers, split into two fp16 parts and laid out as MFMA A operands, so
+// The 128 x 128 weights of the two inner layers, split into three bf16 parts and laid out as MFMA A operands, so
 // that hidden_kernel fetches them with coalesced 16-byte loads and no arithmetic:
-// wsplit[mlp][layer][part][wave w][K step ks][lane (i, h)] = 8 fp16 of row 32 w + i, K = 16 ks + 8 h .. + 7, and behind the parts the
-// reciprocal 2^-(e + 13) of each row's scale and the activations'.
-// The d x 128 output projection likewise, for the hidden kernel that goes on to project:
-// w3split[mlp][part][32-channel tile][K step ks][lane (i, h)] = 8 fp16 of row 32 tile + i, K = 16 ks + 8 h .. + 7, then d reciprocals.
+// wsplit[mlp][layer][part][wave w][K step ks][lane (i, h)] = 8 bf16 of row 32 w + i, K = 16 ks + 8 h .. + 7.
+// The d x 128 output projection likewise in two fp16 parts, for the hidden kernel that goes on to project, and with it
+// w3scale[mlp][row], the reciprocal 2^-(e + 13) of the row's scale and the activations':
+// w3split[mlp][part][32-channel tile][K step ks][lane (i, h)] = 8 fp16 of row 32 tile + i, K = 16 ks + 8 h .. + 7.
 // A workgroup of 512 threads takes the 32 rows of one (mlp, layer, wave) or one (mlp, tile).
-constexpr int kSplitPerLayer = 2 * kOrder * kOrder + 2 * kOrder;      // fp16-sized elements per (mlp, layer)
-__host__ __device__ constexpr long w3_split_elems(int d) { return 2l * d * kOrder + 2l * d; }      // and per mlp
+constexpr int kSplitPerLayer = 3 * kOrder * kOrder;      // bf16 elements per (mlp, layer)
 template <class TAB>
 __global__ __launch_bounds__(512) void split_weights_kernel(TAB tab, int nmlp, int d, uint16_t* __restrict__ wsplit,
-                                                            uint16_t* __restrict__ w3split) {
-  __shared__ float most[8][32];
+                                                            uint16_t* __restrict__ w3split, float* __restrict__ w3scale) {
   const int inner = nmlp * 2 * 4;
   const int lane = threadIdx.x & 63, i32 = lane & 31, ks = threadIdx.x >> 6;
-  const float* rows;
-  u32x4* dst;
-  float* scales;
-  int part;                                       // 16-byte pieces per part
   if ((int)blockIdx.x < inner) {
     const int w = blockIdx.x & 3, layer = (blockIdx.x >> 2) & 1, m = blockIdx.x >> 3;
     const MlpPtrs& W = tab.at(m >> 1).mlp[m & 1];
     if (W.w0 == nullptr) return;
-    rows = (layer == 0 ? W.w1 : W.w2) + 32l * w * kOrder;
-    uint16_t* out = wsplit + ((long)(m * 2 + layer)) * kSplitPerLayer;
-    dst = reinterpret_cast<u32x4*>(out) + (w * 8 + ks) * 64 + lane;
-    scales = reinterpret_cast<float*>(out + 2 * kOrder * kOrder) + 32 * w;
-    part = kOrder * kOrder / 8;
-  } else {
-    const int ct = ((int)blockIdx.x - inner) % (d / 32), m = ((int)blockIdx.x - inner) / (d / 32);
-    const MlpPtrs& W = tab.at(m >> 1).mlp[m & 1];
-    if (W.w3 == nullptr) return;
-    rows = W.w3 + 32l * ct * kOrder;
-    uint16_t* out = w3split + m * w3_split_elems(d);
-    dst = reinterpret_cast<u32x4*>(out) + (ct * 8 + ks) * 64 + lane;
-    scales = reinterpret_cast<float*>(out + 2l * d * kOrder) + 32 * ct;
-    part = d * kOrder / 8;
+    const float* src = (layer == 0 ? W.w1 : W.w2) + (long)(32 * w + i32) * kOrder + 16 * ks + 8 * (lane >> 5);
+    u32x4 vh, vm, vl;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      float h[2], md[2], l[2];
+      split3(src[2 * j], h[0], md[0], l[0]);
+      split3(src[2 * j + 1], h[1], md[1], l[1]);
+      vh[j] = pack_bf16x2(h[0], h[1]);
+      vm[j] = pack_bf16x2(md[0], md[1]);
+      vl[j] = pack_bf16x2(l[0], l[1]);
+    }
+    u32x4* dst = reinterpret_cast<u32x4*>(wsplit + ((long)(m * 2 + layer)) * kSplitPerLayer) + (w * 8 + ks) * 64 + lane;
+    dst[0] = vh;
+    dst[kOrder * kOrder / 8] = vm;
+    dst[2 * kOrder * kOrder / 8] = vl;
+    return;
   }
-  const float* src = rows + (long)i32 * kOrder + 16 * ks + 8 * (lane >> 5);
+  __shared__ float most[8][32];
+  const int ct = ((int)blockIdx.x - inner) % (d / 32), m = ((int)blockIdx.x - inner) / (d / 32);
+  const MlpPtrs& W = tab.at(m >> 1).mlp[m & 1];
+  if (W.w3 == nullptr) return;
+  const float* src = W.w3 + (long)(32 * ct + i32) * kOrder + 16 * ks + 8 * (lane >> 5);
   float v[8], top = 0.f;
 #pragma unroll
   for (int j = 0; j < 8; ++j) {
@@ -102,22 +102,23 @@ __global__ __launch_bounds__(512) void split_weights_kernel(TAB tab, int nmlp, i
     hi[j] = h;
     lo[j] = l;
   }
+  u32x4* dst = reinterpret_cast<u32x4*>(w3split + (long)m * 2 * d * kOrder) + (ct * 8 + ks) * 64 + lane;
   dst[0] = hi;
-  dst[part] = lo;
-  if (threadIdx.x < 32) scales[threadIdx.x] = 1.f / (scale * kActScale);
+  dst[d * kOrder / 8] = lo;
+  if (threadIdx.x < 32) w3scale[(long)m * d + 32 * ct + threadIdx.x] = 1.f / (scale * kActScale);
 }
 
-constexpr int kActRowB = 2 * kOrder + 16;     // bytes per padded fp16 row of an activation part (conflict-free 16-byte reads)
+constexpr int kActRowB = 2 * kOrder + 16;     // bytes per padded 16-bit row of an activation part (conflict-free 16-byte reads)
 
 // grid (L / (32 TILES), 2 * nfilters), block 256 = 4 waves.  Wave w owns the output neurons [32 w, 32 w + 32) of all
-// TILES tiles of 32 positions of the workgroup.  The activations live in LDS as two fp16 parts (2^13 h = hi + lo) and every layer
-// overwrites them in place; the two 128 x 128 layers are three-product split-fp16 MFMA GEMMs, their
-// weights pre-split by split_weights_kernel and held in registers for all tiles (fetching them is what a short run
-// of positions per workgroup pays most for: 64 KB per workgroup and layer from L2).  Within a layer the products of
+// TILES tiles of 32 positions of the workgroup.  The activations live in LDS as three bf16 parts (hi, mid, lo:
+// together the fp32 value) and every layer overwrites them in place; the two 128 x 128 layers are six-product
+// split-bf16 MFMA GEMMs, their weights pre-split by split_weights_kernel and held in registers for all tiles (fetching them is what a short run
+// of positions per workgroup pays most for: 96 KB per workgroup and layer from L2).  Within a layer the products of
 // tile i + 1 are issued together with the sin epilogue of tile i, so that matrix pipe and vector ALU overlap.
 //
 // PROJECT = true: the same workgroup goes on to the 128 -> d output projection of its positions (the last hidden
-// layer's activations stay in LDS as hi / lo parts instead of travelling through memory): wave w takes the
+// layer's activations stay in LDS as fp16 hi / lo parts instead of travelling through memory): wave w takes the
 // 32-channel tiles w, w + 4, ..., fetches the tile's pre-split weight rows (hi / lo parts in operand layout, from L2:
 // every workgroup reads all of them once), multiplies (three products: W_hi h_hi + W_hi h_lo + W_lo h_hi), applies
 // exp(-t |delta|) + shift and stores the taps channel-major with streaming stores, forward taps at [0, L), reverse taps
@@ -127,10 +128,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
                                                      const uint16_t* __restrict__ wsplit,
                                                      uint16_t* __restrict__ h_hi /* (2 nf, L, 128) fp16 */,
                                                      uint16_t* __restrict__ h_lo /* (2 nf, L, 128) fp16 */,
-                                                     int d, float shift, const uint16_t* __restrict__ w3split,
+                                                     int d, float shift, const uint16_t* __restrict__ w3split, const float* __restrict__ w3scale,
                                                      float* __restrict__ taps /* (nf, d, 2L) */) {
   constexpr int P = 32 * TILES;
-  __shared__ __attribute__((aligned(16))) unsigned char act[2][P * kActRowB];
+  __shared__ __attribute__((aligned(16))) unsigned char act[3][P * kActRowB];
   __shared__ float zt[P * kMaxEmb];
   const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63, i32 = lane & 31, half = lane >> 5;
   const int fi = blockIdx.y >> 1, dir = blockIdx.y & 1;
@@ -145,6 +146,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     return;
   }
 
+  auto put3 = [&](int pos, int o, const float (&s)[4]) __attribute__((always_inline)) {
+    float h[4], m[4], l[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) split3(s[j], h[j], m[j], l[j]);
+    const int off = pos * kActRowB + 2 * o;
+    *reinterpret_cast<uint2*>(&act[0][off]) = make_uint2(pack_bf16x2(h[0], h[1]), pack_bf16x2(h[2], h[3]));
+    *reinterpret_cast<uint2*>(&act[1][off]) = make_uint2(pack_bf16x2(m[0], m[1]), pack_bf16x2(m[2], m[3]));
+    *reinterpret_cast<uint2*>(&act[2][off]) = make_uint2(pack_bf16x2(l[0], l[1]), pack_bf16x2(l[2], l[3]));
+  };
   auto put2 = [&](int pos, int o, const float (&s)[4]) __attribute__((always_inline)) {
     uint32_t h0, h1, l0, l1;
     split2(s[0] * kActScale, s[1] * kActScale, h0, l0);
@@ -155,14 +165,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   };
 
   // Weights of an inner layer -> registers.  Requested one phase early (layer 1's before the vector-ALU layer, layer
-  // 2's before the last epilogue of layer 1), so that the 16 KB per wave arrive behind other work.
-  f16x8 ah[8], al[8];
+  // 2's before the last epilogue of layer 1), so that the 24 KB per wave arrive behind other work.
+  bf16x8 ah[8], am[8], al[8];
   auto load_weights = [&](int layer) __attribute__((always_inline)) {
     const u32x4* wp = reinterpret_cast<const u32x4*>(wsplit + ((long)(blockIdx.y * 2 + layer)) * kSplitPerLayer) + w * 8 * 64 + lane;
 #pragma unroll
     for (int ks = 0; ks < 8; ++ks) {
-      ah[ks] = __builtin_bit_cast(f16x8, wp[ks * 64]);
-      al[ks] = __builtin_bit_cast(f16x8, wp[ks * 64 + kOrder * kOrder / 8]);
+      ah[ks] = __builtin_bit_cast(bf16x8, wp[ks * 64]);
+      am[ks] = __builtin_bit_cast(bf16x8, wp[ks * 64 + kOrder * kOrder / 8]);
+      al[ks] = __builtin_bit_cast(bf16x8, wp[ks * 64 + 2 * kOrder * kOrder / 8]);
     }
   };
   load_weights(0);
@@ -192,7 +203,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         for (int e = 0; e < kMaxEmb; ++e) acc += wt[j][e] * zt[pos * emb + e];      // pos emb + e < P emb + 8 <= P kMaxEmb
         s[j] = sin_reduced(fo[j] * acc);
       }
-      put2(pos, o, s);
+      put3(pos, o, s);
     }
   }
   // layers 1, 2: D[o'][pos] = sum_o W[o'][o] act[pos][o].  A = weight rows 32 w + i32 (registers), B = positions of the
@@ -203,29 +214,29 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     const int boff = (32 * tile + i32) * kActRowB + 16 * half;
 #pragma unroll
     for (int ks = 0; ks < 8; ++ks) {
-      const f16x8 bh = __builtin_bit_cast(f16x8, *reinterpret_cast<const u32x4*>(&act[0][boff + 32 * ks]));
-      const f16x8 bl = __builtin_bit_cast(f16x8, *reinterpret_cast<const u32x4*>(&act[1][boff + 32 * ks]));
-      acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(al[ks], bh, acc, 0, 0, 0);
-      acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah[ks], bl, acc, 0, 0, 0);
-      acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah[ks], bh, acc, 0, 0, 0);
+      const bf16x8 bh = __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4*>(&act[0][boff + 32 * ks]));
+      const bf16x8 bm = __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4*>(&act[1][boff + 32 * ks]));
+      const bf16x8 bl = __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4*>(&act[2][boff + 32 * ks]));
+      // smallest terms first
+      acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(al[ks], bh, acc, 0, 0, 0);
+      acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah[ks], bl, acc, 0, 0, 0);
+      acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(am[ks], bm, acc, 0, 0, 0);
+      acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(am[ks], bh, acc, 0, 0, 0);
+      acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah[ks], bm, acc, 0, 0, 0);
+      acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah[ks], bh, acc, 0, 0, 0);
     }
   };
   // accumulator element v: neuron 32 w + 8 (v / 4) + 4 half + v % 4, position i32 of the tile
-  // (the scale r of a row goes into frequency and bias, exactly: freq (r acc + b) = (freq r) (acc + b / r))
   float fr[16], bs[16];
   auto load_scales = [&](int layer) __attribute__((always_inline)) {
     const float* bias = layer == 0 ? W.b1 : W.b2;
-    const float* rows = reinterpret_cast<const float*>(wsplit + ((long)(blockIdx.y * 2 + layer)) * kSplitPerLayer + 2 * kOrder * kOrder);
 #pragma unroll
     for (int vq = 0; vq < 4; ++vq) {
       const int o = 32 * w + 8 * vq + 4 * half;
       const float4 fq = *reinterpret_cast<const float4*>(F.freq + o);
       const float4 bq = *reinterpret_cast<const float4*>(bias + o);
-      const float4 rq = *reinterpret_cast<const float4*>(rows + o);
-      fr[4 * vq] = w_mod * fq.x * rq.x; fr[4 * vq + 1] = w_mod * fq.y * rq.y; fr[4 * vq + 2] = w_mod * fq.z * rq.z; fr[4 * vq + 3] = w_mod * fq.w * rq.w;
-      auto inverse = [](float r) { return __uint_as_float(0x7f000000u - __float_as_uint(r)); };      // of a power of two
-      bs[4 * vq] = bq.x * inverse(rq.x); bs[4 * vq + 1] = bq.y * inverse(rq.y);
-      bs[4 * vq + 2] = bq.z * inverse(rq.z); bs[4 * vq + 3] = bq.w * inverse(rq.w);
+      fr[4 * vq] = w_mod * fq.x; fr[4 * vq + 1] = w_mod * fq.y; fr[4 * vq + 2] = w_mod * fq.z; fr[4 * vq + 3] = w_mod * fq.w;
+      bs[4 * vq] = bq.x; bs[4 * vq + 1] = bq.y; bs[4 * vq + 2] = bq.z; bs[4 * vq + 3] = bq.w;
     }
   };
   auto epilogue = [&](auto ll, int tile, const floatx16& acc) __attribute__((always_inline)) {
@@ -237,7 +248,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       float s[4];
 #pragma unroll
       for (int j = 0; j < 4; ++j) s[j] = sin_reduced(fr[4 * vq + j] * (acc[4 * vq + j] + bs[4 * vq + j]));
-      if constexpr (layer == 0 || PROJECT) {      // (PROJECT: h3 stays in LDS for the projection)
+      if constexpr (layer == 0) {
+        put3(pos, o, s);
+      } else if constexpr (PROJECT) {           // h3 stays in LDS (parts 0 and 1) for the projection
         put2(pos, o, s);
       } else {
         const long hrow = ((long)blockIdx.y * L + l0 + pos) * kOrder;
@@ -274,8 +287,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   if constexpr (PROJECT) {
     // the barrier that ended the last layer says h3 (hi in act[0], lo in act[1]) is complete for all P positions
     float* out = taps + (long)fi * d * 2 * L;
-    const u32x4* w3 = reinterpret_cast<const u32x4*>(w3split + blockIdx.y * w3_split_elems(d)) + lane;
-    const float* w3scale = reinterpret_cast<const float*>(w3split + blockIdx.y * w3_split_elems(d) + 2l * d * kOrder);
+    const u32x4* w3 = reinterpret_cast<const u32x4*>(w3split + (long)blockIdx.y * 2 * d * kOrder) + lane;
+    const float* back = w3scale + (long)blockIdx.y * d;
     float tl[TILES];
 #pragma unroll
     for (int t = 0; t < TILES; ++t) tl[t] = F.t[l0 + 32 * t + i32];
@@ -294,7 +307,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll
       for (int vq = 0; vq < 4; ++vq) {
         o.dq[vq] = *reinterpret_cast<const float4*>(F.deltas + 32 * ct + 8 * vq + 4 * half);
-        o.rq[vq] = *reinterpret_cast<const float4*>(w3scale + 32 * ct + 8 * vq + 4 * half);
+        o.rq[vq] = *reinterpret_cast<const float4*>(back + 32 * ct + 8 * vq + 4 * half);
       }
     };
     auto project_tile = [&](int ct, const TileOps& o) __attribute__((always_inline)) {
@@ -332,8 +345,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         }
       }
     };
-    // Two register sets: the next tile's operands are requested before the products of this one (they fit beside them since the
-    // inner layers' weights are two parts instead of three).
+    // two register sets: the next tile's operands are requested before the products of this one
     TileOps o[2];
     const int last = d / 32 - 1;
     auto fetch = [&](int ct, TileOps& into) __attribute__((always_inline)) { fetch_tile(ct < last ? ct : last, into); };      // (never beyond the weights)
@@ -491,40 +503,39 @@ using namespace m2;
 
 extern "C" size_t m2_hyena_filter_workspace_bytes(int nfilters, int L, int d, int order) {
   if (nfilters <= 0 || L <= 0 || d <= 0 || order <= 0) return 0;
-  // h3 in two parts; the output projections of the 2 nfilters MLPs in two; their inner-layer weights in two and the scales of both, in
-  // the room of the three parts that the inner layers had when the documented sizes were laid down
-  size_t inner = (size_t)2 * 3 * order * order;
-  if (inner < 2 * (size_t)kSplitPerLayer + 2 * (size_t)d) inner = 2 * (size_t)kSplitPerLayer + 2 * (size_t)d;
-  return (size_t)2 * nfilters * L * order * sizeof(float) + (size_t)2 * nfilters * inner * sizeof(uint16_t) +
+  // h3 in two fp16 parts; the inner-layer weights of the 2 nfilters MLPs as three bf16 parts each; their output
+  // projections as two fp16 parts
+  return (size_t)2 * nfilters * L * order * sizeof(float) + (size_t)2 * nfilters * 2 * 3 * order * order * sizeof(uint16_t) +
          (size_t)2 * nfilters * 2 * d * order * sizeof(uint16_t);
 }
+
+// Hidden layers and projection as one kernel, whose h3 never leaves the chip.  (No more channels than the room of h3, which is free
+// then, has for their scales where a caller's workspace of the documented size is all there is.)
+static bool project_with_hidden(int L, int d) { return L >= 1024 && L % 64 == 0 && d <= kOrder * L; }
 
 // The two or three launches of a batch of filters (weight re-split, hidden layers, projection + decay), the table coming
 // either by value or from device memory.  `w3split` / `taps` null: the projection is left to the caller (the fused
 // projection + spectrum kernel of short sequences).  Kernels that keep a projection's weights in registers split them themselves.
 template <class TAB>
 static int filter_launches(TAB tab, int nfilters, int L, int d, int emb_dim, float w_mod, float shift, uint16_t* h_hi,
-                           uint16_t* h_lo, uint16_t* wsplit, uint16_t* w3split, float* taps, hipStream_t s) {
-  const bool one_kernel = taps && L >= 1024 && L % 64 == 0;      // hidden layers and projection
+                           uint16_t* h_lo, uint16_t* wsplit, uint16_t* w3split, float* w3scale, float* taps, hipStream_t s) {
+  const bool one_kernel = taps && project_with_hidden(L, d);
   const int split_blocks = 2 * nfilters * 2 * 4 + (one_kernel ? 2 * nfilters * (d / 32) : 0);
-  hipLaunchKernelGGL(split_weights_kernel<TAB>, dim3(split_blocks), dim3(512), 0, s, tab, 2 * nfilters, d, wsplit, w3split);
+  hipLaunchKernelGGL(split_weights_kernel<TAB>, dim3(split_blocks), dim3(512), 0, s, tab, 2 * nfilters, d, wsplit, w3split,
+                     w3scale);
   int rc = check_launch("hyena split_weights_kernel");
   if (rc) return rc;
-  // Positions per workgroup: longer runs amortise the weight fetch (64 KB per workgroup and layer, 520 bytes per channel for the
-  // projection), short sequences need the workgroups spread over the chip.  From L = 1024 on hidden layers and projection are one
-  // kernel, h3 never leaves the chip; us for hidden layers + projection + spectra of 12 mixers, d = 768, with 128 and with 64
-  // positions: L = 1024 158 / 157, 4096 514 / 534, 8192 947 / 994; three bf16 parts and 64 positions: 190 / 587 / 1078.
+  // Positions per workgroup: longer runs amortise the weight fetch (96 KB per workgroup and layer, 520 bytes per channel for the
+  // projection), short sequences need the workgroups spread over the chip.  128 positions would leave one workgroup on a compute unit
+  // (104 KB of activations) and half of them idle for a single mixer.  us for the spectra of 1 / 12 mixers, d = 768: L = 1024 44 / 155,
+  // 4096 60 / 501, 8192 94 / 967; with inner layers in two fp16 parts and 128 positions 56 / 151, 71 / 457, 93 / 869.
   if (one_kernel) {
-    if (L % 128 == 0)
-      hipLaunchKernelGGL((hidden_kernel<4, TAB, true>), dim3(L / 128, 2 * nfilters), dim3(256), 0, s, tab, L, emb_dim, w_mod, wsplit,
-                         h_hi, h_lo, d, shift, w3split, taps);
-    else
-      hipLaunchKernelGGL((hidden_kernel<2, TAB, true>), dim3(L / 64, 2 * nfilters), dim3(256), 0, s, tab, L, emb_dim, w_mod, wsplit,
-                         h_hi, h_lo, d, shift, w3split, taps);
+    hipLaunchKernelGGL((hidden_kernel<2, TAB, true>), dim3(L / 64, 2 * nfilters), dim3(256), 0, s, tab, L, emb_dim, w_mod, wsplit,
+                       h_hi, h_lo, d, shift, w3split, w3scale, taps);
     return check_launch("hyena hidden + project kernel");
   }
   hipLaunchKernelGGL((hidden_kernel<1, TAB, false>), dim3(L / 32, 2 * nfilters), dim3(256), 0, s, tab, L, emb_dim, w_mod, wsplit,
-                     h_hi, h_lo, 0, 0.f, nullptr, nullptr);
+                     h_hi, h_lo, 0, 0.f, nullptr, nullptr, nullptr);
   rc = check_launch("hyena hidden_kernel");
   if (rc || !taps) return rc;
   hipLaunchKernelGGL(project_kernel<TAB>, dim3((L + kPosPerWg - 1) / kPosPerWg, (d + 127) / 128, 2 * nfilters), dim3(256), 0, s, tab, L, d, shift,
@@ -569,7 +580,8 @@ static int hyena_filter_launch(const char* who, const m2_hyena_filter_params* pa
   uint16_t* h_lo = h_hi + (size_t)2 * nfilters * L * order;
   uint16_t* wsplit = h_lo + (size_t)2 * nfilters * L * order;
   uint16_t* w3split = wsplit + (size_t)2 * nfilters * 2 * kSplitPerLayer;
-  return filter_launches(tab, nfilters, L, d, emb_dim, w_mod, shift, h_hi, h_lo, wsplit, w3split, taps, (hipStream_t)stream);
+  float* w3scale = reinterpret_cast<float*>(workspace);      // (h3 and these are never in memory in the same call)
+  return filter_launches(tab, nfilters, L, d, emb_dim, w_mod, shift, h_hi, h_lo, wsplit, w3split, w3scale, taps, (hipStream_t)stream);
 }
 
 extern "C" int m2_hyena_filter_fwd(const m2_hyena_filter_params* params, int nfilters, int L, int d, int order,
@@ -640,7 +652,7 @@ extern "C" int m2_hyena_filter_fwd_static(const m2_hyena_filter_params* params, 
 // ---------------------------------------------------------------------------------------------
 namespace {
 struct BatchLayout {
-  size_t h_lo, wsplit, w3split, taps, total;      // byte offsets into the workspace (h_hi at 0)
+  size_t h_lo, wsplit, w3split, w3scale, taps, total;      // byte offsets into the workspace (h_hi at 0)
   bool fused;                                     // projection + spectrum as one kernel, taps never in memory
 };
 BatchLayout batch_layout(int nmixers, int fpm, int L, int d) {
@@ -651,7 +663,8 @@ BatchLayout batch_layout(int nmixers, int fpm, int L, int d) {
   b.h_lo = up(2 * nf * L * kOrder * sizeof(uint16_t));
   b.wsplit = b.h_lo + up(2 * nf * L * kOrder * sizeof(uint16_t));
   b.w3split = b.wsplit + up(2 * nf * 2 * (size_t)kSplitPerLayer * sizeof(uint16_t));
-  b.taps = b.w3split + (b.fused ? 0 : up(2 * nf * (size_t)w3_split_elems(d) * sizeof(uint16_t)));
+  b.w3scale = b.w3split + (b.fused ? 0 : up(2 * nf * 2 * (size_t)d * kOrder * sizeof(uint16_t)));
+  b.taps = b.w3scale + (b.fused ? 0 : up(2 * nf * (size_t)d * sizeof(float)));
   b.total = b.taps + (b.fused ? 0 : up(nf * (size_t)d * 2 * L * sizeof(float)));
   return b;
 }
@@ -684,10 +697,11 @@ extern "C" int m2_mixer_filters_fwd(const m2_hyena_filter_params* params_dev, co
   uint16_t* h_lo = reinterpret_cast<uint16_t*>(ws + lay.h_lo);
   uint16_t* wsplit = reinterpret_cast<uint16_t*>(ws + lay.wsplit);
   uint16_t* w3split = lay.fused ? nullptr : reinterpret_cast<uint16_t*>(ws + lay.w3split);
+  float* w3scale = lay.fused ? nullptr : reinterpret_cast<float*>(ws + lay.w3scale);
   float* taps = lay.fused ? nullptr : reinterpret_cast<float*>(ws + lay.taps);
   TabByPointer tab{reinterpret_cast<const FilterPtrs*>(params_dev)};
   hipStream_t s = (hipStream_t)stream;
-  rc = filter_launches(tab, nf, L, d, emb_dim, w_mod, shift, h_hi, h_lo, wsplit, w3split, taps, s);
+  rc = filter_launches(tab, nf, L, d, emb_dim, w_mod, shift, h_hi, h_lo, wsplit, w3split, w3scale, taps, s);
   if (rc) return rc;
   const long spec_stride = (long)(m2_filter_spectrum_bytes(d, L) / sizeof(float));
   if (lay.fused)

@@ -52,3 +52,34 @@ def test_taps_of_infinite_and_large_weights(gpu):
     taps = fn.to(gpu).bidirectional_taps(L).cpu()[:, :L]
     bad = ~torch.isfinite(taps).all(dim=1)
     assert bad[2] and bad[6] and int(bad.sum()) == 2
+
+
+@pytest.mark.parametrize("L", [128, 1024])
+def test_inner_layers_keep_all_bits(gpu, L):
+    """Weights and activations of the inner layers whose mantissas lie between two numbers of 11 bits, one product per neuron and a last
+    sine of arguments up to 128, which shows the relative error of that product: sine, two products and two more sines are five
+    roundings of 2^-24 at most, below 2 x 2^-24 in the root mean square.  (Operands in two fp16 parts without the product of the low
+    ones would be 2^-22 off, all in one direction.)"""
+    import m2_amd
+    d = n = 128
+    g = torch.Generator().manual_seed(L)
+    between = 1 + 0.97 * 2.0 ** -11
+    sign = torch.randint(0, 2, (n,), generator=g) * 2.0 - 1
+    b0 = (0.01 + 0.01 * torch.rand(n, generator=g)).float()
+    w1 = (torch.asin(between * 2.0 ** -7 * sign.double()) / torch.sin(b0.double())).float()
+    w2 = between * 2.0 ** torch.randint(12, 15, (n,), generator=g).float()
+    fn = m2_amd.HyenaFilter(d, emb_dim=5, order=n, seq_len=L, bidirectional=True, w=1)
+    with torch.no_grad():
+        for name, p in fn.named_parameters():
+            if "implicit_filter" in name and not name.endswith("freq"):
+                p.zero_()
+        fn.modulation.deltas.zero_()
+        for mlp in (fn.implicit_filter, fn.implicit_filter_rev):
+            mlp[0].bias.copy_(b0)
+            mlp[2].weight.copy_(torch.diag(w1))
+            mlp[4].weight.copy_(torch.diag(w2))
+            mlp[6].weight.copy_(torch.eye(n))
+    taps = fn.to(gpu).bidirectional_taps(L).double().cpu()
+    arg = w2.double() * torch.sin(w1.double() * torch.sin(b0.double()))
+    err = (taps - torch.sin(arg)[:, None]) / arg[:, None]
+    assert err.pow(2).mean().sqrt() <= 2 * 2.0 ** -24
