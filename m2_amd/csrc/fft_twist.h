@@ -97,6 +97,13 @@ __device__ __forceinline__ void sync_threads() {
   }
 }
 
+// The thread's number, to the compiler another value each time: what is formed from it is formed anew and not kept in registers across
+// the passes, which would spill it.
+__device__ __forceinline__ int anew(int t) {
+  asm volatile("" : "+v"(t));
+  return t;
+}
+
 // ------------------------------------------------------------------------------------------
 // radix-R transforms in registers.  The factor of stage S (blocks of R / 2^S), number e < max(1, 2^(S-1)), at shift sigma is
 // exp(-i pi (sigma + e) / 2^S); the other half of a stage's factors are these times -i.
@@ -248,6 +255,8 @@ struct TwistForward {            // of the last forward pass: group k1 R2 + k2 h
         last[decltype(ii)::value].init(8 * (g / P::R2 + P::R1 * (g % P::R2)) + S8, 8 * P::R1 * P::R2);
       });
   }
+  template <int I>
+  __device__ __forceinline__ const Factors<P::R3>& group() const { return last[I]; }
 };
 template <class P>
 struct TwistInverse {            // of the last inverse pass
@@ -352,10 +361,10 @@ __device__ __forceinline__ void load_group(cf (&x)[P::E], int t, const float2* r
   const float2* pg = row + P::phys(P::R3 * (t + P::T * I));
   static_for<0, P::R3>([&](auto jj) { x[I * P::R3 + decltype(jj)::value] = lds_get(pg, decltype(jj)::value); });
 }
-template <class P, int S8, int I>
-__device__ __forceinline__ void fwd_group(cf (&x)[P::E], int t, const float2* tab, const TwistForward<P, S8>& tf) {
+template <class P, int I, class TF>
+__device__ __forceinline__ void fwd_group(cf (&x)[P::E], int t, const float2* tab, const TF& tf) {
   if constexpr (P::THREE) {
-    tf.last[I].use([&](auto&& w) __attribute__((always_inline)) { fwd_factors<P::R3, I * P::R3>(x, w, KeepAll{}); });
+    tf.template group<I>().use([&](auto&& w) __attribute__((always_inline)) { fwd_factors<P::R3, I * P::R3>(x, w, KeepAll{}); });
   } else {
     TableRow<P::R3> w;
     w.load(tab + (t + P::T * I) * P::FS);
@@ -418,12 +427,16 @@ __device__ __forceinline__ void store_spectrum(const cf (&x)[P::E], float scale,
   });
 }
 
+struct Nothing {
+  __device__ __forceinline__ void operator()() const {}
+};
 // One signal: registers in first-pass layout -> spectrum product -> registers in first-pass layout, still shifted.  Enters and
 // leaves by LDS slots of the thread's own, so one may follow another without a barrier.  The groups of the last pass are a thread's
-// own too: transformed, multiplied and transformed back one after the other.
-template <class P, int S8, bool REAL>
-__device__ __forceinline__ void convolve(cf (&x)[P::E], int t, float2* row, const float2* tab, const TwistForward<P, S8>& tf,
-                                         const TwistInverse<P>& ti, const float4* __restrict__ sp) {
+// own too: transformed, multiplied and transformed back one after the other.  `before_last` is called ahead of the last pass, where
+// the spectrum's registers are free again: loads that it issues travel under that pass.
+template <class P, int S8, bool REAL, class TF, class F = Nothing>
+__device__ __forceinline__ void convolve(cf (&x)[P::E], int t, float2* row, const float2* tab, const TF& tf,
+                                         const TwistInverse<P>& ti, const float4* __restrict__ sp, F&& before_last = Nothing{}) {
   float4 K[P::R3 / 2];
   if constexpr (!P::THREE) load_spectrum<P, 0>(K, sp, t);      // requested a pass ahead of its use
   fwd_first<P, S8, REAL>(x, t, row);
@@ -436,7 +449,7 @@ __device__ __forceinline__ void convolve(cf (&x)[P::E], int t, float2* row, cons
   static_for<0, P::NG>([&](auto gg) { load_group<P, decltype(gg)::value>(x, t, row); });
   static_for<0, P::NG>([&](auto gg) {
     constexpr int g = decltype(gg)::value;
-    fwd_group<P, S8, g>(x, t, tab, tf);
+    fwd_group<P, g>(x, t, tab, tf);
     multiply<P, g>(x, K);
     if constexpr (g + 1 < P::NG) load_spectrum<P, g + 1>(K, sp, t);
     inv_group<P, g>(x, t, row);
@@ -446,6 +459,7 @@ __device__ __forceinline__ void convolve(cf (&x)[P::E], int t, float2* row, cons
     second<P, true>(x, t, row, tab);
     sync_threads<P::T>();
   }
+  before_last();
   inv_first<P>(x, t, row, tab, ti);
 }
 // the forward half: the spectrum of registers in first-pass layout
@@ -458,7 +472,7 @@ __device__ __forceinline__ void transform(cf (&x)[P::E], int t, float2* row, con
     sync_threads<P::T>();
   }
   static_for<0, P::NG>([&](auto gg) { load_group<P, decltype(gg)::value>(x, t, row); });
-  static_for<0, P::NG>([&](auto gg) { fwd_group<P, S8, decltype(gg)::value>(x, t, tab, tf); });
+  static_for<0, P::NG>([&](auto gg) { fwd_group<P, decltype(gg)::value>(x, t, tab, tf); });
 }
 
 // half transforms and rows by sequence length; the shift of one signal's ring (z^L = -i) in eighths

@@ -9,14 +9,19 @@
 //   spec[channel][signal][half][register pair 0 .. 15][T]  float4, as in fftconv_kernels.hip
 //
 // One workgroup of 512 threads fills a compute unit.  A thread holds 32 samples of either half of the row in the layout of the first
-// pass (positions t + 512 j and H + t + 512 j), which u is read in directly, consecutive lanes consecutive floats.  The product of
-// the short convolutions, the gate and the results are staged through the transform's buffer (32768 floats are the 16384 complex
-// slots), 64 consecutive time steps per thread on the global side.
+// pass (positions t + 512 j and H + t + 512 j), which u and the input of a plain convolution are read in directly, consecutive lanes
+// consecutive samples.  The product of the short convolutions, the gate and the results of the mixer are staged through the transform's
+// buffer (32768 floats are the 16384 complex slots), 64 consecutive time steps per thread on the global side.
 //
-// 268 us at B = 1, d = 768 in bf16 (318 in fp32), against 338 (405) with the polyphase form that this took over from, whose product
-// paired mirrored frequencies at nine times the multiplications: 124 us of vector instructions, 700 MB of memory traffic, and with one
-// workgroup per unit the two hardly overlap.  Requesting the next row's inputs or u ahead needs more registers than there are: with
-// 100 of them spilled the kernel took 305 us.
+// What bounds it: 124 us of vector instructions and 700 MB of memory traffic (B = 1, d = 768, bf16), which with one workgroup per unit
+// overlap only where loads are requested ahead of a pass, and registers: a row's state takes 128 - 192 of 256, and what the compiler
+// keeps beside it is spilled, each reload a wait for every load and store before it.  So what only depends on the thread is formed
+// anew where it is used (`anew`, fft_twist.h) or kept in LDS: 232 bytes of scratch per lane became 12.
+// us at d = 768, with addresses and factors kept / now, and of the polyphase form that this took over from, whose product paired
+// mirrored frequencies at nine times the multiplications: B = 1 bf16 268 / 232 / 338, fp32 316 / 271 / 397; without u 145 / 122 / 140, fp32
+// 191 / 165 / 170; plain convolution, which was staged too, 149 / 86 / 102, fp32 173 / 105 / 125.
+// Requesting the next row's inputs or u ahead with both signals needs more registers than there are: with 100 of them spilled the kernel
+// took 305 us.
 //
 // Stands in for the same reference code as fftconv_kernels.hip (bert/src/mm/hyena_utils.py:16-42,
 // 231-236; bert/src/mm/monarch_mixer_sequence_mixer.py:112-147).
@@ -49,52 +54,70 @@ __device__ __forceinline__ void short_conv8(const float (&in)[10], const float (
   });
 }
 
-// the factors at shift 5/8 from those at 1/8
+// The factors of the last forward pass at shift S8 / 8 from those at shift 1/8 by one constant, where they are used: four numbers in
+// registers and not eight.
+template <class P, int S8>
+struct HalfForward {
+  const TwistForward<P, 1>& at1;
+  template <int I>
+  __device__ __forceinline__ Factors<P::R3> group() const {
+    cf f = at1.last[I].fine, m = at1.last[I].mid;
+    asm volatile("" : "+v"(f.re), "+v"(f.im), "+v"(m.re), "+v"(m.im));
+    return {mul_root<S8 - 1, 8 * P::H>(f), mul_root<S8 - 1, 8 * P::H / 4>(m)};
+  }
+};
+
+// Buffer and tables in LDS; behind them a thread's two factors that remove the shifts, which are read where they are used.
 template <class P>
-__device__ __forceinline__ TwistForward<P, 5> shifted(const TwistForward<P, 1>& a) {
-  TwistForward<P, 5> b;
-  static_for<0, P::NG>([&](auto ii) {
-    constexpr int i = decltype(ii)::value;
-    b.last[i].fine = mul_root<4, 8 * P::H>(a.last[i].fine);
-    b.last[i].mid = mul_root<4, 2 * P::H>(a.last[i].mid);
-  });
-  return b;
+constexpr size_t real_lds_bytes() { return (size_t)(P::ROW + 2 * P::TAB + 2 * P::T) * sizeof(float2); }
+template <class P>
+__device__ __forceinline__ float4* ends_init(float2* lds, int t) {
+  static_assert((P::ROW + 2 * P::TAB) % 2 == 0 && P::NB1 == 1, "16-byte slots, one factor each");
+  float4* ends = reinterpret_cast<float4*>(lds + P::ROW + 2 * P::TAB);
+  TwistEnd<P, 1> te1;
+  TwistEnd<P, 5> te5;
+  te1.init(t);
+  te5.init(t);
+  ends[t] = make_float4(te1.f[0].re, te1.f[0].im, te5.f[0].re, te5.f[0].im);
+  return ends;
 }
 
-// acc += the convolution of (lo, hi) held in first-pass layout; sp: the signal's two blocks.  `again` provides lo and hi for the
-// second half (registers or memory).
-template <class P, class A>
-__device__ __forceinline__ void convolve_halves(float (&lo)[32], float (&hi)[32], A&& again, cf (&acc)[32], int t, float2* row, const float2* tab1,
-                                                const float2* tab5, const TwistForward<P, 1>& tf1,
-                                                const TwistInverse<P>& ti, const TwistEnd<P, 1>& te1, const TwistEnd<P, 5>& te5,
-                                                const float4* __restrict__ sp) {
+// acc += the convolution of the signal whose samples in first-pass layout are lo(r) and hi(r); sp: the signal's two blocks.  The
+// second half asks for them again: at(kUnder1st) is called under the last pass of the first half, at(kBetween) behind it, at(kUnder2nd)
+// under the last pass of the second half.
+enum { kUnder1st, kBetween, kUnder2nd };
+template <class P, class LO, class HI, class F>
+__device__ __forceinline__ void convolve_halves(LO&& lo, HI&& hi, F&& at, cf (&acc)[32], int t, float2* row,
+                                                const float2* tab1, const float2* tab5, const TwistForward<P, 1>& tf1,
+                                                const TwistInverse<P>& ti, const float4* ends, const float4* __restrict__ sp) {
   cf x[32];
   static_for<0, 32>([&](auto rr) {
-    constexpr int r = decltype(rr)::value;
-    const float v = kRho * hi[r];
-    x[r] = {lo[r] + v, -v};
+    const float v = kRho * hi(rr);
+    x[decltype(rr)::value] = {lo(rr) + v, -v};
   });
-  convolve<P, 1, false>(x, t, row, tab1, tf1, ti, sp);
+  convolve<P, 1, false>(x, anew(t), row, tab1, HalfForward<P, 1>{tf1}, ti, sp, [&]() __attribute__((always_inline)) { at(ic<kUnder1st>{}); });
   // acc.re: first half of the row, acc.im: second.  P without its shift is f v; P / r = f v exp(i pi / 4)
+  const float2 end1 = *reinterpret_cast<const float2*>(ends + anew(t));
   static_for<0, 32>([&](auto rr) {
-    constexpr int r = decltype(rr)::value, i = r / P::R1, j = r % P::R1;
-    const cf v = mul_root<j, 8 * P::R1, true>(x[r]);
-    const float re = te1.f[i].re * v.re - te1.f[i].im * v.im, im = te1.f[i].re * v.im + te1.f[i].im * v.re;
+    constexpr int r = decltype(rr)::value;
+    const cf v = mul_root<r, 8 * P::R1, true>(x[r]);
+    const float re = end1.x * v.re - end1.y * v.im, im = end1.x * v.im + end1.y * v.re;
     acc[r].re += re;
     acc[r].im = fmaf(kRho, re - im, acc[r].im);
   });
   __builtin_amdgcn_sched_barrier(0);
-  again(lo, hi);
+  at(ic<kBetween>{});
+  static_for<0, 32>([&](auto rr) {
+    const float v = kRho * hi(rr);
+    x[decltype(rr)::value] = {lo(rr) - v, v};
+  });
+  convolve<P, 5, false>(x, anew(t), row, tab5, HalfForward<P, 5>{tf1}, ti, sp + real_spec_block<P>() / 4,
+                        [&]() __attribute__((always_inline)) { at(ic<kUnder2nd>{}); });
+  const float2 end5 = reinterpret_cast<const float2*>(ends + anew(t))[1];
   static_for<0, 32>([&](auto rr) {
     constexpr int r = decltype(rr)::value;
-    const float v = kRho * hi[r];
-    x[r] = {lo[r] - v, v};
-  });
-  convolve<P, 5, false>(x, t, row, tab5, shifted(tf1), ti, sp + real_spec_block<P>() / 4);
-  static_for<0, 32>([&](auto rr) {
-    constexpr int r = decltype(rr)::value, i = r / P::R1, j = r % P::R1;
-    const cf v = mul_root<5 * j, 8 * P::R1, true>(x[r]);
-    const float re = te5.f[i].re * v.re - te5.f[i].im * v.im, im = te5.f[i].re * v.im + te5.f[i].im * v.re;
+    const cf v = mul_root<5 * r, 8 * P::R1, true>(x[r]);
+    const float re = end5.x * v.re - end5.y * v.im, im = end5.x * v.im + end5.y * v.re;
     acc[r].re += re;
     acc[r].im = fmaf(-kRho, re - im, acc[r].im);
   });
@@ -103,9 +126,9 @@ __device__ __forceinline__ void convolve_halves(float (&lo)[32], float (&hi)[32]
 // ------------------------------------------------------------------------------------------
 // the fused mixer core, sequence length 2 P::H
 // ------------------------------------------------------------------------------------------
-// FULL: short convolutions and gates (sw, sb non-null); otherwise a plain long convolution of one input.
-// HAS_U: the residual long convolution of the layer input u (uin non-null).
-template <class P, typename ACT, bool FULL, bool HAS_U>
+// HAS_U: the residual long convolution of the layer input u (uin non-null).  Without it there are registers for the gate's inputs to
+// be requested under the last pass and the next row's under the epilogue.
+template <class P, typename ACT, bool HAS_U>
 __global__ __launch_bounds__(P::T) __attribute__((amdgpu_waves_per_eu(2, 2))) void mixer_real_kernel(
     const ACT* __restrict__ xproj,      // (3d, B, LS): x1 | x2 | v, channel-major
     long ldx,                           // elements between two channels of xproj, B L or more
@@ -123,72 +146,74 @@ __global__ __launch_bounds__(P::T) __attribute__((amdgpu_waves_per_eu(2, 2))) vo
   float2* row = lds;
   float* stage = reinterpret_cast<float*>(lds);
   const float2 *tab1 = lds + P::ROW, *tab5 = tab1 + P::TAB;
-  const int t = threadIdx.x, n0 = 64 * t;
+  const int t = threadIdx.x;
 
   tables_init<P, 1>(lds + P::ROW);
   tables_init<P, 5>(lds + P::ROW + P::TAB);
   TwistForward<P, 1> tf1;
   TwistInverse<P> ti;
-  TwistEnd<P, 1> te1;
-  TwistEnd<P, 5> te5;
   tf1.init(t);
   ti.init(t);
-  te1.init(t);
-  te5.init(t);
+  float4* ends = ends_init<P>(lds, t);
   sync_threads<T>();
 
   // workgroup -> (channel, batch row) as in mixer_pair_kernel: XCD e takes the channels c = e (mod 8)
   const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3, slots = gridDim.x >> 3;
   const int rows_per_xcd = (d >> 3) * B;
+  RawRow<ACT, 8, true> r1, rv, r2;
+  auto fetch = [&](RawRow<ACT, 8, true>& r, int third, int j) __attribute__((always_inline)) {
+    const int c = __builtin_amdgcn_readfirstlane((j / B) * 8 + xcd), bb = __builtin_amdgcn_readfirstlane(j % B);
+    const ACT* p = xproj + ((long)third * d + c) * ldx + (long)bb * LS;
+    const int n0 = 64 * anew(t);
+    static_for<0, 8>([&](auto qq) { r.template fetch<decltype(qq)::value>(p, n0 + 8 * decltype(qq)::value); });
+  };
+  if constexpr (!HAS_U) {
+    if (slot < rows_per_xcd) {
+      fetch(r1, 0, slot);
+      fetch(rv, 2, slot);
+    }
+  }
   for (int j = slot; j < rows_per_xcd; j += slots) {
     // the same for every lane: say so, so that row base addresses live in scalar registers
     const int c = __builtin_amdgcn_readfirstlane((j / B) * 8 + xcd), bb = __builtin_amdgcn_readfirstlane(j % B);
     const float4* sp = reinterpret_cast<const float4*>(spec + (long)c * 4 * BLK);
     float lo[32], hi[32];
+    auto get_lo = [&](auto rr) __attribute__((always_inline)) { return lo[decltype(rr)::value]; };
+    auto get_hi = [&](auto rr) __attribute__((always_inline)) { return hi[decltype(rr)::value]; };
     cf acc[32];
     static_for<0, 32>([&](auto rr) { acc[decltype(rr)::value] = {0.f, 0.f}; });
 
-    // ---- first signal: a = sc(x1) sc(v)  (or the plain input), convolved with filter 1
+    // ---- first signal: a = sc(x1) sc(v), convolved with filter 1
     {
-      RawRow<ACT, 8, true> r1, rv;
-      const ACT* px = FULL ? xproj + (long)(0 * d + c) * ldx + (long)bb * LS : xproj + (long)c * ldx + (long)bb * LS;
-      const ACT* pv = xproj + (long)(2 * d + c) * ldx + (long)bb * LS;
-      static_for<0, 8>([&](auto qq) {
-        constexpr int q = decltype(qq)::value;
-        r1.template fetch<q>(px, n0 + 8 * q);
-        if constexpr (FULL) rv.template fetch<q>(pv, n0 + 8 * q);
-      });
-      float w1[3], wv[3], p1 = 0.f, pbv = 0.f, f1 = 0.f, fv = 0.f;
-      if constexpr (FULL) {
-#pragma unroll
-        for (int k = 0; k < 3; ++k) {
-          w1[k] = sw[(long)c * 3 + k];
-          wv[k] = sw[((long)2 * d + c) * 3 + k];
-        }
-        if (pbias) { p1 = pbias[c]; pbv = pbias[2 * d + c]; }
-        f1 = sb[c] + p1 * (w1[0] + w1[1] + w1[2]);
-        fv = sb[2 * d + c] + pbv * (wv[0] + wv[1] + wv[2]);
+      if constexpr (HAS_U) {
+        fetch(r1, 0, j);
+        fetch(rv, 2, j);
       }
+      float w1[3], wv[3], p1 = 0.f, pbv = 0.f;
+#pragma unroll
+      for (int k = 0; k < 3; ++k) {
+        w1[k] = sw[(long)c * 3 + k];
+        wv[k] = sw[((long)2 * d + c) * 3 + k];
+      }
+      if (pbias) { p1 = pbias[c]; pbv = pbias[2 * d + c]; }
+      const float f1 = sb[c] + p1 * (w1[0] + w1[1] + w1[2]), fv = sb[2 * d + c] + pbv * (wv[0] + wv[1] + wv[2]);
+      const int n0 = 64 * anew(t);
       __builtin_amdgcn_sched_barrier(0);
       static_for<0, 8>([&](auto qq) {
         constexpr int q = decltype(qq)::value;
         const int n = n0 + 8 * q;
         float in[10], a[8], v[8];
         r1.template expand<q>(n, in);
-        if constexpr (FULL) {
-          short_conv8(in, w1, f1, a);
-          rv.template expand<q>(n, in);
-          short_conv8(in, wv, fv, v);
-          if constexpr (q == 0) {
-            if (t == 0) {      // time steps 0 and 1: taps that fall on the zero padding, outside the biased signal
-              a[0] -= p1 * (w1[0] + w1[1]); a[1] -= p1 * w1[0];
-              v[0] -= pbv * (wv[0] + wv[1]); v[1] -= pbv * wv[0];
-            }
+        short_conv8(in, w1, f1, a);
+        rv.template expand<q>(n, in);
+        short_conv8(in, wv, fv, v);
+        if constexpr (q == 0) {
+          if (t == 0) {      // time steps 0 and 1: taps that fall on the zero padding, outside the biased signal
+            a[0] -= p1 * (w1[0] + w1[1]); a[1] -= p1 * w1[0];
+            v[0] -= pbv * (wv[0] + wv[1]); v[1] -= pbv * wv[0];
           }
-          static_for<0, 8>([&](auto ee) { a[decltype(ee)::value] *= v[decltype(ee)::value]; });
-        } else {
-          static_for<0, 8>([&](auto ee) { a[decltype(ee)::value] = in[decltype(ee)::value + 2]; });
         }
+        static_for<0, 8>([&](auto ee) { a[decltype(ee)::value] *= v[decltype(ee)::value]; });
         float4* dst = reinterpret_cast<float4*>(stage + stage_phys(n0) + 8 * q);
         dst[0] = make_float4(a[0], a[1], a[2], a[3]);
         dst[1] = make_float4(a[4], a[5], a[6], a[7]);
@@ -197,7 +222,7 @@ __global__ __launch_bounds__(P::T) __attribute__((amdgpu_waves_per_eu(2, 2))) vo
     }
     sync_threads<T>();
     auto from_stage = [&](auto&& put) __attribute__((always_inline)) {
-      const float* pl = stage + stage_phys(t);
+      const float* pl = stage + stage_phys(anew(t));
       static_for<0, 32>([&](auto rr) {
         constexpr int r = decltype(rr)::value;
         put(rr, pl[stage_phys(512 * r)], pl[stage_phys(H + 512 * r)]);
@@ -208,39 +233,37 @@ __global__ __launch_bounds__(P::T) __attribute__((amdgpu_waves_per_eu(2, 2))) vo
       hi[decltype(rr)::value] = h;
     });
     sync_threads<T>();                     // the transform's slots overlap the staged row
-    convolve_halves<P>(lo, hi, [](float (&)[32], float (&)[32]) {}, acc, t, row, tab1, tab5, tf1, ti, te1, te5, sp);
-
-    // u, read twice rather than kept across the first half transform
-    const float* pu = HAS_U ? uin + ((long)c * B + bb) * LS : nullptr;
-    auto load_u = [&](float (&l)[32], float (&h)[32]) __attribute__((always_inline)) {
-      int again = 0;
-      asm volatile("" : "+s"(again));      // a second load, not the first one's registers kept across the half transform
-      const float* p = pu + again;
-      static_for<0, 32>([&](auto rr) {
-        constexpr int r = decltype(rr)::value;
-        l[r] = (p + 512 * r)[(unsigned)t];
-        h[r] = (p + H + 512 * r)[(unsigned)t];
-      });
-    };
+    convolve_halves<P>(get_lo, get_hi, [&](auto when) __attribute__((always_inline)) {
+      if constexpr (!HAS_U && decltype(when)::value == kUnder2nd) fetch(r2, 1, j);
+    }, acc, t, row, tab1, tab5, tf1, ti, ends, sp);
 
     // ---- gate: acc = y1 * sc(x2), by way of the stage
-    if constexpr (FULL) {
-      RawRow<ACT, 8, true> r2;
-      const ACT* p2 = xproj + (long)(1 * d + c) * ldx + (long)bb * LS;
-      static_for<0, 8>([&](auto qq) { r2.template fetch<decltype(qq)::value>(p2, n0 + 8 * decltype(qq)::value); });
+    {
+      if constexpr (HAS_U) fetch(r2, 1, j);
       float w2[3], pb2 = 0.f;
 #pragma unroll
       for (int k = 0; k < 3; ++k) w2[k] = sw[((long)d + c) * 3 + k];
       if (pbias) pb2 = pbias[d + c];
       const float f2 = sb[d + c] + pb2 * (w2[0] + w2[1] + w2[2]);
       sync_threads<T>();                   // everybody has read the last pass's slots
-      float* ps = stage + stage_phys(t);
+      float* ps = stage + stage_phys(anew(t));
       static_for<0, 32>([&](auto rr) {
         constexpr int r = decltype(rr)::value;
         ps[stage_phys(512 * r)] = acc[r].re;
         ps[stage_phys(H + 512 * r)] = acc[r].im;
       });
+      if constexpr (!HAS_U) {
+        __builtin_amdgcn_sched_barrier(0);
+        if (j + slots < rows_per_xcd) {
+          fetch(r1, 0, j + slots);
+          fetch(rv, 2, j + slots);
+        } else {      // (values of their own here too: otherwise this row's inputs would stay in registers up to this point)
+          static_for<0, 8>([&](auto qq) { r1.clear(qq); rv.clear(qq); });
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
       sync_threads<T>();
+      const int n0 = 64 * anew(t);
       static_for<0, 8>([&](auto qq) {
         constexpr int q = decltype(qq)::value;
         float in[10], g[8];
@@ -260,27 +283,40 @@ __global__ __launch_bounds__(P::T) __attribute__((amdgpu_waves_per_eu(2, 2))) vo
         }
         __builtin_amdgcn_sched_barrier(0);
       });
-      sync_threads<T>();
+      sync_threads<T>();                   // the next row's prologue overwrites what has just been read
       if constexpr (HAS_U) {
         from_stage([&](auto rr, float l, float h) __attribute__((always_inline)) { acc[decltype(rr)::value] = {l, h}; });
         sync_threads<T>();
       }
     }
 
-    // ---- second signal: the layer input u, convolved with filter 2 on top of it
+    // ---- second signal: the layer input u, convolved with filter 2 on top of it; read twice rather than kept across the first half
     if constexpr (HAS_U) {
-      load_u(lo, hi);
-      convolve_halves<P>(lo, hi, load_u, acc, t, row, tab1, tab5, tf1, ti, te1, te5, sp + BLK / 2);
-    }
-    if constexpr (HAS_U || !FULL) {        // results to 64 consecutive time steps per thread
+      const float* pu = uin + ((long)c * B + bb) * LS;
+      auto load_u = [&]() __attribute__((always_inline)) {
+        int again = 0;
+        asm volatile("" : "+s"(again));      // a second load, not the first one's registers kept across the half transform
+        const float* p = pu + again;
+        static_for<0, 32>([&](auto rr) {
+          constexpr int r = decltype(rr)::value;
+          lo[r] = (p + 512 * r)[(unsigned)t];
+          hi[r] = (p + H + 512 * r)[(unsigned)t];
+        });
+      };
+      load_u();
+      convolve_halves<P>(get_lo, get_hi, [&](auto when) __attribute__((always_inline)) {
+        if constexpr (decltype(when)::value == kBetween) load_u();
+      }, acc, t, row, tab1, tab5, tf1, ti, ends, sp + BLK / 2);
+      // results to 64 consecutive time steps per thread
       sync_threads<T>();
-      float* ps = stage + stage_phys(t);
+      float* ps = stage + stage_phys(anew(t));
       static_for<0, 32>([&](auto rr) {
         constexpr int r = decltype(rr)::value;
         ps[stage_phys(512 * r)] = acc[r].re;
         ps[stage_phys(H + 512 * r)] = acc[r].im;
       });
       sync_threads<T>();
+      const int n0 = 64 * anew(t);
       static_for<0, 8>([&](auto qq) {
         constexpr int q = decltype(qq)::value;
         const float4* at = reinterpret_cast<const float4*>(stage + stage_phys(n0) + 8 * q);
@@ -290,6 +326,71 @@ __global__ __launch_bounds__(P::T) __attribute__((amdgpu_waves_per_eu(2, 2))) vo
       });
       sync_threads<T>();                   // the next row's prologue overwrites what has just been read
     }
+  }
+}
+
+// A plain long convolution of one input, without short convolutions and gates: samples go straight from memory to the layout of the
+// first pass and back, consecutive lanes consecutive samples, so that nothing is staged and no barrier stands between rows; the
+// samples are read twice, the second time and the next row's first under a last pass.
+template <class P, typename ACT>
+__global__ __launch_bounds__(P::T) __attribute__((amdgpu_waves_per_eu(2, 2))) void conv_real_kernel(
+    const ACT* __restrict__ x, const float* __restrict__ spec, ACT* __restrict__ y, int B, int d) {
+  constexpr int T = P::T, H = P::H;
+  constexpr long LS = 2L * H, BLK = real_spec_block<P>();
+  static_assert(T == 512 && P::E == 32 && P::NB1 == 1 && P::S1 == 512, "first-pass layout");
+  extern __shared__ float2 lds[];
+  float2* row = lds;
+  const float2 *tab1 = lds + P::ROW, *tab5 = tab1 + P::TAB;
+  const int t = threadIdx.x;
+
+  tables_init<P, 1>(lds + P::ROW);
+  tables_init<P, 5>(lds + P::ROW + P::TAB);
+  TwistForward<P, 1> tf1;
+  TwistInverse<P> ti;
+  tf1.init(t);
+  ti.init(t);
+  float4* ends = ends_init<P>(lds, t);
+  sync_threads<T>();
+
+  const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3, slots = gridDim.x >> 3;
+  const int rows_per_xcd = (d >> 3) * B;
+  ACT lo[32], hi[32];
+  auto value = [](ACT v) __attribute__((always_inline)) -> float {
+    if constexpr (sizeof(ACT) == 2) return bf16_to_f32(v); else return v;
+  };
+  auto get_lo = [&](auto rr) __attribute__((always_inline)) { return value(lo[decltype(rr)::value]); };
+  auto get_hi = [&](auto rr) __attribute__((always_inline)) { return value(hi[decltype(rr)::value]); };
+  auto load = [&](int j) __attribute__((always_inline)) {
+    const int c = __builtin_amdgcn_readfirstlane((j / B) * 8 + xcd), bb = __builtin_amdgcn_readfirstlane(j % B);
+    int again = 0;
+    asm volatile("" : "+s"(again));      // a load of its own, not an earlier one's registers kept
+    const ACT* p = x + ((long)c * B + bb) * LS + again;
+    static_for<0, 32>([&](auto rr) {
+      constexpr int r = decltype(rr)::value;
+      lo[r] = (p + 512 * r)[(unsigned)t];
+      hi[r] = (p + H + 512 * r)[(unsigned)t];
+    });
+  };
+  if (slot < rows_per_xcd) load(slot);
+  for (int j = slot; j < rows_per_xcd; j += slots) {
+    const int c = __builtin_amdgcn_readfirstlane((j / B) * 8 + xcd), bb = __builtin_amdgcn_readfirstlane(j % B);
+    cf acc[32];
+    static_for<0, 32>([&](auto rr) { acc[decltype(rr)::value] = {0.f, 0.f}; });
+    convolve_halves<P>(get_lo, get_hi, [&](auto when) __attribute__((always_inline)) {
+      if constexpr (decltype(when)::value == kUnder1st) load(j);
+      if constexpr (decltype(when)::value == kUnder2nd) load(j + slots < rows_per_xcd ? j + slots : j);
+    }, acc, t, row, tab1, tab5, tf1, ti, ends, reinterpret_cast<const float4*>(spec + (long)c * 4 * BLK));
+    ACT* py = y + ((long)c * B + bb) * LS;
+    static_for<0, 32>([&](auto rr) {
+      constexpr int r = decltype(rr)::value;
+      if constexpr (sizeof(ACT) == 2) {
+        (py + 512 * r)[(unsigned)t] = f32_to_bf16(acc[r].re);
+        (py + H + 512 * r)[(unsigned)t] = f32_to_bf16(acc[r].im);
+      } else {
+        (py + 512 * r)[(unsigned)t] = acc[r].re;
+        (py + H + 512 * r)[(unsigned)t] = acc[r].im;
+      }
+    });
   }
 }
 
@@ -371,19 +472,22 @@ template <typename ACT>
 static int launch_mixer_real(const void* xproj, long ldx, const float* u, const float* sw, const float* sb, const float* pbias,
                              const float* spec, void* y, int B, int d, hipStream_t stream) {
   typedef RealPlan P;
-  const size_t lds_bytes = (size_t)(P::ROW + 2 * P::TAB) * sizeof(float2);
-  auto kern = sw ? (u ? mixer_real_kernel<P, ACT, true, true> : mixer_real_kernel<P, ACT, true, false>)
-                 : mixer_real_kernel<P, ACT, false, false>;
+  const size_t lds_bytes = real_lds_bytes<P>();
+  const void* kern = !sw ? (const void*)conv_real_kernel<P, ACT>
+                         : u ? (const void*)mixer_real_kernel<P, ACT, true> : (const void*)mixer_real_kernel<P, ACT, false>;
   if (!sw && u) return set_error(M2_ERR_ARG, "mixer_real: a plain convolution takes no second input");
-  hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes);
+  hipError_t e = hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes);
   if (e != hipSuccess) return set_error(M2_ERR_LAUNCH, "hipFuncSetAttribute(mixer_real): %s", hipGetErrorString(e));
   const int rows_per_xcd = (d / 8) * B;
-  int slots = num_cus() / 8;          // one workgroup per compute unit (140 KB of LDS)
+  int slots = num_cus() / 8;          // one workgroup per compute unit (158 KB of LDS)
   if (slots > rows_per_xcd) slots = rows_per_xcd;
   const int rounds = (rows_per_xcd + slots - 1) / slots;      // every workgroup the same number of rows
   slots = (rows_per_xcd + rounds - 1) / rounds;
-  hipLaunchKernelGGL(kern, dim3(8 * slots), dim3(P::T), lds_bytes, stream, (const ACT*)xproj, ldx, u, sw, sb, pbias, spec,
-                     (ACT*)y, B, d);
+  if (!sw)
+    hipLaunchKernelGGL((conv_real_kernel<P, ACT>), dim3(8 * slots), dim3(P::T), lds_bytes, stream, (const ACT*)xproj, spec, (ACT*)y, B, d);
+  else
+    hipLaunchKernelGGL((u ? mixer_real_kernel<P, ACT, true> : mixer_real_kernel<P, ACT, false>), dim3(8 * slots), dim3(P::T), lds_bytes,
+                       stream, (const ACT*)xproj, ldx, u, sw, sb, pbias, spec, (ACT*)y, B, d);
   return check_launch("mixer_real");
 }
 
