@@ -8,7 +8,8 @@
 //
 // us (bf16, d = 768), against two half transforms of both signals packed: L = 8192, B = 4 171 / 184 (15 % fewer vector instructions;
 // the ALU is 72 % busy, LDS a third of the time, and the two overlap only across the workgroups of a unit), L = 16384, B = 2 189 / 218.
-// Requesting the next row's inputs under the epilogue gained nothing measurable at B = 4 and 3 % with fp32 inputs.
+// Requesting the next row's inputs under the epilogue gained nothing measurable at B = 4 and 3 % with fp32 inputs.  Addresses are formed
+// anew where they are used: kept, they had up to 108 bytes per lane spilled (fp32, L = 16384, B = 1 / 2: 145 / 263, now 130 / 248).
 //
 // Stands in for the same reference code as fftconv_kernels.hip (bert/src/mm/hyena_utils.py:16-42,
 // 231-236; bert/src/mm/monarch_mixer_sequence_mixer.py:112-147).
@@ -41,7 +42,6 @@ __global__ __launch_bounds__(P::T) __attribute__((amdgpu_waves_per_eu(2, 2))) vo
   float2* row = lds;
   const float2* tab = lds + P::ROW;
   const int t = threadIdx.x;
-  const int n0 = 32 * t;
 
   tables_init<P, kQuarter>(lds + P::ROW);
   TwistForward<P, kQuarter> tf;
@@ -61,7 +61,7 @@ __global__ __launch_bounds__(P::T) __attribute__((amdgpu_waves_per_eu(2, 2))) vo
   RawRow<ACT, 4, true> r1, r2, rv;      // the four accesses of a thread are consecutive
   f32x4_t ru[8];
   auto fetch_row = [&](int j) __attribute__((always_inline)) {
-    const int c = (j / B) * 8 + xcd, bb = j % B;
+    const int c = (j / B) * 8 + xcd, bb = j % B, n0 = 32 * anew(t);
     static_for<0, 4>([&](auto qq) {
       constexpr int q = decltype(qq)::value;
       const int n = n0 + 8 * q;
@@ -106,6 +106,7 @@ __global__ __launch_bounds__(P::T) __attribute__((amdgpu_waves_per_eu(2, 2))) vo
       // of a row, where one or two taps fall on the zero padding (outside the biased signal): those are corrected.
       const float f1 = b1 + p1 * (w1[0] + w1[1] + w1[2]), f2 = b2 + p2 * (w2[0] + w2[1] + w2[2]),
                   fv = bv + pv * (wv[0] + wv[1] + wv[2]);
+      const int n0 = 32 * anew(t);
       __builtin_amdgcn_sched_barrier(0);
       static_for<0, 4>([&](auto qq) {
         constexpr int q = decltype(qq)::value;
@@ -160,9 +161,10 @@ __global__ __launch_bounds__(P::T) __attribute__((amdgpu_waves_per_eu(2, 2))) vo
     const float4* sp = spec + (long)c * 2 * (E / 2) * T;
     cf x[E];
     float u[E], ya[E];
+    const int t0 = anew(t);
     static_for<0, P::NB1>([&](auto ii) {
       constexpr int i = decltype(ii)::value;
-      const float2* pb = row + P::phys(t + T * i);
+      const float2* pb = row + P::phys(t0 + T * i);
       static_for<0, P::R1>([&](auto jj) {
         constexpr int r = i * P::R1 + decltype(jj)::value;
         const cf v = lds_get(pb, P::phys(decltype(jj)::value * P::S1));
@@ -170,16 +172,17 @@ __global__ __launch_bounds__(P::T) __attribute__((amdgpu_waves_per_eu(2, 2))) vo
         u[r] = v.im;
       });
     });
-    convolve<P, kQuarter, true>(x, t, row, tab, tf, ti, sp);
+    convolve<P, kQuarter, true>(x, anew(t), row, tab, tf, ti, sp);
     static_for<0, E>([&](auto rr) {
       constexpr int r = decltype(rr)::value;
       ya[r] = end_real<P, kQuarter, r>(x, te);
       x[r] = {u[r], 0.f};
     });
-    if constexpr (HAS_U) convolve<P, kQuarter, true>(x, t, row, tab, tf, ti, sp + (E / 2) * T);
+    if constexpr (HAS_U) convolve<P, kQuarter, true>(x, anew(t), row, tab, tf, ti, sp + (E / 2) * T);
+    const int t1 = anew(t);
     static_for<0, P::NB1>([&](auto ii) {
       constexpr int i = decltype(ii)::value;
-      float2* pb = row + P::phys(t + T * i);
+      float2* pb = row + P::phys(t1 + T * i);
       static_for<0, P::R1>([&](auto jj) {
         constexpr int r = i * P::R1 + decltype(jj)::value;
         lds_put(pb, P::phys(decltype(jj)::value * P::S1), cf{ya[r], HAS_U ? end_real<P, kQuarter, r>(x, te) : 0.f});
@@ -200,6 +203,7 @@ __global__ __launch_bounds__(P::T) __attribute__((amdgpu_waves_per_eu(2, 2))) vo
     sync_threads<T>();
 
     // ---- epilogue: 32 consecutive outputs per thread
+    const int n0 = 32 * anew(t);
     static_for<0, 4>([&](auto qq) {
       constexpr int q = decltype(qq)::value;
       const int n = n0 + 8 * q;
