@@ -41,15 +41,17 @@ constexpr double cos_quadrant(double x) {
   }
   return sum;
 }
-constexpr float root_cos(long k, long n) {
+constexpr double root_cos64(long k, long n) {
   k = ((k % n) + n) % n;
   const long quadrant = 4 * k / n, rest = 4 * k - quadrant * n;      // angle = pi / 2 (quadrant + rest / n)
   const double half_pi = 1.57079632679489661923;
   // an angle and its distance to the next quadrant: the cosine of the one is the sine of the other
   const double c = rest == 0 ? 1.0 : cos_quadrant(half_pi * (double)rest / (double)n);
   const double s = rest == 0 ? 0.0 : cos_quadrant(half_pi * (double)(n - rest) / (double)n);
-  return (float)(quadrant == 0 ? c : quadrant == 1 ? -s : quadrant == 2 ? -c : s);
+  return quadrant == 0 ? c : quadrant == 1 ? -s : quadrant == 2 ? -c : s;
 }
+constexpr double root_sin64(long k, long n) { return root_cos64(4 * k - n, 4 * n); }
+constexpr float root_cos(long k, long n) { return (float)root_cos64(k, n); }
 constexpr float root_sin(long k, long n) { return root_cos(4 * k - n, 4 * n); }
 
 // v exp(-2 pi i K / N), or with CONJ v exp(+2 pi i K / N)

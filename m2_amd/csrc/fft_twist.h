@@ -475,6 +475,108 @@ __device__ __forceinline__ void transform(cf (&x)[P::E], int t, float2* row, con
   static_for<0, P::NG>([&](auto gg) { fwd_group<P, decltype(gg)::value>(x, t, tab, tf); });
 }
 
+// The forward half with fp64 butterflies, for the spectra of the shortest rows: values are rounded to fp32 between the passes and at
+// the end.  A signal meets its transform's rounding once, a filter's errors every signal alike: with these spectra the
+// core at L = 128 is 1.9e-7 from fp64, with fp32 butterflies 2.2e-7 where the transform of 2 L points of both signals packed, which
+// this took over from, had 1.9e-7; from L = 256 on fp32 butterflies come out no further off than that one.  (us for the filters
+// of 1 / 12 mixers of 768 channels: 27 / 54, with fp32 butterflies 28 / 51.5, with the packed transform 27 / 53.4.)
+template <class P>
+constexpr bool fine_spectrum() { return P::H == 128; }
+struct cd {
+  double re, im;
+};
+// factors of the last pass as in tables_init: row r, stage and number
+template <class P, int S8>
+struct FineTable {
+  double v[P::R1][P::R3 / 2][2];
+  constexpr FineTable() : v{} {
+    for (int r = 0; r < P::R1; ++r)
+      for (int n = 0; n < P::R3 / 2; ++n) {
+        const int S = ilog2(2 * n + 1), e = n == 0 ? 0 : n - (1 << (S - 1));
+        v[r][n][0] = root_cos64(8 * r + S8 + e * 8 * P::R1, 16 * P::R1 << S);
+        v[r][n][1] = -root_sin64(8 * r + S8 + e * 8 * P::R1, 16 * P::R1 << S);
+      }
+  }
+};
+template <class P, int S8>
+__device__ constexpr FineTable<P, S8> kFineTable{};
+// the factors of the thread's group
+template <class P, int S8>
+struct FineForward {
+  cd f[P::R3 / 2];
+  __device__ __forceinline__ void load(int t) {
+    static_for<0, P::R3 / 2>([&](auto nn) {
+      constexpr int n = decltype(nn)::value;
+      f[n] = {kFineTable<P, S8>.v[t][n][0], kFineTable<P, S8>.v[t][n][1]};
+    });
+  }
+};
+__device__ __forceinline__ void butterfly(cd& a, cd& b, double wr, double wi) {
+  const cd s = {fma(-wi, b.im, fma(wr, b.re, a.re)), fma(wi, b.re, fma(wr, b.im, a.im))};
+  b = {fma(2.0, a.re, -s.re), fma(2.0, a.im, -s.im)};
+  a = s;
+}
+template <class P, int S8>
+__device__ __forceinline__ void transform_fine(cf (&x)[P::E], int t, float2* row, const FineForward<P, S8>& ff) {
+  static_for<0, P::NB1>([&](auto ii) {
+    constexpr int i = decltype(ii)::value, R = P::R1;
+    cd z[R];
+    static_for<0, R>([&](auto rr) { z[decltype(rr)::value] = {x[i * R + decltype(rr)::value].re, x[i * R + decltype(rr)::value].im}; });
+    static_for<0, ilog2(R)>([&](auto ss) {
+      constexpr int S = decltype(ss)::value, h = R >> (S + 1);
+      static_for<0, (1 << S)>([&](auto bb) {
+        constexpr int b = decltype(bb)::value, k = S8 + 8 * bitrev(b, S), n = 16 << S, at = 2 * h * b;
+        constexpr double wr = root_cos64(k, n), wi = -root_sin64(k, n);
+        static_for<0, h>([&](auto jj) { butterfly(z[at + decltype(jj)::value], z[at + h + decltype(jj)::value], wr, wi); });
+      });
+    });
+    float2* pb = row + P::phys(t + P::T * i);
+    static_for<0, R>([&](auto rr) {
+      constexpr int r = decltype(rr)::value;
+      lds_put(pb, P::phys(bitrev(r, ilog2(R)) * P::S1), cf{(float)z[r].re, (float)z[r].im});
+    });
+  });
+  sync_threads<P::T>();
+  constexpr int R = P::R3;
+  static_assert(P::NG == 1, "one group per thread");
+  cd z[R];
+  const float2* pg = row + P::phys(R * t);
+  static_for<0, R>([&](auto jj) {
+    const cf v = lds_get(pg, decltype(jj)::value);
+    z[decltype(jj)::value] = {v.re, v.im};
+  });
+  static_for<0, ilog2(R)>([&](auto ss) {
+    constexpr int S = decltype(ss)::value, h = R >> (S + 1);
+    static_for<0, (1 << S)>([&](auto bb) {
+      constexpr int b = decltype(bb)::value, e = bitrev(b, S), half = S > 0 ? (1 << S) / 2 : 1, at = 2 * h * b;
+      const cd w = ff.f[S == 0 ? 0 : half + e % half];
+      constexpr bool rot = S > 0 && e >= half;      // the other half of a stage's factors: times -i
+      static_for<0, h>([&](auto jj) {
+        butterfly(z[at + decltype(jj)::value], z[at + h + decltype(jj)::value], rot ? w.im : w.re, rot ? -w.re : w.im);
+      });
+    });
+  });
+  static_for<0, R>([&](auto rr) { x[decltype(rr)::value] = {(float)z[decltype(rr)::value].re, (float)z[decltype(rr)::value].im}; });
+}
+// the forward transform of a spectrum kernel: what it keeps, and the passes
+template <class P, int S8>
+struct SpectrumForward {
+  typename std::conditional<fine_spectrum<P>(), FineForward<P, S8>, TwistForward<P, S8>>::type tf;
+  // (by all threads of the workgroup; a barrier has to follow)
+  __device__ __forceinline__ void init(int t, float2* tab) {
+    if constexpr (fine_spectrum<P>()) {
+      tf.load(t);
+    } else {
+      tables_init<P, S8>(tab);
+      tf.init(t);
+    }
+  }
+  __device__ __forceinline__ void operator()(cf (&x)[P::E], int t, float2* row, const float2* tab) const {
+    if constexpr (fine_spectrum<P>()) transform_fine<P, S8>(x, t, row, tf);
+    else transform<P, S8>(x, t, row, tab, tf);
+  }
+};
+
 // half transforms and rows by sequence length; the shift of one signal's ring (z^L = -i) in eighths
 constexpr int kQuarter = 2;
 typedef TwistPlan<7, 8, 1, 16, 16> Twist128;

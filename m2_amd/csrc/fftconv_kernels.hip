@@ -289,9 +289,8 @@ __global__ __launch_bounds__(SpectrumLayout<P>::WG) __attribute__((amdgpu_waves_
     select_mixer(sb, d, 2 * L, taps1, taps2, D1, D2, sp);
     spec = reinterpret_cast<float4*>(sp);
   }
-  tables_init<P, kQuarter>(lds + RPW * P::ROW);
-  TwistForward<P, kQuarter> tf;
-  tf.init(t);
+  SpectrumForward<P, kQuarter> forward;
+  forward.init(t, lds + RPW * P::ROW);
   __syncthreads();
 
   for (int i0 = blockIdx.x * RPW; i0 < 2 * d; i0 += gridDim.x * RPW) {
@@ -310,7 +309,7 @@ __global__ __launch_bounds__(SpectrumLayout<P>::WG) __attribute__((amdgpu_waves_
       static_for<0, E>([&](auto rr) { x[decltype(rr)::value] = {0.f, 0.f}; });
     }
     sync_threads<T>();                       // the item before has been read
-    transform<P, kQuarter>(x, t, row, tab, tf);
+    forward(x, t, row, tab);
     if (i0 + rloc < 2 * d) store_spectrum<P>(x, 1.f / (float)L, spec + (long)item * (E / 2) * T + t);
   }
 }

@@ -34,8 +34,9 @@ __global__ __launch_bounds__(2 * kFusedRows * P::T) void project_spectrum_kernel
   constexpr int L = P::H, T = P::T, NT = 2 * kFusedRows * T, NW = NT / 64;
   extern __shared__ float2 lds[];
   float2* factors = lds + 2 * kFusedRows * P::ROW;
-  tables_init<P, kQuarter>(factors);
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, i16 = lane & 15, q4 = lane >> 4;
+  SpectrumForward<P, kQuarter> forward;
+  forward.init(tid % T, factors);
   const int mixer = blockIdx.y, c0 = blockIdx.x * kFusedRows;
   const int nmlp = 2 * fpm;
 
@@ -128,8 +129,6 @@ __global__ __launch_bounds__(2 * kFusedRows * P::T) void project_spectrum_kernel
   // ---- phase 2: one row per T threads ----
   const int rloc = threadIdx.x / T, t = threadIdx.x % T, which = rloc & 1, c = c0 + (rloc >> 1);
   float2* row = lds + rloc * P::ROW;
-  TwistForward<P, kQuarter> tf;
-  tf.init(t);
   __syncthreads();
   cf x[P::E];
   static_for<0, P::E>([&](auto rr) {
@@ -140,7 +139,7 @@ __global__ __launch_bounds__(2 * kFusedRows * P::T) void project_spectrum_kernel
     const float* D = skip[mixer * fpm + which];
     if (D) x[0].re += D[c];
   }
-  transform<P, kQuarter>(x, t, row, factors, tf);
+  forward(x, t, row, factors);
   store_spectrum<P>(x, 1.f / (float)L, spec + (long)mixer * spec_stride4 + ((long)c * 2 + which) * (P::E / 2) * T + t);
 }
 

@@ -37,3 +37,16 @@ def test_mixer_core_rows(gpu, L, d, B, act):
     plain = ops.fftconv(u.to(act).to(gpu), spec, B, L, d).double().cpu()
     ref = _conv(u.to(act).double(), taps[0], D[0])
     assert (plain - ref).norm() <= tol * ref.norm()
+
+
+def test_spectra_of_the_shortest_rows(gpu):
+    """At L = 128 the filters' transform is rounded twice and not in every stage: what is left are the two transforms of the signal, 14
+    stages of two and a half roundings of 2^-25 in the root mean square, and half a dozen others.  (With a filter transform in
+    fp32 the 8192 rows come out at 2.1e-7.)"""
+    from m2_amd import ops
+    L, d, B = 128, 256, 32
+    g = torch.Generator(device=gpu).manual_seed(0)
+    k, x = torch.randn(d, 2 * L, generator=g, device=gpu), torch.randn(d, B, L, generator=g, device=gpu)
+    y = ops.fftconv(x, ops.filter_spectrum(k, None, None, None), B, L, d)
+    ref = _conv(x.double(), k, torch.zeros(d, device=gpu))
+    assert (y - ref).norm() <= (2.5 * 14 + 6) ** 0.5 * 2.0 ** -25 * ref.norm()
