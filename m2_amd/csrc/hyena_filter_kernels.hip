@@ -43,6 +43,13 @@ __device__ __forceinline__ float sin_reduced(float x) {
   return __uint_as_float(__float_as_uint(s) ^ ((uint32_t)static_cast<int>(n) << 31));      // odd n: the other sign
 }
 
+// The last hidden layer's, whose fp16 parts end at 8: beyond |x| = 3e7 the reduction leaves arguments of any size, and what the polynomial
+// makes of them is no sine, but it has to stay a number.  NaN stays NaN.
+__device__ __forceinline__ float sin_bounded(float x) {
+  const float s = sin_reduced(x);
+  return fabsf(s) > 2.f ? copysignf(1.f, s) : s;
+}
+
 // The 128 x 128 weights of the two inner layers, split into three bf16 parts and laid out as MFMA A operands, so
 // that hidden_kernel fetches them with coalesced 16-byte loads and no arithmetic:
 // wsplit[mlp][layer][part][wave w][K step ks][lane (i, h)] = 8 bf16 of row 32 w + i, K = 16 ks + 8 h .. + 7.
@@ -247,7 +254,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       const int o = 32 * w + 8 * vq + 4 * half;
       float s[4];
 #pragma unroll
-      for (int j = 0; j < 4; ++j) s[j] = sin_reduced(fr[4 * vq + j] * (acc[4 * vq + j] + bs[4 * vq + j]));
+      for (int j = 0; j < 4; ++j) {
+        const float arg = fr[4 * vq + j] * (acc[4 * vq + j] + bs[4 * vq + j]);
+        s[j] = layer == 0 ? sin_reduced(arg) : sin_bounded(arg);
+      }
       if constexpr (layer == 0) {
         put3(pos, o, s);
       } else if constexpr (PROJECT) {           // h3 stays in LDS (parts 0 and 1) for the projection

@@ -83,3 +83,26 @@ def test_inner_layers_keep_all_bits(gpu, L):
     arg = w2.double() * torch.sin(w1.double() * torch.sin(b0.double()))
     err = (taps - torch.sin(arg)[:, None]) / arg[:, None]
     assert err.pow(2).mean().sqrt() <= 2 * 2.0 ** -24
+
+
+@pytest.mark.parametrize("L,d", [(128, 64), (1024, 64)])
+def test_arguments_without_a_sine_left(gpu, L, d):
+    """fp32 arguments beyond 3e7 leave the sines wrong, but the taps finite and no larger than sines make them, on every route; NaN
+    stays NaN."""
+    import m2_amd
+    g = torch.Generator().manual_seed(L)
+    mixer = m2_amd.MonarchMixerSequenceMixing(d, l_max=L, bidirectional=True, hyena_emb_dim=5, hyena_filter_order=128,
+                                              residual_long_conv=True)
+    fn = mixer.filter_fn
+    with torch.no_grad():
+        for f in (fn, mixer.filter_fn2):
+            for mlp in (f.implicit_filter, f.implicit_filter_rev):
+                mlp[4].weight.normal_(0.0, 1.0, generator=g).mul_(10.0 ** torch.randint(6, 12, (128, 1), generator=g))
+    most = torch.stack([m[6].weight.detach().abs().sum(1) for m in (fn.implicit_filter, fn.implicit_filter_rev)]).amax(0).to(gpu)
+    mixer = mixer.to(gpu)
+    taps = fn.bidirectional_taps(L)
+    assert (taps.abs() <= 1.001 * most[:, None] * (1 + abs(float(fn.modulation.shift)))).all()
+    assert torch.isfinite(mixer.filter_spectrum(L)).all()
+    with torch.no_grad():
+        fn.implicit_filter[4].bias[0] = float("nan")
+    assert not torch.isfinite(fn.bidirectional_taps(L)[:, :L]).any()
