@@ -290,7 +290,8 @@ class BertLayer(nn.Module):
         d = at.d_model
         if at.hyena_training_additions:      # extra input LayerNorm: needs the fp32 form, replaces h16 / hT
             _, h16, hT = at.pre_norm(h32, want_f32=False, want_bf16=True)
-        xproj = at.projected(h16, B, L)              # channel-major, bias added in the core
+        # channel-major, bias added in the core; an attention module of a caller's own need only have project_in, core and project_out
+        xproj = at.projected(h16, B, L) if isinstance(at, MonarchMixerSequenceMixing) else at.project_in(h16).view(3 * d, B, L)
         if spec_ready is not None:
             torch.cuda.current_stream().wait_event(spec_ready)
         y = at.core(xproj, hT.view(d, B, L) if at.residual_long_conv else None, B, L, spec=spec)

@@ -140,9 +140,9 @@ class MonarchMixerSequenceMixing(nn.Module):
 
     def projected(self, x: torch.Tensor, B: int, L: int) -> torch.Tensor:
         """project_in as the core takes it: (3d, B, L), or (3d, row) where a row a little longer than B L is faster to write.  (A class
-        of a caller's own may have a core or a projection that knows no such rows.)"""
+        of a caller's own, or a method put in the place of one of these two, may know no such rows.)"""
         M, d = x.shape
-        if type(self) is MonarchMixerSequenceMixing and x.dtype == torch.bfloat16 and ops.channels_row(M, d) != M:
+        if x.dtype == torch.bfloat16 and ops.channels_row(M, d) != M and knows_rows(self):
             return self.project_in(x, wide=True)
         return self.project_in(x).view(3 * d, B, L)
 
@@ -208,7 +208,8 @@ class MonarchMixerSequenceMixing(nn.Module):
                 xproj = ops.split_to_channels(parts, w_in, B * L, 3 * d, d).view(3 * d, B, L)
                 u_cm = x_cm if u_cm is None else u_cm
             else:
-                xproj = self.projected(x, B, L)                                          # (3d, B, L), bias added in the core
+                # (3d, B, L), bias added in the core
+                xproj = self.projected(x, B, L) if low else self.project_in(x).view(3 * d, B, L)
             if u_cm is None and self.residual_long_conv:
                 u_cm = u2.float().t().contiguous()                                       # (d, B*L)
             if not self.residual_long_conv:
@@ -216,3 +217,13 @@ class MonarchMixerSequenceMixing(nn.Module):
             y = self.core(xproj, None if u_cm is None else u_cm.view(d, B, L), B, L)
             out = self.project_out(y.view(d, B * L), w_out)                             # (B*L, d)
         return out.view(B, L, d), None
+
+
+_OWN = MonarchMixerSequenceMixing.project_in, MonarchMixerSequenceMixing.core
+
+
+def knows_rows(mixer) -> bool:
+    """Whether the mixer's projection and core are the ones of this file, which agree on rows longer than B L."""
+    cls = type(mixer)
+    return (cls is MonarchMixerSequenceMixing and (cls.project_in, cls.core) == _OWN
+            and not {"project_in", "core"} & mixer.__dict__.keys())
