@@ -6,12 +6,8 @@ import torch
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("L,d", [(128, 64), (1024, 64), (1088, 192), (1024, 320), (2048, 192)])
-def test_taps_of_rows_of_any_size(gpu, L, d):
-    import m2_amd
-    from oracle import m2_oracle as O
-    g = torch.Generator().manual_seed(L + d)
-    fn = m2_amd.HyenaFilter(d, emb_dim=5, order=128, seq_len=L, bidirectional=True, w=10)
+def _uneven(fn, d, g):
+    """Weights of the implicit filters whose rows are of very different sizes."""
     with torch.no_grad():
         for name, p in fn.named_parameters():
             leaf = name.rsplit(".", 1)[-1]
@@ -26,17 +22,57 @@ def test_taps_of_rows_of_any_size(gpu, L, d):
                 p[5, 7] *= 64.0
                 if not last:
                     p[9] *= 2.0 ** -60
-    sd = {k: v.detach().clone().double() for k, v in fn.state_dict().items()}
+
+
+def _reference(fn, L, dtype, bidirectional=True):
+    from oracle import m2_oracle as O
+    sd = {k: v.detach().cpu().to(dtype) for k, v in fn.state_dict().items()}
+    fwd, rev = (O.hyena_filter_taps(sd, "", L, rev=r)[0].T if bidirectional or not r else None for r in (False, True))
+    return O.bidirectional_kernel(fwd, torch.zeros_like(fwd) if rev is None else rev, L)
+
+
+@pytest.mark.parametrize("L,d", [(128, 64), (1024, 64), (1088, 192), (1024, 320), (2048, 192)])
+def test_taps_of_rows_of_any_size(gpu, L, d):
+    import m2_amd
+    g = torch.Generator().manual_seed(L + d)
+    fn = m2_amd.HyenaFilter(d, emb_dim=5, order=128, seq_len=L, bidirectional=True, w=10)
+    _uneven(fn, d, g)
+    ref, ref32 = _reference(fn, L, torch.float64), _reference(fn, L, torch.float32).double()
     taps = fn.to(gpu).bidirectional_taps(L).double().cpu()
-    ref = O.bidirectional_kernel(*(O.hyena_filter_taps(sd, "", L, rev=r)[0].T for r in (False, True)), L)
-    sd32 = {k: v.float() for k, v in sd.items()}
-    ref32 = O.bidirectional_kernel(*(O.hyena_filter_taps(sd32, "", L, rev=r)[0].T for r in (False, True)), L).double()
     assert torch.isfinite(taps).all()
     # channel by channel: products good to a few 2^-24 each, and what fp32 arithmetic itself makes of sin(10 x)
     norm = ref.norm(dim=1)
     err, err32 = (taps - ref).norm(dim=1), (ref32 - ref).norm(dim=1)
     assert (err <= 8 * 2.0 ** -24 * norm + 4 * err32).all(), (err / norm.clamp_min(1e-300)).max()
     assert not taps[3].any()
+
+
+@pytest.mark.parametrize("bidirectional", [True, False])
+@pytest.mark.parametrize("fpm", [1, 2])
+@pytest.mark.parametrize("L", [128, 256, 512])
+def test_spectra_of_rows_of_any_size(gpu, L, fpm, bidirectional):
+    """The kernel that projects and transforms in one, on two mixers with such rows: against spectra of fp64 taps, channel by channel
+    and filter by filter."""
+    import m2_amd
+    from m2_amd import ops
+    d, g = 64, torch.Generator().manual_seed(L + fpm)
+    fns = [m2_amd.HyenaFilter(d, emb_dim=5, order=128, seq_len=L, bidirectional=bidirectional, w=10) for _ in range(2 * fpm)]
+    for fn in fns:
+        _uneven(fn, d, g)
+    refs = [[_reference(fn, L, t, bidirectional).float().to(gpu) for t in (torch.float64, torch.float32)] for fn in fns]
+    groups = [fns[i:i + fpm] for i in range(0, 2 * fpm, fpm)]
+    table = ops.FilterTable([[f.to(gpu).kernel_params("both") for f in m] for m in groups], [[None] * fpm] * 2, L, d, 128, 5)
+    spectra = ops.mixer_filter_spectra(table, w_mod=1.0, shift=float(fns[0].modulation.shift)).view(2, d, 2, 2 * L).double()
+    for m in range(2):
+        for f in range(2):
+            if f >= fpm:
+                assert not spectra[m, :, f].any()
+                continue
+            want, want32 = (ops.filter_spectrum(t, None, None, None).view(d, 2, 2 * L)[:, 0].double() for t in refs[m * fpm + f])
+            norm, err, err32 = want.norm(dim=1), (spectra[m, :, f] - want).norm(dim=1), (want32 - want).norm(dim=1)
+            # as for the taps, and the roundings of either transform
+            assert (err <= 12 * 2.0 ** -24 * norm + 4 * err32).all(), (m, f, (err / norm.clamp_min(1e-30)).max())
+            assert not spectra[m, 3, f].any()
 
 
 def test_taps_of_infinite_and_large_weights(gpu):
