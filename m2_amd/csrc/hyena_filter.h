@@ -46,9 +46,11 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 //
 // The two 128 x 128 layers: either operand as three bf16 parts, x = hi + mid + lo, which hold all 24 bits of an fp32 value of any size,
 // and the six products down to 2^-24 of the whole one (mid lo, lo mid and lo lo, below 2^-24, are left out).  What such a layer loses,
-// sin(freq x) of the next one amplifies by its argument.  (Two fp16 parts and three products, as below, save half of the matrix
-// instructions, 5 to 10 % of filter generation, and with operands whose mantissas lie between two numbers of 11 bits they put every
-// argument off by 2.6e-7 of itself where fp32 products leave 0.6e-7.)
+// sin(freq x) of the next one amplifies by its argument.  So the five small products of a sum are added apart from the leading ones: in
+// one sum of all six each is a rounding of the whole, which leaves an argument off by 0.9e-7 of itself where it is 0.2e-7 now, and a
+// whole fp32 mixer 3.8e-7 from fp64 where it is 2.9e-7 now (L = 128; 4.3e-7 and 3.7e-7 at 8192).  (Two fp16 parts and three products, as
+// below, save half of the matrix instructions, 5 to 10 % of filter generation, and with operands whose mantissas lie between two numbers
+// of 11 bits they put every argument off by 2.6e-7 of itself.)
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 __device__ __forceinline__ void split3(float x, float& hi, float& mid, float& lo) {
   hi = bf16_to_f32(f32_to_bf16(x));
@@ -60,8 +62,9 @@ __device__ __forceinline__ void split3(float x, float& hi, float& mid, float& lo
 // The output projection, whose result nothing amplifies: two fp16 parts, x 2^e = hi + lo, three products (hi lo, lo hi, hi hi).  The
 // parts hold a value to 2^-23 of itself and the product left out is at most 2^-22 of the whole one (the error of a product is 2^-21
 // at most and 2^-23.7 in the root mean square).  fp16 has five bits of exponent: every row of the weight is scaled so that its largest
-// entry lies in [2^12, 2^13), activations by 2^13.  What is below 2^-13 of the largest has its low part among fp16's subnormal numbers
-// and is held to 2^-38 of the largest.  Two bf16 parts (16 bits, the same matrix instructions) left the taps at 4e-6 from fp64, these
+// entry lies in [2^12, 2^13), activations, of which 1 is the largest possible, by 2^13.  What is below 2^-13 of the largest has its low
+// part among fp16's subnormal numbers and is held to 2^-38 of the largest: of activations 2^-38, whatever their size (two bf16 parts
+// held 2^-17 of any value, which is more for activations that are all below 2^-21).  Two bf16 parts (16 bits, the same matrix instructions) left the taps at 4e-6 from fp64, these
 // leave them where fp32 arithmetic does, at 2e-7; a third part would double the instructions.
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
@@ -75,7 +78,7 @@ __device__ __forceinline__ void split2(float a, float b, uint32_t& hi, uint32_t&
   hi = __builtin_bit_cast(uint32_t, h);
   lo = __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{a - back.x, b - back.y}, f16x2));
 }
-// Scale of a row whose largest magnitude is m: 2^e.  (A row below 2^-47 is scaled by 2^60, no more: its reciprocal multiplies biases.)
+// Scale of a row whose largest magnitude is m: 2^e.  (A row below 2^-47 is scaled by 2^60, no more.)
 __device__ __forceinline__ float row_scale(float m) {
   int e = 12 - (int)((__float_as_uint(m) >> 23) & 0xff) + 127;      // -116 (infinity) ...
   e = e > 60 ? 60 : e;

@@ -216,8 +216,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   // layers 1, 2: D[o'][pos] = sum_o W[o'][o] act[pos][o].  A = weight rows 32 w + i32 (registers), B = positions of the
   // tile (LDS); lane (i32, half) holds K = 16 ks + 8 half .. + 7 of both.
   auto products = [&](int tile, floatx16& acc) __attribute__((always_inline)) {
+    floatx16 small;      // the products below the leading one, added at the end: the sum is rounded at its full size once a K step
 #pragma unroll
-    for (int v = 0; v < 16; ++v) acc[v] = 0.f;
+    for (int v = 0; v < 16; ++v) acc[v] = small[v] = 0.f;
     const int boff = (32 * tile + i32) * kActRowB + 16 * half;
 #pragma unroll
     for (int ks = 0; ks < 8; ++ks) {
@@ -225,13 +226,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       const bf16x8 bm = __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4*>(&act[1][boff + 32 * ks]));
       const bf16x8 bl = __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4*>(&act[2][boff + 32 * ks]));
       // smallest terms first
-      acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(al[ks], bh, acc, 0, 0, 0);
-      acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah[ks], bl, acc, 0, 0, 0);
-      acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(am[ks], bm, acc, 0, 0, 0);
-      acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(am[ks], bh, acc, 0, 0, 0);
-      acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah[ks], bm, acc, 0, 0, 0);
+      small = __builtin_amdgcn_mfma_f32_32x32x16_bf16(al[ks], bh, small, 0, 0, 0);
+      small = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah[ks], bl, small, 0, 0, 0);
+      small = __builtin_amdgcn_mfma_f32_32x32x16_bf16(am[ks], bm, small, 0, 0, 0);
+      small = __builtin_amdgcn_mfma_f32_32x32x16_bf16(am[ks], bh, small, 0, 0, 0);
+      small = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah[ks], bm, small, 0, 0, 0);
       acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah[ks], bh, acc, 0, 0, 0);
     }
+#pragma unroll
+    for (int v = 0; v < 16; ++v) acc[v] += small[v];
   };
   // accumulator element v: neuron 32 w + 8 (v / 4) + 4 half + v % 4, position i32 of the tile
   float fr[16], bs[16];
@@ -537,8 +540,8 @@ static int filter_launches(TAB tab, int nfilters, int L, int d, int emb_dim, flo
   if (rc) return rc;
   // Positions per workgroup: longer runs amortise the weight fetch (96 KB per workgroup and layer, 520 bytes per channel for the
   // projection), short sequences need the workgroups spread over the chip.  128 positions would leave one workgroup on a compute unit
-  // (104 KB of activations) and half of them idle for a single mixer.  us for the spectra of 1 / 12 mixers, d = 768: L = 1024 44 / 155,
-  // 4096 60 / 501, 8192 94 / 967; with inner layers in two fp16 parts and 128 positions 56 / 151, 71 / 457, 93 / 869.
+  // (104 KB of activations) and half of them idle for a single mixer.  us for the spectra of 1 / 12 mixers, d = 768: L = 1024 44 / 159,
+  // 4096 60 / 508, 8192 93 / 979; with inner layers in two fp16 parts and 128 positions 56 / 151, 71 / 457, 93 / 869.
   if (one_kernel) {
     hipLaunchKernelGGL((hidden_kernel<2, TAB, true>), dim3(L / 64, 2 * nfilters), dim3(256), 0, s, tab, L, emb_dim, w_mod, wsplit,
                        h_hi, h_lo, d, shift, w3split, w3scale, taps);

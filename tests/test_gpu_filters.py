@@ -121,6 +121,33 @@ def test_inner_layers_keep_all_bits(gpu, L):
     assert err.pow(2).mean().sqrt() <= 2 * 2.0 ** -24
 
 
+@pytest.mark.parametrize("L", [128, 1024])
+def test_inner_layers_round_their_sums_once_a_step(gpu, L):
+    """Sums of 128 positive products whose last sine, at arguments around 90, shows the sums' relative error.  The leading products
+    of a sum are added in eight steps, each a rounding (0.41 x 2^-24 in the root mean square) of what is there by then:
+    0.82 sqrt(sum (k / 8)^2) = 1.3 x 2^-25; the other 40 products are added apart.  (In one sum, 48 roundings would leave 3 x 2^-25.)"""
+    import m2_amd
+    d = n = 128
+    g = torch.Generator().manual_seed(L)
+    b0 = 0.01 + 0.01 * torch.rand(n, generator=g)
+    w1, w2 = 0.9 + 0.2 * torch.rand(n, generator=g), 32.0 + 32.0 * torch.rand(n, n, generator=g)
+    fn = m2_amd.HyenaFilter(d, emb_dim=5, order=n, seq_len=L, bidirectional=True, w=1)
+    with torch.no_grad():
+        for name, p in fn.named_parameters():
+            if "implicit_filter" in name and not name.endswith("freq"):
+                p.zero_()
+        fn.modulation.deltas.zero_()
+        for mlp in (fn.implicit_filter, fn.implicit_filter_rev):
+            mlp[0].bias.copy_(b0)
+            mlp[2].weight.copy_(torch.diag(w1))
+            mlp[4].weight.copy_(w2)
+            mlp[6].weight.copy_(torch.eye(n))
+    taps = fn.to(gpu).bidirectional_taps(L).double().cpu()
+    arg = w2.double() @ torch.sin(w1.double() * torch.sin(b0.double()))
+    err = (taps - torch.sin(arg)[:, None]) / arg[:, None]
+    assert err.pow(2).mean().sqrt() <= 1.5 * 2.0 ** -25
+
+
 @pytest.mark.parametrize("L,d", [(128, 64), (1024, 64)])
 def test_arguments_without_a_sine_left(gpu, L, d):
     """fp32 arguments beyond 3e7 leave the sines wrong, but the taps finite and no larger than sines make them, on every route; NaN
