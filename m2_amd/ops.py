@@ -290,22 +290,25 @@ def fftconv(x: Tensor, spec: Tensor, B: int, L: int, d: int) -> Tensor:
 
 
 # The library's own projection kernels against torch's (hipBLASLt), MI355X, us per call (own / torch):
-#   to_channels    d = 768: M = 2048 15 / 16, 4096 20 / 27, 8192 30 / 47, 16384 50 / 62, 31744 93 / 124; d = 960: 4096 27 / 25,
-#                  8192 49 / 49, 16384 101 / 85; d = 1536: 2048 36 / 30, 4096 66 / 58, 8192 120 / 102; d = 1792: 2048 42 / 46,
-#                  4096 91 / 72.  Below that torch's call costs 19 us whatever the size (its host side), own 8 .. 20.
+#   to_channels    d = 768 (kernels alone): M = 512 8.4 / 8.7, 1536 12.0 / 10.5, 2048 14.7 / 15.2, 3072 17.6 / 15.6, 4096 20 / 25, 5632 24.0 /
+#                  21.5, 6144 24.1 / 22.5, 7168 26.5 / 25.0, 8192 30 / 46, 10240 35 / 39, 16384 51 / 59, 32768 94 / 117, 49152 159 / 169,
+#                  57344 192 / 188, 65536 216 / 210, 81920 270 / 274, 131072 420 / 413; d = 960: 4096 27 / 25, 8192 49 / 49,
+#                  16384 101 / 85; d = 1536: 2048 36 / 30, 4096 66 / 58, 8192 120 / 102; d = 1792: 2048 42 / 46, 4096 91 / 72.
+#                  Below that torch's call costs 19 us whatever the size (its host side), own 8 .. 20.
 #   from_channels  d = 768: 4096 13 / 20, 16384 25 / 27, 32768 45 / 49; d = 960: 8192 23 / 29, 16384 36 / 48, 32768 69 / 74;
 #                  d = 1536: 2048 22 / 20, 4096 30 / 27, 8192 41 / 41, 16384 84 / 77; d = 1792: 4096 35 / 32, 8192 58 / 51.
-# So the own kernels serve products of up to about 29 GFLOP and every one of d = 768, whose weights fit the registers (to_channels),
-# and every one of d <= 1024 (from_channels).  At d >= 960 a
-# single product near that line is up to 20 % faster in the library; own ones serve it all the same, because a forward that uses them
+# So the own kernels serve products of up to about 29 GFLOP and those of d = 768, whose weights fit the registers, up to 49152 rows, beyond
+# which the two are within 4 % of each other either way (to_channels), and every one of d <= 1024 (from_channels).  At d >= 960 a
+# single product near that line is up to 20 % faster in the library, at d = 768 one of 1500 to 7200 rows up to 14 %; own ones serve it all the same, because a forward that uses them
 # for both projections is enqueued natively, and with them the streaming GLU and wo of few rows.  Whole forwards as captured graphs,
 # where the host costs nothing, all steps before / these (ms): 24 x 1536 M = 1024 3.98 / 2.70, 2048 4.37 / 3.74; 12 x 960 M = 2048
 # 1.57 / 1.13, 4096 1.97 / 1.79; 12 x 1792 M = 2048 3.14 / 2.22.
 _OWN_DENSE_FLOPS = 2.95e10
+_OWN_REGISTER_ROWS = 49152
 
 
 def own_to_channels(M: int, d: int) -> bool:
-    return (d == 768 or 6.0 * M * d * d <= _OWN_DENSE_FLOPS) and bool(lib.m2_dense_supported(M, 3 * d, d))
+    return (M <= _OWN_REGISTER_ROWS if d == 768 else 6.0 * M * d * d <= _OWN_DENSE_FLOPS) and bool(lib.m2_dense_supported(M, 3 * d, d))
 
 
 def native_rows(M: int, d: int) -> bool:

@@ -74,3 +74,18 @@ def test_layer_with_an_attention_module_of_another_class(gpu):
         want = layer.fused(*args)[0]
         layer.attention = _Other(layer.attention)
         assert torch.equal(layer.fused(*args)[0], want)
+
+
+@pytest.mark.parametrize("M,own", [(49152, True), (49280, False), (57344, False)])
+def test_projections_of_very_many_rows(gpu, M, own):
+    """On either side of the line beyond which the library's product takes over; a row a line apart is asked for on both."""
+    import m2_amd
+    from m2_amd import ops
+    assert ops.own_to_channels(M, 768) == own
+    g = torch.Generator(device=gpu).manual_seed(M)
+    mixer = m2_amd.MonarchMixerSequenceMixing(768, l_max=128, hyena_filter_order=128, hyena_emb_dim=5).to(gpu)
+    x = torch.randn(M, 768, generator=g, device=gpu).bfloat16()
+    with torch.no_grad():
+        got = mixer.projected(x, M // 128, 128).flatten(1)[:, :M]
+    want = mixer.in_linear.weight.detach().bfloat16().float() @ x.float().t()
+    assert (got.float() - want).norm() <= 2.0 ** -9 * want.norm() and (got.float() - want).abs().max() <= 2.0 ** -8 * want.abs().max()
