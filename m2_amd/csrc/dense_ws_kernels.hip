@@ -58,6 +58,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
   constexpr int K = 32 * KS, KG = (KS + 3) / 4, kSlab = KG * 8192, LD = 2 * KG, D = 3;
   static_assert(KS % D == 0 && KS % 4 == 0, "the operand ring closes over a slab; whole 256-byte pieces of a row");
   constexpr int kBar = KS - D + 1, kAcc = 64 / TJ;      // k steps whose weights sit in the accumulation registers
+  static_assert(3 * TJ >= 8, "the products between the last of a sum (k step KS - 1) and its reading (behind those of tile 0 of k step 1)");
+  static_assert(TJ + 1 < kBar, "results leave in k steps 1 .. TJ, the loads behind them and ahead of the barrier");
+  static_assert((STAGES - 2) * LD + TJ < 64 && 2 * TJ < 64, "what the waits count");
+  static_assert(8 * 16 * TJ * 128 <= kSlab + 16384, "the weights' way through LDS: the last stage and the room behind it");
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   const int tid = threadIdx.x, lane = tid & 63, i16 = lane & 15, q4 = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);

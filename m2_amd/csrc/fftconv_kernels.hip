@@ -106,8 +106,8 @@ __global__ __launch_bounds__(PairLayout<P>::WG) __attribute__((amdgpu_waves_per_
   // registers of batch i have been consumed by its prologue, and travel while batch i is transformed.  Without
   // this the workgroups of a compute unit, which start together, stay in step: all load, then all compute, and
   // memory time adds to arithmetic time instead of hiding behind it.
-  RawRow<ACT, Q, true> r1, r2, rv;
-  RawRow<float, Q, true> ru;
+  RawRow<ACT, Q> r1, r2, rv;
+  RawRow<float, Q> ru;
   static_for<0, Q>([&](auto q) { ru.a[decltype(q)::value] = ru.b[decltype(q)::value] = f32x4_t{0.f, 0.f, 0.f, 0.f}; });
   float cst = 0.f;
   auto fetch_batch = [&](int j0) __attribute__((always_inline)) {

@@ -58,7 +58,7 @@ __global__ __launch_bounds__(P::T) __attribute__((amdgpu_waves_per_eu(2, 2))) vo
   const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3, slots = gridDim.x >> 3;
   const int rows_per_xcd = (d >> 3) * B;
 
-  RawRow<ACT, 4, true> r1, r2, rv;      // the four accesses of a thread are consecutive
+  RawRow<ACT, 4> r1, r2, rv;      // the four accesses of a thread are consecutive
   f32x4_t ru[8];
   auto fetch_row = [&](int j) __attribute__((always_inline)) {
     const int c = (j / B) * 8 + xcd, bb = j % B, n0 = 32 * anew(t);

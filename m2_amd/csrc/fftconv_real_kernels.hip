@@ -160,8 +160,8 @@ __global__ __launch_bounds__(P::T) __attribute__((amdgpu_waves_per_eu(2, 2))) vo
   // workgroup -> (channel, batch row) as in mixer_pair_kernel: XCD e takes the channels c = e (mod 8)
   const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3, slots = gridDim.x >> 3;
   const int rows_per_xcd = (d >> 3) * B;
-  RawRow<ACT, 8, true> r1, rv, r2;
-  auto fetch = [&](RawRow<ACT, 8, true>& r, int third, int j) __attribute__((always_inline)) {
+  RawRow<ACT, 8> r1, rv, r2;
+  auto fetch = [&](RawRow<ACT, 8>& r, int third, int j) __attribute__((always_inline)) {
     const int c = __builtin_amdgcn_readfirstlane((j / B) * 8 + xcd), bb = __builtin_amdgcn_readfirstlane(j % B);
     const ACT* p = xproj + ((long)third * d + c) * ldx + (long)bb * LS;
     const int n0 = 64 * anew(t);

@@ -24,19 +24,17 @@ __device__ __forceinline__ void store8(uint16_t* p, int n0, const float (&v)[8])
 }
 
 // 8 consecutive activations starting at element n0 (n0 % 8 == 0) plus the two before them, as fp32:
-// out[0], out[1] = in[n0-2], in[n0-1] (zero when n0 == 0), out[2..10) = in[n0 .. n0+8); `add` is added to every
-// element that exists (the two before n0 == 0 stay zero: that is the convolution's zero padding, which sits
-// outside the biased signal).  Split into the loads (`fetch`, raw bits) and the conversion (`expand`), so that a
+// out[0], out[1] = in[n0-2], in[n0-1] (zero when n0 == 0), out[2..10) = in[n0 .. n0+8).  Split into the loads (`fetch`, raw bits) and the conversion (`expand`), so that a
 // kernel can put all loads of a row in flight before it starts converting.
 typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
 typedef float f32x2_t __attribute__((ext_vector_type(2)));
 // Raw registers of one access.  Kept as separate arrays of plain vectors (RawRow<ACT, Q>::a / b / h), not as
 // an array of structs: only the former are reliably promoted to registers.
-// CHAINED: the Q accesses are consecutive (access I starts where access I - 1 ends), so only access 0 fetches the
-// two elements before it; the others take them from the registers of their predecessor.
-template <typename ACT, int Q, bool CHAINED = false> struct RawRow;
-template <int Q, bool CHAINED> struct RawRow<float, Q, CHAINED> {
+// The Q accesses are consecutive (access I starts where access I - 1 ends): only access 0 fetches the two elements before it, the
+// others take them from the registers of their predecessor.
+template <typename ACT, int Q> struct RawRow;
+template <int Q> struct RawRow<float, Q> {
   f32x4_t a[Q], b[Q];
   f32x2_t h[Q];
   template <int I> __device__ __forceinline__ void clear(std::integral_constant<int, I>) {
@@ -46,21 +44,13 @@ template <int Q, bool CHAINED> struct RawRow<float, Q, CHAINED> {
   template <int I> __device__ __forceinline__ void fetch(const float* p, int n0) {
     a[I] = *reinterpret_cast<const f32x4_t*>(p + n0);
     b[I] = *reinterpret_cast<const f32x4_t*>(p + n0 + 4);
-    if constexpr (!(CHAINED && I > 0))
+    if constexpr (I == 0)
       h[I] = *reinterpret_cast<const f32x2_t*>(p + (n0 > 0 ? n0 - 2 : 0));      // unused when n0 == 0
   }
   template <int I> __device__ __forceinline__ f32x2_t before() const {
-    if constexpr (CHAINED && I > 0) return f32x2_t{b[I - 1].z, b[I - 1].w};
+    if constexpr (I > 0) return f32x2_t{b[I - 1].z, b[I - 1].w};
     else return h[I];
   }
-  template <int I> __device__ __forceinline__ void expand(int n0, float add, float (&o)[10]) const {
-    const f32x2_t hh = before<I>();
-    o[0] = n0 > 0 ? hh.x + add : 0.f;
-    o[1] = n0 > 0 ? hh.y + add : 0.f;
-    o[2] = a[I].x + add; o[3] = a[I].y + add; o[4] = a[I].z + add; o[5] = a[I].w + add;
-    o[6] = b[I].x + add; o[7] = b[I].y + add; o[8] = b[I].z + add; o[9] = b[I].w + add;
-  }
-  // the same without the addend (no add instructions at all)
   template <int I> __device__ __forceinline__ void expand(int n0, float (&o)[10]) const {
     const f32x2_t hh = before<I>();
     o[0] = n0 > 0 ? hh.x : 0.f;
@@ -69,7 +59,7 @@ template <int Q, bool CHAINED> struct RawRow<float, Q, CHAINED> {
     o[6] = b[I].x; o[7] = b[I].y; o[8] = b[I].z; o[9] = b[I].w;
   }
 };
-template <int Q, bool CHAINED> struct RawRow<uint16_t, Q, CHAINED> {
+template <int Q> struct RawRow<uint16_t, Q> {
   u32x4_t a[Q];
   uint32_t h[Q];
   template <int I> __device__ __forceinline__ void clear(std::integral_constant<int, I>) {
@@ -78,21 +68,12 @@ template <int Q, bool CHAINED> struct RawRow<uint16_t, Q, CHAINED> {
   }
   template <int I> __device__ __forceinline__ void fetch(const uint16_t* p, int n0) {
     a[I] = *reinterpret_cast<const u32x4_t*>(p + n0);
-    if constexpr (!(CHAINED && I > 0))
+    if constexpr (I == 0)
       h[I] = *reinterpret_cast<const uint32_t*>(p + (n0 > 0 ? n0 - 2 : 0));     // unused when n0 == 0
   }
   template <int I> __device__ __forceinline__ uint32_t before() const {
-    if constexpr (CHAINED && I > 0) return a[I - 1].w;
+    if constexpr (I > 0) return a[I - 1].w;
     else return h[I];
-  }
-  template <int I> __device__ __forceinline__ void expand(int n0, float add, float (&o)[10]) const {
-    const uint32_t hh = before<I>();
-    o[0] = n0 > 0 ? __uint_as_float(hh << 16) + add : 0.f;
-    o[1] = n0 > 0 ? __uint_as_float(hh & 0xffff0000u) + add : 0.f;
-    o[2] = __uint_as_float(a[I].x << 16) + add; o[3] = __uint_as_float(a[I].x & 0xffff0000u) + add;
-    o[4] = __uint_as_float(a[I].y << 16) + add; o[5] = __uint_as_float(a[I].y & 0xffff0000u) + add;
-    o[6] = __uint_as_float(a[I].z << 16) + add; o[7] = __uint_as_float(a[I].z & 0xffff0000u) + add;
-    o[8] = __uint_as_float(a[I].w << 16) + add; o[9] = __uint_as_float(a[I].w & 0xffff0000u) + add;
   }
   template <int I> __device__ __forceinline__ void expand(int n0, float (&o)[10]) const {
     const uint32_t hh = before<I>();

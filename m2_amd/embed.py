@@ -77,8 +77,8 @@ class M2BertTextEncoder:
         return out.numpy()
 
     def _assemble(self, token_ids: Sequence, attention_masks: Optional[Sequence], lo: int, hi: int):
-        """Texts [lo, hi) as padded or cut (hi - lo, max_seq_len) ids and mask.  Rows are written into two arrays; a torch tensor
-        per text, its mask, both padded and all of them concatenated took 60 us a text, 3 ms of the 12 of 75 texts of up to 512 tokens."""
+        """Texts [lo, hi) as padded or cut (hi - lo, max_seq_len) ids and mask.  Rows are written into two arrays, 7 us a
+        text of up to 512 tokens; a torch tensor per text, its mask, both padded and all of them concatenated took 41 (3 ms of 75 texts)."""
         L = self.max_seq_len
         ids_b, mask_b = np.zeros((hi - lo, L), np.int64), np.zeros((hi - lo, L), np.int64)
         for k in range(lo, hi):
