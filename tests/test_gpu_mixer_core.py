@@ -27,9 +27,12 @@ def test_mixer_core_rows(gpu, L, d, B, act):
     x = torch.nn.functional.pad(xproj.double() + pb.double()[:, None, None], (2, 0))
     s = sb.double()[:, None, None] + sum(sw.double()[:, k, None, None] * x[..., k:k + L] for k in range(3))
     first, second = _conv(s[:d] * s[2 * d:], taps[0], D[0]) * s[d:2 * d], _conv(u.double(), taps[1], D[1])
-    # fp32: two roundings of 2^-24 per stage of either transform, a few in the convolutions and the gate.  bf16: the gate and the
-    # result are rounded to 2^-9, here relative to a result of which they are a part
-    tol = (4 * (L.bit_length() - 1) + 12) * 2.0 ** -24 if act == torch.float32 else 2.0 ** -8
+    # fp32: the roundings are independent, two and a half in a stage of each of the three transforms (signal, filter, back) and a
+    # dozen in the convolutions, the gate and the factors; each is below 2^-25 of its value in the root mean square, and their
+    # squares add up.  Twice that for what a few rows leave to chance.  bf16: the gate and the result are rounded to 2^-9, here
+    # relative to a result of which they are a part
+    stages = 3 * (L.bit_length() - 1)
+    tol = 2 * (2.5 * stages + 12) ** 0.5 * 2.0 ** -25 if act == torch.float32 else 2.0 ** -8
     for second_signal in (True, False):
         y = ops.mixer_core(xproj.to(gpu), u.to(gpu) if second_signal else None, sw.to(gpu), sb.to(gpu), spec, B, L, d, proj_bias=pb.to(gpu))
         ref = first + second if second_signal else first
