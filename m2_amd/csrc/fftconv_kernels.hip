@@ -55,13 +55,13 @@ struct PairLayout {
 // the layout of the first pass, as plain rows of floats in the buffers of the two transforms.
 //
 // What bounds it is the vector ALU: at L = 128, d = 1536, B = 64 about 1300 vector instructions per wave and batch of four rows are
-// 52 us at full issue, the kernel takes 49; at L = 2048 and 4096 the ALU is 84 - 90 % busy.  So the split follows the instruction
+// 52 us at full issue, the kernel takes 49; by counter the ALU is 80 % busy there and 81 % at L = 1024, B = 31.  So the split follows the instruction
 // count: 16 or 32 points per thread, so that a row up to L = 1024 is two passes inside one wavefront without a barrier, and both
 // signals at once, so that a signal that waits costs no registers and the next rows' inputs can travel in them.  us, against the
 // transform of 2 L points per row of both signals packed (three passes): L = 128, d = 768, B = 32 15.5 / 21.3; d = 1536, B = 64
 // 49 / 68; L = 512, B = 32 56 / 78; L = 1024, B = 31 117 / 166; L = 2048, d = 960, B = 16 184 / 221; L = 4096, B = 1 28 / 32, B = 8
-// 159 / 171.  Relative error of the fp32 core against fp64, now / then: 2.0e-7 / 1.7e-7 at L = 128, 2.2e-7 / 3.6e-7 at 512, 2.7e-7 /
-// 6.6e-7 at 2048, 3.0e-7 / 1.2e-6 at 16384.
+// 159 / 171.  Relative error of the fp32 core against fp64, now / then (N(0, 1) signals and taps): 1.9e-7 / 1.9e-7 at L = 128, 2.4e-7 /
+// 2.4e-7 at 256, 2.5e-7 / 4.0e-7 at 512, 3.0e-7 / 6.8e-7 at 2048, 3.4e-7 / 1.2e-6 at 8192.
 // FULL: short convolutions and gates (sw, sb non-null); otherwise a plain long convolution of one input.
 template <class P, typename ACT, bool FULL>
 __global__ __launch_bounds__(PairLayout<P>::WG) __attribute__((amdgpu_waves_per_eu(P::E == 16 ? 3 : 2, P::E == 16 ? 3 : 2))) void mixer_pair_kernel(

@@ -7,7 +7,7 @@
 // them side by side again.
 //
 // us (bf16, d = 768), against two half transforms of both signals packed: L = 8192, B = 4 171 / 184 (15 % fewer vector instructions;
-// the ALU is 72 % busy, LDS a third of the time, and the two overlap only across the workgroups of a unit), L = 16384, B = 2 189 / 218.
+// the ALU is 72 % busy by counter, and LDS and memory overlap with it only across the workgroups of a unit), L = 16384, B = 2 189 / 218.
 // Requesting the next row's inputs under the epilogue gained nothing measurable at B = 4 and 3 % with fp32 inputs.  Addresses are formed
 // anew where they are used: kept, they had up to 108 bytes per lane spilled (fp32, L = 16384, B = 1 / 2: 145 / 263, now 130 / 248).
 //
