@@ -577,6 +577,26 @@ struct SpectrumForward {
   }
 };
 
+// Workgroups per XCD for `pieces` equal pieces of work that slot s takes at s, s + slots, ... : `cus` compute units, `most` workgroups
+// on them at a time.  The unit with the most pieces ends last, and a piece goes faster with its unit to itself, so what counts is how
+// many pieces the fullest unit has; among equals the fewest workgroups.  (Only the second rule, "no more workgroups than the rounds need",
+// put four rows on half of the units and two on the others where three each were possible.  us of the core, d = 768, bf16, by that
+// rule / by this one: L = 512, B = 11 30.1 / 27.7, 1024, 3 21.8 / 19.0, 2048, 3 37.1 / 32.6, 4096, 1 28.4 / 24.9, 4096, 3 63.3 / 56.6.)
+inline int slots_for(int pieces, int most, int cus) {
+  if (pieces <= most) return pieces;
+  const int rounds = (pieces + most - 1) / most, few = (pieces + rounds - 1) / rounds;
+  auto fullest = [&](int slots) {
+    int worst = 0;
+    for (int u = 0; u < cus && u < slots; ++u) {
+      int n = 0;
+      for (int s = u; s < slots; s += cus) n += (pieces - s + slots - 1) / slots;
+      worst = n > worst ? n : worst;
+    }
+    return worst;
+  };
+  return fullest(most) < fullest(few) ? most : few;
+}
+
 // half transforms and rows by sequence length; the shift of one signal's ring (z^L = -i) in eighths
 constexpr int kQuarter = 2;
 typedef TwistPlan<7, 8, 1, 16, 16> Twist128;

@@ -339,11 +339,7 @@ static int launch_mixer_pair(const void* xproj, long ldx, const float* u, const 
     resident = n;
   }
   const int per_cu = resident;
-  int slots = (num_cus() / 8) * (per_cu > 8 ? 8 : per_cu);          // workgroups per XCD
-  if (slots > slots_needed) slots = slots_needed;
-  // every workgroup the same number of row batches: the fewest workgroups that need no extra round
-  const int rounds = (slots_needed + slots - 1) / slots;
-  slots = (slots_needed + rounds - 1) / rounds;
+  const int cus = num_cus() / 8, slots = slots_for(slots_needed, cus * (per_cu > 8 ? 8 : per_cu), cus);          // per XCD
   hipLaunchKernelGGL(kern, dim3(8 * slots), dim3(Lay::WG), Lay::lds_bytes, stream, (const ACT*)xproj, ldx, u, sw, sb, pbias,
                      (const float4*)spec, (ACT*)y, B, d);
   return check_launch("mixer_pair");

@@ -233,10 +233,7 @@ static int launch_mixer_long(const void* xproj, long ldx, const float* u, const 
   int per_cu = (int)((160 * 1024) / lds_bytes);
   if (per_cu < 1) per_cu = 1;
   if (per_cu > 512 / P::T) per_cu = 512 / P::T;  // two waves per SIMD at 256 registers
-  int slots = (num_cus() / 8) * per_cu;          // workgroups per XCD
-  if (slots > rows_per_xcd) slots = rows_per_xcd;
-  const int rounds = (rows_per_xcd + slots - 1) / slots;      // every workgroup the same number of rows
-  slots = (rows_per_xcd + rounds - 1) / rounds;
+  const int cus = num_cus() / 8, slots = slots_for(rows_per_xcd, cus * per_cu, cus);          // workgroups per XCD
   hipLaunchKernelGGL(kern, dim3(8 * slots), dim3(P::T), lds_bytes, stream, (const ACT*)xproj, ldx, u, sw, sb, pbias,
                      (const float4*)spec, (ACT*)y, B, d);
   return check_launch("mixer_long");

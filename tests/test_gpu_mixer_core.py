@@ -53,3 +53,17 @@ def test_spectra_of_the_shortest_rows(gpu):
     y = ops.fftconv(x, ops.filter_spectrum(k, None, None, None), B, L, d)
     ref = _conv(x.double(), k, torch.zeros(d, device=gpu))
     assert (y - ref).norm() <= (2.5 * 14 + 6) ** 0.5 * 2.0 ** -25 * ref.norm()
+
+
+@pytest.mark.parametrize("L,d,B", [(512, 768, 11), (2048, 768, 3), (4096, 768, 1), (8192, 768, 1)])
+def test_rows_dealt_unevenly(gpu, L, d, B):
+    """Row counts at which some workgroups take one batch of rows more than others: every row is there and is itself (the rows of fp64
+    transforms; bound as above)."""
+    from m2_amd import ops
+    g = torch.Generator(device=gpu).manual_seed(L + B)
+    rn = lambda *s: torch.randn(*s, generator=g, device=gpu)      # noqa: E731
+    k, x = rn(d, 2 * L) / L ** 0.5, rn(d, B, L)
+    y = ops.fftconv(x, ops.filter_spectrum(k, None, None, None), B, L, d)
+    ref = _conv(x.double(), k, torch.zeros(d, device=gpu))
+    tol = 2 * (2.5 * 3 * (L.bit_length() - 1) + 6) ** 0.5 * 2.0 ** -25
+    assert ((y - ref).norm(dim=2) <= tol * ref.norm(dim=2)).all()
