@@ -110,6 +110,12 @@ int m2_mixer_filters_fwd(const m2_hyena_filter_params* params_dev, const float* 
                          int filters_per_mixer, int L, int d, int order, int emb_dim, float w_mod, float shift,
                          void* workspace, float* spec, void* stream);
 
+/* The taps of the same filters, without the skip weights: taps (nmixers, filters_per_mixer, d, 2L) fp32, what m2_mixer_core_taps_fwd
+ * reads.  L a multiple of 64 from 1024 on; the other arguments as above, the workspace of its own size. */
+size_t m2_mixer_taps_workspace_bytes(int nmixers, int filters_per_mixer, int L, int d, int order);
+int m2_mixer_taps_fwd(const m2_hyena_filter_params* params_dev, int nmixers, int filters_per_mixer, int L, int d, int order, int emb_dim,
+                      float w_mod, float shift, void* workspace, float* taps, void* stream);
+
 /* ---------------------------------------------------------------------------------------------
  * Long convolution: filter spectra and the fused mixer core.
  * Stand in for: bert/src/mm/hyena_utils.py:16-42 (fftconv_ref), :219-248 (HyenaFilter.forward) and
@@ -149,6 +155,14 @@ int m2_mixer_core_fwd(const void* xproj, const float* proj_bias, const float* u,
 /* The same with the rows of xproj (channels) xproj_row >= B * L elements apart, a multiple of 8. */
 int m2_mixer_core_rows_fwd(const void* xproj, long xproj_row, const float* proj_bias, const float* u, const float* short_w,
                            const float* short_b, const float* spec, void* y, int B, int L, int d, int act_dtype, void* stream);
+
+/* The same for bf16 rows with the filters as taps, (nfilters, d, 2L) fp32, which are transformed for every row: faster than spectra
+ * where few rows share them (m2_mixer_core_taps_pays, host code).  skip_dev: DEVICE array of nfilters pointers to the (d) skip
+ * weights, entries may be null; NULL for none.  nfilters 2, or 1 (the second filter is zero; u NULL).  L = 1024 .. 16384. */
+int m2_mixer_core_taps_pays(int B, int L);
+int m2_mixer_core_taps_fwd(const void* xproj, long xproj_row, const float* proj_bias, const float* u, const float* short_w,
+                           const float* short_b, const float* taps, const float* const* skip_dev, int nfilters, void* y, int B, int L,
+                           int d, void* stream);
 
 /* Plain long convolution y[c,b,:] = fftconv(x[c,b,:]; k1)[:L] + D1[c] x[c,b,:] with the first filter
  * of `spec` (HyenaFilter.forward on its own, bert/src/mm/hyena_utils.py:219-248).
@@ -343,6 +357,11 @@ size_t m2_encoder_layers_workspace_bytes(int M, int d, int intermediate);
 int m2_encoder_layers_fwd(const m2_layer_params* layers, int nlayers, const float* spectra, const void* h16,
                           const float* h_channel_major, float* const* out_f32, void* workspace, int B, int L, int d,
                           int intermediate, int nblocks, float eps, void* stream);
+/* The same with the filters as taps (m2_mixer_taps_fwd) and their skip weights (as m2_mixer_filters_fwd takes them), where
+ * m2_mixer_core_taps_fwd serves L. */
+int m2_encoder_layers_taps_fwd(const m2_layer_params* layers, int nlayers, const float* taps, const float* const* skip_dev,
+                               int filters_per_mixer, const void* h16, const float* h_channel_major, float* const* out_f32,
+                               void* workspace, int B, int L, int d, int intermediate, int nblocks, float eps, void* stream);
 
 #ifdef __cplusplus
 }

@@ -70,6 +70,14 @@ def _load() -> ctypes.CDLL:
     lib.m2_mixer_filters_fwd.restype = c_int
     lib.m2_mixer_filters_fwd.argtypes = [c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_float, c_float,
                                          c_void_p, c_void_p, c_void_p]
+    lib.m2_mixer_taps_workspace_bytes.restype = ctypes.c_size_t
+    lib.m2_mixer_taps_workspace_bytes.argtypes = [c_int] * 5
+    lib.m2_mixer_taps_fwd.restype = c_int
+    lib.m2_mixer_taps_fwd.argtypes = [c_void_p] + [c_int] * 6 + [c_float, c_float] + [c_void_p] * 3
+    lib.m2_mixer_core_taps_pays.restype = c_int
+    lib.m2_mixer_core_taps_pays.argtypes = [c_int, c_int]
+    lib.m2_mixer_core_taps_fwd.restype = c_int
+    lib.m2_mixer_core_taps_fwd.argtypes = [c_void_p, c_long] + [c_void_p] * 6 + [c_int, c_void_p] + [c_int] * 3 + [c_void_p]
     lib.m2_dense_supported.restype = c_int
     lib.m2_dense_supported.argtypes = [c_int] * 3
     lib.m2_dense_to_channels_fwd.restype = c_int
@@ -138,15 +146,17 @@ def _load() -> ctypes.CDLL:
     lib.m2_encoder_layers_workspace_bytes.argtypes = [c_int] * 3
     lib.m2_encoder_layers_fwd.restype = c_int
     lib.m2_encoder_layers_fwd.argtypes = [c_void_p, c_int] + [c_void_p] * 5 + [c_int] * 5 + [c_float, c_void_p]
+    lib.m2_encoder_layers_taps_fwd.restype = c_int
+    lib.m2_encoder_layers_taps_fwd.argtypes = [c_void_p, c_int] + [c_void_p] * 2 + [c_int] + [c_void_p] * 4 + [c_int] * 5 + [c_float, c_void_p]
     return lib
 
 
 lib = _load()
 
-EXPORTS = ["m2_version", "m2_last_error", "m2_hyena_filter_workspace_bytes", "m2_hyena_filter_fwd", "m2_hyena_filter_fwd_static", "m2_mixer_filters_workspace_bytes", "m2_mixer_filters_fwd",
-           "m2_fftconv_supported_seqlen", "m2_filter_spectrum_bytes", "m2_filter_spectrum_fwd", "m2_mixer_core_fwd", "m2_mixer_core_rows_fwd",
+EXPORTS = ["m2_version", "m2_last_error", "m2_hyena_filter_workspace_bytes", "m2_hyena_filter_fwd", "m2_hyena_filter_fwd_static", "m2_mixer_filters_workspace_bytes", "m2_mixer_filters_fwd", "m2_mixer_taps_workspace_bytes", "m2_mixer_taps_fwd",
+           "m2_fftconv_supported_seqlen", "m2_filter_spectrum_bytes", "m2_filter_spectrum_fwd", "m2_mixer_core_fwd", "m2_mixer_core_rows_fwd", "m2_mixer_core_taps_pays", "m2_mixer_core_taps_fwd",
            "m2_fftconv_fwd", "m2_dense_supported", "m2_dense_to_channels_fwd", "m2_dense_to_channels_rows_fwd", "m2_dense_channels_row", "m2_dense_from_channels_fwd", "m2_blockdiag_glu_fwd", "m2_blockdiag_glu_few_rows", "m2_blockdiag_linear_fwd", "m2_blockdiag_linear_f32_fwd", "m2_mlp_fused_supported", "m2_mlp_fused_packed_bytes", "m2_mlp_fused_pack", "m2_mlp_fused_fwd", "m2_glu_stream_supported", "m2_glu_stream_packed_bytes", "m2_glu_stream_pack", "m2_glu_stream_fwd", "m2_layernorm_fwd", "m2_layernorm_bf16_fwd", "m2_input_forms_fwd",
-           "m2_embed_layernorm_fwd", "m2_blockdiag_linear_layernorm_supported", "m2_blockdiag_linear_layernorm_fwd", "m2_encoder_layers_workspace_bytes", "m2_encoder_layers_fwd",
+           "m2_embed_layernorm_fwd", "m2_blockdiag_linear_layernorm_supported", "m2_blockdiag_linear_layernorm_fwd", "m2_encoder_layers_workspace_bytes", "m2_encoder_layers_fwd", "m2_encoder_layers_taps_fwd",
            "m2_split_bytes", "m2_split_rows_fwd", "m2_split_jobs_fwd", "m2_split_channels_fwd", "m2_split_to_channels_fwd", "m2_split_linear_fwd", "m2_split_glu_fwd"]
 
 

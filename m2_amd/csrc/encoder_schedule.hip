@@ -38,11 +38,11 @@ extern "C" size_t m2_encoder_layers_workspace_bytes(int M, int d, int intermedia
   return layout(M, d, intermediate).total;
 }
 
-extern "C" int m2_encoder_layers_fwd(const m2_layer_params* layers, int nlayers, const float* spectra, const void* h16,
-                                     const float* h_channel_major, float* const* out_f32, void* workspace, int B, int L,
-                                     int d, int intermediate, int nblocks, float eps, void* stream) {
-  const char* who = "m2_encoder_layers_fwd";
-  if (!layers || !spectra || !h16 || !h_channel_major || !out_f32 || !workspace) return set_error(M2_ERR_ARG, "%s: null pointer", who);
+// filters: spectra, or with fpm > 0 the taps of fpm filters per layer
+static int encoder_layers(const char* who, const m2_layer_params* layers, int nlayers, const float* filters, int fpm, const float* const* skip,
+                          const void* h16, const float* h_channel_major, float* const* out_f32, void* workspace, int B, int L, int d,
+                          int intermediate, int nblocks, float eps, void* stream) {
+  if (!layers || !filters || !h16 || !h_channel_major || !out_f32 || !workspace) return set_error(M2_ERR_ARG, "%s: null pointer", who);
   if (nlayers < 1 || B < 1 || L < 1 || d < 1 || intermediate < 1)
     return set_error(M2_ERR_ARG, "%s: sizes must be positive (layers=%d B=%d L=%d d=%d I=%d)", who, nlayers, B, L, d, intermediate);
   if ((long)B * L > 0x7fffffffL) return set_error(M2_ERR_UNSUPPORTED, "%s: B * L = %ld does not fit an int", who, (long)B * L);
@@ -57,13 +57,15 @@ extern "C" int m2_encoder_layers_fwd(const m2_layer_params* layers, int nlayers,
   unsigned char* ws = (unsigned char*)workspace;
   void *xproj = ws + l.xproj, *y = ws + l.y, *a = ws + l.a, *g = ws + l.g, *s = ws + l.s, *nh = ws + l.h16;
   float* nt = (float*)(ws + l.hT);
-  const size_t spec_stride = m2_filter_spectrum_bytes(d, L) / sizeof(float);
+  const size_t stride = fpm ? (size_t)fpm * d * 2 * L : m2_filter_spectrum_bytes(d, L) / sizeof(float);
   for (int i = 0; i < nlayers; ++i) {
     const m2_layer_params& p = layers[i];
     int rc = m2_dense_to_channels_rows_fwd(h16, p.in_w, xproj, l.xrow, M, 3 * d, d, stream);
     if (rc) return rc;
-    rc = m2_mixer_core_rows_fwd(xproj, l.xrow, p.in_b, p.residual ? h_channel_major : nullptr, p.short_w, p.short_b, spectra + i * spec_stride,
-                                y, B, L, d, M2_DTYPE_BF16, stream);
+    const float* u = p.residual ? h_channel_major : nullptr;
+    rc = fpm ? m2_mixer_core_taps_fwd(xproj, l.xrow, p.in_b, u, p.short_w, p.short_b, filters + i * stride, skip ? skip + i * fpm : nullptr, fpm, y,
+                                      B, L, d, stream)
+             : m2_mixer_core_rows_fwd(xproj, l.xrow, p.in_b, u, p.short_w, p.short_b, filters + i * stride, y, B, L, d, M2_DTYPE_BF16, stream);
     if (rc) return rc;
     rc = m2_dense_from_channels_fwd(y, p.out_w, p.out_b, a, M, d, d, stream);
     if (rc) return rc;
@@ -83,4 +85,21 @@ extern "C" int m2_encoder_layers_fwd(const m2_layer_params* layers, int nlayers,
     h_channel_major = nt;
   }
   return M2_OK;
+}
+
+extern "C" int m2_encoder_layers_fwd(const m2_layer_params* layers, int nlayers, const float* spectra, const void* h16,
+                                     const float* h_channel_major, float* const* out_f32, void* workspace, int B, int L,
+                                     int d, int intermediate, int nblocks, float eps, void* stream) {
+  return encoder_layers("m2_encoder_layers_fwd", layers, nlayers, spectra, 0, nullptr, h16, h_channel_major, out_f32, workspace, B, L, d,
+                        intermediate, nblocks, eps, stream);
+}
+
+extern "C" int m2_encoder_layers_taps_fwd(const m2_layer_params* layers, int nlayers, const float* taps, const float* const* skip_dev,
+                                          int filters_per_mixer, const void* h16, const float* h_channel_major, float* const* out_f32,
+                                          void* workspace, int B, int L, int d, int intermediate, int nblocks, float eps, void* stream) {
+  const char* who = "m2_encoder_layers_taps_fwd";
+  if (filters_per_mixer < 1 || filters_per_mixer > 2)
+    return set_error(M2_ERR_ARG, "%s: filters_per_mixer=%d must be 1 or 2", who, filters_per_mixer);
+  return encoder_layers(who, layers, nlayers, taps, filters_per_mixer, skip_dev, h16, h_channel_major, out_f32, workspace, B, L, d, intermediate,
+                        nblocks, eps, stream);
 }

@@ -427,6 +427,23 @@ __device__ __forceinline__ void store_spectrum(const cf (&x)[P::E], float scale,
   });
 }
 
+// taps (2 L of one filter and channel) in first-pass layout: lo + i hi, the two halves of the window
+template <class P>
+__device__ __forceinline__ void load_taps(cf (&x)[P::E], const float* __restrict__ p, int t) {
+  static_for<0, P::E>([&](auto rr) {
+    constexpr int r = decltype(rr)::value, n = P::T * (r / P::R1) + P::S1 * (r % P::R1);
+    x[r] = {(p + n)[(unsigned)t], (p + n + P::H)[(unsigned)t]};
+  });
+}
+
+// Where a mixer core finds its filters: spectra from memory (m2_filter_spectrum_fwd), or taps that it transforms itself, filter f of
+// channel c at taps + (f d + c) 2 L, with skip[f][c] on tap 0.
+struct FilterTaps {
+  const float* taps;
+  const float* const* skip;      // one pointer per filter (entries, or the table, may be null)
+  int nfilters;                  // 1: the second filter is zero
+};
+
 struct Nothing {
   __device__ __forceinline__ void operator()() const {}
 };
@@ -460,6 +477,31 @@ __device__ __forceinline__ void convolve(cf (&x)[P::E], int t, float2* row, cons
     sync_threads<P::T>();
   }
   before_last();
+  inv_first<P>(x, t, row, tab, ti);
+}
+// The same with the spectrum in registers, as `transform` leaves it.  `behind_product` is called where those registers are free again.
+template <class P, int S8, bool REAL, class F>
+__device__ __forceinline__ void convolve_held(cf (&x)[P::E], int t, float2* row, const float2* tab, const TwistForward<P, S8>& tf,
+                                              const TwistInverse<P>& ti, const cf (&K)[P::E], F&& behind_product) {
+  fwd_first<P, S8, REAL>(x, t, row);
+  sync_threads<P::T>();
+  if constexpr (P::THREE) {
+    second<P, false>(x, t, row, tab);
+    sync_threads<P::T>();
+  }
+  static_for<0, P::NG>([&](auto gg) { load_group<P, decltype(gg)::value>(x, t, row); });
+  static_for<0, P::NG>([&](auto gg) {
+    constexpr int g = decltype(gg)::value;
+    fwd_group<P, g>(x, t, tab, tf);
+    static_for<g * P::R3, (g + 1) * P::R3>([&](auto rr) { x[decltype(rr)::value] = cmul(x[decltype(rr)::value], K[decltype(rr)::value]); });
+    inv_group<P, g>(x, t, row);
+  });
+  behind_product();
+  sync_threads<P::T>();
+  if constexpr (P::THREE) {
+    second<P, true>(x, t, row, tab);
+    sync_threads<P::T>();
+  }
   inv_first<P>(x, t, row, tab, ti);
 }
 // the forward half: the spectrum of registers in first-pass layout

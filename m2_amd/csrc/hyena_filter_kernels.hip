@@ -689,18 +689,23 @@ extern "C" size_t m2_mixer_filters_workspace_bytes(int nmixers, int filters_per_
   return batch_layout(nmixers, filters_per_mixer, L, d).total;
 }
 
-extern "C" int m2_mixer_filters_fwd(const m2_hyena_filter_params* params_dev, const float* const* skip_dev, int nmixers,
-                                    int filters_per_mixer, int L, int d, int order, int emb_dim, float w_mod,
-                                    float shift, void* workspace, float* spec, void* stream) {
-  const char* who = "m2_mixer_filters_fwd";
-  if (!params_dev || !workspace || !spec) return set_error(M2_ERR_ARG, "%s: null pointer", who);
+// validation of a batch of mixers, for the entry points whose table lives in device memory
+static int check_mixers(const char* who, int nmixers, int filters_per_mixer, int L, int d, int order, int emb_dim) {
   if (filters_per_mixer < 1 || filters_per_mixer > 2)
     return set_error(M2_ERR_ARG, "%s: filters_per_mixer=%d must be 1 or 2", who, filters_per_mixer);
   // the MLPs of the batch (two per filter) are one grid dimension of the hidden-layer launch
   if (nmixers < 1 || (long)nmixers * filters_per_mixer * 2 > 65535)
     return set_error(M2_ERR_ARG, "%s: nmixers=%d with %d filters each: at most 65535 MLPs (two per filter) per call", who, nmixers,
                      filters_per_mixer);
-  int rc = check_filter_sizes(who, L, d, order, emb_dim);
+  return check_filter_sizes(who, L, d, order, emb_dim);
+}
+
+extern "C" int m2_mixer_filters_fwd(const m2_hyena_filter_params* params_dev, const float* const* skip_dev, int nmixers,
+                                    int filters_per_mixer, int L, int d, int order, int emb_dim, float w_mod,
+                                    float shift, void* workspace, float* spec, void* stream) {
+  const char* who = "m2_mixer_filters_fwd";
+  if (!params_dev || !workspace || !spec) return set_error(M2_ERR_ARG, "%s: null pointer", who);
+  int rc = check_mixers(who, nmixers, filters_per_mixer, L, d, order, emb_dim);
   if (rc) return rc;
   if (!m2_fftconv_supported_seqlen(L))
     return set_error(M2_ERR_UNSUPPORTED, "%s: L=%d unsupported (need L a power of two in [128, 32768])", who, L);
@@ -722,4 +727,26 @@ extern "C" int m2_mixer_filters_fwd(const m2_hyena_filter_params* params_dev, co
     return launch_project_spectrum(tab.p, skip_dev, nmixers, filters_per_mixer, L, d, shift, h_hi, h_lo, spec, spec_stride, s);
   SpectrumBatch sb{taps, skip_dev, filters_per_mixer, spec_stride};
   return launch_filter_spectrum_any(nullptr, nullptr, nullptr, nullptr, spec, d, L, sb, nmixers, s);
+}
+
+// The taps alone, for a mixer core that transforms them itself: the same two launches, no room for taps in the workspace.
+extern "C" size_t m2_mixer_taps_workspace_bytes(int nmixers, int filters_per_mixer, int L, int d, int order) {
+  if (nmixers <= 0 || filters_per_mixer < 1 || filters_per_mixer > 2 || d <= 0 || order != kOrder || !project_with_hidden(L, d)) return 0;
+  const BatchLayout lay = batch_layout(nmixers, filters_per_mixer, L, d);
+  return lay.taps - lay.wsplit;      // (h3 does not leave the chip)
+}
+
+extern "C" int m2_mixer_taps_fwd(const m2_hyena_filter_params* params_dev, int nmixers, int filters_per_mixer, int L, int d, int order,
+                                 int emb_dim, float w_mod, float shift, void* workspace, float* taps, void* stream) {
+  const char* who = "m2_mixer_taps_fwd";
+  if (!params_dev || !workspace || !taps) return set_error(M2_ERR_ARG, "%s: null pointer", who);
+  int rc = check_mixers(who, nmixers, filters_per_mixer, L, d, order, emb_dim);
+  if (rc) return rc;
+  if (!project_with_hidden(L, d)) return set_error(M2_ERR_UNSUPPORTED, "%s: L=%d unsupported (need a multiple of 64 from 1024 on)", who, L);
+  const BatchLayout lay = batch_layout(nmixers, filters_per_mixer, L, d);
+  unsigned char* ws = reinterpret_cast<unsigned char*>(workspace);
+  TabByPointer tab{reinterpret_cast<const FilterPtrs*>(params_dev)};
+  return filter_launches(tab, nmixers * filters_per_mixer, L, d, emb_dim, w_mod, shift, nullptr, nullptr, reinterpret_cast<uint16_t*>(ws),
+                         reinterpret_cast<uint16_t*>(ws + lay.w3split - lay.wsplit), reinterpret_cast<float*>(ws + lay.w3scale - lay.wsplit),
+                         taps, (hipStream_t)stream);
 }

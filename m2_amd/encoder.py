@@ -28,7 +28,7 @@ import torch.nn as nn
 from . import ops, schedule
 from .blockdiag import BlockdiagLinear
 from .config import M2BertConfig
-from .mixer import MonarchMixerSequenceMixing
+from .mixer import MonarchMixerSequenceMixing, takes_taps
 
 
 class BertEmbeddings(nn.Module):
@@ -302,6 +302,9 @@ class BertLayer(nn.Module):
         return self.mlp.normed(a16, want_f32, not (pre or last), not (pre or last))
 
 
+_OWN_FUSED = BertLayer.fused
+
+
 class BertEncoder(nn.Module):
     """`use_hip_graph=True` captures the whole stack of layers into one HIP graph per input shape and replays
     it: at short sequence lengths the forward is launch-bound (about ten small kernels per layer) and the
@@ -412,12 +415,17 @@ class BertEncoder(nn.Module):
                     side = self._filter_stream
                     side.wait_stream(cur)
                 with torch.cuda.stream(side if side is not None else cur):
+                    # (layers and mixers of a caller's own are given spectra)
+                    filters_of = ops.mixer_filter_spectra
+                    if ops.taps_pay(B, L, torch.bfloat16) and all(
+                            type(lay) is BertLayer and type(lay).fused is _OWN_FUSED and "fused" not in lay.__dict__
+                            and takes_taps(lay.attention) for lay in self.layer):
+                        filters_of = ops.mixer_filter_taps
                     for first, count in groups:
-                        sp = ops.mixer_filter_spectra(table, w_mod=float(f0.w_mod), shift=float(f0.modulation.shift),
-                                                      first=first, count=count)
+                        sp = filters_of(table, w_mod=float(f0.w_mod), shift=float(f0.modulation.shift), first=first, count=count)
                         ev = None
                         if side is not None:
-                            sp.record_stream(cur)
+                            sp[0].record_stream(cur)      # (one piece of memory for all of them)
                             ev = torch.cuda.Event()
                             ev.record(side)
                         ahead += [(sp[j], ev) for j in range(count)]

@@ -105,9 +105,9 @@ class MonarchMixerSequenceMixing(nn.Module):
             skips.append(b if (b.dtype == torch.float32 and b.is_contiguous()) else b.float().contiguous())
         return filters, skips
 
-    def _generate_spectrum(self, L: int, fns) -> torch.Tensor:
+    def _generate_spectrum(self, L: int, fns, taps: bool = False):
         """All of filter generation in one library call: hidden layers, projection + decay, window, skip weight,
-        transform (for L <= 512 the taps never reach memory)."""
+        transform (for L <= 512 the taps never reach memory).  taps: without the last two, an ops.MixerTaps."""
         f0 = self.filter_fn
         filters, skips = self.filter_table_entry()
         table = self._filter_table
@@ -116,7 +116,8 @@ class MonarchMixerSequenceMixing(nn.Module):
         if table is None or table[0] != key_probe:
             table = (key_probe, ops.FilterTable([filters], [skips], L, self.d_model, f0.order, f0.emb_dim))
             self._filter_table = table
-        return ops.mixer_filter_spectra(table[1], w_mod=float(f0.w_mod), shift=float(f0.modulation.shift))[0]
+        generate = ops.mixer_filter_taps if taps else ops.mixer_filter_spectra
+        return generate(table[1], w_mod=float(f0.w_mod), shift=float(f0.modulation.shift))[0]
 
     def core(self, xproj: torch.Tensor, u_cm: Optional[torch.Tensor], B: int, L: int,
              spec: Optional[torch.Tensor] = None) -> torch.Tensor:
@@ -124,7 +125,10 @@ class MonarchMixerSequenceMixing(nn.Module):
         in_linear.bias as it loads), u_cm (d, B, L) fp32 -> y (d, B, L).  xproj may also be (3d, row), row >= B L, the values of a
         channel at the start of its row."""
         if spec is None:
-            spec = self.filter_spectrum(L)
+            if ops.taps_pay(B, L, xproj.dtype) and not self.cache_filters and takes_taps(self):
+                spec = self._generate_spectrum(L, [self.filter_fn] + ([self.filter_fn2] if self.residual_long_conv else []), taps=True)
+            else:
+                spec = self.filter_spectrum(L)
         sw = self._cast("short_w", self.short_filter.weight, torch.float32).view(3 * self.d_model, 3)
         sb = self._cast("short_b", self.short_filter.bias, torch.float32)
         pb = self._cast("in_b32", self.in_linear.bias, torch.float32)
@@ -220,6 +224,7 @@ class MonarchMixerSequenceMixing(nn.Module):
 
 
 _OWN = MonarchMixerSequenceMixing.project_in, MonarchMixerSequenceMixing.core
+_OWN_FILTERS = MonarchMixerSequenceMixing.core, MonarchMixerSequenceMixing.filter_spectrum, MonarchMixerSequenceMixing._generate_spectrum
 
 
 def knows_rows(mixer) -> bool:
@@ -227,3 +232,10 @@ def knows_rows(mixer) -> bool:
     cls = type(mixer)
     return (cls is MonarchMixerSequenceMixing and (cls.project_in, cls.core) == _OWN
             and not {"project_in", "core"} & mixer.__dict__.keys())
+
+
+def takes_taps(mixer) -> bool:
+    """Whether the mixer's core and filters are the ones of this file, so that taps may stand in the place of spectra between them."""
+    cls = type(mixer)
+    return (cls is MonarchMixerSequenceMixing and (cls.core, cls.filter_spectrum, cls._generate_spectrum) == _OWN_FILTERS
+            and not {"core", "filter_spectrum", "_generate_spectrum"} & mixer.__dict__.keys())

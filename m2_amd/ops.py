@@ -241,6 +241,38 @@ def mixer_filter_spectra(table: FilterTable, w_mod: float = 1.0, shift: float = 
     return out
 
 
+class MixerTaps:
+    """Taps (filters, d, 2L) fp32 of one mixer's filters with the device pointers of their skip weights: what `mixer_core` takes in the
+    place of spectra where it transforms them itself."""
+
+    def __init__(self, taps: Tensor, skip: int, table: FilterTable):
+        self.taps, self.skip, self.table = taps, skip, table
+
+    def record_stream(self, stream) -> None:
+        self.taps.record_stream(stream)
+
+
+def taps_pay(B: int, L: int, dtype) -> bool:
+    """Rows whose core is faster on taps than on spectra."""
+    return dtype == torch.bfloat16 and bool(lib.m2_mixer_core_taps_pays(B, L))
+
+
+def mixer_filter_taps(table: FilterTable, w_mod: float = 1.0, shift: float = 0.0, first: int = 0,
+                      count: Optional[int] = None) -> Sequence[MixerTaps]:
+    """The taps of the mixers [first, first + count) of `table`, generated like `mixer_filter_spectra`."""
+    count = table.nmixers - first if count is None else count
+    if first < 0 or count < 1 or first + count > table.nmixers:
+        raise ValueError(f"mixers [{first}, {first + count}) outside the table of {table.nmixers}")
+    dev = table.table.device
+    stream = _stream()
+    table.use_on(stream)
+    taps = torch.empty(count, table.fpm, table.d, 2 * table.L, dtype=torch.float32, device=dev)
+    workspace = torch.empty(lib.m2_mixer_taps_workspace_bytes(count, table.fpm, table.L, table.d, table.order), dtype=torch.uint8, device=dev)
+    check(lib.m2_mixer_taps_fwd(ctypes.c_void_p(table.table.data_ptr() + first * table.fpm * 18 * 8), count, table.fpm, table.L, table.d,
+                                table.order, table.emb_dim, float(w_mod), float(shift), _ptr(workspace), _ptr(taps), stream))
+    return [MixerTaps(taps[i], table.skip.data_ptr() + (first + i) * table.fpm * 8, table) for i in range(count)]
+
+
 def filter_spectrum(taps1: Tensor, taps2: Optional[Tensor], D1: Optional[Tensor], D2: Optional[Tensor]) -> Tensor:
     """Opaque spectrum buffer for `mixer_core` from (d, 2L) taps of one or two filters."""
     d, n = taps1.shape
@@ -260,7 +292,7 @@ def mixer_core(xproj: Tensor, u: Optional[Tensor], short_w: Tensor, short_b: Ten
                d: int, out: Optional[Tensor] = None, proj_bias: Optional[Tensor] = None, row: Optional[int] = None) -> Tensor:
     """y (d, B, L) from the channel-major in-projection (3d, B, L) and layer input (d, B, L).
     `proj_bias` (3d) fp32 is added to xproj on load (pass the in_linear bias when the GEMM ran without it).
-    `row`: xproj is (3d, row), the B L values of a channel at the start of its row."""
+    `row`: xproj is (3d, row), the B L values of a channel at the start of its row.  `spec`: spectra, or a `MixerTaps` (bf16)."""
     _require(xproj, "xproj", None, (3 * d, B, L) if row is None else (3 * d, row))
     code = _act_code(xproj.dtype)
     if proj_bias is not None:
@@ -269,11 +301,21 @@ def mixer_core(xproj: Tensor, u: Optional[Tensor], short_w: Tensor, short_b: Ten
         _require(u, "u", torch.float32, (d, B, L))
     _require(short_w, "short_w", torch.float32, (3 * d, 3))
     _require(short_b, "short_b", torch.float32, (3 * d,))
-    _require(spec, "spec", torch.float32, (lib.m2_filter_spectrum_bytes(d, L) // 4,))
+    if isinstance(spec, MixerTaps):
+        _require(xproj, "xproj", torch.bfloat16)
+        _require(spec.taps, "taps", torch.float32, (spec.table.fpm, d, 2 * L))
+    else:
+        _require(spec, "spec", torch.float32, (lib.m2_filter_spectrum_bytes(d, L) // 4,))
     if out is None:
         out = torch.empty(d, B, L, dtype=xproj.dtype, device=xproj.device)
     else:
         _require(out, "out", xproj.dtype, (d, B, L))
+    if isinstance(spec, MixerTaps):
+        stream = _stream()
+        spec.table.use_on(stream)
+        check(lib.m2_mixer_core_taps_fwd(_ptr(xproj), B * L if row is None else row, _ptr(proj_bias), _ptr(u), _ptr(short_w), _ptr(short_b),
+                                         _ptr(spec.taps), spec.skip, spec.table.fpm, _ptr(out), B, L, d, stream))
+        return out
     check(lib.m2_mixer_core_rows_fwd(_ptr(xproj), B * L if row is None else row, _ptr(proj_bias), _ptr(u), _ptr(short_w),
                                      _ptr(short_b), _ptr(spec), _ptr(out), B, L, d, code, _stream()))
     return out

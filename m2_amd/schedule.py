@@ -221,6 +221,7 @@ class StackPlan(NoPlan):
         self.L = L
         self.spec_bytes = lib.m2_filter_spectrum_bytes(self.d, L)
         self.filter_ws = lib.m2_mixer_filters_workspace_bytes(n, self.table.fpm, L, self.d, self.table.order)
+        self.taps_ws = lib.m2_mixer_taps_workspace_bytes(n, self.table.fpm, L, self.d, self.table.order)
         self.filter_ws_layer = max(1, lib.m2_mixer_filters_workspace_bytes(1, self.table.fpm, L, self.d, self.table.order))
 
     @staticmethod
@@ -263,8 +264,9 @@ class StackPlan(NoPlan):
         route[1].use_on(current)
         stream = ctypes.c_void_p(current)
         up = lambda v: (v + 255) & ~255      # noqa: E731
-        o_spec = up(self.filter_ws)
-        o_act = o_spec + up(n * self.spec_bytes)
+        taps = ops.taps_pay(B, L, torch.bfloat16)
+        o_spec = up(self.taps_ws if taps else self.filter_ws)
+        o_act = o_spec + up(n * (8 * t.fpm * d * L if taps else self.spec_bytes))
         o_in = o_act + up(lib.m2_encoder_layers_workspace_bytes(M, d, self.I))
         ws = torch.empty(o_in + (up(2 * M * d) + 4 * M * d if ids is not None else 0), dtype=torch.uint8, device=dev)
         base = ws.data_ptr()
@@ -272,15 +274,22 @@ class StackPlan(NoPlan):
         ptrs = (ctypes.c_void_p * n)()
         for i, o in enumerate(outs):
             ptrs[n - len(outs) + i] = o.data_ptr()
-        check(lib.m2_mixer_filters_fwd(t.table.data_ptr(), t.skip.data_ptr(), n, t.fpm, L, d, t.order, t.emb_dim, self.w_mod, self.shift,
-                                       base, base + o_spec, stream))
+        if taps:
+            check(lib.m2_mixer_taps_fwd(t.table.data_ptr(), n, t.fpm, L, d, t.order, t.emb_dim, self.w_mod, self.shift, base, base + o_spec, stream))
+        else:
+            check(lib.m2_mixer_filters_fwd(t.table.data_ptr(), t.skip.data_ptr(), n, t.fpm, L, d, t.order, t.emb_dim, self.w_mod, self.shift,
+                                           base, base + o_spec, stream))
         if ids is not None:
             p16, pT = base + o_in, base + o_in + up(2 * M * d)
             check(lib.m2_embed_layernorm_fwd(ids.data_ptr(), None if tt is None else tt.data_ptr(), None if pos is None else pos.data_ptr(),
                                              *part.args, None, p16, pT, part.bad_index, B, L, d, stream))
         else:
             p16, pT = h16.data_ptr(), hT.data_ptr()
-        check(lib.m2_encoder_layers_fwd(route[0], n, base + o_spec, p16, pT, ptrs, base + o_act, B, L, d, self.I, self.nb, self.eps, stream))
+        if taps:
+            check(lib.m2_encoder_layers_taps_fwd(route[0], n, base + o_spec, t.skip.data_ptr(), t.fpm, p16, pT, ptrs, base + o_act, B, L, d,
+                                                 self.I, self.nb, self.eps, stream))
+        else:
+            check(lib.m2_encoder_layers_fwd(route[0], n, base + o_spec, p16, pT, ptrs, base + o_act, B, L, d, self.I, self.nb, self.eps, stream))
         return outs
 
 

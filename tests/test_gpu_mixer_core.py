@@ -67,3 +67,61 @@ def test_rows_dealt_unevenly(gpu, L, d, B):
     ref = _conv(x.double(), k, torch.zeros(d, device=gpu))
     tol = 2 * (2.5 * 3 * (L.bit_length() - 1) + 6) ** 0.5 * 2.0 ** -25
     assert ((y - ref).norm(dim=2) <= tol * ref.norm(dim=2)).all()
+
+
+@pytest.mark.parametrize("L,d,B", [(1024, 8, 1), (1024, 24, 3), (2048, 16, 1), (4096, 768, 1), (4096, 8, 2), (8192, 16, 1), (8192, 768, 1), (16384, 8, 1)])
+@pytest.mark.parametrize("nfilters", [1, 2])
+def test_mixer_core_on_taps(gpu, L, d, B, nfilters):
+    """The core that transforms its filters itself, in part filled workgroups and with workgroups that take several rows, against fp64 transforms
+    and against the core on spectra: fp32 sums of the same numbers whose rounding to bf16 falls the other way now and then."""
+    from m2_amd import ops
+    g = torch.Generator(device=gpu).manual_seed(L + d + B)
+    rn = lambda *s: torch.randn(*s, generator=g, device=gpu)      # noqa: E731
+    taps, D = rn(nfilters, d, 2 * L) / L ** 0.5, rn(nfilters, d)
+    row = B * L + 64
+    xproj, u = rn(3 * d, row).bfloat16(), rn(d, B, L)
+    sw, sb, pb = rn(3 * d, 3), rn(3 * d), rn(3 * d)
+
+    class Table:
+        fpm = nfilters
+
+        def use_on(self, handle):
+            pass
+
+    for skips in (True, False):
+        skip = torch.tensor([D[f].data_ptr() if skips else 0 for f in range(nfilters)], dtype=torch.int64).to(gpu)
+        zero = torch.zeros_like(D)
+        Ds = D if skips else zero
+        x = torch.nn.functional.pad(xproj[:, :B * L].view(3 * d, B, L).double() + pb.double()[:, None, None], (2, 0))
+        s = sb.double()[:, None, None] + sum(sw.double()[:, k, None, None] * x[..., k:k + L] for k in range(3))
+        ref = _conv(s[:d] * s[2 * d:], taps[0], Ds[0]) * s[d:2 * d]
+        if nfilters == 2:
+            ref = ref + _conv(u.double(), taps[1], Ds[1])
+        second = u if nfilters == 2 else None
+        y = ops.mixer_core(xproj, second, sw, sb, ops.MixerTaps(taps, skip.data_ptr(), Table()), B, L, d, proj_bias=pb, row=row)
+        spec = ops.filter_spectrum(taps[0], taps[1] if nfilters == 2 else None, Ds[0], Ds[1] if nfilters == 2 else None)
+        z = ops.mixer_core(xproj, second, sw, sb, spec, B, L, d, proj_bias=pb, row=row)
+        assert (y.double() - ref).norm() <= 2.0 ** -8 * ref.norm()      # (the gate and the result are rounded to 2^-9)
+        assert (y.double() - z.double()).norm() <= 2.0 ** -12 * ref.norm()
+
+
+def test_core_on_taps_refuses(gpu):
+    from m2_amd import ops
+    L, d = 1024, 8
+    x, taps = torch.randn(3 * d, 1, L, device=gpu), torch.randn(2, d, 2 * L, device=gpu)
+    sw, sb = torch.randn(3 * d, 3, device=gpu), torch.randn(3 * d, device=gpu)
+
+    class Table:
+        fpm = 2
+
+        def use_on(self, handle):
+            pass
+
+    filters = ops.MixerTaps(taps, None, Table())
+    with pytest.raises(TypeError):
+        ops.mixer_core(x, None, sw, sb, filters, 1, L, d)                       # fp32 rows read spectra
+    with pytest.raises(ValueError):
+        ops.mixer_core(x.bfloat16()[:, :, :512].contiguous(), None, sw, sb, filters, 1, 512, d)
+    short = ops.MixerTaps(taps[:, :, :1024].contiguous(), None, Table())
+    with pytest.raises(RuntimeError):
+        ops.mixer_core(x.bfloat16()[:, :, :512].contiguous(), None, sw, sb, short, 1, 512, d)

@@ -1,0 +1,76 @@
+"""Forwards of one sequence, whose mixer cores read filter taps, against the same ones on spectra."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _spectra_only(call):
+    """The call with every core on spectra, and how many cores were on taps without that."""
+    from m2_amd import ops, schedule  # noqa: F401
+    kept, asked = ops.taps_pay, []
+    ops.taps_pay = lambda B, L, dtype: (asked.append(kept(B, L, dtype)), False)[1]
+    try:
+        return call(), sum(asked)
+    finally:
+        ops.taps_pay = kept
+
+
+def _close(a, b):
+    # fp32 sums in another order ahead of bf16 roundings, of which a few fall the other way: two layers of 2^-9, mostly the same
+    return (a.double() - b.double()).norm() <= 2.0 ** -8 * b.double().norm()
+
+
+@pytest.mark.parametrize("helper,L,residual", [("m2_bert_80m", 1024, True), ("m2_bert_80m", 2048, False), ("m2_bert_80m", 16384, True),
+                                               ("m2_bert_110m", 4096, True), ("m2_bert_large", 2048, True)])
+def test_one_sequence(gpu, helper, L, residual):
+    import m2_amd
+    cfg = getattr(m2_amd, helper)(L)
+    cfg.num_hidden_layers, cfg.residual_long_conv = 2, residual
+    model = m2_amd.BertModel(cfg)
+    model.load_state_dict(m2_amd.seeded_state_dict(cfg, 3))
+    model = model.to(gpu).eval()
+    ids = torch.randint(0, cfg.vocab_size, (1, L), generator=torch.Generator().manual_seed(4)).to(gpu)
+    with torch.no_grad():
+        (want, pooled), taps = _spectra_only(lambda: model(ids))
+        assert taps
+        got, gpooled = model(ids)
+        assert _close(got, want) and _close(gpooled, pooled)
+        model.encoder.native_schedule = False
+        for overlap in (None, False):
+            model.encoder.overlap_filters = overlap
+            assert torch.equal(model(ids)[0], got)
+        model.encoder.overlap_filters = None
+        layer = model.encoder.layer[0]
+        u = torch.randn(1, L, cfg.hidden_size, generator=torch.Generator().manual_seed(5)).to(gpu).bfloat16()
+        want, taps = _spectra_only(lambda: layer.attention(u)[0])
+        assert taps == 1 and _close(layer.attention(u)[0], want)
+
+
+def test_mixers_of_a_callers_own_are_given_spectra(gpu):
+    """A core put in the place of the module's, and kept spectra, see tensors as before; a graph of the taps route replays."""
+    import m2_amd
+    L = 1024
+    cfg = m2_amd.m2_bert_80m(L)
+    cfg.num_hidden_layers = 2
+    model = m2_amd.BertModel(cfg, use_hip_graph=True)
+    model.load_state_dict(m2_amd.seeded_state_dict(cfg, 6))
+    model = model.to(gpu).eval()
+    ids = [torch.randint(0, cfg.vocab_size, (1, L), generator=torch.Generator().manual_seed(s)).to(gpu) for s in (7, 8, 9)]
+    with torch.no_grad():
+        graphed = [model(i)[0] for i in ids]
+        model.encoder.use_hip_graph = False
+        assert all(torch.equal(model(i)[0], g) for i, g in zip(ids, graphed))
+        model.encoder.native_schedule = False
+        at, seen = model.encoder.layer[1].attention, []
+        core = type(at).core
+
+        def own(xproj, u, B, L, spec=None):
+            seen.append(type(spec))
+            return core(at, xproj, u, B, L, spec=spec)
+
+        at.core = own
+        assert _close(model(ids[0])[0], graphed[0]) and seen == [torch.Tensor]
+        del at.core
+        at.cache_filters = True
+        assert _close(model(ids[0])[0], graphed[0]) and isinstance(at._spec_cache[1], torch.Tensor)
