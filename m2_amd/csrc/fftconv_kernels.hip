@@ -66,7 +66,7 @@ __global__ __launch_bounds__(SpectrumLayout<P>::WG) __attribute__((amdgpu_waves_
   for (int i0 = blockIdx.x * RPW; i0 < 2 * d; i0 += gridDim.x * RPW) {
     const int item = i0 + rloc < 2 * d ? i0 + rloc : 2 * d - 1, c = item >> 1;
     const float* taps = item & 1 ? taps2 : taps1;
-    const float* D = item & 1 ? D2 : D1;
+    gfloat* D = in_global(item & 1 ? D2 : D1);
     cf x[E];
     if (taps) {
       const float* p = taps + (long)c * 2 * L + t;

@@ -429,7 +429,7 @@ __global__ __launch_bounds__(P::T) __attribute__((amdgpu_waves_per_eu(2, 2))) vo
   for (int item = blockIdx.x; item < 2 * d; item += gridDim.x) {
     const int c = item >> 1;
     const float* taps = item & 1 ? taps2 : taps1;
-    const float* D = item & 1 ? D2 : D1;
+    gfloat* D = in_global(item & 1 ? D2 : D1);
     float4* blk = reinterpret_cast<float4*>(spec + (long)item * 2 * BLK) + t;
     if (!taps) {
       static_for<0, 2>([&](auto hh) {

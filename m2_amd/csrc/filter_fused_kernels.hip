@@ -50,20 +50,19 @@ __global__ __launch_bounds__(2 * kFusedRows * P::T) void project_spectrum_kernel
 
   // ---- phase 1: projection + decay into the window ----
   {
-    const int m = wave % nmlp, which = m >> 1, dir = m & 1;
+    const int m = __builtin_amdgcn_readfirstlane(wave) % nmlp, which = m >> 1, dir = m & 1;
     const int f = mixer * fpm + which;
-    const FilterPtrs& F = tab[f];
-    const float* W3 = F.mlp[dir].w3;
+    gfloat *const W3 = in_global(tab[f].mlp[dir].w3), *const tt = in_global(tab[f].t), *const deltas = in_global(tab[f].deltas);
     if (W3 != nullptr) {
       f16x8 ahi[kOrder / 32], alo[kOrder / 32];
       float rs[4];                     // reciprocal scales of the lane's four channels
       {
-        const float* wrow = W3 + (long)(c0 + i16) * kOrder + 8 * q4;
+        gfloat* wrow = W3 + (long)(c0 + i16) * kOrder + 8 * q4;
         float v[kOrder / 4], top = 0.f;
 #pragma unroll
         for (int ks = 0; ks < kOrder / 32; ++ks) {
-          const float4 v0 = *reinterpret_cast<const float4*>(wrow + 32 * ks);
-          const float4 v1 = *reinterpret_cast<const float4*>(wrow + 32 * ks + 4);
+          const floatx4 v0 = *(gfloatx4*)(wrow + 32 * ks);
+          const floatx4 v1 = *(gfloatx4*)(wrow + 32 * ks + 4);
           v[8 * ks] = v0.x; v[8 * ks + 1] = v0.y; v[8 * ks + 2] = v0.z; v[8 * ks + 3] = v0.w;
           v[8 * ks + 4] = v1.x; v[8 * ks + 5] = v1.y; v[8 * ks + 6] = v1.z; v[8 * ks + 7] = v1.w;
         }
@@ -90,7 +89,7 @@ __global__ __launch_bounds__(2 * kFusedRows * P::T) void project_spectrum_kernel
       }
       float adelta[4];
 #pragma unroll
-      for (int j = 0; j < 4; ++j) adelta[j] = -fabsf(F.deltas[c0 + 4 * q4 + j]) * 1.44269504088896341f;
+      for (int j = 0; j < 4; ++j) adelta[j] = -fabsf(deltas[c0 + 4 * q4 + j]) * 1.44269504088896341f;
       const uint16_t* gh = h_hi + ((long)(2 * f + dir) * L + i16) * kOrder + 8 * q4;
       const uint16_t* gl = h_lo + ((long)(2 * f + dir) * L + i16) * kOrder + 8 * q4;
       // the waves that share an MLP take its 16-position tiles in turn
@@ -102,7 +101,7 @@ __global__ __launch_bounds__(2 * kFusedRows * P::T) void project_spectrum_kernel
           bl[ks] = *reinterpret_cast<const u32x4*>(gl + (long)pt * 16 * kOrder + 32 * ks);
         }
         const int p = 16 * pt + i16;
-        const float tl = F.t[p];
+        const float tl = tt[p];
         floatx4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int ks = 0; ks < kOrder / 32; ++ks) {      // smallest terms first
@@ -136,7 +135,7 @@ __global__ __launch_bounds__(2 * kFusedRows * P::T) void project_spectrum_kernel
     x[r] = lds_get(row + P::phys(t + T * (r / P::R1)), P::phys(P::S1 * (r % P::R1)));
   });
   if (t == 0 && skip != nullptr && which < fpm) {      // the skip weight D is one more tap at lag 0
-    const float* D = skip[mixer * fpm + which];
+    gfloat* D = in_global(skip[mixer * fpm + which]);
     if (D) x[0].re += D[c];
   }
   forward(x, t, row, factors);

@@ -38,8 +38,15 @@ struct TabByPointer {
   __device__ __forceinline__ const FilterPtrs& at(int i) const { return p[i]; }
 };
 
+// The tables hold plain pointers, of which a kernel cannot know that they point to device memory.  Loads through them were flat ones,
+// whose results come back out of order with LDS reads: every wait for an LDS read was a wait for them too; and where a kernel stores,
+// the pointer itself was loaded again for each use, in a wait for all that was in flight.  So kernels take a filter's pointers
+// out of the table once, at their start, through in_global.  us for the filters of a mixer of 768 channels, with the 64-bit vector address
+// that each store of a tap had, before / now: 12 mixers at once L = 1024 13.4 / 12.9, 4096 45.2 / 43.4, 8192 82.2 / 80.1, three at 32768
+// 336 / 326; one mixer 512 55.0 / 52.9, 1024 45.7 / 43.8, 4096 61.7 / 59.6, 8192 96.8 / 92.5.
 typedef float floatx16 __attribute__((ext_vector_type(16)));
 typedef float floatx4 __attribute__((ext_vector_type(4)));
+typedef const __attribute__((address_space(1))) floatx4 gfloatx4;
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 // The matrix products of the filter MLPs, fp32 accumulation.

@@ -65,9 +65,9 @@ __global__ __launch_bounds__(512) void split_weights_kernel(TAB tab, int nmlp, i
   const int lane = threadIdx.x & 63, i32 = lane & 31, ks = threadIdx.x >> 6;
   if ((int)blockIdx.x < inner) {
     const int w = blockIdx.x & 3, layer = (blockIdx.x >> 2) & 1, m = blockIdx.x >> 3;
-    const MlpPtrs& W = tab.at(m >> 1).mlp[m & 1];
+    const MlpPtrs W = tab.at(m >> 1).mlp[m & 1];
     if (W.w0 == nullptr) return;
-    const float* src = (layer == 0 ? W.w1 : W.w2) + (long)(32 * w + i32) * kOrder + 16 * ks + 8 * (lane >> 5);
+    gfloat* src = in_global(layer == 0 ? W.w1 : W.w2) + (long)(32 * w + i32) * kOrder + 16 * ks + 8 * (lane >> 5);
     u32x4 vh, vm, vl;
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
@@ -86,9 +86,9 @@ __global__ __launch_bounds__(512) void split_weights_kernel(TAB tab, int nmlp, i
   }
   __shared__ float most[8][32];
   const int ct = ((int)blockIdx.x - inner) % (d / 32), m = ((int)blockIdx.x - inner) / (d / 32);
-  const MlpPtrs& W = tab.at(m >> 1).mlp[m & 1];
+  const MlpPtrs W = tab.at(m >> 1).mlp[m & 1];
   if (W.w3 == nullptr) return;
-  const float* src = W.w3 + (long)(32 * ct + i32) * kOrder + 16 * ks + 8 * (lane >> 5);
+  gfloat* src = in_global(W.w3) + (long)(32 * ct + i32) * kOrder + 16 * ks + 8 * (lane >> 5);
   float v[8], top = 0.f;
 #pragma unroll
   for (int j = 0; j < 8; ++j) {
@@ -140,10 +140,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   constexpr int P = 32 * TILES;
   __shared__ __attribute__((aligned(16))) unsigned char act[3][P * kActRowB];
   __shared__ float zt[P * kMaxEmb];
-  const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63, i32 = lane & 31, half = lane >> 5;
+  const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, i32 = lane & 31, half = lane >> 5;
   const int fi = blockIdx.y >> 1, dir = blockIdx.y & 1;
   const FilterPtrs& F = tab.at(fi);
-  const MlpPtrs& W = F.mlp[dir];
+  const MlpPtrs W = F.mlp[dir];
+  gfloat *const z = in_global(F.z), *const tt = in_global(F.t), *const freq = in_global(F.freq), *const deltas = in_global(F.deltas);
+  gfloat *const w0 = in_global(W.w0), *const b0 = in_global(W.b0), *const b1 = in_global(W.b1), *const b2 = in_global(W.b2);
   const int l0 = blockIdx.x * P;
   if (W.w0 == nullptr) {                        // not bidirectional: nothing to compute for dir == 1 ...
     if constexpr (PROJECT) {                    // ... and the reverse half of the window is zero
@@ -175,12 +177,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   // 2's before the last epilogue of layer 1), so that the 24 KB per wave arrive behind other work.
   bf16x8 ah[8], am[8], al[8];
   auto load_weights = [&](int layer) __attribute__((always_inline)) {
-    const u32x4* wp = reinterpret_cast<const u32x4*>(wsplit + ((long)(blockIdx.y * 2 + layer)) * kSplitPerLayer) + w * 8 * 64 + lane;
+    const u32x4* wp = reinterpret_cast<const u32x4*>(wsplit + ((long)(blockIdx.y * 2 + layer)) * kSplitPerLayer) + w * 8 * 64;
 #pragma unroll
     for (int ks = 0; ks < 8; ++ks) {
-      ah[ks] = __builtin_bit_cast(bf16x8, wp[ks * 64]);
-      am[ks] = __builtin_bit_cast(bf16x8, wp[ks * 64 + kOrder * kOrder / 8]);
-      al[ks] = __builtin_bit_cast(bf16x8, wp[ks * 64 + 2 * kOrder * kOrder / 8]);
+      ah[ks] = __builtin_bit_cast(bf16x8, (wp + ks * 64)[(unsigned)lane]);
+      am[ks] = __builtin_bit_cast(bf16x8, (wp + ks * 64 + kOrder * kOrder / 8)[(unsigned)lane]);
+      al[ks] = __builtin_bit_cast(bf16x8, (wp + ks * 64 + 2 * kOrder * kOrder / 8)[(unsigned)lane]);
     }
   };
   load_weights(0);
@@ -188,15 +190,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   // layer 0 (emb -> 128) on the vector ALU: thread = (4 neurons, P / 8 positions).  The embeddings of the tile
   // (P x emb consecutive floats) go through LDS; weights beyond emb are zero so the dot product has a fixed length.
   {
-    for (int i = tid; i < P * kMaxEmb; i += 256) zt[i] = i < P * emb ? F.z[(long)l0 * emb + i] : 0.f;
+    for (int i = tid; i < P * kMaxEmb; i += 256) zt[i] = i < P * emb ? z[(long)l0 * emb + i] : 0.f;
     const int o = 4 * (tid & 31), p0 = tid >> 5;          // positions p0, p0 + 8, ...
     float wt[4][kMaxEmb], bb[4], fo[4];
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
 #pragma unroll
-      for (int e = 0; e < kMaxEmb; ++e) wt[j][e] = e < emb ? W.w0[(o + j) * emb + e] : 0.f;
-      bb[j] = W.b0[o + j];
-      fo[j] = w_mod * F.freq[o + j];
+      for (int e = 0; e < kMaxEmb; ++e) wt[j][e] = e < emb ? w0[(o + j) * emb + e] : 0.f;
+      bb[j] = b0[o + j];
+      fo[j] = w_mod * freq[o + j];
     }
     __syncthreads();
 #pragma unroll 4
@@ -239,12 +241,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   // accumulator element v: neuron 32 w + 8 (v / 4) + 4 half + v % 4, position i32 of the tile
   float fr[16], bs[16];
   auto load_scales = [&](int layer) __attribute__((always_inline)) {
-    const float* bias = layer == 0 ? W.b1 : W.b2;
+    gfloat* bias = layer == 0 ? b1 : b2;
 #pragma unroll
     for (int vq = 0; vq < 4; ++vq) {
       const int o = 32 * w + 8 * vq + 4 * half;
-      const float4 fq = *reinterpret_cast<const float4*>(F.freq + o);
-      const float4 bq = *reinterpret_cast<const float4*>(bias + o);
+      const floatx4 fq = *(gfloatx4*)(freq + o);
+      const floatx4 bq = *(gfloatx4*)(bias + o);
       fr[4 * vq] = w_mod * fq.x; fr[4 * vq + 1] = w_mod * fq.y; fr[4 * vq + 2] = w_mod * fq.z; fr[4 * vq + 3] = w_mod * fq.w;
       bs[4 * vq] = bq.x; bs[4 * vq + 1] = bq.y; bs[4 * vq + 2] = bq.z; bs[4 * vq + 3] = bq.w;
     }
@@ -300,27 +302,27 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   if constexpr (PROJECT) {
     // the barrier that ended the last layer says h3 (hi in act[0], lo in act[1]) is complete for all P positions
     float* out = taps + (long)fi * d * 2 * L;
-    const u32x4* w3 = reinterpret_cast<const u32x4*>(w3split + (long)blockIdx.y * 2 * d * kOrder) + lane;
+    const u32x4* w3 = reinterpret_cast<const u32x4*>(w3split + (long)blockIdx.y * 2 * d * kOrder);
     const float* back = w3scale + (long)blockIdx.y * d;
     float tl[TILES];
 #pragma unroll
-    for (int t = 0; t < TILES; ++t) tl[t] = F.t[l0 + 32 * t + i32];
+    for (int t = 0; t < TILES; ++t) tl[t] = tt[l0 + 32 * t + i32];
     // A operand of a channel tile: weight rows 32 ct + i32, K = 16 ks + 8 half + {0..7}, hi / lo parts as
     // split_weights_kernel left them, and the decay rates and scales of the lane's 16 channels
     struct TileOps {
       f16x8 ahi[kOrder / 16], alo[kOrder / 16];
-      float4 dq[4], rq[4];
+      floatx4 dq[4], rq[4];
     };
     auto fetch_tile = [&](int ct, TileOps& o) __attribute__((always_inline)) {
 #pragma unroll
       for (int ks = 0; ks < kOrder / 16; ++ks) {
-        o.ahi[ks] = __builtin_bit_cast(f16x8, w3[(ct * 8 + ks) * 64]);
-        o.alo[ks] = __builtin_bit_cast(f16x8, w3[(ct * 8 + ks) * 64 + d * kOrder / 8]);
+        o.ahi[ks] = __builtin_bit_cast(f16x8, (w3 + (ct * 8 + ks) * 64)[(unsigned)lane]);
+        o.alo[ks] = __builtin_bit_cast(f16x8, (w3 + (ct * 8 + ks) * 64 + d * kOrder / 8)[(unsigned)lane]);
       }
 #pragma unroll
       for (int vq = 0; vq < 4; ++vq) {
-        o.dq[vq] = *reinterpret_cast<const float4*>(F.deltas + 32 * ct + 8 * vq + 4 * half);
-        o.rq[vq] = *reinterpret_cast<const float4*>(back + 32 * ct + 8 * vq + 4 * half);
+        o.dq[vq] = ((gfloatx4*)(deltas + 32 * ct + 8 * vq))[(unsigned)half];
+        o.rq[vq] = reinterpret_cast<const floatx4*>(back + 32 * ct + 8 * vq)[(unsigned)half];
       }
     };
     auto project_tile = [&](int ct, const TileOps& o) __attribute__((always_inline)) {
@@ -348,13 +350,20 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         }
         // accumulator element v of lane: channel 32 ct + 8 (v / 4) + 4 half + v % 4, position l0 + 32 t + i32
         const int l = l0 + 32 * t + i32;
-        float* po = out + (long)(32 * ct + 4 * half) * 2 * L + (dir == 0 ? l : (2L * L - 1 - l));
+        // A row is the same for all lanes: its address walks along in scalar registers (kept by the asm, which the compiler would turn into
+        // sixteen vector addresses), the lane's place in it is a 32-bit offset.
+        typedef __attribute__((address_space(1))) char gbyte;
+        gbyte* po = (gbyte*)out + (long)(32 * ct) * 8 * L;
+        unsigned at = 4u * (4u * half * 2 * L + (dir == 0 ? l : 2 * L - 1 - l));
+        asm volatile("" : "+v"(at));
 #pragma unroll
         for (int v = 0; v < 16; ++v) {
+          asm volatile("" : "+s"(po));
           // (exp(-t |delta|) + shift) r, r the reciprocal scale of the channel; the bare hardware exp2 flushes results below 2^-126 to zero, which is the value to
           // 1e-38 absolute.  Streaming store: the taps are read once, by a later kernel
           const float decay = fmaf(__builtin_amdgcn_exp2f(tl[t] * adelta[v]), rs[v], shift * rs[v]);
-          __builtin_nontemporal_store(acc[v] * decay, po + (long)(8 * (v >> 2) + (v & 3)) * 2 * L);
+          __builtin_nontemporal_store(acc[v] * decay, (__attribute__((address_space(1))) float*)(po + at));
+          po += (v & 3) == 3 ? 40l * L : 8l * L;      // channels 8 (v / 4) + v % 4 of the tile
         }
       }
     };
@@ -392,12 +401,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 4))) voi
   __shared__ float4 rate[4][8], back[4][8];        // of a wave's 32 channels: -|delta| log2(e), reciprocal scale
   const int fi = blockIdx.z >> 1, dir = blockIdx.z & 1;
   const FilterPtrs& F = tab.at(fi);
+  gfloat *const w3 = in_global(F.mlp[dir].w3), *const tt = in_global(F.t), *const deltas = in_global(F.deltas);
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, i32 = lane & 31, half = lane >> 5;
   const int c0 = blockIdx.y * 128 + wave * 32;
   const bool active = c0 < d;                      // d is a multiple of 64: a wave is all in or all out
   const int lbase = blockIdx.x * kPosPerWg;
   float* out = taps + (long)fi * d * 2 * L;
-  if (F.mlp[dir].w3 == nullptr) {
+  if (w3 == nullptr) {
     // not bidirectional: the reverse half of the window is zero
     if (active)
       for (int r = 0; r < 32; ++r)
@@ -436,7 +446,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 4))) voi
   // parts, read a second time for the splitting, it took 1.4 us more (taps of one filter, d = 768: L = 128 21.7 us, 512 36.2, 8224 54)
   f16x8 ahi[kOrder / 16], alo[kOrder / 16];
   if (active) {
-    const float* row = F.mlp[dir].w3 + (long)(c0 + i32) * kOrder + 8 * half;
+    gfloat* row = w3 + (long)(c0 + i32) * kOrder + 8 * half;
     float top = 0.f;
 #pragma unroll
     for (int ks = 0; ks < kOrder / 16; ++ks)
@@ -458,7 +468,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 4))) voi
       alo[ks] = __builtin_bit_cast(f16x8, vl);
     }
     if (half == 0) {
-      reinterpret_cast<float*>(rate[wave])[i32] = -fabsf(F.deltas[c0 + i32]) * 1.44269504088896341f;
+      reinterpret_cast<float*>(rate[wave])[i32] = -fabsf(deltas[c0 + i32]) * 1.44269504088896341f;
       reinterpret_cast<float*>(back[wave])[i32] = 1.f / (scale * kActScale);
     }
   }
@@ -486,7 +496,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 4))) voi
       }
       // accumulator element v of lane: channel c0 + 8 (v / 4) + 4 half + v % 4, position i32
       const int l = lbase + pt * 32 + i32;
-      const float tl = F.t[l];
+      const float tl = tt[l];
       float* po = out + (long)(c0 + 4 * half) * 2 * L + (dir == 0 ? l : (2L * L - 1 - l));
 #pragma unroll
       for (int vq = 0; vq < 4; ++vq) {

@@ -29,6 +29,10 @@ int blockdiag_linear_engine(const void* x, const void* w, const float* bias, con
 bool dense_ws_serves(int M, int N, int K);
 int dense_ws_launch(const void* x, const void* w, void* out, int M, int N, long ldo, hipStream_t stream);
 
+// A pointer that was read from memory, said to point to device memory: loads through it are global ones and not flat ones.
+typedef const __attribute__((address_space(1))) float gfloat;
+__device__ __forceinline__ gfloat* in_global(const float* p) { return (gfloat*)p; }
+
 // round-to-nearest-even float -> bfloat16 bits (NaN stays NaN)
 // float -> bf16 bits, round to nearest even (host restatement of what v_cvt_pk_bf16_f32 does)
 __host__ __device__ __forceinline__ uint16_t f32_to_bf16_bits(float f) {

@@ -93,7 +93,7 @@ __global__ __launch_bounds__(P::T) __attribute__((amdgpu_waves_per_eu(2, 2))) vo
     load_taps<P>(K, filters.taps + ((long)f * d + c) * (2L * L), anew(t));
   };
   auto transform_taps = [&](int c, int f) __attribute__((always_inline)) {
-    const float* D = filters.skip ? filters.skip[f] : nullptr;
+    gfloat* D = filters.skip ? in_global(filters.skip[f]) : nullptr;
     if (D && t == 0) K[0].re += D[c];      // the skip weight is one more tap at lag 0
     transform<P, kQuarter>(K, anew(t), row, tab, tf);
   };

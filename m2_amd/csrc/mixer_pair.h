@@ -141,7 +141,7 @@ __global__ __launch_bounds__(PairLayout<P>::WG) __attribute__((amdgpu_waves_per_
       fetch_batch(j0);                     // (travels while the taps are transformed)
       __builtin_amdgcn_sched_barrier(0);
       if (sig < filters.nfilters) {
-        const float* D = filters.skip ? filters.skip[sig] : nullptr;
+        gfloat* D = filters.skip ? in_global(filters.skip[sig]) : nullptr;
         if (D && t == 0) K[0].re += D[c];      // the skip weight is one more tap at lag 0
       } else {
         static_for<0, E>([&](auto rr) { K[decltype(rr)::value] = {0.f, 0.f}; });
