@@ -91,7 +91,7 @@ __global__ __launch_bounds__(256) void mlp_fused_pack_kernel(const uint16_t* __r
 }
 
 // WAVES = 8: the kernel as described above.  WAVES = 4: the same with workgroups of four waves and 64 rows, for row
-// counts at which 128-row tiles would leave compute units without work (M < 8192: one wave per SIMD, every wave
+// counts of which those make no more workgroups than there are compute units (M <= 4096: one wave per SIMD, every wave
 // copies 9 of a chunk's 36 blocks).
 template <typename OUT, int WAVES>
 __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(WAVES / 4, 2))) void mlp_fused_kernel(
@@ -403,9 +403,10 @@ extern "C" int m2_mlp_fused_fwd(const void* x, const void* w_packed, const float
                      "m2_mlp_fused_fwd: built for nblocks=4, in_features=768 and intermediate a multiple of 128 "
                      "(got nblocks=%d in=%d intermediate=%d); use m2_blockdiag_glu_fwd + m2_blockdiag_linear_fwd",
                      nblocks, in_features, intermediate);
-  // 128-row tiles and eight waves per workgroup; 64-row tiles and four waves where the 128-row tiles of the four
-  // output blocks would not occupy the compute units (M < 8192 on 256 of them)
-  const bool small = 4 * ((M + kFRows - 1) / kFRows) < num_cus();
+  // 128-row tiles and eight waves per workgroup; 64-row tiles and four waves where one round of those does (M up to 4096 on 256 compute
+  // units).  Beyond, two rounds of those take longer than one of the large ones: M = 4104 40.4 / 29.7 us, 5632 41.2 / 30.4, 8000
+  // 43.4 / 34.9; one round of the small ones 22.6 at M = 2048, 24.6 at 4096.
+  const bool small = 4l * ((M + kFRows / 2 - 1) / (kFRows / 2)) <= num_cus();
   const int rows = small ? kFRows / 2 : kFRows;
   const int ntiles = (M + rows - 1) / rows;
   // one persistent workgroup per compute unit (144 KB of LDS each), an even number per XCD
