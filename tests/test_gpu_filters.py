@@ -169,3 +169,21 @@ def test_arguments_without_a_sine_left(gpu, L, d):
     with torch.no_grad():
         fn.implicit_filter[4].bias[0] = float("nan")
     assert not torch.isfinite(fn.bidirectional_taps(L)[:, :L]).any()
+
+
+@pytest.mark.parametrize("bidirectional", [True, False])
+@pytest.mark.parametrize("fpm", [1, 2])
+@pytest.mark.parametrize("L", [128, 256, 512])
+def test_spectra_of_many_mixers_at_once(gpu, L, fpm, bidirectional):
+    """Enough mixers for workgroups of 32 channels: the same bits as one mixer at a time, whose workgroups have 16."""
+    import m2_amd
+    from m2_amd import ops
+    d, n = 768, 6
+    torch.manual_seed(L + fpm)
+    mixers = [m2_amd.MonarchMixerSequenceMixing(d, l_max=L, bidirectional=bidirectional, hyena_emb_dim=5, hyena_filter_order=128,
+                                                residual_long_conv=fpm == 2).to(gpu) for _ in range(n)]
+    entries = [m.filter_table_entry() for m in mixers]
+    table = ops.FilterTable([e[0] for e in entries], [e[1] for e in entries], L, d, 128, 5)
+    together = ops.mixer_filter_spectra(table)
+    for i in range(n):
+        assert torch.equal(together[i], ops.mixer_filter_spectra(table, first=i, count=1)[0])
