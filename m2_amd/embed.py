@@ -9,6 +9,7 @@ token ids directly to `encode_token_ids`.
 from __future__ import annotations
 
 from array import array
+from collections import deque
 from typing import Callable, Dict, Iterable, List, Optional, Sequence
 
 import numpy as np
@@ -65,27 +66,74 @@ class M2BertTextEncoder:
         """token_ids: one 1-D sequence of ids per text (any lengths, may be empty); returns (len(token_ids), d)
         fp32.  Without attention_masks every given token counts as real and the padding as masked."""
         out = [torch.empty(0, self.model.config.hidden_size)]
-        for lo in range(0, len(token_ids), batch_size):
-            hi = min(lo + batch_size, len(token_ids))
-            ids_b, mask_b = self._assemble(token_ids, attention_masks, lo, hi)
-            with torch.no_grad():
-                _, pooled = self.model(input_ids=ids_b.to(self.device), attention_mask=mask_b.to(self.device))
-            out.append(pooled.detach().float().cpu())
+        if self._plain_model():
+            self._run_ahead(token_ids, batch_size, attention_masks, out)
+        else:
+            for lo in range(0, len(token_ids), batch_size):
+                hi = min(lo + batch_size, len(token_ids))
+                ids_b, mask_b = self._assemble(token_ids, attention_masks, lo, hi)
+                with torch.no_grad():
+                    _, pooled = self.model(input_ids=ids_b.to(self.device), attention_mask=mask_b.to(self.device))
+                out.append(pooled.detach().float().cpu())
         out = torch.cat(out, 0)
         if torch.isnan(out).any():
             raise ValueError("NaNs in the encoded texts")
         return out.numpy()
 
-    def _assemble(self, token_ids: Sequence, attention_masks: Optional[Sequence], lo: int, hi: int):
-        """Texts [lo, hi) as padded or cut (hi - lo, max_seq_len) ids and mask.  Rows are written into two arrays, 7 us a
+    def _plain_model(self) -> bool:
+        """The model's forward is the one of this package, with nothing around it that would see its arguments."""
+        m = self.model
+        return (type(m).forward is BertModel.forward and "forward" not in m.__dict__ and not m._forward_hooks and not m._forward_pre_hooks
+                and torch.device(self.device).type == "cuda")
+
+    def _run_ahead(self, token_ids: Sequence, batch_size: int, attention_masks: Optional[Sequence], out: List[torch.Tensor]) -> None:
+        """The batches enqueued up to two ahead of the GPU: while one is computed the next is put together, in pinned memory that the GPU
+        fetches by itself, and nothing is waited for but the batch before the last (waiting for each batch's copies and for its check
+        of the token ids left the GPU idle for 0.7 ms between two batches of 32 x 512: 75 texts 9.7 ms, now 8.7; 512 texts 60.9, now 48.1).  The ids are checked
+        once, behind the last batch or ahead of another error."""
+        emb, pending = self.model.embeddings, deque()
+
+        def finish():
+            host, done = pending.popleft()
+            done.synchronize()
+            out.append(host)
+
+        try:
+            for lo in range(0, len(token_ids), batch_size):
+                hi = min(lo + batch_size, len(token_ids))
+                both = torch.empty(2, hi - lo, self.max_seq_len, dtype=torch.int64, pin_memory=True)
+                self._assemble(token_ids, attention_masks, lo, hi, both)
+                with torch.no_grad():
+                    ids_b, mask_b = both.to(self.device, non_blocking=True).unbind(0)
+                    _, pooled = self.model(input_ids=ids_b, attention_mask=mask_b, ids_checked_later=True)
+                host = torch.empty(pooled.shape, dtype=torch.float32, pin_memory=True)
+                host.copy_(pooled.detach().float(), non_blocking=True)
+                done = torch.cuda.Event()
+                done.record(torch.cuda.current_stream(pooled.device))
+                pending.append((host, done))
+                if len(pending) > 2:
+                    finish()
+            while pending:
+                finish()
+        finally:
+            if self.model.validate_ids:
+                emb.check_indices()
+
+    def _assemble(self, token_ids: Sequence, attention_masks: Optional[Sequence], lo: int, hi: int, into: Optional[torch.Tensor] = None):
+        """Texts [lo, hi), in the two halves of `into` where given, as padded or cut (hi - lo, max_seq_len) ids and mask.  Rows are written into two arrays, 7 us a
         text of up to 512 tokens; a torch tensor per text, its mask, both padded and all of them concatenated took 41 (3 ms of 75 texts)."""
         L = self.max_seq_len
-        ids_b, mask_b = np.zeros((hi - lo, L), np.int64), np.zeros((hi - lo, L), np.int64)
+        both = np.empty((2, hi - lo, L), np.int64) if into is None else into.numpy()
+        both[...] = 0
+        ids_b, mask_b = both
         for k in range(lo, hi):
             ids = _host_row(token_ids[k])
             mask = None if attention_masks is None else _host_row(attention_masks[k])
             if ids is None or (mask is None and attention_masks is not None):
-                return self._assemble_tensors(token_ids, attention_masks, lo, hi)
+                rows = self._assemble_tensors(token_ids, attention_masks, lo, hi)
+                if into is not None:
+                    torch.stack(rows, out=into)
+                return rows
             if mask is not None and mask.shape != ids.shape:
                 raise ValueError(f"text {k}: {ids.shape[0]} token ids but {mask.shape[0]} mask entries")
             n = min(ids.shape[0], L)

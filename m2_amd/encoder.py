@@ -706,6 +706,6 @@ class BertModel(nn.Module):
         finally:
             # last, behind everything that is to be enqueued: it waits for the stream.  Also when the pooler raises: a bad id is
             # this forward's error and not the next one's
-            if self.validate_ids and not torch.cuda.is_current_stream_capturing():
+            if self.validate_ids and not kwargs.get("ids_checked_later") and not torch.cuda.is_current_stream_capturing():
                 self.embeddings.check_indices()
         return (enc if output_all_encoded_layers else enc[-1]), pooled

@@ -1,0 +1,60 @@
+"""Texts encoded with batches enqueued ahead of the GPU: the results and the errors of one batch after the other."""
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _encoder(gpu, length=128):
+    import m2_amd
+    cfg = m2_amd.m2_bert_80m(length)
+    cfg.num_hidden_layers = 2
+    model = m2_amd.BertModel(cfg)
+    model.load_state_dict(m2_amd.seeded_state_dict(cfg, 11))
+    return m2_amd.M2BertTextEncoder(model.to(gpu), max_seq_len=length)
+
+
+def _texts(n, vocab=30000):
+    g = torch.Generator().manual_seed(n)
+    return [torch.randint(1, vocab, (int(k),), generator=g).tolist() for k in torch.randint(1, 160, (n,), generator=g)]
+
+
+@pytest.mark.parametrize("n,batch", [(0, 4), (1, 4), (23, 3), (9, 1), (40, 16)])
+def test_same_as_one_batch_at_a_time(gpu, n, batch):
+    enc = _encoder(gpu)
+    texts = _texts(n)
+    got = enc.encode_token_ids(texts, batch)
+    hook = enc.model.register_forward_hook(lambda *a: None)      # (a hook sees what it always saw)
+    want = enc.encode_token_ids(texts, batch)
+    hook.remove()
+    assert got.shape == (n, 768) and got.dtype == np.float32 and np.array_equal(got, want)
+    assert np.array_equal(enc.encode_token_ids([torch.tensor(t) for t in texts], batch), got)
+    odd = [t if i % 3 else np.array(t) for i, t in enumerate(texts)]      # rows that torch.as_tensor is asked about
+    assert np.array_equal(enc.encode_token_ids(odd, batch), got)
+    masks = [[1] * len(t) for t in texts]
+    assert np.array_equal(enc.encode_token_ids(texts, batch, attention_masks=masks), got)
+
+
+def test_errors(gpu):
+    enc = _encoder(gpu)
+    texts = _texts(20)
+    want = enc.encode_token_ids(texts, 4)
+    bad = list(texts)
+    bad[9] = [5, 10 ** 6, 7]
+    with pytest.raises(IndexError):
+        enc.encode_token_ids(bad, 4)
+    masks = [[1] * len(t) for t in texts]
+    masks[18] = [1]
+    texts[18] = [1, 2, 3]
+    with pytest.raises(ValueError, match="text 18"):
+        enc.encode_token_ids(texts, 4, attention_masks=masks)
+    with pytest.raises(IndexError):                               # of an earlier batch, ahead of a later one's
+        enc.encode_token_ids(bad[:18] + texts[18:], 4, attention_masks=[[1] * len(t) for t in bad[:18]] + masks[18:])
+    texts = _texts(20)
+    assert np.array_equal(enc.encode_token_ids(texts, 4), want)  # nothing of it is left
+    enc.model.validate_ids = False
+    assert np.isfinite(enc.encode_token_ids(bad, 4)).all()
+    enc.model.validate_ids = True
+    with pytest.raises(IndexError):                               # what nobody asked about is still there
+        enc.model.embeddings.check_indices()
