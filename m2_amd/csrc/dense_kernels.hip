@@ -153,6 +153,186 @@ static int launch_small(GemmArgs g, hipStream_t st) {
   return check_launch("small_gemm");
 }
 
+// ---------------------------------------------------------------------------------------------
+// LayerNorm and in_linear of few rows as one kernel: rows of s (M, d) bf16 are normalised on their way into the product
+//   out (N, M) = w (N, d) LayerNorm(s)^T
+// A workgroup has 32 rows and 16 JT output channels.  The rows come whole into LDS (48 KB at d = 768), where every wave takes the
+// statistics of four as layernorm_kernel does, column by column and lane by lane and by the same expressions, so that the rows have its bits;
+// then every wave normalises its eighth of K in operand layout, and products and sums are small_gemm_kernel's.  The channel-major fp32
+// form that the mixer core reads is written by the workgroups of the first d channels' worth of tiles, 32 of its channels each.
+//
+// What it takes away is a launch in a chain of dependent ones, and a kernel that is a load, a reduction and a store long with 16
+// workgroups.  us per forward, two kernels / one, batches of L = 128: 12 x 768 B = 1 551 / 508, 2 617 / 583, 12 x 960 B = 1 605 / 549,
+// 24 x 1536 B = 1 1757 / 1724, 2 2018 / 1980, 12 x 1792 B = 1 1098 / 1055, 2 1243 / 1225 (6 to 10 us of the first three are the filters').
+// ---------------------------------------------------------------------------------------------
+template <int PER, int JT>
+struct LnGemmShape {
+  static constexpr int d = 64 * PER, KS = (d / 32 + 7) / 8, PITCH = d + 8;      // bf16 per row in LDS: 16-byte accesses of 16 rows spread over the banks
+  static constexpr int kRows = 32 * PITCH * 2, kRed = 8 * 16 * JT * kRedRow * 4;
+  static constexpr int kLds = (kRows > kRed ? kRows : kRed) + 32 * 8;
+};
+template <int PER, int JT>
+__global__ __launch_bounds__(512) void ln_gemm_kernel(const uint16_t* __restrict__ s, const float* __restrict__ gamma, const float* __restrict__ beta,
+                                                      float eps, const uint16_t* __restrict__ w, uint16_t* __restrict__ out, long ldo,
+                                                      float* __restrict__ out_t /* (d, M) or null */, int M, int N, int ti, int tj) {
+  using S = LnGemmShape<PER, JT>;
+  constexpr int d = S::d, KS = S::KS, PITCH = S::PITCH, NKS = d / 32;
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  uint16_t* rows = reinterpret_cast<uint16_t*>(smem);
+  float2* stats = reinterpret_cast<float2*>(smem + (S::kLds - 32 * 8));      // sum, 1 / deviation
+  const int tid = threadIdx.x, lane = tid & 63, i16 = lane & 15, q4 = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  // the tiles of an XCD keep the weights' rows together: they are read by one L2 only
+  const int ntiles = ti * tj, xcd = blockIdx.x & 7;
+  const int tile = (int)((long)xcd * ntiles / 8) + (int)(blockIdx.x >> 3);
+  if (tile >= (int)((long)(xcd + 1) * ntiles / 8)) return;
+  const int jt = __builtin_amdgcn_readfirstlane(tile / ti), i0 = 32 * (tile - jt * ti), j0 = 16 * JT * jt;
+  const int s0 = wave * NKS / 8, ns = (wave + 1) * NKS / 8 - s0;
+  const u32x4 zero = {0u, 0u, 0u, 0u};
+  // value - mean with one rounding (what the compiler makes of layernorm_kernel's two steps)
+  auto centred = [](float v, float sum) __attribute__((always_inline)) { return fmaf(-sum, 1.0f / (float)d, v); };
+
+  // everything that is read is requested here: rows, weights, the scales of this wave's columns
+  constexpr int kPieces = 32 * d / 8, kLoads = (kPieces + 511) / 512;
+  u32x4 raw[kLoads];
+  static_for<0, kLoads>([&](auto ll) {
+    constexpr int l = decltype(ll)::value;
+    const int p = tid + 512 * l, r = p / (d / 8), c = p % (d / 8);
+    int m = i0 + r;
+    m = m < M ? m : M - 1;
+    if (512 * (l + 1) <= kPieces || p < kPieces) raw[l] = *reinterpret_cast<const u32x4*>(s + (long)m * d + 8 * c);
+  });
+  u32x4 qf[JT][KS];
+  static_for<0, JT>([&](auto jj) {
+    int j = j0 + 16 * decltype(jj)::value + i16;
+    j = j < N ? j : N - 1;
+    static_for<0, KS>([&](auto ss) {
+      constexpr int k = decltype(ss)::value;
+      qf[decltype(jj)::value][k] = zero;
+      if (k < ns) qf[decltype(jj)::value][k] = *reinterpret_cast<const u32x4*>(w + (long)j * d + 32 * (s0 + k) + 8 * q4);
+    });
+  });
+  float g[KS][8], b[KS][8];
+  static_for<0, KS>([&](auto ss) {
+    constexpr int k = decltype(ss)::value;
+    const int at = k < ns ? 32 * (s0 + k) + 8 * q4 : 0;
+    static_for<0, 2>([&](auto hh) {
+      constexpr int h = decltype(hh)::value;
+      const floatx4 gv = *reinterpret_cast<const floatx4*>(gamma + at + 4 * h), bv = *reinterpret_cast<const floatx4*>(beta + at + 4 * h);
+      static_for<0, 4>([&](auto e) {
+        g[k][4 * h + decltype(e)::value] = gv[decltype(e)::value];
+        b[k][4 * h + decltype(e)::value] = bv[decltype(e)::value];
+      });
+    });
+  });
+  static_for<0, kLoads>([&](auto ll) {
+    constexpr int l = decltype(ll)::value;
+    const int p = tid + 512 * l, r = p / (d / 8), c = p % (d / 8);
+    if (512 * (l + 1) <= kPieces || p < kPieces) *reinterpret_cast<u32x4*>(rows + r * PITCH + 8 * c) = raw[l];
+  });
+  __syncthreads();
+
+  // ---- statistics of the wave's four rows, as in layernorm_kernel
+  {
+    float v[4][PER], sum[4], sq[4];
+    static_for<0, 4>([&](auto rr) {
+      constexpr int r = decltype(rr)::value;
+      static_for<0, PER>([&](auto ii) { v[r][decltype(ii)::value] = bf16_to_f32(rows[(4 * wave + r) * PITCH + lane + 64 * decltype(ii)::value]); });
+      float t = 0.f;
+      static_for<0, PER>([&](auto ii) { t += v[r][decltype(ii)::value]; });
+      sum[r] = t;
+    });
+    for (int o = 32; o > 0; o >>= 1) static_for<0, 4>([&](auto rr) { sum[decltype(rr)::value] += __shfl_xor(sum[decltype(rr)::value], o); });
+    static_for<0, 4>([&](auto rr) {
+      constexpr int r = decltype(rr)::value;
+      float t = 0.f;
+      static_for<0, PER>([&](auto ii) {
+        const float c = centred(v[r][decltype(ii)::value], sum[r]);
+        t += c * c;
+      });
+      sq[r] = t;
+    });
+    for (int o = 32; o > 0; o >>= 1) static_for<0, 4>([&](auto rr) { sq[decltype(rr)::value] += __shfl_xor(sq[decltype(rr)::value], o); });
+    static_for<0, 4>([&](auto rr) {
+      constexpr int r = decltype(rr)::value;
+      if (lane == r) stats[4 * wave + r] = make_float2(sum[r], rsqrtf(fmaf(sq[r], 1.0f / (float)d, eps)));
+    });
+  }
+  __syncthreads();
+
+  // ---- the wave's operands: row 8 (i16 / 4) + 4 t + i16 % 4 of the tile, K = 32 (s0 + k) + 8 q4 .. + 7
+  u32x4 pf[2][KS];
+  static_for<0, 2>([&](auto tt) {
+    constexpr int t = decltype(tt)::value;
+    const int r = 8 * (i16 >> 2) + 4 * t + (i16 & 3);
+    const float2 st = stats[r];
+    static_for<0, KS>([&](auto ss) {
+      constexpr int k = decltype(ss)::value;
+      const u32x4 x = *reinterpret_cast<const u32x4*>(rows + r * PITCH + (k < ns ? 32 * (s0 + k) + 8 * q4 : 0));
+      static_for<0, 4>([&](auto e) {
+        constexpr int i = decltype(e)::value;
+        const float lo = fmaf(centred(__uint_as_float(x[i] << 16), st.x) * st.y, g[k][2 * i], b[k][2 * i]);
+        const float hi = fmaf(centred(__uint_as_float(x[i] & 0xffff0000u), st.x) * st.y, g[k][2 * i + 1], b[k][2 * i + 1]);
+        pf[t][k][i] = k < ns ? pack_bf16x2(lo, hi) : 0u;
+      });
+    });
+  });
+  floatx4 acc[2][JT];
+  static_for<0, 2>([&](auto tt) {
+    constexpr int t = decltype(tt)::value;
+    static_for<0, JT>([&](auto jj) {
+      constexpr int u = decltype(jj)::value;
+      floatx4 a = {0.f, 0.f, 0.f, 0.f};
+      static_for<0, KS>([&](auto ss) {
+        constexpr int k = decltype(ss)::value;
+        a = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, pf[t][k]), __builtin_bit_cast(bf16x8, qf[u][k]), a, 0, 0, 0);
+      });
+      acc[t][u] = a;
+    });
+  });
+  if (out_t && jt < d / 32) {
+    const int c = 32 * jt + (tid >> 4), r = 2 * (tid & 15);
+    if (i0 + r < M) {      // (M is even)
+      const float gc = gamma[c], bc = beta[c];
+      const float2 sa = stats[r], sb = stats[r + 1];
+      const float va = fmaf(centred(bf16_to_f32(rows[r * PITCH + c]), sa.x) * sa.y, gc, bc),
+                  vb = fmaf(centred(bf16_to_f32(rows[(r + 1) * PITCH + c]), sb.x) * sb.y, gc, bc);
+      *reinterpret_cast<float2*>(out_t + (long)c * M + i0 + r) = make_float2(va, vb);
+    }
+  }
+  __syncthreads();      // the partial sums take the rows' place
+  float* red = reinterpret_cast<float*>(smem);
+  static_for<0, 2>([&](auto tt) {
+    constexpr int t = decltype(tt)::value;
+    static_for<0, JT>([&](auto jj) {
+      constexpr int u = decltype(jj)::value;
+      *reinterpret_cast<floatx4*>(red + (wave * 16 * JT + 16 * u + i16) * kRedRow + 8 * q4 + 4 * t) = acc[t][u];
+    });
+  });
+  __syncthreads();
+  const int j = tid >> 3, i4 = 4 * (tid & 7);
+  if (j >= 16 * JT || j0 + j >= N || i0 + i4 >= M) return;
+  floatx4 v = {0.f, 0.f, 0.f, 0.f};
+  static_for<0, 8>([&](auto ww) { v += *reinterpret_cast<const floatx4*>(red + (decltype(ww)::value * 16 * JT + j) * kRedRow + i4); });
+  u32x2 pk = {pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
+  *reinterpret_cast<u32x2*>(out + (long)(j0 + j) * ldo + i0 + i4) = pk;
+}
+
+template <int PER, int JT>
+static int launch_ln_gemm(const void* s, const float* gamma, const float* beta, float eps, const void* w, void* out, long ldo, float* out_t,
+                          int M, int N, hipStream_t st) {
+  using S = LnGemmShape<PER, JT>;
+  auto kern = ln_gemm_kernel<PER, JT>;
+  if (S::kLds > 64 * 1024) {
+    hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, S::kLds);
+    if (e != hipSuccess) return set_error(M2_ERR_LAUNCH, "hipFuncSetAttribute(ln_gemm): %s", hipGetErrorString(e));
+  }
+  const int ti = (M + 31) / 32, tj = (N + 16 * JT - 1) / (16 * JT), nt = ti * tj;
+  hipLaunchKernelGGL(kern, dim3(8 * ((nt + 7) / 8)), dim3(512), S::kLds, st, (const uint16_t*)s, gamma, beta, eps, (const uint16_t*)w,
+                     (uint16_t*)out, ldo, out_t, M, N, ti, tj);
+  return check_launch("ln_gemm");
+}
+
 template <int BI, int BJ, int WI, int WJ, int STAGES, bool QKM, int OCC>
 static int launch_engine(GemmArgs g, hipStream_t st) {
   using S = GemmShape<BI, BJ, WI, WJ, STAGES, QKM>;
@@ -330,4 +510,36 @@ extern "C" int m2_dense_from_channels_fwd(const void* x, const void* w, const fl
   if (rc) return rc;
   GemmArgs g{(const uint16_t*)w, (const uint16_t*)x, (uint16_t*)out, bias, nullptr, K, M, N, N, M, K, 1, 0, 0, 0, 0};
   return dense_launch<true>(pick_variant(g, true), g, (hipStream_t)stream);
+}
+
+// LayerNorm and in_linear as one kernel where in_linear alone would be the kernel of few rows: every tile normalises its rows again, which
+// hides behind the launch it saves only there (up to 256 or 384 rows; figures above).
+extern "C" int m2_layernorm_to_channels_supported(int M, int N, int K) {
+  if (!m2_dense_supported(M, N, K) || N != 3 * K || (K != 768 && K != 960 && K != 1536 && K != 1792) || dense_ws_serves(M, N, K)) return 0;
+  const GemmArgs g{nullptr, nullptr, nullptr, nullptr, nullptr, K, K, M, M, N, K, 1, 0, 0, 0, 1};
+  return pick_variant(g, false) == kVarSmall ? 1 : 0;
+}
+
+extern "C" int m2_layernorm_to_channels_fwd(const void* s, const float* gamma, const float* beta, float eps, const void* w, void* out, long out_row,
+                                            float* out_channel_major, int M, int N, int K, void* stream) {
+  const char* who = "m2_layernorm_to_channels_fwd";
+  if (!gamma || !beta) return set_error(M2_ERR_ARG, "%s: null pointer", who);
+  const int rc = check_dense(who, s, w, out, M, N, K);
+  if (rc) return rc;
+  if (out_row < M || out_row % 8) return set_error(M2_ERR_ARG, "%s: rows of the output %ld apart, need a multiple of 8 from M = %d on", who, out_row, M);
+  if (N != 3 * K) return set_error(M2_ERR_UNSUPPORTED, "%s: N=%d must be 3 K=%d", who, N, 3 * K);
+  if (!aligned16(gamma, beta, out_channel_major)) return set_error(M2_ERR_UNSUPPORTED, "%s: operands must be 16-byte aligned", who);
+  // 16 JT output channels: the fullest compute unit has the fewest operand rows to fetch
+  const long ti = (M + 31) / 32, cus = num_cus();
+  auto fetched = [&](long jt) { return (ti * ((N + 16 * jt - 1) / (16 * jt)) + cus - 1) / cus * (32 + 16 * jt); };
+  const bool three = fetched(3) < fetched(2);
+  hipStream_t st = (hipStream_t)stream;
+  switch (K) {
+#define X(PER)                                                                                                                          \
+  case 64 * PER: return three ? launch_ln_gemm<PER, 3>(s, gamma, beta, eps, w, out, out_row, out_channel_major, M, N, st)               \
+                              : launch_ln_gemm<PER, 2>(s, gamma, beta, eps, w, out, out_row, out_channel_major, M, N, st);
+    X(12) X(15) X(24) X(28)
+#undef X
+  }
+  return set_error(M2_ERR_UNSUPPORTED, "%s: K=%d, built for 768, 960, 1536 and 1792", who, K);
 }

@@ -57,10 +57,14 @@ static int encoder_layers(const char* who, const m2_layer_params* layers, int nl
   unsigned char* ws = (unsigned char*)workspace;
   void *xproj = ws + l.xproj, *y = ws + l.y, *a = ws + l.a, *g = ws + l.g, *s = ws + l.s, *nh = ws + l.h16;
   float* nt = (float*)(ws + l.hT);
+  // a layer's LayerNorm and the next one's in_linear as one kernel, where nobody else reads the normalised rows
+  const bool joined = m2_layernorm_to_channels_supported(M, 3 * d, d);
+  const m2_layer_params* norm = nullptr;      // of the layer whose sum is still to be normalised
   const size_t stride = fpm ? (size_t)fpm * d * 2 * L : m2_filter_spectrum_bytes(d, L) / sizeof(float);
   for (int i = 0; i < nlayers; ++i) {
     const m2_layer_params& p = layers[i];
-    int rc = m2_dense_to_channels_rows_fwd(h16, p.in_w, xproj, l.xrow, M, 3 * d, d, stream);
+    int rc = norm ? m2_layernorm_to_channels_fwd(s, norm->ln_gamma, norm->ln_beta, eps, p.in_w, xproj, l.xrow, nt, M, 3 * d, d, stream)
+                  : m2_dense_to_channels_rows_fwd(h16, p.in_w, xproj, l.xrow, M, 3 * d, d, stream);
     if (rc) return rc;
     const float* u = p.residual ? h_channel_major : nullptr;
     rc = fpm ? m2_mixer_core_taps_fwd(xproj, l.xrow, p.in_b, u, p.short_w, p.short_b, filters + i * stride, skip ? skip + i * fpm : nullptr, fpm, y,
@@ -79,10 +83,12 @@ static int encoder_layers(const char* who, const m2_layer_params* layers, int nl
     }
     if (rc) return rc;
     const bool last = i == nlayers - 1;
+    h_channel_major = nt;
+    norm = joined && !last && !out_f32[i] && aligned16(p.ln_gamma, p.ln_beta) ? &p : nullptr;
+    if (norm) continue;
     rc = m2_layernorm_bf16_fwd(s, p.ln_gamma, p.ln_beta, eps, out_f32[i], last ? nullptr : nh, last ? nullptr : nt, M, d, stream);
     if (rc) return rc;
     h16 = nh;
-    h_channel_major = nt;
   }
   return M2_OK;
 }
