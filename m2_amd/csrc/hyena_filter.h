@@ -47,6 +47,8 @@ struct TabByPointer {
 typedef float floatx16 __attribute__((ext_vector_type(16)));
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 typedef const __attribute__((address_space(1))) floatx4 gfloatx4;
+typedef floatx4 floatx4_any __attribute__((aligned(4)));      // at any address of a float
+typedef const __attribute__((address_space(1))) floatx4_any gfloatx4_any;
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 // The matrix products of the filter MLPs, fp32 accumulation.

@@ -7,7 +7,7 @@
 // filter_rev, :231-236 placement of the forward and the flipped reverse taps in a 2L window.)
 //
 // Three kernels.  `split_weights_kernel` re-splits the weights into parts in MFMA operand layout (hyena_filter.h; a few
-// microseconds, once per call).  `hidden_kernel` evaluates the three sin layers for 32 or 64 positions per workgroup: the first
+// microseconds, once per call) where the next kernel has many workgroups to read them.  `hidden_kernel` evaluates the three sin layers for 32 or 64 positions per workgroup: the first
 // (emb -> 128) on the vector ALU, the two 128 x 128 layers as six-product split-bf16 MFMA GEMMs (v_mfma_f32_32x32x16_bf16 on the
 // three parts of weights and activations: fp32 products, which matters because sin(freq * x) amplifies any rounding of
 // x) with the activations resident in LDS; it writes h3 in two fp16 parts.  `project_kernel` is the 128 -> d projection, three
@@ -175,14 +175,44 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 
   // Weights of an inner layer -> registers.  Requested one phase early (layer 1's before the vector-ALU layer, layer
   // 2's before the last epilogue of layer 1), so that the 24 KB per wave arrive behind other work.
+  // PROJECT: from the split copy.  Otherwise a workgroup splits its own rows, 64 values a lane and layer (about 2 us of vector
+  // instructions in all, where a launch ahead of this one took 3 to 7): it has one tile, and few of them share a compute unit.
   bf16x8 ah[8], am[8], al[8];
+  floatx4 raw[PROJECT ? 1 : 16];
+  gfloat *const w1 = in_global(W.w1), *const w2 = in_global(W.w2);
   auto load_weights = [&](int layer) __attribute__((always_inline)) {
-    const u32x4* wp = reinterpret_cast<const u32x4*>(wsplit + ((long)(blockIdx.y * 2 + layer)) * kSplitPerLayer) + w * 8 * 64;
+    if constexpr (PROJECT) {
+      const u32x4* wp = reinterpret_cast<const u32x4*>(wsplit + ((long)(blockIdx.y * 2 + layer)) * kSplitPerLayer) + w * 8 * 64;
 #pragma unroll
-    for (int ks = 0; ks < 8; ++ks) {
-      ah[ks] = __builtin_bit_cast(bf16x8, (wp + ks * 64)[(unsigned)lane]);
-      am[ks] = __builtin_bit_cast(bf16x8, (wp + ks * 64 + kOrder * kOrder / 8)[(unsigned)lane]);
-      al[ks] = __builtin_bit_cast(bf16x8, (wp + ks * 64 + 2 * kOrder * kOrder / 8)[(unsigned)lane]);
+      for (int ks = 0; ks < 8; ++ks) {
+        ah[ks] = __builtin_bit_cast(bf16x8, (wp + ks * 64)[(unsigned)lane]);
+        am[ks] = __builtin_bit_cast(bf16x8, (wp + ks * 64 + kOrder * kOrder / 8)[(unsigned)lane]);
+        al[ks] = __builtin_bit_cast(bf16x8, (wp + ks * 64 + 2 * kOrder * kOrder / 8)[(unsigned)lane]);
+      }
+    } else {
+      gfloat* row = (layer == 0 ? w1 : w2) + (32 * w + i32) * kOrder + 8 * half;
+#pragma unroll
+      for (int i = 0; i < 16; ++i) raw[i] = *(gfloatx4_any*)(row + 16 * (i >> 1) + 4 * (i & 1));
+    }
+  };
+  auto split_weights = [&]() __attribute__((always_inline)) {
+    if constexpr (!PROJECT) {
+#pragma unroll
+      for (int ks = 0; ks < 8; ++ks) {
+        u32x4 vh, vm, vl;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          float h[2], md[2], l[2];
+#pragma unroll
+          for (int e = 0; e < 2; ++e) split3(raw[2 * ks + j / 2][2 * (j & 1) + e], h[e], md[e], l[e]);
+          vh[j] = pack_bf16x2(h[0], h[1]);
+          vm[j] = pack_bf16x2(md[0], md[1]);
+          vl[j] = pack_bf16x2(l[0], l[1]);
+        }
+        ah[ks] = __builtin_bit_cast(bf16x8, vh);
+        am[ks] = __builtin_bit_cast(bf16x8, vm);
+        al[ks] = __builtin_bit_cast(bf16x8, vl);
+      }
     }
   };
   load_weights(0);
@@ -294,9 +324,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     __syncthreads();
   };
   load_scales(0);
+  split_weights();
   __syncthreads();                     // layer 0's activations are complete
   layer_pass(ic<0>{});
   load_scales(1);
+  split_weights();
   layer_pass(ic<1>{});
 
   if constexpr (PROJECT) {
@@ -544,11 +576,12 @@ template <class TAB>
 static int filter_launches(TAB tab, int nfilters, int L, int d, int emb_dim, float w_mod, float shift, uint16_t* h_hi,
                            uint16_t* h_lo, uint16_t* wsplit, uint16_t* w3split, float* w3scale, float* taps, hipStream_t s) {
   const bool one_kernel = taps && project_with_hidden(L, d);
-  const int split_blocks = 2 * nfilters * 2 * 4 + (one_kernel ? 2 * nfilters * (d / 32) : 0);
-  hipLaunchKernelGGL(split_weights_kernel<TAB>, dim3(split_blocks), dim3(512), 0, s, tab, 2 * nfilters, d, wsplit, w3split,
-                     w3scale);
-  int rc = check_launch("hyena split_weights_kernel");
-  if (rc) return rc;
+  if (one_kernel) {
+    hipLaunchKernelGGL(split_weights_kernel<TAB>, dim3(2 * nfilters * 2 * 4 + 2 * nfilters * (d / 32)), dim3(512), 0, s, tab, 2 * nfilters, d,
+                       wsplit, w3split, w3scale);
+    const int rc = check_launch("hyena split_weights_kernel");
+    if (rc) return rc;
+  }
   // Positions per workgroup: longer runs amortise the weight fetch (96 KB per workgroup and layer, 520 bytes per channel for the
   // projection), short sequences need the workgroups spread over the chip.  128 positions would leave one workgroup on a compute unit
   // (104 KB of activations) and half of them idle for a single mixer.  us for the spectra of 1 / 12 mixers, d = 768: L = 1024 44 / 159,
@@ -560,7 +593,7 @@ static int filter_launches(TAB tab, int nfilters, int L, int d, int emb_dim, flo
   }
   hipLaunchKernelGGL((hidden_kernel<1, TAB, false>), dim3(L / 32, 2 * nfilters), dim3(256), 0, s, tab, L, emb_dim, w_mod, wsplit,
                      h_hi, h_lo, 0, 0.f, nullptr, nullptr, nullptr);
-  rc = check_launch("hyena hidden_kernel");
+  const int rc = check_launch("hyena hidden_kernel");
   if (rc || !taps) return rc;
   hipLaunchKernelGGL(project_kernel<TAB>, dim3((L + kPosPerWg - 1) / kPosPerWg, (d + 127) / 128, 2 * nfilters), dim3(256), 0, s, tab, L, d, shift,
                      h_hi, h_lo, taps);
