@@ -10,7 +10,8 @@
 // us, d = 768, bf16, core and its spectra (of one mixer / a twelfth of twelve mixers' at once) against the core on taps: L = 1024, B = 1
 // 10.4 + 8.4 / 6 against 13.5, 2048 15.6 + 11.0 / 9 against 22.1, 4096 25.2 + 20.1 / 17.4 against 37.1, 8192 46.4 + 37.9 / 36.5 against 73.9,
 // 16384 104.8 + 90.5 against 154.8; B = 2 12.5, 23.4, 41.7, 81.7, 195.4 against 16.6, 32.3, 57.6, 112.2, 289.0 (up to 5 % of both, or a loss),
-// B = 3 19.0, 32.3, 56.5, 136.9, 288.6 against 25.5, 46.2, 79.7, 173.7, 421.1.  So: one row to a channel.  Whole forwards of 12 x 768, B = 1:
+// B = 3 19.0, 32.3, 56.5, 136.9, 288.6 against 25.5, 46.2, 79.7, 173.7, 421.1.  So: one row to a channel, and two where whole forwards
+// gain by it too: 12 x 768, B = 2, L = 1024 1090 / 1102, 2048 1531 / 1550, 4096 2295 / 2264, 8192 4837 / 4704.  Whole forwards of 12 x 768, B = 1:
 // L = 1024 1011 / 971, 2048 1230 / 1208, 4096 1793 / 1723, 8192 2814 / 2680, 16384 6030 / 5720; 24 x 1536, 2048 4786 / 4541.
 // fp32 rows, whose inputs take twice the registers, spill beside a spectrum (52 bytes a lane and more) and read spectra; at L = 32768 a
 // half transform's inputs would have to be formed twice from all the taps.
@@ -37,7 +38,7 @@ static int launch_mixer_taps(const void* xproj, long ldx, const float* u, const 
 using namespace m2;
 
 extern "C" int m2_mixer_core_taps_pays(int B, int L) {
-  return B == 1 && L >= 1024 && L <= 16384 && m2_fftconv_supported_seqlen(L);
+  return m2_fftconv_supported_seqlen(L) && L >= 1024 && ((B == 1 && L <= 16384) || (B == 2 && L >= 4096 && L <= 8192));
 }
 
 extern "C" int m2_mixer_core_taps_fwd(const void* xproj, long xproj_row, const float* proj_bias, const float* u, const float* short_w,

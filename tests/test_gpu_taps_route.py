@@ -1,4 +1,4 @@
-"""Forwards of one sequence, whose mixer cores read filter taps, against the same ones on spectra."""
+"""Forwards of one or two sequences, whose mixer cores read filter taps, against the same ones on spectra."""
 import pytest
 import torch
 
@@ -21,16 +21,16 @@ def _close(a, b):
     return (a.double() - b.double()).norm() <= 2.0 ** -8 * b.double().norm()
 
 
-@pytest.mark.parametrize("helper,L,residual", [("m2_bert_80m", 1024, True), ("m2_bert_80m", 2048, False), ("m2_bert_80m", 16384, True),
-                                               ("m2_bert_110m", 4096, True), ("m2_bert_large", 2048, True)])
-def test_one_sequence(gpu, helper, L, residual):
+@pytest.mark.parametrize("helper,L,residual,B", [("m2_bert_80m", 1024, True, 1), ("m2_bert_80m", 2048, False, 1), ("m2_bert_80m", 16384, True, 1),
+                                                 ("m2_bert_110m", 4096, True, 1), ("m2_bert_large", 2048, True, 1), ("m2_bert_80m", 8192, True, 2)])
+def test_few_sequences(gpu, helper, L, residual, B):
     import m2_amd
     cfg = getattr(m2_amd, helper)(L)
     cfg.num_hidden_layers, cfg.residual_long_conv = 2, residual
     model = m2_amd.BertModel(cfg)
     model.load_state_dict(m2_amd.seeded_state_dict(cfg, 3))
     model = model.to(gpu).eval()
-    ids = torch.randint(0, cfg.vocab_size, (1, L), generator=torch.Generator().manual_seed(4)).to(gpu)
+    ids = torch.randint(0, cfg.vocab_size, (B, L), generator=torch.Generator().manual_seed(4)).to(gpu)
     with torch.no_grad():
         (want, pooled), taps = _spectra_only(lambda: model(ids))
         assert taps
@@ -42,7 +42,7 @@ def test_one_sequence(gpu, helper, L, residual):
             assert torch.equal(model(ids)[0], got)
         model.encoder.overlap_filters = None
         layer = model.encoder.layer[0]
-        u = torch.randn(1, L, cfg.hidden_size, generator=torch.Generator().manual_seed(5)).to(gpu).bfloat16()
+        u = torch.randn(B, L, cfg.hidden_size, generator=torch.Generator().manual_seed(5)).to(gpu).bfloat16()
         want, taps = _spectra_only(lambda: layer.attention(u)[0])
         assert taps == 1 and _close(layer.attention(u)[0], want)
 
