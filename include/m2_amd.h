@@ -278,6 +278,10 @@ int m2_layernorm_bf16_fwd(const void* x, const float* gamma, const float* beta, 
  * (hidden states given to a stack of layers).  Needs d % 64 == 0. */
 int m2_input_forms_fwd(const float* x, void* out_bf16, float* out_channel_major, int M, int d, void* stream);
 
+/* The pooler: out (B, d) = tanh(h w^T + bias), fp32; h: B rows of d values h_row elements apart (the first token of each sequence), w (d, d),
+ * bias (d) or NULL.  d a multiple of 8, h_row of 4; h and w 16-byte aligned.  (bert/src/bert_layers.py:816-859) */
+int m2_pooler_fwd(const float* h, long h_row, const float* w, const float* bias, float* out, int B, int d, void* stream);
+
 /* out = LayerNorm(blockdiag_multiply(x, w) + bias + residual) in one kernel: m2_blockdiag_linear_fwd followed by
  * m2_layernorm_fwd without the fp32 intermediate (bert/src/bert_layers.py:504-506: wo, dropout, residual,
  * layernorm).  Arguments as in those two; any of the three outputs may be NULL.

@@ -123,6 +123,8 @@ def _load() -> ctypes.CDLL:
     lib.m2_layernorm_fwd.restype = c_int
     lib.m2_layernorm_fwd.argtypes = [c_void_p, c_void_p, c_void_p, c_float, c_void_p, c_void_p, c_void_p, c_int, c_int,
                                      c_void_p]
+    lib.m2_pooler_fwd.restype = c_int
+    lib.m2_pooler_fwd.argtypes = [c_void_p, c_long] + [c_void_p] * 3 + [c_int, c_int, c_void_p]
     lib.m2_input_forms_fwd.restype = c_int
     lib.m2_input_forms_fwd.argtypes = [c_void_p] * 3 + [c_int] * 2 + [c_void_p]
     lib.m2_blockdiag_linear_layernorm_supported.restype = c_int
@@ -159,7 +161,7 @@ lib = _load()
 
 EXPORTS = ["m2_version", "m2_last_error", "m2_hyena_filter_workspace_bytes", "m2_hyena_filter_fwd", "m2_hyena_filter_fwd_static", "m2_mixer_filters_workspace_bytes", "m2_mixer_filters_fwd", "m2_mixer_taps_workspace_bytes", "m2_mixer_taps_fwd",
            "m2_fftconv_supported_seqlen", "m2_filter_spectrum_bytes", "m2_filter_spectrum_fwd", "m2_mixer_core_fwd", "m2_mixer_core_rows_fwd", "m2_mixer_core_taps_pays", "m2_mixer_core_taps_fwd",
-           "m2_fftconv_fwd", "m2_dense_supported", "m2_dense_to_channels_fwd", "m2_dense_to_channels_rows_fwd", "m2_dense_channels_row", "m2_dense_from_channels_fwd", "m2_layernorm_to_channels_supported", "m2_layernorm_to_channels_fwd", "m2_blockdiag_glu_fwd", "m2_blockdiag_glu_few_rows", "m2_blockdiag_linear_fwd", "m2_blockdiag_linear_f32_fwd", "m2_mlp_fused_supported", "m2_mlp_fused_packed_bytes", "m2_mlp_fused_pack", "m2_mlp_fused_fwd", "m2_glu_stream_supported", "m2_glu_stream_packed_bytes", "m2_glu_stream_pack", "m2_glu_stream_fwd", "m2_layernorm_fwd", "m2_layernorm_bf16_fwd", "m2_input_forms_fwd",
+           "m2_fftconv_fwd", "m2_dense_supported", "m2_dense_to_channels_fwd", "m2_dense_to_channels_rows_fwd", "m2_dense_channels_row", "m2_dense_from_channels_fwd", "m2_layernorm_to_channels_supported", "m2_layernorm_to_channels_fwd", "m2_blockdiag_glu_fwd", "m2_blockdiag_glu_few_rows", "m2_blockdiag_linear_fwd", "m2_blockdiag_linear_f32_fwd", "m2_mlp_fused_supported", "m2_mlp_fused_packed_bytes", "m2_mlp_fused_pack", "m2_mlp_fused_fwd", "m2_glu_stream_supported", "m2_glu_stream_packed_bytes", "m2_glu_stream_pack", "m2_glu_stream_fwd", "m2_layernorm_fwd", "m2_layernorm_bf16_fwd", "m2_input_forms_fwd", "m2_pooler_fwd",
            "m2_embed_layernorm_fwd", "m2_blockdiag_linear_layernorm_supported", "m2_blockdiag_linear_layernorm_fwd", "m2_encoder_layers_workspace_bytes", "m2_encoder_layers_fwd", "m2_encoder_layers_taps_fwd",
            "m2_split_bytes", "m2_split_rows_fwd", "m2_split_jobs_fwd", "m2_split_channels_fwd", "m2_split_to_channels_fwd", "m2_split_linear_fwd", "m2_split_glu_fwd"]
 

@@ -599,6 +599,9 @@ class BertPooler(nn.Module):
         return self.activation(self.dense(mean))
 
 
+_OWN_POOLER = BertPooler.forward
+
+
 class BertModel(nn.Module):
     """Embeddings + encoder + pooler; returns (sequence output or list of layer outputs, pooled output or None)
     like the reference (bert/src/bert_layers.py:880-1010)."""
@@ -643,6 +646,21 @@ class BertModel(nn.Module):
             return None
         plan, route = found
         return plan.run(route, B, all_layers, None, None, part, ids.contiguous(), tt, pos)
+
+    def _pool(self, hidden: torch.Tensor, mask: torch.Tensor) -> torch.Tensor:
+        """The pooler's output: by one kernel where it is the plain module, in fp32 and nobody asks for gradients, for batches up to
+        256 (beyond, the library's product shares its weights among more rows)."""
+        p = self.pooler
+        if (type(p) is BertPooler and type(p).forward is _OWN_POOLER and "forward" not in p.__dict__ and not p.pool_all
+                and hidden.shape[0] <= 256 and hidden.dtype == torch.float32 and not torch.is_autocast_enabled()
+                and type(p.dense) is nn.Linear and type(p.activation) is nn.Tanh
+                and not any(m._forward_hooks or m._forward_pre_hooks or "forward" in m.__dict__ for m in (p, p.dense, p.activation))):
+            w, b, d = p.dense.weight, p.dense.bias, hidden.shape[2]
+            plain = all(t.dtype == torch.float32 and t.is_contiguous() and t.device == hidden.device and not (t.requires_grad and torch.is_grad_enabled())
+                        for t in (w, b) if t is not None)
+            if plain and w.shape == (d, d) and (b is None or b.shape == (d,)) and d % 8 == 0 and (hidden.data_ptr() | w.data_ptr()) % 16 == 0:
+                return ops.pooler(hidden.detach()[:, 0], w.detach(), None if b is None else b.detach())
+        return p(hidden, mask=mask)
 
     def get_input_embeddings(self):
         return self.embeddings.word_embeddings
@@ -702,7 +720,7 @@ class BertModel(nn.Module):
             if self.pooler is not None:
                 if attention_mask is None:
                     attention_mask = torch.ones_like(input_ids)
-                pooled = self.pooler(enc[-1], mask=attention_mask)
+                pooled = self._pool(enc[-1], attention_mask)
         finally:
             # last, behind everything that is to be enqueued: it waits for the stream.  Also when the pooler raises: a bad id is
             # this forward's error and not the next one's

@@ -638,6 +638,19 @@ def layernorm(x: Tensor, gamma: Tensor, beta: Tensor, eps: float, want_f32: bool
     return o32, o16, ot
 
 
+def pooler(h: Tensor, w: Tensor, bias: Optional[Tensor]) -> Tensor:
+    """tanh(h @ w^T + bias): h (B, d) fp32, rows contiguous and any distance apart, w (d, d)."""
+    B, d = h.shape
+    if not h.is_cuda or h.dtype != torch.float32 or h.stride(1) != 1:
+        raise ValueError("h: fp32 rows on the GPU")
+    _require(w, "w", torch.float32, (d, d))
+    if bias is not None:
+        _require(bias, "bias", torch.float32, (d,))
+    out = torch.empty(B, d, dtype=torch.float32, device=h.device)
+    check(lib.m2_pooler_fwd(_ptr(h), h.stride(0) if B > 1 else d, _ptr(w), _ptr(bias), _ptr(out), B, d, _stream()))
+    return out
+
+
 def input_forms(x: Tensor):
     """x (M, d) fp32, d a multiple of 64 -> (bf16 (M, d), f32 (d, M)) in one pass."""
     _require(x, "x", torch.float32)

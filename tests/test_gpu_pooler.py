@@ -1,0 +1,53 @@
+"""The pooler as one kernel against fp64 and against the module, whose place it takes where that is plain."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("d", [8, 264, 768, 960, 1536, 1792])
+@pytest.mark.parametrize("B", [1, 2, 8, 9, 31, 256])
+def test_against_fp64(gpu, B, d):
+    from m2_amd import ops
+    g = torch.Generator(device=gpu).manual_seed(B + d)
+    rn = lambda *s: torch.randn(*s, generator=g, device=gpu)      # noqa: E731
+    h, w, b = rn(B, 3, d), rn(d, d) / d ** 0.5, rn(d)
+    h[0, 0, 0] = float("nan") if B > 1 else 1.0
+    for bias in (b, None):
+        got = ops.pooler(h[:, 0], w, bias)
+        s = h[:, 0].double() @ w.double().t() + (0 if bias is None else bias.double())
+        ref, size = s.tanh(), (h[:, 0].double().abs() @ w.double().abs().t() + 1)
+        # sums of d products in fp32, in the root mean square far below d / 64 roundings of their size; tanh to two ulp
+        bad = torch.isnan(ref)
+        assert torch.equal(torch.isnan(got), bad)
+        assert ((got.double() - ref).abs()[~bad] <= ((d / 64 + 8) * 2.0 ** -24 * size)[~bad]).all()
+
+
+def test_stands_for_the_module_only_where_it_is_plain(gpu):
+    import m2_amd
+    from m2_amd import ops
+    cfg = m2_amd.m2_bert_80m(128)
+    cfg.num_hidden_layers = 1
+    model = m2_amd.BertModel(cfg)
+    model.load_state_dict(m2_amd.seeded_state_dict(cfg, 2))
+    model = model.to(gpu).eval()
+    ids = torch.randint(0, cfg.vocab_size, (3, 128), generator=torch.Generator().manual_seed(1)).to(gpu)
+    calls, own = [], ops.pooler
+    ops.pooler = lambda *a: (calls.append(1), own(*a))[1]
+    try:
+        with torch.no_grad():
+            seq, pooled = model(ids)
+            want = model.pooler(seq, mask=torch.ones_like(ids))
+            assert len(calls) == 1 and (pooled - want).abs().max() < 1e-6
+            with torch.autocast("cuda", dtype=torch.bfloat16):
+                low = model(ids)[1]
+            assert len(calls) == 1 and low.dtype == model.pooler.activation(torch.zeros(1, dtype=torch.bfloat16)).dtype
+            hook = model.pooler.dense.register_forward_hook(lambda m, i, o: o + 1)
+            assert (model(ids)[1] - (torch.atanh(want.double()) + 1).tanh()).abs().max() < 1e-4 and len(calls) == 1
+            hook.remove()
+        pooled = model(ids)[1]
+        assert pooled.requires_grad and len(calls) == 1          # the module's own graph
+        model.pooler.requires_grad_(False)
+        assert not model(ids)[1].requires_grad and len(calls) == 2
+    finally:
+        ops.pooler = own
