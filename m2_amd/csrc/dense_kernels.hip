@@ -11,17 +11,19 @@ namespace m2 {
 // ---------------------------------------------------------------------------------------------
 constexpr int kRedRow = 36;      // floats between two j of a partial tile
 
-template <int NW, int KSMAX, bool QKM, bool GLU>
+// JT: 16-wide tiles along j of a workgroup.
+template <int NW, int KSMAX, bool QKM, bool GLU, int JT>
 struct SmallShape {
   static constexpr int kProd = GLU ? 2 : 1;
-  static constexpr int kRed = NW * kProd * 32 * kRedRow * 4;
+  static constexpr int kRed = NW * kProd * 16 * JT * kRedRow * 4;
   static constexpr int kStage = QKM ? NW * KSMAX * 2048 : 0;
   static constexpr int kLds = kRed > kStage ? kRed : kStage;
 };
 
-template <int NW, int KSMAX, bool QKM, bool GLU>
+template <int NW, int KSMAX, bool QKM, bool GLU, int JT>
 __global__ __launch_bounds__(64 * NW) void small_gemm_kernel(GemmArgs g) {
-  using S = SmallShape<NW, KSMAX, QKM, GLU>;
+  using S = SmallShape<NW, KSMAX, QKM, GLU, JT>;
+  static_assert(JT == 2 || !QKM, "64-byte rows of a channel-major operand");
   static_assert(!(QKM && GLU), "the gated product reads row-major activations");
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   const int tid = threadIdx.x, lane = tid & 63, i16 = lane & 15, q4 = lane >> 4;
@@ -31,12 +33,12 @@ __global__ __launch_bounds__(64 * NW) void small_gemm_kernel(GemmArgs g) {
   const int tile = (int)((long)xcd * ntiles / 8) + (int)(blockIdx.x >> 3);
   if (tile >= (int)((long)(xcd + 1) * ntiles / 8)) return;
   int i0, j0, blk;
-  tile_origin<32, 32>(g, tile, i0, j0, blk);
+  tile_origin<32, 16 * JT>(g, tile, i0, j0, blk);
   const int nks = (g.nk + 31) / 32;
   const int s0 = wave * nks / NW, ns = (wave + 1) * nks / NW - s0;
   const u32x4 zero = {0u, 0u, 0u, 0u};
 
-  u32x4 pf[S::kProd][KSMAX][2], qf[S::kProd][KSMAX][2];
+  u32x4 pf[S::kProd][KSMAX][2], qf[S::kProd][KSMAX][JT];
   static_for<0, S::kProd>([&](auto dd) {
     constexpr int D = decltype(dd)::value;
     // GLU: gated columns of weight block blk (gate, read against the same block of Q) and of block blk + nblk (value)
@@ -52,10 +54,10 @@ __global__ __launch_bounds__(64 * NW) void small_gemm_kernel(GemmArgs g) {
       static_for<0, KSMAX>([&](auto ss) {
         constexpr int s = decltype(ss)::value;
         pf[D][s][t] = zero;
-        if constexpr (!QKM) qf[D][s][t] = zero;
+        if constexpr (!QKM && t < JT) qf[D][s][t] = zero;
         if (s < ns && 32 * (s0 + s) + 8 * q4 < g.nk) {
           pf[D][s][t] = *reinterpret_cast<const u32x4*>(pb + (long)i * g.ldp + 32 * s);
-          if constexpr (!QKM) qf[D][s][t] = *reinterpret_cast<const u32x4*>(qbase + (long)j * g.ldq + 32 * s);
+          if constexpr (!QKM && t < JT) qf[D][s][t] = *reinterpret_cast<const u32x4*>(qbase + (long)j * g.ldq + 32 * s);
         }
       });
     });
@@ -85,11 +87,11 @@ __global__ __launch_bounds__(64 * NW) void small_gemm_kernel(GemmArgs g) {
       });
     });
   }
-  floatx4 acc[S::kProd][2][2];
+  floatx4 acc[S::kProd][2][JT];
   static_for<0, S::kProd>([&](auto dd) {
     constexpr int D = decltype(dd)::value;
-    static_for<0, 4>([&](auto tt) {
-      constexpr int t = decltype(tt)::value >> 1, u = decltype(tt)::value & 1;
+    static_for<0, 2 * JT>([&](auto tt) {
+      constexpr int t = decltype(tt)::value / JT, u = decltype(tt)::value % JT;
       floatx4 a = {0.f, 0.f, 0.f, 0.f};
       static_for<0, KSMAX>([&](auto ss) {
         constexpr int s = decltype(ss)::value;
@@ -102,20 +104,20 @@ __global__ __launch_bounds__(64 * NW) void small_gemm_kernel(GemmArgs g) {
   if constexpr (QKM) __syncthreads();      // every wave has read its stage: the partial sums take its place
   static_for<0, S::kProd>([&](auto dd) {
     constexpr int D = decltype(dd)::value;
-    static_for<0, 4>([&](auto tt) {
-      constexpr int t = decltype(tt)::value >> 1, u = decltype(tt)::value & 1;
-      *reinterpret_cast<floatx4*>(red + ((wave * S::kProd + D) * 32 + 16 * u + i16) * kRedRow + 8 * q4 + 4 * t) = acc[D][t][u];
+    static_for<0, 2 * JT>([&](auto tt) {
+      constexpr int t = decltype(tt)::value / JT, u = decltype(tt)::value % JT;
+      *reinterpret_cast<floatx4*>(red + ((wave * S::kProd + D) * 16 * JT + 16 * u + i16) * kRedRow + 8 * q4 + 4 * t) = acc[D][t][u];
     });
   });
   __syncthreads();
-  if (tid >= 256) return;
+  if (tid >= 128 * JT) return;
   const int j = tid >> 3, i4 = 4 * (tid & 7);
   floatx4 sum[S::kProd];
   static_for<0, S::kProd>([&](auto dd) {
     constexpr int D = decltype(dd)::value;
     floatx4 v = {0.f, 0.f, 0.f, 0.f};
     static_for<0, NW>([&](auto ww) {
-      v += *reinterpret_cast<const floatx4*>(red + ((decltype(ww)::value * S::kProd + D) * 32 + j) * kRedRow + i4);
+      v += *reinterpret_cast<const floatx4*>(red + ((decltype(ww)::value * S::kProd + D) * 16 * JT + j) * kRedRow + i4);
     });
     sum[D] = v;
   });
@@ -138,12 +140,12 @@ __global__ __launch_bounds__(64 * NW) void small_gemm_kernel(GemmArgs g) {
   *reinterpret_cast<u32x2*>(g.out + o) = pk;
 }
 
-template <int NW, int KSMAX, bool QKM, bool GLU>
-static int launch_small(GemmArgs g, hipStream_t st) {
-  using S = SmallShape<NW, KSMAX, QKM, GLU>;
-  auto kern = small_gemm_kernel<NW, KSMAX, QKM, GLU>;
+template <int NW, int KSMAX, bool QKM, bool GLU, int JT>
+static int launch_small_j(GemmArgs g, hipStream_t st) {
+  using S = SmallShape<NW, KSMAX, QKM, GLU, JT>;
+  auto kern = small_gemm_kernel<NW, KSMAX, QKM, GLU, JT>;
   g.ti = g.nblk * ((g.ni + 31) / 32);
-  g.tj = (g.nj + 31) / 32;
+  g.tj = (g.nj + 16 * JT - 1) / (16 * JT);
   if (S::kLds > 64 * 1024) {
     hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, S::kLds);
     if (e != hipSuccess) return set_error(M2_ERR_LAUNCH, "hipFuncSetAttribute(small_gemm): %s", hipGetErrorString(e));
@@ -151,6 +153,15 @@ static int launch_small(GemmArgs g, hipStream_t st) {
   const int nt = g.ti * g.tj;
   hipLaunchKernelGGL(kern, dim3(8 * ((nt + 7) / 8)), dim3(64 * NW), S::kLds, st, g);
   return check_launch("small_gemm");
+}
+// 32 x 16 tiles where 32 x 32 ones leave half of the compute units without one: a workgroup fetches 48 operand rows instead of 64.
+// us per forward, L = 128, B = 1 (`wo`, 96 tiles of 32 x 32), before / now: 12 x 768 494 / 485, 12 x 960 532 / 520.
+template <int NW, int KSMAX, bool QKM, bool GLU>
+static int launch_small(const GemmArgs& g, hipStream_t st) {
+  if constexpr (!QKM && !GLU) {
+    if (2l * g.nblk * ((g.ni + 31) / 32) * ((g.nj + 31) / 32) <= num_cus()) return launch_small_j<NW, KSMAX, QKM, GLU, 1>(g, st);
+  }
+  return launch_small_j<NW, KSMAX, QKM, GLU, 2>(g, st);
 }
 
 // ---------------------------------------------------------------------------------------------
