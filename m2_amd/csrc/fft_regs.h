@@ -9,10 +9,12 @@ struct cf {            // complex float; kept as two scalars so that nothing is 
   float re, im;
 };
 
+// a b with its roundings said: of the two products of each sum the one with a.re goes into the sum unrounded.  Left to the compiler, which of
+// them that was depended on where b came from (memory, or the thread's own transform), and with it the last bit of the result.
 __device__ __forceinline__ cf cmul(cf a, cf b) {
-  return {a.re * b.re - a.im * b.im, a.re * b.im + a.im * b.re};
+  return {fmaf(a.re, b.re, -(a.im * b.im)), fmaf(a.re, b.im, a.im * b.re)};
 }
-__device__ __forceinline__ cf csquare(cf a) { return {a.re * a.re - a.im * a.im, (a.re + a.re) * a.im}; }
+__device__ __forceinline__ cf csquare(cf a) { return {fmaf(a.re, a.re, -(a.im * a.im)), (a.re + a.re) * a.im}; }
 
 template <int I> using ic = std::integral_constant<int, I>;
 
@@ -65,6 +67,21 @@ __device__ __forceinline__ cf mul_root(cf v) {
     if constexpr (c == 0.f) return {-s * v.im, s * v.re};
     else if constexpr (s == 0.f) return {c * v.re, c * v.im};
     else return {c * v.re - s * v.im, c * v.im + s * v.re};
+  }
+}
+
+// v exp(-2 pi i K / N), 0 <= K < N / 4, with its roundings said: of the two products of each sum the one with the smaller of cosine and sine
+// (LARGE: with the larger one; where they are equal, with v.im) goes into the sum unrounded.
+template <int K, int N, bool LARGE>
+__device__ __forceinline__ cf mul_root_rounded(cf v) {
+  static_assert(K >= 0 && 4 * K < N, "an angle of the first quadrant");
+  if constexpr (K == 0) {
+    return v;
+  } else {
+    constexpr float c = root_cos(K, N), s = root_sin(K, N);
+    if constexpr (8 * K == N) return {fmaf(s, v.im, c * v.re), fmaf(c, v.im, -(s * v.re))};
+    else if constexpr ((8 * K < N) == LARGE) return {fmaf(c, v.re, s * v.im), fmaf(c, v.im, -(s * v.re))};
+    else return {fmaf(s, v.im, c * v.re), fmaf(-s, v.re, c * v.im)};
   }
 }
 

@@ -218,7 +218,8 @@ __device__ __forceinline__ void inv_factors(cf (&x)[NREG], W&& w, OUT&& out) {
 }
 
 // All factors of a radix-R pass from two of them held in registers, those with e = 0 of the last stage and of the last but two:
-// the others are squares of these (one or two steps) and constant multiples.
+// the others are squares of these (one or two steps) and constant multiples.  Their roundings are said, and with them the last bit of what is
+// transformed: filters' spectra (LARGE, mul_root_rounded) come out the same from the kernel that stores them and in a core that makes its own.
 template <int R>
 struct Factors {
   cf fine, mid;
@@ -227,7 +228,7 @@ struct Factors {
     fine = unit_root(num, den * R);
     mid = unit_root(num, den * (R / 4));
   }
-  template <class F>
+  template <bool LARGE, class F>
   __device__ __forceinline__ void use(F&& body) const {
     constexpr int last = ilog2(R) - 1;
     cf f = fine, m = mid;
@@ -239,7 +240,7 @@ struct Factors {
     if constexpr (last > 2) t[last - 3] = csquare(m);
     if constexpr (last > 3) t[last - 4] = csquare(t[last - 3]);
     body([&](auto ss, auto ee) __attribute__((always_inline)) {
-      return mul_root<decltype(ee)::value, (2 << decltype(ss)::value)>(t[decltype(ss)::value]);
+      return mul_root_rounded<decltype(ee)::value, (2 << decltype(ss)::value), LARGE>(t[decltype(ss)::value]);
     });
   }
 };
@@ -361,10 +362,10 @@ __device__ __forceinline__ void load_group(cf (&x)[P::E], int t, const float2* r
   const float2* pg = row + P::phys(P::R3 * (t + P::T * I));
   static_for<0, P::R3>([&](auto jj) { x[I * P::R3 + decltype(jj)::value] = lds_get(pg, decltype(jj)::value); });
 }
-template <class P, int I, class TF>
+template <class P, int I, bool LARGE, class TF>
 __device__ __forceinline__ void fwd_group(cf (&x)[P::E], int t, const float2* tab, const TF& tf) {
   if constexpr (P::THREE) {
-    tf.template group<I>().use([&](auto&& w) __attribute__((always_inline)) { fwd_factors<P::R3, I * P::R3>(x, w, KeepAll{}); });
+    tf.template group<I>().template use<LARGE>([&](auto&& w) __attribute__((always_inline)) { fwd_factors<P::R3, I * P::R3>(x, w, KeepAll{}); });
   } else {
     TableRow<P::R3> w;
     w.load(tab + (t + P::T * I) * P::FS);
@@ -389,7 +390,7 @@ __device__ __forceinline__ void inv_first(cf (&x)[P::E], int t, const float2* ro
       x[i * P::R1 + r] = lds_get(pb, P::phys(bitrev(r, ilog2(P::R1)) * P::S1));
     });
     if constexpr (P::THREE) {
-      ti.first[i].use([&](auto&& w) __attribute__((always_inline)) { inv_factors<P::R1, i * P::R1>(x, w, KeepAll{}); });
+      ti.first[i].template use<false>([&](auto&& w) __attribute__((always_inline)) { inv_factors<P::R1, i * P::R1>(x, w, KeepAll{}); });
     } else {
       TableRow<P::R1> w;
       w.load(tab + P::R1 * P::FS + (t + P::T * i) * P::IS);
@@ -466,7 +467,7 @@ __device__ __forceinline__ void convolve(cf (&x)[P::E], int t, float2* row, cons
   static_for<0, P::NG>([&](auto gg) { load_group<P, decltype(gg)::value>(x, t, row); });
   static_for<0, P::NG>([&](auto gg) {
     constexpr int g = decltype(gg)::value;
-    fwd_group<P, g>(x, t, tab, tf);
+    fwd_group<P, g, false>(x, t, tab, tf);
     multiply<P, g>(x, K);
     if constexpr (g + 1 < P::NG) load_spectrum<P, g + 1>(K, sp, t);
     inv_group<P, g>(x, t, row);
@@ -479,7 +480,7 @@ __device__ __forceinline__ void convolve(cf (&x)[P::E], int t, float2* row, cons
   before_last();
   inv_first<P>(x, t, row, tab, ti);
 }
-// The same with the spectrum in registers, as `transform` leaves it.  `behind_product` is called where those registers are free again.
+// The same with the spectrum in registers, as `held_spectrum` leaves it.  `behind_product` is called where those registers are free again.
 template <class P, int S8, bool REAL, class F>
 __device__ __forceinline__ void convolve_held(cf (&x)[P::E], int t, float2* row, const float2* tab, const TwistForward<P, S8>& tf,
                                               const TwistInverse<P>& ti, const cf (&K)[P::E], F&& behind_product) {
@@ -492,7 +493,7 @@ __device__ __forceinline__ void convolve_held(cf (&x)[P::E], int t, float2* row,
   static_for<0, P::NG>([&](auto gg) { load_group<P, decltype(gg)::value>(x, t, row); });
   static_for<0, P::NG>([&](auto gg) {
     constexpr int g = decltype(gg)::value;
-    fwd_group<P, g>(x, t, tab, tf);
+    fwd_group<P, g, false>(x, t, tab, tf);
     static_for<g * P::R3, (g + 1) * P::R3>([&](auto rr) { x[decltype(rr)::value] = cmul(x[decltype(rr)::value], K[decltype(rr)::value]); });
     inv_group<P, g>(x, t, row);
   });
@@ -505,7 +506,7 @@ __device__ __forceinline__ void convolve_held(cf (&x)[P::E], int t, float2* row,
   inv_first<P>(x, t, row, tab, ti);
 }
 // the forward half: the spectrum of registers in first-pass layout
-template <class P, int S8>
+template <class P, int S8, bool LARGE>
 __device__ __forceinline__ void transform(cf (&x)[P::E], int t, float2* row, const float2* tab, const TwistForward<P, S8>& tf) {
   fwd_first<P, S8, false>(x, t, row);
   sync_threads<P::T>();
@@ -514,7 +515,14 @@ __device__ __forceinline__ void transform(cf (&x)[P::E], int t, float2* row, con
     sync_threads<P::T>();
   }
   static_for<0, P::NG>([&](auto gg) { load_group<P, decltype(gg)::value>(x, t, row); });
-  static_for<0, P::NG>([&](auto gg) { fwd_group<P, decltype(gg)::value>(x, t, tab, tf); });
+  static_for<0, P::NG>([&](auto gg) { fwd_group<P, decltype(gg)::value, LARGE>(x, t, tab, tf); });
+}
+// The spectrum of taps in first-pass layout, kept in registers: what the spectrum kernels leave in memory, value by value.
+template <class P, int S8>
+__device__ __forceinline__ void held_spectrum(cf (&x)[P::E], int t, float2* row, const float2* tab, const TwistForward<P, S8>& tf) {
+  transform<P, S8, true>(x, t, row, tab, tf);
+  constexpr float scale = 1.f / (float)P::H;
+  static_for<0, P::E>([&](auto rr) { x[decltype(rr)::value] = {scale * x[decltype(rr)::value].re, scale * x[decltype(rr)::value].im}; });
 }
 
 // The forward half with fp64 butterflies, for the spectra of the shortest rows: values are rounded to fp32 between the passes and at
@@ -615,7 +623,7 @@ struct SpectrumForward {
   }
   __device__ __forceinline__ void operator()(cf (&x)[P::E], int t, float2* row, const float2* tab) const {
     if constexpr (fine_spectrum<P>()) transform_fine<P, S8>(x, t, row, tf);
-    else transform<P, S8>(x, t, row, tab, tf);
+    else transform<P, S8, true>(x, t, row, tab, tf);
   }
 };
 

@@ -456,11 +456,11 @@ __global__ __launch_bounds__(P::T) __attribute__((amdgpu_waves_per_eu(2, 2))) vo
       });
     }
     sync_threads<T>();                      // the item before has been read
-    transform<P, 1>(x, t, row, tab1, tf1);
+    transform<P, 1, false>(x, t, row, tab1, tf1);
     store_spectrum<P>(x, scale, blk);
     sync_threads<T>();
     static_for<0, 32>([&](auto rr) { x[decltype(rr)::value] = q[decltype(rr)::value]; });
-    transform<P, 5>(x, t, row, tab5, tf5);
+    transform<P, 5, false>(x, t, row, tab5, tf5);
     store_spectrum<P>(x, scale, blk + BLK / 4);
   }
 }

@@ -53,10 +53,6 @@ __global__ __launch_bounds__(P::T) __attribute__((amdgpu_waves_per_eu(2, 2))) vo
   tf.init(t);
   ti.init(t);
   te.init(t);
-  if constexpr (TAPS) static_for<0, P::NB1>([&](auto ii) {      // (1 / L, which the spectra hold otherwise)
-    te.f[decltype(ii)::value].re *= 1.f / (float)L;
-    te.f[decltype(ii)::value].im *= 1.f / (float)L;
-  });
   sync_threads<T>();
 
   // Workgroup ids are dealt round-robin to the 8 XCDs (one L2 each).  XCD e takes the channels
@@ -95,7 +91,7 @@ __global__ __launch_bounds__(P::T) __attribute__((amdgpu_waves_per_eu(2, 2))) vo
   auto transform_taps = [&](int c, int f) __attribute__((always_inline)) {
     gfloat* D = filters.skip ? in_global(filters.skip[f]) : nullptr;
     if (D && t == 0) K[0].re += D[c];      // the skip weight is one more tap at lag 0
-    transform<P, kQuarter>(K, anew(t), row, tab, tf);
+    held_spectrum<P, kQuarter>(K, anew(t), row, tab, tf);
   };
   if constexpr (TAPS) {
     if (slot < rows_per_xcd) fetch_taps(slot, 0);

@@ -73,10 +73,6 @@ __global__ __launch_bounds__(PairLayout<P>::WG) __attribute__((amdgpu_waves_per_
   tf.init(t);
   ti.init(t);
   te.init(t);
-  if constexpr (TAPS) static_for<0, P::NB1>([&](auto ii) {      // (1 / L, which the spectra hold otherwise)
-    te.f[decltype(ii)::value].re *= 1.f / (float)L;
-    te.f[decltype(ii)::value].im *= 1.f / (float)L;
-  });
   __syncthreads();
 
   // Workgroup ids are dealt round-robin to the 8 XCDs (one L2 each).  XCD e takes the channels
@@ -146,7 +142,7 @@ __global__ __launch_bounds__(PairLayout<P>::WG) __attribute__((amdgpu_waves_per_
       } else {
         static_for<0, E>([&](auto rr) { K[decltype(rr)::value] = {0.f, 0.f}; });
       }
-      transform<P, kQuarter>(K, anew(t), row, tab, tf);      // (the prologue's first barrier stands between its reads and the stage)
+      held_spectrum<P, kQuarter>(K, anew(t), row, tab, tf);      // (the prologue's first barrier stands between its reads and the stage)
     }
 
     // ---- prologue: 8 Q consecutive time steps per thread: short conv, gate, stage a and u in LDS ----

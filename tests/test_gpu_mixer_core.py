@@ -73,7 +73,7 @@ def test_rows_dealt_unevenly(gpu, L, d, B):
 @pytest.mark.parametrize("nfilters", [1, 2])
 def test_mixer_core_on_taps(gpu, L, d, B, nfilters):
     """The core that transforms its filters itself, in part filled workgroups and with workgroups that take several rows, against fp64 transforms
-    and against the core on spectra: fp32 sums of the same numbers whose rounding to bf16 falls the other way now and then."""
+    and against the core on spectra, whose bits it has."""
     from m2_amd import ops
     g = torch.Generator(device=gpu).manual_seed(L + d + B)
     rn = lambda *s: torch.randn(*s, generator=g, device=gpu)      # noqa: E731
@@ -102,7 +102,7 @@ def test_mixer_core_on_taps(gpu, L, d, B, nfilters):
         spec = ops.filter_spectrum(taps[0], taps[1] if nfilters == 2 else None, Ds[0], Ds[1] if nfilters == 2 else None)
         z = ops.mixer_core(xproj, second, sw, sb, spec, B, L, d, proj_bias=pb, row=row)
         assert (y.double() - ref).norm() <= 2.0 ** -8 * ref.norm()      # (the gate and the result are rounded to 2^-9)
-        assert (y.double() - z.double()).norm() <= 2.0 ** -12 * ref.norm()
+        assert torch.equal(y, z)
 
 
 def test_core_on_taps_refuses(gpu):
@@ -125,3 +125,29 @@ def test_core_on_taps_refuses(gpu):
     short = ops.MixerTaps(taps[:, :, :1024].contiguous(), None, Table())
     with pytest.raises(RuntimeError):
         ops.mixer_core(x.bfloat16()[:, :, :512].contiguous(), None, sw, sb, short, 1, 512, d)
+
+
+@pytest.mark.parametrize("L", [1024, 2048, 4096, 8192, 16384])
+def test_core_on_taps_beyond_ordinary_numbers(gpu, L):
+    """The bits of the core on spectra also next to the ends of fp32 (products that only the factor 1 / L of a spectrum keeps below the upper one), and
+    where a row has an infinity or a NaN."""
+    from m2_amd import ops
+    d, B = 64, 2
+    g = torch.Generator(device=gpu).manual_seed(L)
+    rn = lambda *s: torch.randn(*s, generator=g, device=gpu)      # noqa: E731
+    taps, xproj, u = rn(2, d, 2 * L) / L ** 0.5, rn(3 * d, B, L).bfloat16(), rn(d, B, L)
+    u[:16] *= 1e35
+    u[16:32] *= 1e-37
+    u[40, 0, 5], u[41, 1, 7] = float("inf"), float("nan")
+    sw, sb = rn(3 * d, 3), rn(3 * d)
+
+    class Table:
+        fpm = 2
+
+        def use_on(self, handle):
+            pass
+
+    y = ops.mixer_core(xproj, u, sw, sb, ops.MixerTaps(taps, None, Table()), B, L, d)
+    z = ops.mixer_core(xproj, u, sw, sb, ops.filter_spectrum(taps[0], taps[1], None, None), B, L, d)
+    assert torch.equal(torch.isnan(y), torch.isnan(z)) and torch.equal(y.nan_to_num(7.0), z.nan_to_num(7.0))
+    assert bool(torch.isfinite(y[:40]).all()) and not bool(torch.isfinite(y[40, 0]).all())
