@@ -102,9 +102,12 @@ class M2BertTextEncoder:
             for lo in range(0, len(token_ids), batch_size):
                 hi = min(lo + batch_size, len(token_ids))
                 both = torch.empty(2, hi - lo, self.max_seq_len, dtype=torch.int64, pin_memory=True)
-                self._assemble(token_ids, attention_masks, lo, hi, both)
+                rows = self._assemble(token_ids, attention_masks, lo, hi, both)
                 with torch.no_grad():
-                    ids_b, mask_b = both.to(self.device, non_blocking=True).unbind(0)
+                    if rows[0].data_ptr() == both.data_ptr():
+                        ids_b, mask_b = both.to(self.device, non_blocking=True).unbind(0)
+                    else:      # (put together from tensors, wherever those are)
+                        ids_b, mask_b = (t.to(self.device) for t in rows)
                     _, pooled = self.model(input_ids=ids_b, attention_mask=mask_b, ids_checked_later=True)
                 host = torch.empty(pooled.shape, dtype=torch.float32, pin_memory=True)
                 host.copy_(pooled.detach().float(), non_blocking=True)
@@ -120,8 +123,9 @@ class M2BertTextEncoder:
                 emb.check_indices()
 
     def _assemble(self, token_ids: Sequence, attention_masks: Optional[Sequence], lo: int, hi: int, into: Optional[torch.Tensor] = None):
-        """Texts [lo, hi), in the two halves of `into` where given, as padded or cut (hi - lo, max_seq_len) ids and mask.  Rows are written into two arrays, 7 us a
-        text of up to 512 tokens; a torch tensor per text, its mask, both padded and all of them concatenated took 41 (3 ms of 75 texts)."""
+        """Texts [lo, hi) as padded or cut (hi - lo, max_seq_len) ids and mask.  Rows are written into two arrays, the halves of `into` where
+        given, 7 us a text of up to 512 tokens; a torch tensor per text, its mask, both padded and all of them concatenated took 41 (3 ms of
+        75 texts).  Rows that no array can be written from (on the GPU, of floats, ...) come as tensors of their own."""
         L = self.max_seq_len
         both = np.empty((2, hi - lo, L), np.int64) if into is None else into.numpy()
         both[...] = 0
@@ -130,10 +134,7 @@ class M2BertTextEncoder:
             ids = _host_row(token_ids[k])
             mask = None if attention_masks is None else _host_row(attention_masks[k])
             if ids is None or (mask is None and attention_masks is not None):
-                rows = self._assemble_tensors(token_ids, attention_masks, lo, hi)
-                if into is not None:
-                    torch.stack(rows, out=into)
-                return rows
+                return self._assemble_tensors(token_ids, attention_masks, lo, hi)
             if mask is not None and mask.shape != ids.shape:
                 raise ValueError(f"text {k}: {ids.shape[0]} token ids but {mask.shape[0]} mask entries")
             n = min(ids.shape[0], L)

@@ -36,6 +36,20 @@ def test_same_as_one_batch_at_a_time(gpu, n, batch):
     assert np.array_equal(enc.encode_token_ids(texts, batch, attention_masks=masks), got)
 
 
+def test_ids_and_masks_on_the_gpu(gpu):
+    enc = _encoder(gpu)
+    texts = _texts(11)
+    masks = [[1 - i % 2 for i in range(len(t))] for t in texts]
+    want = enc.encode_token_ids(texts, 4, attention_masks=masks)
+    there = [torch.tensor(t).to(gpu) for t in texts]
+    mthere = [torch.tensor(m).to(gpu) for m in masks]
+    assert np.array_equal(enc.encode_token_ids(there, 4), want)      # (the mask is not used by the plain pooler)
+    assert np.array_equal(enc.encode_token_ids(there, 4, attention_masks=mthere), want)
+    assert np.array_equal(enc.encode_token_ids(there, 4, attention_masks=masks), want)
+    assert np.array_equal(enc.encode_token_ids(texts, 4, attention_masks=mthere), want)
+    assert np.array_equal(enc.encode_token_ids([t.int() for t in there], 4), want)
+
+
 def test_errors(gpu):
     enc = _encoder(gpu)
     texts = _texts(20)
