@@ -96,7 +96,7 @@ class M2BertTextEncoder:
         def finish():
             host, done = pending.popleft()
             done.synchronize()
-            out.append(host)
+            out.append(host.clone())      # (pageable: the pinned block goes back for the batch after the next)
 
         try:
             for lo in range(0, len(token_ids), batch_size):

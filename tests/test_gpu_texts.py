@@ -1,4 +1,6 @@
 """Texts encoded with batches enqueued ahead of the GPU: the results and the errors of one batch after the other."""
+import weakref
+
 import numpy as np
 import pytest
 import torch
@@ -48,6 +50,23 @@ def test_ids_and_masks_on_the_gpu(gpu):
     assert np.array_equal(enc.encode_token_ids(there, 4, attention_masks=masks), want)
     assert np.array_equal(enc.encode_token_ids(texts, 4, attention_masks=mthere), want)
     assert np.array_equal(enc.encode_token_ids([t.int() for t in there], 4), want)
+
+
+def test_pinned_memory_does_not_grow_with_the_texts(gpu, monkeypatch):
+    enc = _encoder(gpu)
+    texts, kept, most, empty = _texts(60), [], [0], torch.empty
+
+    def counting(*args, **kw):
+        t = empty(*args, **kw)
+        if kw.get("pin_memory"):
+            kept.append(weakref.ref(t))
+            most[0] = max(most[0], sum(r() is not None for r in kept))
+        return t
+
+    monkeypatch.setattr(torch, "empty", counting)
+    enc.encode_token_ids(texts, 2)
+    # ids of the batch being put together and of the last, results of three
+    assert len(kept) == 60 and most[0] <= 5 and not any(r() is not None for r in kept)
 
 
 def test_errors(gpu):
