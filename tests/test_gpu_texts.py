@@ -91,3 +91,14 @@ def test_errors(gpu):
     enc.model.validate_ids = True
     with pytest.raises(IndexError):                               # what nobody asked about is still there
         enc.model.embeddings.check_indices()
+    assert np.isfinite(enc.encode_token_ids(texts, 4)).all()
+    # ... and is not the error of a call that has looked nothing up
+    enc.model.validate_ids = False
+    enc.encode_token_ids(bad, 4)
+    enc.model.validate_ids = True
+    assert enc.encode_token_ids([], 4).shape == (0, 768)
+    with pytest.raises(ValueError, match="text 0"):
+        enc.encode_token_ids([[1, 2]], 4, attention_masks=[[1]])
+    with pytest.raises(IndexError):
+        enc.encode_token_ids(texts, 4)
+    assert np.array_equal(enc.encode_token_ids(texts, 4), want)
