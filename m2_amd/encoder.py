@@ -23,7 +23,10 @@ from functools import partial
 from typing import List, Optional
 
 import torch
+import torch.autograd.forward_ad as forward_ad
 import torch.nn as nn
+from torch.overrides import _get_current_function_mode_stack
+from torch.utils._device import DeviceContext
 
 from . import ops, schedule
 from .blockdiag import BlockdiagLinear
@@ -602,6 +605,28 @@ class BertPooler(nn.Module):
 _OWN_POOLER = BertPooler.forward
 
 
+def called_plainly(*modules: nn.Module) -> bool:
+    """Whether a call of each module is its class's forward and nothing of a caller's own: no hooks (nor any for all modules), no forward
+    of the instance, no compiled one."""
+    every = torch.nn.modules.module
+    if every._global_forward_hooks or every._global_forward_pre_hooks or every._global_backward_hooks or every._global_backward_pre_hooks:
+        return False
+    return not any(m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks or m._compiled_call_impl is not None
+                   or "forward" in m.__dict__ for m in modules)
+
+
+def only_values(*tensors: torch.Tensor) -> bool:
+    """Whether a kernel that is given the tensors' memory is all that the product of them would be: nobody asks for gradients of them (backward or
+    forward), traces, transforms functions (vmap, jvp, ...) or has a mode of its own around torch's operations."""
+    c = torch._C
+    if c._are_functorch_transforms_active() or c._get_tracing_state() is not None or c._len_torch_dispatch_stack():
+        return False
+    if any(type(m) is not DeviceContext for m in _get_current_function_mode_stack()):
+        return False
+    return not any(type(t) not in (torch.Tensor, nn.Parameter) or (t.requires_grad and torch.is_grad_enabled())
+                   or forward_ad.unpack_dual(t).tangent is not None for t in tensors)
+
+
 class BertModel(nn.Module):
     """Embeddings + encoder + pooler; returns (sequence output or list of layer outputs, pooled output or None)
     like the reference (bert/src/bert_layers.py:880-1010)."""
@@ -648,18 +673,18 @@ class BertModel(nn.Module):
         return plan.run(route, B, all_layers, None, None, part, ids.contiguous(), tt, pos)
 
     def _pool(self, hidden: torch.Tensor, mask: torch.Tensor) -> torch.Tensor:
-        """The pooler's output: by one kernel where it is the plain module, in fp32 and nobody asks for gradients, for batches up to
+        """The pooler's output: by one kernel where it is the plain module, in fp32 and nobody asks for more than values, for batches up to
         256 (beyond, the library's product shares its weights among more rows)."""
         p = self.pooler
-        if (type(p) is BertPooler and type(p).forward is _OWN_POOLER and "forward" not in p.__dict__ and not p.pool_all
-                and hidden.shape[0] <= 256 and hidden.dtype == torch.float32 and not torch.is_autocast_enabled()
-                and type(p.dense) is nn.Linear and type(p.activation) is nn.Tanh
-                and not any(m._forward_hooks or m._forward_pre_hooks or "forward" in m.__dict__ for m in (p, p.dense, p.activation))):
-            w, b, d = p.dense.weight, p.dense.bias, hidden.shape[2]
-            plain = all(t.dtype == torch.float32 and t.is_contiguous() and t.device == hidden.device and not (t.requires_grad and torch.is_grad_enabled())
-                        for t in (w, b) if t is not None)
-            if plain and w.shape == (d, d) and (b is None or b.shape == (d,)) and d % 8 == 0 and (hidden.data_ptr() | w.data_ptr()) % 16 == 0:
-                return ops.pooler(hidden.detach()[:, 0], w.detach(), None if b is None else b.detach())
+        if (type(p) is BertPooler and type(p).forward is _OWN_POOLER and not p.pool_all and type(p.dense) is nn.Linear and type(p.activation) is nn.Tanh
+                and called_plainly(p, p.dense, p.activation) and not torch.is_autocast_enabled()):
+            w, b = p.dense.weight, p.dense.bias
+            given = [t for t in (w, b) if t is not None]
+            if (only_values(hidden, *given) and hidden.dtype == torch.float32 and hidden.shape[0] <= 256
+                    and all(t.dtype == torch.float32 and t.is_contiguous() and t.device == hidden.device for t in given)):
+                d = hidden.shape[2]
+                if w.shape == (d, d) and (b is None or b.shape == (d,)) and d % 8 == 0 and (hidden.data_ptr() | w.data_ptr()) % 16 == 0:
+                    return ops.pooler(hidden.detach()[:, 0], w.detach(), None if b is None else b.detach())
         return p(hidden, mask=mask)
 
     def get_input_embeddings(self):

@@ -23,6 +23,79 @@ def test_against_fp64(gpu, B, d):
         assert ((got.double() - ref).abs()[~bad] <= ((d / 64 + 8) * 2.0 ** -24 * size)[~bad]).all()
 
 
+@pytest.fixture
+def counted(gpu):
+    """(a one-layer model, how often the kernel has run)"""
+    import m2_amd
+    from m2_amd import ops
+    cfg = m2_amd.m2_bert_80m(128)
+    cfg.num_hidden_layers = 1
+    model = m2_amd.BertModel(cfg)
+    model.load_state_dict(m2_amd.seeded_state_dict(cfg, 2))
+    calls, own = [], ops.pooler
+    ops.pooler = lambda *a: (calls.append(1), own(*a))[1]
+    yield model.to(gpu).eval(), calls
+    ops.pooler = own
+
+
+def _hidden(gpu, B=3):
+    return torch.randn(B, 128, 768, generator=torch.Generator().manual_seed(B)).to(gpu)
+
+
+def test_transforms_and_modes_see_the_module(gpu, counted):
+    import torch.autograd.forward_ad as fw
+    from torch.func import functional_call, jvp, vmap
+    from torch.utils.flop_counter import FlopCounterMode
+    model, calls = counted
+    model.pooler.requires_grad_(False)
+    h, p = _hidden(gpu), model.pooler
+    w, dw = p.dense.weight.detach(), torch.randn_like(p.dense.weight)
+    s = h[:, 0].double() @ w.double().t() + p.dense.bias.double()
+    tangent = (h[:, 0].double() @ dw.double().t()) / s.cosh() ** 2
+
+    class Pool(torch.nn.Module):
+        def __init__(self):
+            super().__init__()
+            self.model = model
+
+        def forward(self, h):
+            return self.model._pool(h, None)
+
+    m = Pool()
+    assert torch.allclose(m(h).double(), s.tanh(), atol=1e-4) and len(calls) == 1
+    with torch.device(gpu):                                       # (a default device is no such mode)
+        m(h)
+    assert len(calls) == 2
+    name = "model.pooler.dense.weight"
+    with fw.dual_level():
+        out = fw.unpack_dual(functional_call(m, {name: fw.make_dual(w, dw)}, (h,)))
+        assert torch.allclose(out.tangent.double(), tangent, atol=1e-3)
+        out = fw.unpack_dual(m(fw.make_dual(h, torch.zeros_like(h))))
+        assert out.tangent is not None
+    out, t = jvp(lambda x: functional_call(m, {name: x}, (h,)), (w,), (dw,))
+    assert torch.allclose(t.double(), tangent, atol=1e-3)
+    many = vmap(lambda x: functional_call(m, {name: x}, (h,)))(torch.stack([w, 2 * w]))
+    assert torch.allclose(many[0].double(), s.tanh(), atol=1e-4) and many.shape == (2, 3, 768)
+    h.requires_grad_()
+    assert m(h).requires_grad
+    h.requires_grad_(False)
+    with FlopCounterMode(display=False) as flops:
+        m(h)
+    assert flops.get_total_flops() == 2 * 3 * 768 * 768
+    assert len(calls) == 2
+    assert torch.jit.trace(m, (h,), check_trace=False)(2 * h).sub(torch.tanh(p.dense(2 * h[:, 0]))).abs().max() < 1e-5
+    seen = []
+    hook = torch.nn.modules.module.register_module_forward_hook(lambda mod, i, o: seen.append(mod))
+    try:
+        m(h)
+    finally:
+        hook.remove()
+    assert p in seen and p.dense in seen and len(calls) == 2
+    p.dense.compile()                                             # (is not run: only that it is asked for)
+    p.dense._compiled_call_impl = lambda x: x + 1
+    assert torch.equal(m(h), torch.tanh(h[:, 0] + 1)) and len(calls) == 2
+
+
 def test_stands_for_the_module_only_where_it_is_plain(gpu):
     import m2_amd
     from m2_amd import ops
