@@ -627,6 +627,14 @@ def only_values(*tensors: torch.Tensor) -> bool:
                    or forward_ad.unpack_dual(t).tangent is not None for t in tensors)
 
 
+def _rows_of_four(hidden: torch.Tensor) -> bool:
+    """Whether the first token of every sequence of (B, L, d) is a row of consecutive values that a multiple of four lies between."""
+    if hidden.dim() != 3 or 0 in hidden.shape:
+        return False
+    B, _, d = hidden.shape
+    return hidden.stride(2) == 1 and (B == 1 or (hidden.stride(0) >= d and hidden.stride(0) % 4 == 0))
+
+
 class BertModel(nn.Module):
     """Embeddings + encoder + pooler; returns (sequence output or list of layer outputs, pooled output or None)
     like the reference (bert/src/bert_layers.py:880-1010)."""
@@ -680,7 +688,7 @@ class BertModel(nn.Module):
                 and called_plainly(p, p.dense, p.activation) and not torch.is_autocast_enabled()):
             w, b = p.dense.weight, p.dense.bias
             given = [t for t in (w, b) if t is not None]
-            if (only_values(hidden, *given) and hidden.dtype == torch.float32 and hidden.shape[0] <= 256
+            if (only_values(hidden, *given) and hidden.dtype == torch.float32 and hidden.is_cuda and _rows_of_four(hidden) and hidden.shape[0] <= 256
                     and all(t.dtype == torch.float32 and t.is_contiguous() and t.device == hidden.device for t in given)):
                 d = hidden.shape[2]
                 if w.shape == (d, d) and (b is None or b.shape == (d,)) and d % 8 == 0 and (hidden.data_ptr() | w.data_ptr()) % 16 == 0:

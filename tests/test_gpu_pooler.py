@@ -96,6 +96,32 @@ def test_transforms_and_modes_see_the_module(gpu, counted):
     assert torch.equal(m(h), torch.tanh(h[:, 0] + 1)) and len(calls) == 2
 
 
+def test_hidden_states_in_any_layout(gpu, counted):
+    """What a caller's own encoder may return: the kernel takes rows it can read, the module everything else."""
+    model, calls = counted
+    h = _hidden(gpu, 5)
+    with torch.no_grad():
+        want = model.pooler(h)
+        wide = torch.zeros(5, 128, 770, device=gpu)
+        wide[..., :768] = h
+        flat = torch.zeros(5 * (128 * 768 + 2), device=gpu)
+        odd = flat.as_strided((5, 128, 768), (128 * 768 + 2, 768, 1))
+        odd.copy_(h)
+        shifted = torch.zeros(h.numel() + 1, device=gpu)[1:].view(h.shape)
+        shifted.copy_(h)
+        # (layout, sequences, whether the kernel takes it)
+        for x, n, own in [(h, 5, True), (h.transpose(1, 2).contiguous().transpose(1, 2), 5, False), (wide[..., :768], 5, True),
+                          (odd, 5, False), (odd[:1], 1, True), (shifted, 5, False), (h[:1].expand(5, 128, 768), 5, False), (h[::2], 3, True)]:
+            del calls[:]
+            got, ref = model._pool(x, None), model.pooler(x)
+            assert len(calls) == own and got.shape == (n, 768) and (got - ref).abs().max() < 2e-6
+        assert model._pool(h[:0], None).shape == (0, 768) and (model._pool(h, None) - want).abs().max() < 2e-6
+        with pytest.raises(IndexError):                           # no first token
+            model._pool(h[:, :0], None)
+        del calls[:]
+        assert model.cpu()._pool(h.cpu(), None).device.type == "cpu" and not calls
+
+
 def test_stands_for_the_module_only_where_it_is_plain(gpu):
     import m2_amd
     from m2_amd import ops
