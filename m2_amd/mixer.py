@@ -125,7 +125,8 @@ class MonarchMixerSequenceMixing(nn.Module):
         in_linear.bias as it loads), u_cm (d, B, L) fp32 -> y (d, B, L).  xproj may also be (3d, row), row >= B L, the values of a
         channel at the start of its row."""
         if spec is None:
-            if ops.taps_pay(B, L, xproj.dtype) and not self.cache_filters and takes_taps(self):
+            # (a second input without a second filter meets the zero spectrum that spectra have in its place)
+            if ((u_cm is None or self.residual_long_conv) and ops.taps_pay(B, L, xproj.dtype) and not self.cache_filters and takes_taps(self)):
                 spec = self._generate_spectrum(L, [self.filter_fn] + ([self.filter_fn2] if self.residual_long_conv else []), taps=True)
             else:
                 spec = self.filter_spectrum(L)

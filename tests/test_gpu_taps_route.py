@@ -90,3 +90,16 @@ def test_cached_filters_give_the_same_bits(gpu, L, B):
         for layer in model.encoder.layer:
             layer.attention.cache_filters = True
         assert all(torch.equal(model(ids)[0], want) for _ in range(2))
+
+
+def test_a_second_input_without_a_second_filter(gpu):
+    """`core` given an input for the residual convolution that the mixer does not have: as if it had not been given."""
+    import m2_amd
+    L, d = 1024, 768
+    mixer = m2_amd.MonarchMixerSequenceMixing(d, l_max=L, bidirectional=True, hyena_emb_dim=5, hyena_filter_order=128, residual_long_conv=False,
+                                              hyena_w=10).to(gpu).eval()
+    g = torch.Generator().manual_seed(12)
+    x, u = torch.randn(3 * d, 1, L, generator=g).to(gpu).bfloat16(), torch.randn(d, 1, L, generator=g).to(gpu)
+    with torch.no_grad():
+        y, z = mixer.core(x, u, 1, L), mixer.core(x, None, 1, L)
+        assert torch.equal(y, z) and torch.equal(y, mixer.core(x, u, 1, L, spec=mixer.filter_spectrum(L)))
