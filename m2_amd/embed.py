@@ -14,9 +14,10 @@ from typing import Callable, Dict, Iterable, List, Optional, Sequence
 
 import numpy as np
 import torch
+import torch.nn as nn
 import torch.nn.functional as F
 
-from .encoder import BertModel
+from .encoder import BertModel, called_plainly
 
 
 def split_list(items: Sequence, chunk_size: int) -> Iterable[Sequence]:
@@ -81,9 +82,9 @@ class M2BertTextEncoder:
         return out.numpy()
 
     def _plain_model(self) -> bool:
-        """The model's forward is the one of this package, with nothing around it that would see its arguments."""
+        """The model's forward is the one of this package, with nothing around it that would see its call."""
         m = self.model
-        return (type(m).forward is BertModel.forward and "forward" not in m.__dict__ and not m._forward_hooks and not m._forward_pre_hooks
+        return (type(m).forward is BertModel.forward and type(m).__call__ is nn.Module.__call__ and called_plainly(m)
                 and torch.device(self.device).type == "cuda")
 
     def _run_ahead(self, token_ids: Sequence, batch_size: int, attention_masks: Optional[Sequence], out: List[torch.Tensor]) -> None:
@@ -109,7 +110,7 @@ class M2BertTextEncoder:
                     else:      # (put together from tensors, wherever those are)
                         ids_b, mask_b = (t.to(self.device) for t in rows)
                     asked = True
-                    _, pooled = self.model(input_ids=ids_b, attention_mask=mask_b, ids_checked_later=True)
+                    _, pooled = self.model._forward(ids_b, None, mask_b, None, False, None, check_ids=False)
                 host = torch.empty(pooled.shape, dtype=torch.float32, pin_memory=True)
                 host.copy_(pooled.detach().float(), non_blocking=True)
                 done = torch.cuda.Event()

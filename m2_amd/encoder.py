@@ -702,6 +702,11 @@ class BertModel(nn.Module):
                 attention_mask: Optional[torch.Tensor] = None, position_ids: Optional[torch.Tensor] = None,
                 output_all_encoded_layers: Optional[bool] = False, masked_tokens_mask: Optional[torch.Tensor] = None,
                 **kwargs):
+        return self._forward(input_ids, token_type_ids, attention_mask, position_ids, output_all_encoded_layers, masked_tokens_mask,
+                             self.validate_ids)
+
+    def _forward(self, input_ids, token_type_ids, attention_mask, position_ids, output_all_encoded_layers, masked_tokens_mask, check_ids: bool):
+        """The forward; check_ids: wait for the GPU at its end and report ids outside their tables."""
         if masked_tokens_mask is not None:
             raise NotImplementedError("masked_tokens_mask subsetting belongs to the MLM head, which is not built")
         B, L = input_ids.shape
@@ -757,6 +762,6 @@ class BertModel(nn.Module):
         finally:
             # last, behind everything that is to be enqueued: it waits for the stream.  Also when the pooler raises: a bad id is
             # this forward's error and not the next one's
-            if self.validate_ids and not kwargs.get("ids_checked_later") and not torch.cuda.is_current_stream_capturing():
+            if check_ids and not torch.cuda.is_current_stream_capturing():
                 self.embeddings.check_indices()
         return (enc if output_all_encoded_layers else enc[-1]), pooled

@@ -69,6 +69,34 @@ def test_pinned_memory_does_not_grow_with_the_texts(gpu, monkeypatch):
     assert len(kept) == 60 and most[0] <= 5 and not any(r() is not None for r in kept)
 
 
+def test_what_a_caller_put_around_the_model_sees_every_call(gpu):
+    import m2_amd
+    enc = _encoder(gpu)
+    texts, seen = _texts(9), []
+    want = enc.encode_token_ids(texts, 4)
+    hook = torch.nn.modules.module.register_module_forward_pre_hook(lambda m, a: seen.append(m))
+    assert np.abs(enc.encode_token_ids(texts, 4) - want).max() < 2e-6      # (such a hook is to see the pooler's modules too)
+    hook.remove()
+    assert seen.count(enc.model) == 3
+
+    class Counting(m2_amd.BertModel):
+        def __call__(self, *args, **kwargs):
+            seen.append(sorted(kwargs))
+            return super().__call__(*args, **kwargs)
+
+    enc.model.__class__ = Counting
+    del seen[:]
+    assert np.array_equal(enc.encode_token_ids(texts, 4), want) and seen == 3 * [["attention_mask", "input_ids"]]
+    enc.model.__class__ = m2_amd.BertModel
+    enc.model._compiled_call_impl = lambda *args, **kwargs: (seen.append(args), enc.model.forward(*args, **kwargs))[1]
+    del seen[:]
+    assert np.array_equal(enc.encode_token_ids(texts, 4), want) and len(seen) == 3
+    enc.model._compiled_call_impl = None
+    # a forward takes what it always took, and no keyword puts its check off
+    with pytest.raises(IndexError):
+        enc.model(torch.full((1, 128), 10 ** 6, device=gpu), ids_checked_later=True)
+
+
 def test_errors(gpu):
     enc = _encoder(gpu)
     texts = _texts(20)
