@@ -186,9 +186,9 @@ long m2_dense_channels_row(int M, int N, int K);
 int m2_dense_from_channels_fwd(const void* x, const void* w, const float* bias, void* out, int M, int N, int K,
                                void* stream);
 /* LayerNorm and the first projection of few rows as one kernel: out (N, M) = w (N, K) LayerNorm(s)^T for s (M, K) bf16, and the normalised
- * rows channel-major in fp32, out_channel_major (K, M) or NULL: the bits of m2_layernorm_bf16_fwd followed by
- * m2_dense_to_channels_rows_fwd.  N = 3 K, K = 768, 960, 1536 or 1792; all pointers 16-byte aligned.  ..._supported: 1 where it is
- * the faster of the two (host code). */
+ * rows channel-major in fp32, out_channel_major (K, M) or NULL: the rows m2_layernorm_bf16_fwd writes, bit for bit, and their product with
+ * w.  N = 3 K, K = 768, 960, 1536 or 1792; all pointers 16-byte aligned.  ..._supported: 1 where it is faster than the two calls (host
+ * code); there the product too has the bits of m2_dense_to_channels_rows_fwd. */
 int m2_layernorm_to_channels_supported(int M, int N, int K);
 int m2_layernorm_to_channels_fwd(const void* s, const float* gamma, const float* beta, float eps, const void* w, void* out, long out_row,
                                  float* out_channel_major, int M, int N, int K, void* stream);

@@ -168,7 +168,8 @@ static int launch_small(const GemmArgs& g, hipStream_t st) {
 // LayerNorm and in_linear of few rows as one kernel: rows of s (M, d) bf16 are normalised on their way into the product
 //   out (N, M) = w (N, d) LayerNorm(s)^T
 // A workgroup has 32 rows and 16 JT output channels.  The rows come whole into LDS (48 KB at d = 768), where every wave takes the
-// statistics of four as layernorm_kernel does, column by column and lane by lane and by the same expressions, so that the rows have its bits;
+// statistics of four as layernorm_kernel does, column by column and lane by lane and by the same functions (ln_squares, ...), so that the
+// rows have its bits;
 // then every wave normalises its eighth of K in operand layout, and products and sums are small_gemm_kernel's.  The channel-major fp32
 // form that the mixer core reads is written by the workgroups of the first d channels' worth of tiles, 32 of its channels each.
 //
@@ -200,8 +201,6 @@ __global__ __launch_bounds__(512) void ln_gemm_kernel(const uint16_t* __restrict
   const int jt = __builtin_amdgcn_readfirstlane(tile / ti), i0 = 32 * (tile - jt * ti), j0 = 16 * JT * jt;
   const int s0 = wave * NKS / 8, ns = (wave + 1) * NKS / 8 - s0;
   const u32x4 zero = {0u, 0u, 0u, 0u};
-  // value - mean with one rounding (what the compiler makes of layernorm_kernel's two steps)
-  auto centred = [](float v, float sum) __attribute__((always_inline)) { return fmaf(-sum, 1.0f / (float)d, v); };
 
   // everything that is read is requested here: rows, weights, the scales of this wave's columns
   constexpr int kPieces = 32 * d / 8, kLoads = (kPieces + 511) / 512;
@@ -256,17 +255,12 @@ __global__ __launch_bounds__(512) void ln_gemm_kernel(const uint16_t* __restrict
     for (int o = 32; o > 0; o >>= 1) static_for<0, 4>([&](auto rr) { sum[decltype(rr)::value] += __shfl_xor(sum[decltype(rr)::value], o); });
     static_for<0, 4>([&](auto rr) {
       constexpr int r = decltype(rr)::value;
-      float t = 0.f;
-      static_for<0, PER>([&](auto ii) {
-        const float c = centred(v[r][decltype(ii)::value], sum[r]);
-        t += c * c;
-      });
-      sq[r] = t;
+      sq[r] = ln_squares<d>(v[r], sum[r]);
     });
     for (int o = 32; o > 0; o >>= 1) static_for<0, 4>([&](auto rr) { sq[decltype(rr)::value] += __shfl_xor(sq[decltype(rr)::value], o); });
     static_for<0, 4>([&](auto rr) {
       constexpr int r = decltype(rr)::value;
-      if (lane == r) stats[4 * wave + r] = make_float2(sum[r], rsqrtf(fmaf(sq[r], 1.0f / (float)d, eps)));
+      if (lane == r) stats[4 * wave + r] = make_float2(sum[r], ln_rstd<d>(sq[r], eps));
     });
   }
   __syncthreads();
@@ -282,8 +276,8 @@ __global__ __launch_bounds__(512) void ln_gemm_kernel(const uint16_t* __restrict
       const u32x4 x = *reinterpret_cast<const u32x4*>(rows + r * PITCH + (k < ns ? 32 * (s0 + k) + 8 * q4 : 0));
       static_for<0, 4>([&](auto e) {
         constexpr int i = decltype(e)::value;
-        const float lo = fmaf(centred(__uint_as_float(x[i] << 16), st.x) * st.y, g[k][2 * i], b[k][2 * i]);
-        const float hi = fmaf(centred(__uint_as_float(x[i] & 0xffff0000u), st.x) * st.y, g[k][2 * i + 1], b[k][2 * i + 1]);
+        const float lo = ln_value<d>(__uint_as_float(x[i] << 16), st.x, st.y, g[k][2 * i], b[k][2 * i]);
+        const float hi = ln_value<d>(__uint_as_float(x[i] & 0xffff0000u), st.x, st.y, g[k][2 * i + 1], b[k][2 * i + 1]);
         pf[t][k][i] = k < ns ? pack_bf16x2(lo, hi) : 0u;
       });
     });
@@ -306,8 +300,8 @@ __global__ __launch_bounds__(512) void ln_gemm_kernel(const uint16_t* __restrict
     if (i0 + r < M) {      // (M is even)
       const float gc = gamma[c], bc = beta[c];
       const float2 sa = stats[r], sb = stats[r + 1];
-      const float va = fmaf(centred(bf16_to_f32(rows[r * PITCH + c]), sa.x) * sa.y, gc, bc),
-                  vb = fmaf(centred(bf16_to_f32(rows[(r + 1) * PITCH + c]), sb.x) * sb.y, gc, bc);
+      const float va = ln_value<d>(bf16_to_f32(rows[r * PITCH + c]), sa.x, sa.y, gc, bc),
+                  vb = ln_value<d>(bf16_to_f32(rows[(r + 1) * PITCH + c]), sb.x, sb.y, gc, bc);
       *reinterpret_cast<float2*>(out_t + (long)c * M + i0 + r) = make_float2(va, vb);
     }
   }

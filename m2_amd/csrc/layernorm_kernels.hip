@@ -117,24 +117,17 @@ __global__ __launch_bounds__(512) void layernorm_kernel(const IN* __restrict__ x
     static_for<0, RW>([&](auto rr_) { sum[decltype(rr_)::value] += __shfl_xor(sum[decltype(rr_)::value], o); });
   static_for<0, RW>([&](auto rr_) {
     constexpr int rr = decltype(rr_)::value;
-    sum[rr] *= (1.0f / (float)d);
-    float s = 0.f;
-    static_for<0, PER>([&](auto ii) {
-      const float c = v[rr][decltype(ii)::value] - sum[rr];
-      s += c * c;
-    });
-    sq[rr] = s;
+    sq[rr] = ln_squares<d>(v[rr], sum[rr]);
   });
   for (int o = 32; o > 0; o >>= 1)
     static_for<0, RW>([&](auto rr_) { sq[decltype(rr_)::value] += __shfl_xor(sq[decltype(rr_)::value], o); });
   static_for<0, RW>([&](auto rr_) {
     constexpr int rr = decltype(rr_)::value;
     const int m = m0 + wave * RW + rr;
-    const float mean = sum[rr];
-    const float rstd = rsqrtf(sq[rr] * (1.0f / (float)d) + eps);
+    const float rstd = ln_rstd<d>(sq[rr], eps);
     static_for<0, PER>([&](auto ii) {
       constexpr int i = decltype(ii)::value;
-      v[rr][i] = (v[rr][i] - mean) * rstd * g[i] + bt[i];
+      v[rr][i] = ln_value<d>(v[rr][i], sum[rr], rstd, g[i], bt[i]);
       if (m < M) {
         if (out_f32) out_f32[(long)m * d + lane + 64 * i] = v[rr][i];
         if (out_bf16) out_bf16[(long)m * d + lane + 64 * i] = f32_to_bf16(v[rr][i]);

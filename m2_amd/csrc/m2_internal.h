@@ -33,6 +33,28 @@ int dense_ws_launch(const void* x, const void* w, void* out, int M, int N, long 
 typedef const __attribute__((address_space(1))) float gfloat;
 __device__ __forceinline__ gfloat* in_global(const float* p) { return (gfloat*)p; }
 
+// LayerNorm of a row of D values with its roundings said, for the kernels that have to give the same bits.  `sum` and `sq` are the sums over the row of the
+// values and of their squared distances to the mean, of which a lane's N values give ln_squares.
+template <int D>
+__device__ __forceinline__ float ln_centred(float v, float sum) { return fmaf(-sum, 1.0f / (float)D, v); }      // value - mean, one rounding
+template <int D, int N>
+__device__ __forceinline__ float ln_squares(const float (&v)[N], float sum) {
+  const float c0 = ln_centred<D>(v[0], sum);
+  float sq = c0 * c0;
+#pragma unroll
+  for (int i = 1; i < N; ++i) {
+    const float c = ln_centred<D>(v[i], sum);
+    sq = i == 1 ? fmaf(c0, c0, c * c) : fmaf(c, c, sq);
+  }
+  return sq;
+}
+template <int D>
+__device__ __forceinline__ float ln_rstd(float sq, float eps) { return rsqrtf(fmaf(sq, 1.0f / (float)D, eps)); }
+template <int D>
+__device__ __forceinline__ float ln_value(float v, float sum, float rstd, float gamma, float beta) {
+  return fmaf(ln_centred<D>(v, sum) * rstd, gamma, beta);
+}
+
 // round-to-nearest-even float -> bfloat16 bits (NaN stays NaN)
 // float -> bf16 bits, round to nearest even (host restatement of what v_cvt_pk_bf16_f32 does)
 __host__ __device__ __forceinline__ uint16_t f32_to_bf16_bits(float f) {
