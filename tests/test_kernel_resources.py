@@ -36,7 +36,8 @@ def _kernels():
     return found
 
 
-@pytest.mark.parametrize("kernel", ["project_kernel", "hidden_kernel", "project_spectrum_kernel", "mixer_pair_kernel", "mixer_long_kernel", "conv_real_kernel"])
+@pytest.mark.parametrize("kernel", ["project_kernel", "hidden_kernel", "project_spectrum_kernel", "mixer_pair_kernel", "mixer_long_kernel", "conv_real_kernel",
+                                    "small_gemm_kernel", "ln_gemm_kernel", "layernorm_kernel", "pooler_kernel"])
 def test_kernels_without_scratch(kernel):
     mine = {n: k for n, k in _kernels().items() if f"{len(kernel)}{kernel}" in n}
     assert mine, kernel
