@@ -94,7 +94,7 @@ int m2_hyena_filter_fwd_static(const m2_hyena_filter_params* params, int nfilter
  * every mixer of a model at once (bert/src/mm/monarch_mixer_sequence_mixer.py:120-139 with
  * bert/src/mm/hyena_utils.py:201-236 and :24-33; the reference's native filter kernel is batched over filters the
  * same way, csrc/flashmm/flash_mm.cpp:301-338).  Same arithmetic as m2_hyena_filter_fwd followed by
- * m2_filter_spectrum_fwd per mixer, in three or four launches for ALL mixers; for L <= 512 the output projection,
+ * m2_filter_spectrum_fwd per mixer, in two or three launches for ALL mixers; for L <= 512 the output projection,
  * the decay and the transform are one kernel and the taps never exist in memory.
  * params_dev  DEVICE array of nmixers * filters_per_mixer structs (of device pointers): filter_fn of mixer 0,
  *             filter_fn2 of mixer 0 (when filters_per_mixer == 2), filter_fn of mixer 1, ...  All filters share L, d,

@@ -569,9 +569,10 @@ extern "C" size_t m2_hyena_filter_workspace_bytes(int nfilters, int L, int d, in
 // then, has for their scales where a caller's workspace of the documented size is all there is.)
 static bool project_with_hidden(int L, int d) { return L >= 1024 && L % 64 == 0 && d <= kOrder * L; }
 
-// The two or three launches of a batch of filters (weight re-split, hidden layers, projection + decay), the table coming
-// either by value or from device memory.  `w3split` / `taps` null: the projection is left to the caller (the fused
-// projection + spectrum kernel of short sequences).  Kernels that keep a projection's weights in registers split them themselves.
+// The launches of a batch of filters (weight re-split and hidden layers with projection + decay, or hidden layers and projection), the table
+// coming either by value or from device memory.  `taps` null: the projection is left to the caller (the fused
+// projection + spectrum kernel of short sequences).  Only the first form reads split copies (`wsplit`, `w3split`, `w3scale`); other kernels split
+// the weights they keep in registers themselves.
 template <class TAB>
 static int filter_launches(TAB tab, int nfilters, int L, int d, int emb_dim, float w_mod, float shift, uint16_t* h_hi,
                            uint16_t* h_lo, uint16_t* wsplit, uint16_t* w3split, float* w3scale, float* taps, hipStream_t s) {
@@ -591,7 +592,7 @@ static int filter_launches(TAB tab, int nfilters, int L, int d, int emb_dim, flo
                        h_hi, h_lo, d, shift, w3split, w3scale, taps);
     return check_launch("hyena hidden + project kernel");
   }
-  hipLaunchKernelGGL((hidden_kernel<1, TAB, false>), dim3(L / 32, 2 * nfilters), dim3(256), 0, s, tab, L, emb_dim, w_mod, wsplit,
+  hipLaunchKernelGGL((hidden_kernel<1, TAB, false>), dim3(L / 32, 2 * nfilters), dim3(256), 0, s, tab, L, emb_dim, w_mod, nullptr,
                      h_hi, h_lo, 0, 0.f, nullptr, nullptr, nullptr);
   const int rc = check_launch("hyena hidden_kernel");
   if (rc || !taps) return rc;
@@ -698,8 +699,9 @@ extern "C" int m2_hyena_filter_fwd_static(const m2_hyena_filter_params* params, 
   void* ptr = nullptr;
   int rc = static_scratch_for_current_device(&ptr);
   if (rc) return rc;
-  // split_weights_kernel and hidden_kernel write every element the later kernels of the same call read, so nothing
-  // left by an earlier (possibly longer) call is ever read and nothing needs clearing
+  // every element that a kernel reads was written by an earlier kernel of the same call (h3 by hidden_kernel, or the split weights by
+  // split_weights_kernel where h3 does not leave the chip), so nothing left by an earlier (possibly longer) call is ever read and nothing
+  // needs clearing
   return hyena_filter_launch("m2_hyena_filter_fwd_static", params, nfilters, L, d, order, emb_dim, w_mod, shift, ptr,
                              taps, stream);
 }
@@ -719,7 +721,8 @@ BatchLayout batch_layout(int nmixers, int fpm, int L, int d) {
   b.fused = project_spectrum_supported(L);
   b.h_lo = up(2 * nf * L * kOrder * sizeof(uint16_t));
   b.wsplit = b.h_lo + up(2 * nf * L * kOrder * sizeof(uint16_t));
-  b.w3split = b.wsplit + up(2 * nf * 2 * (size_t)kSplitPerLayer * sizeof(uint16_t));
+  // (fused: hidden_kernel and project_spectrum_kernel split their weights themselves)
+  b.w3split = b.wsplit + (b.fused ? 0 : up(2 * nf * 2 * (size_t)kSplitPerLayer * sizeof(uint16_t)));
   b.w3scale = b.w3split + (b.fused ? 0 : up(2 * nf * 2 * (size_t)d * kOrder * sizeof(uint16_t)));
   b.taps = b.w3scale + (b.fused ? 0 : up(2 * nf * (size_t)d * sizeof(float)));
   b.total = b.taps + (b.fused ? 0 : up(nf * (size_t)d * 2 * L * sizeof(float)));
@@ -757,7 +760,7 @@ extern "C" int m2_mixer_filters_fwd(const m2_hyena_filter_params* params_dev, co
   unsigned char* ws = reinterpret_cast<unsigned char*>(workspace);
   uint16_t* h_hi = reinterpret_cast<uint16_t*>(ws);
   uint16_t* h_lo = reinterpret_cast<uint16_t*>(ws + lay.h_lo);
-  uint16_t* wsplit = reinterpret_cast<uint16_t*>(ws + lay.wsplit);
+  uint16_t* wsplit = lay.fused ? nullptr : reinterpret_cast<uint16_t*>(ws + lay.wsplit);
   uint16_t* w3split = lay.fused ? nullptr : reinterpret_cast<uint16_t*>(ws + lay.w3split);
   float* w3scale = lay.fused ? nullptr : reinterpret_cast<float*>(ws + lay.w3scale);
   float* taps = lay.fused ? nullptr : reinterpret_cast<float*>(ws + lay.taps);
