@@ -15,6 +15,9 @@
 // B = 3 19.0, 32.3, 56.5, 136.9, 288.6 against 25.5, 46.2, 79.7, 173.7, 421.1.  So: one row to a channel, and two where whole forwards
 // gain by it too: 12 x 768, B = 2, L = 1024 1090 / 1102, 2048 1531 / 1550, 4096 2295 / 2264, 8192 4837 / 4704.  Whole forwards of 12 x 768, B = 1:
 // L = 1024 1011 / 971, 2048 1230 / 1208, 4096 1793 / 1723, 8192 2814 / 2680, 16384 6030 / 5720; 24 x 1536, 2048 4786 / 4541.
+// The width changes little, as both routes grow with it.  Six layers, spectra / taps: B = 1, L = 1024, 4096, 16384 960 553 / 500, 1111 / 1048,
+// 3685 / 3499, 1536 804 / 770, 1834 / 1716, 6626 / 6168, 1792 918 / 878, 2230 / 2099, 8084 / 7548; B = 2, L = 4096, 8192 768 1091 / 1079, 2053 / 2011,
+// 960 1629 / 1610, 3000 / 2956, 1536 2773 / 2726, 5588 / 5490, 1792 3512 / 3457, 6869 / 6786.
 // fp32 rows, whose inputs take twice the registers, spill beside a spectrum (52 bytes a lane and more) and read spectra; at L = 32768 a
 // half transform's inputs would have to be formed twice from all the taps.
 #include "mixer_long.h"
