@@ -2,7 +2,9 @@
 // W (d, d) (bert/src/bert_layers.py:816-859).
 //
 // A few rows of a 768 x 768 product: what it takes is a launch and one trip to memory, which the library's product and the tanh behind it made
-// twice (9.4 and 4.9 us in a trace).  us per forward, L = 128, B = 1, before / now: 12 x 768 501 / 492, 24 x 1536 1724 / 1709.  A wave has two columns and up to eight rows, its lanes share K, and the sums meet in the lanes.
+// twice (9.4 and 4.9 us in a trace).  us per forward, L = 128, B = 1, before / now: 12 x 768 501 / 492, 24 x 1536 1724 / 1709.  A wave has two columns
+// and up to eight rows, its lanes share K, and the sums meet in the lanes.  Every eight rows read the whole weight again: d = 768 B = 8 7.7 us,
+// 64 10.8, 256 22, where the library's product with its tanh stays at 7.0, 7.2, 9.3; encoder.py sends it eight sequences at most.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 

@@ -115,6 +115,10 @@ def test_hidden_states_in_any_layout(gpu, counted):
             del calls[:]
             got, ref = model._pool(x, None), model.pooler(x)
             assert len(calls) == own and got.shape == (n, 768) and (got - ref).abs().max() < 2e-6
+        many = _hidden(gpu, 9)                                    # beyond what one pass over the weights serves
+        del calls[:]
+        assert torch.equal(model._pool(many, None), model.pooler(many)) and not calls
+        assert model._pool(many[:8], None).shape == (8, 768) and len(calls) == 1
         assert model._pool(h[:0], None).shape == (0, 768) and (model._pool(h, None) - want).abs().max() < 2e-6
         with pytest.raises(IndexError):                           # no first token
             model._pool(h[:, :0], None)
